@@ -274,9 +274,8 @@ enum {
      * shared sequence of wavefronts; without the flag every job shares one sequence. tr_autotune
      * tries both */
     TR_RENDER_PER_JOB = 128u,
-    /* closest-hit launches run node steps and triangle steps in separate wavefront-wide phases: a
-     * node's entered leaves wait until many lanes hold some (keyed 16-bit stack; BVHs of at most
-     * 65,536 nodes, otherwise ignored). Launch tuning; results do not change. */
+    /* accepted, and the same as STACK_KEYED: closest-hit launches always let a lane test its leaves
+     * while others visit nodes. Launch tuning; results do not change. */
     TR_RENDER_POSTPONE_LEAVES = 512u,
     /* camera rays (the first bounce of a single-job render) traced one query per lane like the
      * later bounces, instead of as packets of one pixel's 64 samples per wavefront. Launch tuning
@@ -341,7 +340,7 @@ int tr_batch_render(tr_batch batch, const tr_launch_desc* launch, tr_render_stat
  * Trials render every job with sqrt_spp capped at the smallest value for which the capped batch
  * holds min(all paths, 2^25) paths (about one largest-candidate wavefront), best of two runs each:
  * stage 1 wavefront sizes 2^18..2^25 with and without graph replay, stage 2 traversal / shading
- * blocks per CU, stage 4 the traversal formats (32-bit stack, keyed stack, postponed leaves).
+ * blocks per CU, stage 4 the traversal formats (32-bit stack, keyed stack).
  * Stage 3 renders the FULL jobs once in each batch mode (shared wavefronts; TR_RENDER_PER_JOB), so
  * the call costs at least two complete batch renders plus the trials. A candidate replaces the
  * incumbent only when more than 2 % faster. Every film is cleared afterwards. */

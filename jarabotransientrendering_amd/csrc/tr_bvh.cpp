@@ -569,3 +569,53 @@ float qbvh_plane_bound(const std::vector<Bvh4QNodeHost>& q4)
     }
     return std::nextafter(float(c * (1.0 + 1e-6)), std::numeric_limits<float>::infinity());
 }
+
+Bvh4Device device_bvh4(const std::vector<Bvh4QNodeHost>& q4, size_t n_tris)
+{
+    Bvh4Device d;
+    d.nodes.resize(q4.size());
+    d.tri_order.reserve(n_tris);
+    d.tri_slot.assign(n_tris, 0u);
+    struct Todo {
+        uint32_t from, to;
+    };
+    std::vector<Todo> todo{{0u, 0u}};
+    uint32_t used = 1;
+    while (!todo.empty()) {
+        const Todo t = todo.back();
+        todo.pop_back();
+        const Bvh4QNodeHost& s = q4[t.from];
+        Bvh4DevNode& n = d.nodes[t.to];
+        std::memset(&n, 0, sizeof n);
+        std::memcpy(n.origin, s.origin, sizeof n.origin);
+        const float step[3] = {s.step_x, s.step_y, s.step_z};
+        for (int a = 0; a < 3; ++a) {
+            n.step24[a] = std::ldexp(step[a], 24);
+            if (!(n.step24[a] * 1e21f < std::numeric_limits<float>::infinity())) d.scaled = false;
+        }
+        int order[4], m = 0;
+        for (int pass = 0; pass < 3; ++pass)
+            for (int k = 0; k < 4; ++k) {
+                const uint32_t c = s.ref[k] >> 29;
+                if (pass == (c == 0 ? 0 : c == kQEmpty ? 2 : 1)) order[m++] = k;
+            }
+        n.tri0 = uint32_t(d.tri_order.size());
+        for (int i = 0; i < 4; ++i) {
+            const int k = order[i];
+            for (int w = 0; w < 6; ++w) n.q[4 * w + i] = s.q[4 * w + k];
+            const uint32_t c = s.ref[k] >> 29, index = s.ref[k] & 0x1FFFFFFFu;
+            if (c == 0) ++n.n_inner;
+            if (c == 0 || c == kQEmpty) continue;
+            for (uint32_t j = 0; j < c; ++j) {
+                const uint32_t slot = uint32_t(d.tri_order.size());
+                n.tri_masks |= (1u << (slot - n.tri0)) << (8 * i);
+                d.tri_slot[index + j] = slot;
+                d.tri_order.push_back(index + j);
+            }
+        }
+        n.child0 = used;
+        used += n.n_inner;
+        for (uint32_t i = n.n_inner; i-- > 0;) todo.push_back({s.ref[order[i]] & 0x1FFFFFFFu, n.child0 + i});
+    }
+    return d;
+}

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 #include <cstdint>
+#include <type_traits>
 
 #include "tr_internal.h"
 
@@ -149,11 +150,11 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v)
 
 // ---- ray/box and watertight ray/triangle -----------------------------------------------------
 struct RayPre {
-    f3 o, d, inv;
-    f3 c;       // -(o * inv): slab offset of the quantized 4-wide BVH's node test
-    float k;    // slab margin of that test per unit |inv|
-    f3 o_rot;   // origin components in (kx, ky, kz) order
-    int rot;   // = kx: offset of the (kx, ky, kz) run in a rotated triangle vertex (TriRot)
+    f3 o, inv;
+    f3 c0, c1;            // -(o * inv) -+ k |inv|: slab offsets of entry and exit planes (4-wide BVH)
+    uint32_t sx, sy, sz;  // byte selectors of the entry planes of children 0 and 1, per axis (kPermUp)
+    f3 o_rot;             // origin components in (kx, ky, kz) order
+    uint32_t rot4;        // 4 * kx: byte offset of the (kx, ky, kz) run in a rotated triangle vertex (TriRot)
     float Sx, Sy, Sz;
 };
 
@@ -164,59 +165,79 @@ __device__ __forceinline__ float safe_rcp(float d)
     return 1.0f / (fabsf(d) < 1e-20f ? copysignf(1e-20f, d) : d);
 }
 
+// Entry planes of an axis for a ray going up (down) it: the lower (upper) ones. v_perm_b32 picks
+// them from the (upper, lower) plane words and spreads two of them to 16-bit halves (0x0c is a zero
+// byte); with the words swapped the same selector picks the exit planes. Children 2 and 3 are two
+// bytes further on.
+constexpr uint32_t kPermUp = 0x0c010c00u, kPermDown = 0x0c050c04u, kPermNext = 0x00020002u;
+
 // Offset and margin of the quantized node test. A plane at P = origin + q * step (one rounding
-// on the host) is entered at (P - o) * inv; the node test evaluates it as fma(q, step * inv, b)
-// with b = fma(origin, inv, c), c = -(o * inv), widened to b -+ k |inv| (one fused multiply-add
-// each; entry planes down, exit planes up), so a plane costs one operation and an axis three more
-// per node. The roundings, each at most u = 2^-24 of its result, are: the host plane
-// u (|origin| + 255 step) |inv|, o * inv u |o| |inv| (the negation is exact), b u |b| with
-// |b| <= (|origin| + |o|) |inv| (1 + u), b -+ m u (|b| + m) and the plane distance
-// u (|b| + 255 step |inv| + m), m = k |inv|. With C >= |origin| + 255 step for every node
-// (plane_bound) they sum to at most u |inv| (4 C + 4 |o|) + 2 u m, which m exceeds for
-// k = 6e-7 (C + max |o|) (about 10 u (C + |o|)): the entry plane is never late and the exit plane
-// never early.
+// on the host) is entered at (P - o) * inv; the node test evaluates it as fma(q, step * inv, b) with
+// b = fma(origin, inv, c) and c = -(o * inv) -+ k |inv| (entry planes down, exit planes up), so a plane
+// costs one operation and an axis three more per node. The roundings, each at most u = 2^-24 of
+// its result, are: the host plane u (|origin| + 255 step) |inv|, o * inv and c together
+// u (2 |o| |inv| + m) with m = k |inv|, b u (|origin| |inv| + |o| |inv| + m) and the plane distance
+// u (|b| + 255 step |inv|). With C >= |origin| + 255 step for every node (plane_bound) they sum to at
+// most u |inv| (4 C + 5 |o|) + 3 u m. Exit planes also make up for the 3 ulp by which box_far moves
+// a hit's distance out: 6 u (C + |o|) |inv| more. k = 1e-6 (C + max |o|) (over 16 u (C + |o|))
+// exceeds the sum: the entry plane is never late and the exit plane never early.
 __device__ __forceinline__ RayPre ray_pre(f3 o, f3 d, float plane_bound)
 {
     RayPre r;
     r.o = o;
-    r.d = d;
     r.inv = mk(safe_rcp(d.x), safe_rcp(d.y), safe_rcp(d.z));
-    r.c = mk(-(o.x * r.inv.x), -(o.y * r.inv.y), -(o.z * r.inv.z));
-    r.k = 6e-7f * (plane_bound + fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)));
+    const float k = 1e-6f * (plane_bound + fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)));
+    const f3 c = mk(-(o.x * r.inv.x), -(o.y * r.inv.y), -(o.z * r.inv.z));
+    r.c0 = mk(fmaf(-k, fabsf(r.inv.x), c.x), fmaf(-k, fabsf(r.inv.y), c.y), fmaf(-k, fabsf(r.inv.z), c.z));
+    r.c1 = mk(fmaf(k, fabsf(r.inv.x), c.x), fmaf(k, fabsf(r.inv.y), c.y), fmaf(k, fabsf(r.inv.z), c.z));
+    r.sx = r.inv.x >= 0.0f ? kPermUp : kPermDown;
+    r.sy = r.inv.y >= 0.0f ? kPermUp : kPermDown;
+    r.sz = r.inv.z >= 0.0f ? kPermUp : kPermDown;
     float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
     int kz = (ax > ay) ? (ax > az ? 0 : 2) : (ay > az ? 1 : 2);
     int kx = kz + 1 == 3 ? 0 : kz + 1;
     int ky = kx + 1 == 3 ? 0 : kx + 1;
     // The paper swaps kx and ky when d[kz] < 0 to keep the winding; that only negates U, V, W, det
     // and T (each exactly), so the hit test and T / det are the same without it.
-    r.rot = kx;
+    r.rot4 = 4u * uint32_t(kx);
     r.o_rot = mk(comp(o, kx), comp(o, ky), comp(o, kz));
-    r.Sz = 1.0f / comp(d, kz);
+    // 1 / d[kz]: the slab reciprocal unless that was clamped
+    const float dz = comp(d, kz);
+    r.Sz = comp(r.inv, kz);
+    if (fabsf(dz) < 1e-20f) r.Sz = 1.0f / dz;
     r.Sx = comp(d, kx) * r.Sz;
     r.Sy = comp(d, ky) * r.Sz;
     return r;
 }
 
-// Rotated triangle record (TriRot, 16 floats = 64 bytes, leaf order): vertex v at floats
+// Rotated triangle record (TriRot, 16 floats = 64 bytes, slot order): vertex v at floats
 // [5v, 5v + 5) as (x, y, z, x, y), so that the components (kx, ky, kz) = (kz+1, kz+2, kz) mod 3
 // of any ray are three consecutive floats starting at kx; float 15 = scene triangle index bits.
 struct __attribute__((packed, aligned(4))) Packed3 {
     float x, y, z;
 };
 
+// The far bound of box tests for a hit at distance t: three ulp further, so that a box whose
+// triangle lies at exactly t is still entered.
+__device__ __forceinline__ float box_far(float t) { return t * 1.00000036f; }
+
+// Tests the triangle record at byte offset `off` of `tris` (its slot is `slot`) against the current
+// hit: updates hit (a slot) and tfar; equal-distance ties go to the lower scene triangle index, which
+// is read only for a tie.
+//
 // Woop, Benthin, Wald, "Watertight Ray/Triangle Intersection", JCGT 2(1) 2013, Sec. 4 (no
-// backface culling; double-precision re-evaluation when an edge function is exactly zero), on a
-// rotated triangle record `t`. Returns false when the ray misses the triangle's interior and
-// edges; otherwise the hit distance is T / det (callers divide only for candidate hits).
-__device__ __forceinline__ bool tri_watertight_td(const RayPre& r, const float* __restrict__ t, float* T_out,
-                                                  float* det_out)
+// backface culling; double-precision re-evaluation when an edge function is exactly zero).
+template <class Off>
+__device__ __forceinline__ void tri_hit(const RayPre& r, const char* __restrict__ tris, Off off, int32_t slot,
+                                        float tnear, float& tfar, int32_t& hit)
 {
     // No fused multiply-adds here: an edge shared by two triangles must evaluate to exactly
     // opposite values in both, which fma(Cx, By, -Cy*Bx) vs fma(Bx, Cy, -By*Cx) does not give.
 #pragma clang fp contract(off)
-    const Packed3 a = *reinterpret_cast<const Packed3*>(t + r.rot);
-    const Packed3 b = *reinterpret_cast<const Packed3*>(t + 5 + r.rot);
-    const Packed3 c = *reinterpret_cast<const Packed3*>(t + 10 + r.rot);
+    const char* t = tris + (off + Off(r.rot4));
+    const Packed3 a = *reinterpret_cast<const Packed3*>(t);
+    const Packed3 b = *reinterpret_cast<const Packed3*>(t + 20);
+    const Packed3 c = *reinterpret_cast<const Packed3*>(t + 40);
     float Akx = a.x - r.o_rot.x, Aky = a.y - r.o_rot.y, Akz = a.z - r.o_rot.z;
     float Bkx = b.x - r.o_rot.x, Bky = b.y - r.o_rot.y, Bkz = b.z - r.o_rot.z;
     float Ckx = c.x - r.o_rot.x, Cky = c.y - r.o_rot.y, Ckz = c.z - r.o_rot.z;
@@ -226,46 +247,34 @@ __device__ __forceinline__ bool tri_watertight_td(const RayPre& r, const float* 
     float U = Cx * By - Cy * Bx;
     float V = Ax * Cy - Ay * Cx;
     float W = Bx * Ay - By * Ax;
-    if (U == 0.0f || V == 0.0f || W == 0.0f) {
+    if (fminf(fminf(fabsf(U), fabsf(V)), fabsf(W)) == 0.0f) {
         U = float(double(Cx) * double(By) - double(Cy) * double(Bx));
         V = float(double(Ax) * double(Cy) - double(Ay) * double(Cx));
         W = float(double(Bx) * double(Ay) - double(By) * double(Ax));
     }
-    if ((U < 0.0f || V < 0.0f || W < 0.0f) && (U > 0.0f || V > 0.0f || W > 0.0f)) return false;
-    float det = U + V + W;
-    if (det == 0.0f) return false;
-    *T_out = U * (r.Sz * Akz) + V * (r.Sz * Bkz) + W * (r.Sz * Ckz);
-    *det_out = det;
-    return true;
-}
-
-// Tests triangle record `t` (scene triangle `id`) against the current closest hit: updates hit and
-// tfar; equal-distance ties go to the lower scene triangle index.
-__device__ __forceinline__ void tri_hit(const RayPre& r, const float* __restrict__ t, float tnear, float& tfar,
-                                        int32_t& hit)
-{
-    float T, det;
-    if (!tri_watertight_td(r, t, &T, &det)) return;
+    const bool neg = fminf(fminf(U, V), W) < 0.0f, pos = fmaxf(fmaxf(U, V), W) > 0.0f;
+    const float det = U + V + W;
+    // outside the triangle's interior and edges, or degenerate
+    if ((neg & pos) | (det == 0.0f)) return;
+    const float T = U * (r.Sz * Akz) + V * (r.Sz * Bkz) + W * (r.Sz * Ckz);
     // divide only when an estimate of the distance is near (tnear, tfar]
     const float te = T * __builtin_amdgcn_rcpf(det);
-    if (!(te >= tnear * 0.99999f && te <= tfar * 1.00001f)) return;
+    if (!((te >= tnear * 0.99999f) & (te <= tfar * 1.00001f))) return;
     const float th = T / det;
-    const int32_t id = __float_as_int(t[15]);
-    if (th > tnear && th <= tfar && (th < tfar || hit < 0 || id < hit)) {
-        hit = id;
-        tfar = th;
+    if (!((th > tnear) & (th <= tfar))) return;
+    if (th == tfar && hit >= 0) {
+        const int32_t id = *reinterpret_cast<const int32_t*>(tris + (off + Off(60)));
+        const int32_t id_hit = *reinterpret_cast<const int32_t*>(tris + (Off(uint32_t(hit)) * 64 + 60));
+        if (id >= id_hit) return;
     }
-}
-
-__device__ __forceinline__ int32_t sel4(int32_t a0, int32_t a1, int32_t a2, int32_t a3, int k)
-{
-    return k == 0 ? a0 : (k == 1 ? a1 : (k == 2 ? a2 : a3));
+    hit = slot;
+    tfar = th;
 }
 
 // Closest (ANY = false) or any (ANY = true) hit in (tnear, tfar]. On a closest hit `tfar` is
 // updated. Equal-distance ties resolve to the lower scene triangle index. `stack` points at this
 // thread's first LDS stack slot; consecutive slots are `stride` ints apart.
-// Returns the scene triangle index or -1.
+// Returns the triangle's slot or -1.
 template <bool ANY>
 __device__ __forceinline__ int32_t trace(const float4* __restrict__ nodes, const float4* __restrict__ tris,
                                          const RayPre& r, float tnear, float& tfar, int32_t* stack,
@@ -300,7 +309,7 @@ __device__ __forceinline__ int32_t trace(const float4* __restrict__ nodes, const
             if (h && cnt > 0) {
                 int first = side == 0 ? dd.x : dd.y;
                 for (int i = first; i < first + cnt; ++i) {
-                    tri_hit(r, reinterpret_cast<const float*>(tris + 4 * size_t(i)), tnear, tfar, hit);
+                    tri_hit<size_t>(r, reinterpret_cast<const char*>(tris), size_t(i) * 64, i, tnear, tfar, hit);
                     if (ANY && hit >= 0) return hit;
                 }
                 if (side == 0) hl = false;
@@ -325,7 +334,8 @@ __device__ __forceinline__ int32_t trace(const float4* __restrict__ nodes, const
     return hit;
 }
 
-// Traversal stack entry formats of the 4-wide BVH, kept in LDS, one column per thread:
+// Traversal stack entry formats of the 4-wide BVH, kept in LDS, one column per thread (entry e of
+// thread `tid` is element e * stride + tid):
 //   kStack32   : 32-bit node index;
 //   kStack16   : 16-bit node index (BVHs of at most 65,536 nodes): half the LDS, so more
 //                wavefronts fit on a compute unit;
@@ -334,220 +344,217 @@ __device__ __forceinline__ int32_t trace(const float4* __restrict__ nodes, const
 //                child that starts beyond the current hit without fetching the node.
 enum { kStack32 = 0, kStack16 = 1, kStackKeyed = 2 };
 
-// Same query over the 4-wide BVH (Bvh4NodeHost: 8 float4 per node). Children that the ray enters
-// are visited nearest first; the others are pushed far-to-near. Leaves are tested on the spot.
-// `stack` is the block's LDS stack, `tid` this thread's column and `stride` the block size.
-constexpr uint32_t kQEmptyDev = 7u;  // child reference count of an empty slot (Bvh4QNodeHost)
-
 // Per-lane state of a 4-wide BVH query between node steps.
 struct Trav4 {
-    int32_t node;      // node to visit next (-1: none); while leaves are tested, the node they belong to
-    int32_t sp;        // stack entries
-    int32_t hit;       // closest (or any) hit so far, -1 if none
-    float tfar;        // current far bound (the hit distance once there is a hit)
-    uint32_t tri;      // leaf mode (tri < tri_end): next triangle of the current leaf
-    uint32_t tri_end;  // end of the current leaf's triangles
-    uint32_t leaves;   // leaf mode: entered leaf children of `node` not finished (the lowest bit is current)
-    int32_t pnode;     // postponed leaves (closest hit): the node whose leaves `leaves` are
+    uint32_t node;    // node to visit next
+    uint32_t sp;      // element index of the next free stack entry
+    int32_t hit;      // slot of the closest (or any) hit so far, -1 if none
+    float tfar;       // current far bound (the hit distance once there is a hit)
+    uint32_t leaves;  // leaf mode: triangles of the last node still to test (bit 8 k + j: slot tri0 + j)
+    uint32_t tri0;    // ... and that node's first triangle slot
+    uint32_t p[4];    // closest hit: the node's entered inner children, nearest first, held back in leaf mode
 };
 
-__device__ __forceinline__ void trav4_begin(Trav4& st, float tfar)
+__device__ __forceinline__ void trav4_begin(Trav4& st, float tfar, uint32_t tid)
 {
     st.node = 0;
-    st.sp = 0;
+    st.sp = tid;
     st.hit = -1;
     st.tfar = tfar;
-    st.tri = 0;
-    st.tri_end = 0;
     st.leaves = 0;
-    st.pnode = -1;
+    st.tri0 = 0;
+}
+
+// q * a + b for the 8-bit planes q held in the halves of `p`. A byte in a 16-bit half is the
+// half-precision subnormal q * 2^-24, which v_fma_mix_f32 takes as it is (exactly; a is held scaled
+// by 2^24): no conversion instruction per plane.
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float plane_lo(uint32_t p, float a, float b)
+{
+    return fmaf(float(__builtin_bit_cast(half2v, p).x), a, b);
+}
+__device__ __forceinline__ float plane_hi(uint32_t p, float a, float b)
+{
+    return fmaf(float(__builtin_bit_cast(half2v, p).y), a, b);
+}
+
+// Entry distances t0[k] (at least tnear) of the four child boxes of a node (Bvh4DevNode) and whether
+// the ray meets them in [tnear, tfar_box]. n / f: entry / exit plane pairs per axis, [2 axis] of
+// children 0 and 1, [2 axis + 1] of children 2 and 3.
+__device__ __forceinline__ void slabs4(const RayPre& r, const uint4& w0, const uint4& w3, const uint32_t (&n)[6],
+                                       const uint32_t (&f)[6], float tnear, float tfar_box, float (&t0)[4], bool (&ent)[4])
+{
+    const float ox = __uint_as_float(w0.x), oy = __uint_as_float(w0.y), oz = __uint_as_float(w0.z);
+    const float ax = __uint_as_float(w3.x) * r.inv.x, ay = __uint_as_float(w3.y) * r.inv.y,
+                az = __uint_as_float(w3.z) * r.inv.z;
+    const float bx0 = fmaf(ox, r.inv.x, r.c0.x), by0 = fmaf(oy, r.inv.y, r.c0.y), bz0 = fmaf(oz, r.inv.z, r.c0.z);
+    const float bx1 = fmaf(ox, r.inv.x, r.c1.x), by1 = fmaf(oy, r.inv.y, r.c1.y), bz1 = fmaf(oz, r.inv.z, r.c1.z);
+#define TR_CHILD(k, P, h)                                                                                        \
+    t0[k] = fmaxf(fmaxf(P(n[h], ax, bx0), P(n[2 + h], ay, by0)), fmaxf(P(n[4 + h], az, bz0), tnear));            \
+    ent[k] = t0[k] <= fminf(fminf(P(f[h], ax, bx1), P(f[2 + h], ay, by1)), fminf(P(f[4 + h], az, bz1), tfar_box));
+    TR_CHILD(0, plane_lo, 0)
+    TR_CHILD(1, plane_hi, 0)
+    TR_CHILD(2, plane_lo, 1)
+    TR_CHILD(3, plane_hi, 1)
+#undef TR_CHILD
+}
+
+// the same with each lane's own entry / exit selection
+__device__ __forceinline__ void node_slabs(const RayPre& r, const uint4& w0, const uint4& w1, const uint4& w2,
+                                           const uint4& w3, float tnear, float tfar_box, float (&t0)[4], bool (&ent)[4])
+{
+    const uint32_t sx2 = r.sx + kPermNext, sy2 = r.sy + kPermNext, sz2 = r.sz + kPermNext;
+    const uint32_t n[6] = {__builtin_amdgcn_perm(w1.y, w1.x, r.sx), __builtin_amdgcn_perm(w1.y, w1.x, sx2),
+                           __builtin_amdgcn_perm(w1.w, w1.z, r.sy), __builtin_amdgcn_perm(w1.w, w1.z, sy2),
+                           __builtin_amdgcn_perm(w2.y, w2.x, r.sz), __builtin_amdgcn_perm(w2.y, w2.x, sz2)};
+    const uint32_t f[6] = {__builtin_amdgcn_perm(w1.x, w1.y, r.sx), __builtin_amdgcn_perm(w1.x, w1.y, sx2),
+                           __builtin_amdgcn_perm(w1.z, w1.w, r.sy), __builtin_amdgcn_perm(w1.z, w1.w, sy2),
+                           __builtin_amdgcn_perm(w2.x, w2.y, r.sz), __builtin_amdgcn_perm(w2.x, w2.y, sz2)};
+    slabs4(r, w0, w3, n, f, tnear, tfar_box, t0, ent);
 }
 
 // One step of a closest (ANY = false) or any (ANY = true) hit query over the quantized 4-wide BVH
-// (Bvh4QNodeHost: 4 x 16 bytes per node). A step visits one node: the inner children the ray
-// enters are pushed far-to-near (any hit: in slot order) and the nearest is visited next. A
-// closest-hit query tests the node's entered leaves in the same step and then drops the inner
-// children behind the hit. An any-hit query instead pushes every entered inner child and tests
-// its leaves one triangle per step (leaf mode), popping the next node when they are done: lanes in
-// leaf mode and lanes visiting nodes share each step, so a wavefront does not wait on a few lanes
-// looping over their leaves (7 % faster shadow rays; for closest hits the lost culling costs
-// more). Returns true when the query is complete (st.hit, st.tfar hold the answer). `stack` is the
-// block's LDS stack, `tid` this thread's column and `stride` the block size.
-template <bool ANY, int SK>
+// (Bvh4DevNode: 4 x 16 bytes per node). A lane either visits a node or, while triangles of its last
+// node's entered leaves are left to test, tests one of them (leaf mode), so a wavefront does not wait
+// on the few lanes that loop over their leaves. The inner children the ray enters are pushed
+// far-to-near and the nearest is visited next; a closest-hit query holds them back (st.p) until its
+// triangles are tested and drops those behind the hit, an any-hit query pushes all of them at once,
+// in slot order. Queries that take no leaf mode (32-bit stack entries, or !POS) loop over the node's
+// triangles in the step. Returns true when the query is complete (st.hit, st.tfar hold the
+// answer). `stack` is the block's LDS stack, `tid` this thread's column and `stride` the block size.
+// POS: every tnear of the launch is positive, so that entry distances order like their bits (renders;
+// not the public queries).
+//
+// The step is bound by VALU issue (a wavefront issues an instruction on nearly every cycle of its
+// SIMD, with about half its lanes active), so what counts is instructions per step: planes taken as
+// half-precision subnormals (no conversions), children as (distance, index) words sorted by integer
+// min / max, triangles as one bit mask over consecutive slots, hits kept as slots (no index loads) and
+// addresses in 32 bits took a node visit of a closest-hit query from about 190 to 115 VALU
+// instructions and a triangle test from 90 to 70; leaf mode for closest hits saved a further tenth
+// (holding the children back keeps the culling that pushing them at once loses). On the
+// 81,930-triangle frame of 67 M paths: closest hits 11.8 -> 9.8 ms, any hits 9.9 -> 7.1 ms, frame
+// 31.1 -> 25.5 ms. Lost: any-hit queries that loop over their triangles in the step (7.1 -> 8.7 ms),
+// triangle tests only once 6 to 20 lanes wait for one (extend 9.8 -> 10.5-10.9 ms), keyed entries by
+// default (12.0 ms: twice the LDS), one triangle per leaf (10.0 ms).
+template <bool ANY, int SK, bool POS>
 __device__ __forceinline__ bool trace4_step(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                            const RayPre& r, float tnear, Trav4& st, uint32_t* stack, int tid,
-                                            int stride)
+                                            const RayPre& r, float tnear, Trav4& st, uint32_t* stack, uint32_t tid,
+                                            uint32_t stride)
 {
     static_assert(!(ANY && SK == kStackKeyed), "any-hit queries keep no entry distances");
-    int32_t hit = st.hit;
-    float tfar = st.tfar;
-    int sp = st.sp;
-    auto push = [&](int32_t child, float key) {
-        if constexpr (SK == kStack32) {
-            stack[sp * stride + tid] = uint32_t(child);
-        } else if constexpr (SK == kStack16) {
-            // entries 2k and 2k+1 of a thread share one 32-bit word: no two lanes write one word
-            reinterpret_cast<uint16_t*>(stack)[((sp >> 1) * stride + tid) * 2 + (sp & 1)] = uint16_t(child);
+    static_assert(!(SK == kStackKeyed && !POS), "keyed entries need positive distances");
+    constexpr bool PACKED = !ANY && SK != kStack32 && POS;  // (distance, child) words of 32 bits
+    // 16-bit node indices: at most 65,536 nodes with eight triangles each, so byte offsets fit 32 bits
+    typedef typename std::conditional<SK == kStack32, size_t, uint32_t>::type Off;
+    const char* tri_base = reinterpret_cast<const char*>(tris);
+    auto push = [&](uint32_t e) {
+        if constexpr (SK == kStack16) reinterpret_cast<uint16_t*>(stack)[st.sp] = uint16_t(e);
+        else stack[st.sp] = e;
+        st.sp += stride;
+    };
+    auto top = [&]() -> uint32_t {
+        if constexpr (SK == kStack16) return reinterpret_cast<const uint16_t*>(stack)[st.sp];
+        else return stack[st.sp];
+    };
+    auto test = [&](uint32_t tri0, uint32_t leaves) {
+        const uint32_t slot = tri0 + (uint32_t(__builtin_ctz(leaves)) & 7u);
+        tri_hit<Off>(r, tri_base, Off(slot) * 64, int32_t(slot), tnear, st.tfar, st.hit);
+    };
+    if ((ANY || PACKED) && st.leaves) {
+        test(st.tri0, st.leaves);
+        if (ANY && st.hit >= 0) return true;
+        st.leaves &= st.leaves - 1u;
+    } else {
+        const uint4* nd = reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(nodes) + Off(st.node) * 64);
+        const uint4 w0 = nd[0], w1 = nd[1], w2 = nd[2], w3 = nd[3];
+        const uint32_t child0 = w0.w, meta = w2.z, tri0 = w2.w, n_inner = w3.w;
+        float t0[4];
+        bool ent[4];
+        node_slabs(r, w0, w1, w2, w3, tnear, box_far(st.tfar), t0, ent);
+        // triangles of the entered leaf children: byte k of `meta` marks those of child k
+        uint32_t leaves = ((ent[0] ? 0x000000FFu : 0u) | (ent[1] ? 0x0000FF00u : 0u) | (ent[2] ? 0x00FF0000u : 0u) |
+                           (ent[3] ? 0xFF000000u : 0u)) & meta;
+        if constexpr (ANY) {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k)
+                if (ent[k] & (k < n_inner)) push(child0 + k);
+            st.leaves = leaves;
+            st.tri0 = tri0;
+        } else if constexpr (PACKED) {
+            // (entry distance, child) in one word, the distance truncated to its upper 16 bits: sorted
+            // with integer min / max; ~0: not entered
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                const uint32_t e = (__float_as_uint(t0[k]) & 0xFFFF0000u) | (child0 + k);
+                st.p[k] = (ent[k] & (k < n_inner)) ? e : 0xFFFFFFFFu;
+            }
+#define TR_CSWAP(a, b)                                                                \
+    {                                                                                 \
+        const uint32_t lo = min(st.p[a], st.p[b]), hi = max(st.p[a], st.p[b]);        \
+        st.p[a] = lo;                                                                 \
+        st.p[b] = hi;                                                                 \
+    }
+            TR_CSWAP(0, 1) TR_CSWAP(2, 3) TR_CSWAP(0, 2) TR_CSWAP(1, 3) TR_CSWAP(1, 2)
+#undef TR_CSWAP
+            st.leaves = leaves;
+            st.tri0 = tri0;
         } else {
-            stack[sp * stride + tid] = (__float_as_uint(key) & 0xFFFF0000u) | uint32_t(child);
-        }
-        ++sp;
-    };
-    // next node from the stack; false when the stack is empty (the query is complete). A keyed
-    // entry whose box starts beyond the hit found since it was pushed is dropped (the same
-    // 1 + 2^-21.5 margin as the box test, so no triangle at t <= tfar is skipped).
-    auto pop = [&]() -> bool {
-        while (sp > 0) {
-            --sp;
-            int32_t nd;
-            if constexpr (SK == kStack32) {
-                nd = int32_t(stack[sp * stride + tid]);
-            } else if constexpr (SK == kStack16) {
-                nd = reinterpret_cast<const uint16_t*>(stack)[((sp >> 1) * stride + tid) * 2 + (sp & 1)];
-            } else {
-                const uint32_t e = stack[sp * stride + tid];
-                if (__uint_as_float(e & 0xFFFF0000u) > tfar * 1.00000036f) continue;
-                nd = int32_t(e & 0xFFFFu);
-            }
-            st.node = nd;
-            return true;
-        }
-        return false;
-    };
-    bool done = false;
-    if (ANY && st.tri < st.tri_end) {
-        // leaf mode (any-hit queries): one triangle
-        tri_hit(r, reinterpret_cast<const float*>(tris + 4 * size_t(st.tri)), tnear, tfar, hit);
-        if (ANY && hit >= 0) {
-            st.hit = hit;
-            st.tfar = tfar;
-            return true;
-        }
-        if (++st.tri == st.tri_end) {
-            const uint32_t rest = st.leaves & (st.leaves - 1u);
-            st.leaves = rest;
-            if (rest) {
-                // the next entered leaf of this node: its reference is re-read from the node
-                const uint4 w3 = reinterpret_cast<const uint4*>(nodes)[4 * size_t(st.node) + 3];
-                const int k = __builtin_ctz(rest);
-                const uint32_t ref = uint32_t(sel4(int32_t(w3.x), int32_t(w3.y), int32_t(w3.z), int32_t(w3.w), k));
-                st.tri = ref & 0x1FFFFFFFu;
-                st.tri_end = st.tri + (ref >> 29);
-            } else {
-                done = !pop();
-            }
-        }
-        st.sp = sp;
-        st.hit = hit;
-        st.tfar = tfar;
-        return done;
-    }
-    // quantized node (Bvh4QNodeHost): origin, grid steps, child box bytes, child references
-    const uint4* n = reinterpret_cast<const uint4*>(nodes) + 4 * size_t(st.node);
-    const uint4 w0 = n[0], w1 = n[1], w2 = n[2], w3 = n[3];
-    const float ox = __uint_as_float(w0.x), oy = __uint_as_float(w0.y), oz = __uint_as_float(w0.z);
-    const float sx = __uint_as_float(w2.z), sy = __uint_as_float(w2.w), sz = __uint_as_float(w0.w);
-    const uint32_t ref[4] = {w3.x, w3.y, w3.z, w3.w};
-    int cha[4], cna[4];
+            for (; leaves; leaves &= leaves - 1u) test(tri0, leaves);
+            float key[4];
+            int32_t idx[4];
+            const float lim = box_far(st.tfar);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        cha[k] = int(ref[k] & 0x1FFFFFFFu);
-        const int c = int(ref[k] >> 29);
-        cna[k] = c == int(kQEmptyDev) ? -1 : c;
-    }
-    // Slab distances in ray space: (origin + q * step - o) * inv = q * a + b with a = step * inv
-    // (exact: step is a power of two) and b = origin * inv - o * inv, so each plane costs one fused
-    // multiply-add. The entry plane of an axis (the lower one for inv >= 0) is evaluated with
-    // b - k |inv| and the exit plane with b + k |inv|, a margin that bounds every rounding against
-    // the plane as the host rounds it (ray_pre). Entry and exit need no min / max.
-    const float ax = sx * r.inv.x, ay = sy * r.inv.y, az = sz * r.inv.z;
-    const float bx = fmaf(ox, r.inv.x, r.c.x), by = fmaf(oy, r.inv.y, r.c.y), bz = fmaf(oz, r.inv.z, r.c.z);
-    const float bx0 = fmaf(-r.k, fabsf(r.inv.x), bx), bx1 = fmaf(r.k, fabsf(r.inv.x), bx);
-    const float by0 = fmaf(-r.k, fabsf(r.inv.y), by), by1 = fmaf(r.k, fabsf(r.inv.y), by);
-    const float bz0 = fmaf(-r.k, fabsf(r.inv.z), bz), bz1 = fmaf(r.k, fabsf(r.inv.z), bz);
-    const bool px = r.inv.x >= 0.0f, py = r.inv.y >= 0.0f, pz = r.inv.z >= 0.0f;
-    const uint32_t nx = px ? w1.x : w1.y, fx = px ? w1.y : w1.x;  // entry / exit plane bytes
-    const uint32_t ny = py ? w1.z : w1.w, fy = py ? w1.w : w1.z;
-    const uint32_t nz = pz ? w2.x : w2.y, fz = pz ? w2.y : w2.x;
-    float key[4];
-    int idx[4];
-    uint32_t leaves = 0;  // children whose box the ray enters and that are leaves
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float x0 = fmaf(float((nx >> (8 * k)) & 0xFFu), ax, bx0), x1 = fmaf(float((fx >> (8 * k)) & 0xFFu), ax, bx1);
-        const float y0 = fmaf(float((ny >> (8 * k)) & 0xFFu), ay, by0), y1 = fmaf(float((fy >> (8 * k)) & 0xFFu), ay, by1);
-        const float z0 = fmaf(float((nz >> (8 * k)) & 0xFFu), az, bz0), z1 = fmaf(float((fz >> (8 * k)) & 0xFFu), az, bz1);
-        const float t0 = fmaxf(fmaxf(x0, y0), fmaxf(z0, tnear));
-        const float t1 = fminf(fminf(x1, y1), fminf(z1, tfar)) * 1.00000036f;
-        bool h = t0 <= t1 && cna[k] >= 0;
-        if (h && cna[k] > 0) leaves |= 1u << k;
-        h = h && cna[k] == 0;
-        key[k] = h ? t0 : __int_as_float(0x7f800000);
-        idx[k] = h ? cha[k] : -1;
-    }
-    if (!ANY && leaves) {
-        // closest hit: the triangles of every entered leaf now, one per iteration (a wavefront runs
-        // as many iterations as its busiest lane needs), so that the inner children behind a hit
-        // found here are not entered at all
-        int k = __builtin_ctz(leaves);
-        int i = sel4(cha[0], cha[1], cha[2], cha[3], k);
-        int e = i + sel4(cna[0], cna[1], cna[2], cna[3], k);
-        for (;;) {
-            tri_hit(r, reinterpret_cast<const float*>(tris + 4 * size_t(i)), tnear, tfar, hit);
-            if (++i == e) {
-                leaves &= leaves - 1u;
-                if (!leaves) break;
-                k = __builtin_ctz(leaves);
-                i = sel4(cha[0], cha[1], cha[2], cha[3], k);
-                e = i + sel4(cna[0], cna[1], cna[2], cna[3], k);
+            for (int k = 0; k < 4; ++k) {
+                const bool h = ent[k] & (uint32_t(k) < n_inner) & (t0[k] <= lim);
+                key[k] = h ? t0[k] : __int_as_float(0x7f800000);
+                idx[k] = h ? int32_t(child0 + uint32_t(k)) : -1;
             }
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            if (!(key[c] <= tfar * 1.00000036f)) {
-                key[c] = __int_as_float(0x7f800000);
-                idx[c] = -1;
-            }
-    }
-    if constexpr (!ANY) {
-        // sort (key, idx) ascending: 5-comparator network; nearest child first
+            // sort (key, idx) ascending: 5-comparator network; nearest child first
 #define TR_CSWAP(a, b)                                                            \
     if (key[b] < key[a]) {                                                        \
         float tk = key[a]; key[a] = key[b]; key[b] = tk;                          \
         int ti = idx[a]; idx[a] = idx[b]; idx[b] = ti;                            \
     }
-        TR_CSWAP(0, 1) TR_CSWAP(2, 3) TR_CSWAP(0, 2) TR_CSWAP(1, 3) TR_CSWAP(1, 2)
+            TR_CSWAP(0, 1) TR_CSWAP(2, 3) TR_CSWAP(0, 2) TR_CSWAP(1, 3) TR_CSWAP(1, 2)
 #undef TR_CSWAP
-    } else {
-        // any hit: order does not matter; move an entered child to slot 0
 #pragma unroll
-        for (int c = 1; c < 4; ++c)
-            if (idx[0] < 0 && idx[c] >= 0) {
-                idx[0] = idx[c];
-                idx[c] = -1;
+            for (int k = 3; k >= 1; --k)
+                if (idx[k] >= 0) push(uint32_t(idx[k]));
+            if (idx[0] >= 0) {
+                st.node = uint32_t(idx[0]);
+                return false;
             }
+        }
     }
-    // push the entered inner children (far first); descend into the nearest, or, for an any-hit
-    // query with entered leaves, push every one of them and test the leaves from the next step on
+    if ((ANY || PACKED) && st.leaves) return false;
+    if constexpr (PACKED) {
+        // words above `lim` start behind the hit or are not entered
+        const uint32_t lim = __float_as_uint(box_far(st.tfar)) | 0xFFFFu;
 #pragma unroll
-    for (int k = 3; k >= 1; --k)
-        if (idx[k] >= 0) push(idx[k], key[k]);
-    if (ANY && leaves) {
-        if (idx[0] >= 0) push(idx[0], key[0]);
-        const int k = __builtin_ctz(leaves);
-        st.leaves = leaves;
-        st.tri = uint32_t(sel4(cha[0], cha[1], cha[2], cha[3], k));
-        st.tri_end = st.tri + uint32_t(sel4(cna[0], cna[1], cna[2], cna[3], k));
-    } else if (idx[0] >= 0) {
-        st.node = idx[0];
-    } else {
-        done = !pop();
+        for (int k = 3; k >= 1; --k)
+            if (st.p[k] <= lim) push(st.p[k]);
+        if (st.p[0] <= lim) {
+            st.node = st.p[0] & 0xFFFFu;
+            return false;
+        }
+        if constexpr (SK == kStackKeyed) {
+            while (st.sp != tid) {
+                st.sp -= stride;
+                const uint32_t e = top();
+                if (e <= lim) {
+                    st.node = e & 0xFFFFu;
+                    return false;
+                }
+            }
+            return true;
+        }
     }
-    st.sp = sp;
-    st.hit = hit;
-    st.tfar = tfar;
-    return done;
+    if (st.sp == tid) return true;
+    st.sp -= stride;
+    st.node = top();
+    return false;
 }
+
 // ---- closest hit of a wavefront's rays as one packet ------------------------------------------
 // The camera rays of one pixel's samples nearly share their traversal. Here the wavefront visits one
 // node at a time for all its lanes: a node is visited when the ray of any active lane enters it, so
@@ -558,26 +565,30 @@ __device__ __forceinline__ bool trace4_step(const float4* __restrict__ nodes, co
 // hit. A lane's answer is the one trace4_step gives: the closest hit does not depend on the order of
 // the visits or on visits of boxes the ray misses (equal distances resolve to the lower triangle
 // index). Children are visited nearest first by the entry distances of the first active lane.
-// `col` is the stack column of the wavefront's first lane (all lanes write the same entries).
+// When the directions of all active lanes have the same signs (nearly every pixel), entry and exit
+// planes are the same for every lane and are picked and spread on the scalar unit.
+// `col` is the stack column of the wavefront's first lane (all lanes write the same entries); tnear
+// is positive.
 template <int SK>
 __device__ __forceinline__ void trace4_packet(const float4* __restrict__ nodes, const float4* __restrict__ tris,
                                               const RayPre& r, float tnear, bool active, float& tfar, int32_t& hit,
                                               uint32_t* stack, int col, int stride)
 {
+    typedef typename std::conditional<SK == kStack32, size_t, uint32_t>::type Off;
     const uint64_t amask = __ballot(active);
     if (amask == 0ull) return;
     const int lead = int(__builtin_ctzll(amask));
-    auto push = [&](int sp, int32_t child) {
-        if constexpr (SK == kStack16)
-            reinterpret_cast<uint16_t*>(stack)[((sp >> 1) * stride + col) * 2 + (sp & 1)] = uint16_t(child);
-        else
-            stack[sp * stride + col] = uint32_t(child);
+    const uint64_t upx = __ballot(active && r.sx == kPermUp), upy = __ballot(active && r.sy == kPermUp),
+                   upz = __ballot(active && r.sz == kPermUp);
+    const bool same = (upx == 0ull || upx == amask) && (upy == 0ull || upy == amask) && (upz == 0ull || upz == amask);
+    const char* tri_base = reinterpret_cast<const char*>(tris);
+    auto push = [&](int sp, uint32_t child) {
+        if constexpr (SK == kStack16) reinterpret_cast<uint16_t*>(stack)[sp * stride + col] = uint16_t(child);
+        else stack[sp * stride + col] = child;
     };
-    auto pop = [&](int sp) -> int32_t {
-        if constexpr (SK == kStack16)
-            return int32_t(reinterpret_cast<const uint16_t*>(stack)[((sp >> 1) * stride + col) * 2 + (sp & 1)]);
-        else
-            return int32_t(stack[sp * stride + col] & (SK == kStackKeyed ? 0xFFFFu : 0xFFFFFFFFu));
+    auto pop = [&](int sp) -> uint32_t {
+        if constexpr (SK == kStack16) return uint32_t(reinterpret_cast<const uint16_t*>(stack)[sp * stride + col]);
+        else return stack[sp * stride + col];
     };
     // the node is the same for every lane: the device pass reads it through the constant address
     // space, so that the compiler uses scalar loads (one per wavefront, into scalar registers); the
@@ -587,74 +598,61 @@ __device__ __forceinline__ void trace4_packet(const float4* __restrict__ nodes, 
 #else
     typedef const uint4 cuint4;
 #endif
-    int32_t node = 0;
+    // two plane bytes in the halves of a word, as v_perm_b32 spreads them
+    auto spread01 = [](uint32_t q) { return (q & 0xFFu) | ((q & 0xFF00u) << 8); };
+    auto spread23 = [](uint32_t q) { return ((q >> 16) & 0xFFu) | ((q >> 8) & 0xFF0000u); };
+    uint32_t node = 0;
     int sp = 0;
     for (;;) {
-        node = __builtin_amdgcn_readfirstlane(node);
-        const cuint4* n = (const cuint4*)(reinterpret_cast<const uint4*>(nodes) + 4 * size_t(node));
-        const uint4 w0 = n[0], w1 = n[1], w2 = n[2], w3 = n[3];
-        const float ox = __uint_as_float(w0.x), oy = __uint_as_float(w0.y), oz = __uint_as_float(w0.z);
-        const float sx = __uint_as_float(w2.z), sy = __uint_as_float(w2.w), sz = __uint_as_float(w0.w);
-        const uint32_t ref[4] = {w3.x, w3.y, w3.z, w3.w};
-        int cha[4], cna[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            cha[k] = int(ref[k] & 0x1FFFFFFFu);
-            const int c = int(ref[k] >> 29);
-            cna[k] = c == int(kQEmptyDev) ? -1 : c;
-        }
-        // the slab test of trace4_step (same planes, same margins)
-        const float ax = sx * r.inv.x, ay = sy * r.inv.y, az = sz * r.inv.z;
-        const float bx = fmaf(ox, r.inv.x, r.c.x), by = fmaf(oy, r.inv.y, r.c.y), bz = fmaf(oz, r.inv.z, r.c.z);
-        const float bx0 = fmaf(-r.k, fabsf(r.inv.x), bx), bx1 = fmaf(r.k, fabsf(r.inv.x), bx);
-        const float by0 = fmaf(-r.k, fabsf(r.inv.y), by), by1 = fmaf(r.k, fabsf(r.inv.y), by);
-        const float bz0 = fmaf(-r.k, fabsf(r.inv.z), bz), bz1 = fmaf(r.k, fabsf(r.inv.z), bz);
-        const bool px = r.inv.x >= 0.0f, py = r.inv.y >= 0.0f, pz = r.inv.z >= 0.0f;
-        const uint32_t nx = px ? w1.x : w1.y, fx = px ? w1.y : w1.x;
-        const uint32_t ny = py ? w1.z : w1.w, fy = py ? w1.w : w1.z;
-        const uint32_t nz = pz ? w2.x : w2.y, fz = pz ? w2.y : w2.x;
-        float key[4];
+        node = uint32_t(__builtin_amdgcn_readfirstlane(int(node)));
+        const cuint4* nd = (const cuint4*)(reinterpret_cast<const char*>(nodes) + size_t(node) * 64);
+        const uint4 w0 = nd[0], w1 = nd[1], w2 = nd[2], w3 = nd[3];
+        const uint32_t child0 = w0.w, meta = w2.z, tri0 = w2.w, n_inner = w3.w;
+        float t0[4];
         bool ent[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const float x0 = fmaf(float((nx >> (8 * k)) & 0xFFu), ax, bx0), x1 = fmaf(float((fx >> (8 * k)) & 0xFFu), ax, bx1);
-            const float y0 = fmaf(float((ny >> (8 * k)) & 0xFFu), ay, by0), y1 = fmaf(float((fy >> (8 * k)) & 0xFFu), ay, by1);
-            const float z0 = fmaf(float((nz >> (8 * k)) & 0xFFu), az, bz0), z1 = fmaf(float((fz >> (8 * k)) & 0xFFu), az, bz1);
-            const float t0 = fmaxf(fmaxf(x0, y0), fmaxf(z0, tnear));
-            const float t1 = fminf(fminf(x1, y1), fminf(z1, tfar)) * 1.00000036f;
-            ent[k] = active && t0 <= t1 && cna[k] >= 0;
-            key[k] = t0;
+        if (same) {
+            const uint32_t nx = upx ? w1.x : w1.y, fx = upx ? w1.y : w1.x;
+            const uint32_t ny = upy ? w1.z : w1.w, fy = upy ? w1.w : w1.z;
+            const uint32_t nz = upz ? w2.x : w2.y, fz = upz ? w2.y : w2.x;
+            const uint32_t n[6] = {spread01(nx), spread23(nx), spread01(ny), spread23(ny), spread01(nz), spread23(nz)};
+            const uint32_t f[6] = {spread01(fx), spread23(fx), spread01(fy), spread23(fy), spread01(fz), spread23(fz)};
+            slabs4(r, w0, w3, n, f, tnear, box_far(tfar), t0, ent);
+        } else {
+            node_slabs(r, w0, w1, w2, w3, tnear, box_far(tfar), t0, ent);
         }
         // leaves first: the wavefront loops over the triangles of every leaf some lane entered;
         // each lane tests those of the leaves its ray entered
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            if (cna[k] > 0 && __ballot(ent[k]) != 0ull) {
-                const int i0 = __builtin_amdgcn_readfirstlane(cha[k]), i1 = i0 + __builtin_amdgcn_readfirstlane(cna[k]);
-                for (int i = i0; i < i1; ++i)
-                    if (ent[k]) tri_hit(r, reinterpret_cast<const float*>(tris + 4 * size_t(i)), tnear, tfar, hit);
+        for (uint32_t k = 0; k < 4; ++k) {
+            const bool e = active && ent[k];
+            if (k >= n_inner && __ballot(e) != 0ull) {
+                for (uint32_t m = (meta >> (8 * k)) & 0xFFu; m; m &= m - 1u) {
+                    const uint32_t slot = tri0 + uint32_t(__builtin_ctz(m));
+                    if (e) tri_hit<Off>(r, tri_base, Off(slot) * 64, int32_t(slot), tnear, tfar, hit);
+                }
             }
         }
         // inner children that some lane enters before its hit, ordered by the first active lane's
-        // entry distances (children that lane does not enter last)
-        float uk[4];
-        int ui[4];
+        // entry distances (children that lane does not enter last; distances are positive, so their
+        // bits order like them)
+        const float lim = box_far(tfar);
+        uint32_t uk[4], ui[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const bool e = ent[k] && cna[k] == 0 && key[k] <= tfar * 1.00000036f;
+        for (uint32_t k = 0; k < 4; ++k) {
+            const bool e = active && ent[k] && k < n_inner && t0[k] <= lim;
             const bool any = __ballot(e) != 0ull;
-            const float lk = __shfl(e ? key[k] : __int_as_float(0x7f800000), lead);
-            uk[k] = any ? lk : __int_as_float(0x7f800000);
-            ui[k] = any ? __builtin_amdgcn_readfirstlane(cha[k]) : -1;
+            const uint32_t lk = uint32_t(__builtin_amdgcn_readlane(e ? __float_as_int(t0[k]) : 0x7f800000, lead));
+            uk[k] = any ? lk : 0xFFFFFFFFu;
+            ui[k] = child0 + k;
         }
 #define TR_PSWAP(a, b)                                                                \
-    if (ui[b] >= 0 && (ui[a] < 0 || uk[b] < uk[a])) {                                 \
-        float tk = uk[a]; uk[a] = uk[b]; uk[b] = tk;                                  \
-        int ti = ui[a]; ui[a] = ui[b]; ui[b] = ti;                                    \
+    if (uk[b] < uk[a]) {                                                              \
+        uint32_t tk = uk[a]; uk[a] = uk[b]; uk[b] = tk;                               \
+        uint32_t ti = ui[a]; ui[a] = ui[b]; ui[b] = ti;                               \
     }
         TR_PSWAP(0, 1) TR_PSWAP(2, 3) TR_PSWAP(0, 2) TR_PSWAP(1, 3) TR_PSWAP(1, 2)
 #undef TR_PSWAP
-        if (ui[0] < 0) {
+        if (uk[0] == 0xFFFFFFFFu) {
             if (sp == 0) break;
             --sp;
             node = pop(sp);
@@ -662,7 +660,7 @@ __device__ __forceinline__ void trace4_packet(const float4* __restrict__ nodes, 
         }
 #pragma unroll
         for (int k = 3; k >= 1; --k)
-            if (ui[k] >= 0) {
+            if (uk[k] != 0xFFFFFFFFu) {
                 push(sp, ui[k]);
                 ++sp;
             }
@@ -670,138 +668,14 @@ __device__ __forceinline__ void trace4_packet(const float4* __restrict__ nodes, 
     }
 }
 
-// ---- closest hit with postponed leaves -------------------------------------------------------
-// A closest-hit query whose wavefront runs node steps and triangle steps as separate, wavefront-wide
-// phases: a node step records the node's entered leaves as the lane's pending leaves instead of
-// testing them, and the lane goes on to the nearest inner child (or pops the keyed stack) while
-// its leaves wait; the caller runs a triangle phase (one triangle per lane with pending leaves)
-// once enough lanes hold some, or when no lane can take a node step. A lane that meets a second
-// node with entered leaves while it still holds pending ones waits on that node and visits it
-// again after its leaves are done (with the smaller far bound). Nodes and triangles then run with
-// most lanes active instead of every node step carrying the triangle loop of a few lanes.
-// Needs the keyed stack (kStackKeyed): entries behind a hit found later are dropped on pop.
-
-// true when the lane can take a node step now
-__device__ __forceinline__ bool trav4_pp_can_step(const Trav4& st, bool blocked) { return st.node >= 0 && !blocked; }
-
-// One node step; `blocked` is set when the node has entered leaves while the lane holds pending
-// ones (the state is left unchanged: the node is visited again once they are tested). Returns true
-// when the query is complete.
-template <int SK>
-__device__ __forceinline__ bool trace4_node_pp(const float4* __restrict__ nodes, const RayPre& r, float tnear, Trav4& st,
-                                               uint32_t* stack, int tid, int stride, bool& blocked)
-{
-    static_assert(SK == kStackKeyed || SK == kStack32, "postponed leaves use the keyed (or 32-bit) stack");
-    const float tfar = st.tfar;
-    int sp = st.sp;
-    const uint4* n = reinterpret_cast<const uint4*>(nodes) + 4 * size_t(st.node);
-    const uint4 w0 = n[0], w1 = n[1], w2 = n[2], w3 = n[3];
-    const float ox = __uint_as_float(w0.x), oy = __uint_as_float(w0.y), oz = __uint_as_float(w0.z);
-    const float sx = __uint_as_float(w2.z), sy = __uint_as_float(w2.w), sz = __uint_as_float(w0.w);
-    const uint32_t ref[4] = {w3.x, w3.y, w3.z, w3.w};
-    int cha[4], cna[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        cha[k] = int(ref[k] & 0x1FFFFFFFu);
-        const int c = int(ref[k] >> 29);
-        cna[k] = c == int(kQEmptyDev) ? -1 : c;
-    }
-    // the slab test of trace4_step (same planes, same margins)
-    const float ax = sx * r.inv.x, ay = sy * r.inv.y, az = sz * r.inv.z;
-    const float bx = fmaf(ox, r.inv.x, r.c.x), by = fmaf(oy, r.inv.y, r.c.y), bz = fmaf(oz, r.inv.z, r.c.z);
-    const float bx0 = fmaf(-r.k, fabsf(r.inv.x), bx), bx1 = fmaf(r.k, fabsf(r.inv.x), bx);
-    const float by0 = fmaf(-r.k, fabsf(r.inv.y), by), by1 = fmaf(r.k, fabsf(r.inv.y), by);
-    const float bz0 = fmaf(-r.k, fabsf(r.inv.z), bz), bz1 = fmaf(r.k, fabsf(r.inv.z), bz);
-    const bool px = r.inv.x >= 0.0f, py = r.inv.y >= 0.0f, pz = r.inv.z >= 0.0f;
-    const uint32_t nx = px ? w1.x : w1.y, fx = px ? w1.y : w1.x;
-    const uint32_t ny = py ? w1.z : w1.w, fy = py ? w1.w : w1.z;
-    const uint32_t nz = pz ? w2.x : w2.y, fz = pz ? w2.y : w2.x;
-    float key[4];
-    int idx[4];
-    uint32_t leaves = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const float x0 = fmaf(float((nx >> (8 * k)) & 0xFFu), ax, bx0), x1 = fmaf(float((fx >> (8 * k)) & 0xFFu), ax, bx1);
-        const float y0 = fmaf(float((ny >> (8 * k)) & 0xFFu), ay, by0), y1 = fmaf(float((fy >> (8 * k)) & 0xFFu), ay, by1);
-        const float z0 = fmaf(float((nz >> (8 * k)) & 0xFFu), az, bz0), z1 = fmaf(float((fz >> (8 * k)) & 0xFFu), az, bz1);
-        const float t0 = fmaxf(fmaxf(x0, y0), fmaxf(z0, tnear));
-        const float t1 = fminf(fminf(x1, y1), fminf(z1, tfar)) * 1.00000036f;
-        bool h = t0 <= t1 && cna[k] >= 0;
-        if (h && cna[k] > 0) leaves |= 1u << k;
-        h = h && cna[k] == 0;
-        key[k] = h ? t0 : __int_as_float(0x7f800000);
-        idx[k] = h ? cha[k] : -1;
-    }
-    if (leaves && st.leaves) {
-        blocked = true;  // test the pending leaves first, then visit this node again
-        return false;
-    }
-    if (leaves) {
-        const int k = __builtin_ctz(leaves);
-        st.pnode = st.node;
-        st.leaves = leaves;
-        st.tri = uint32_t(sel4(cha[0], cha[1], cha[2], cha[3], k));
-        st.tri_end = st.tri + uint32_t(sel4(cna[0], cna[1], cna[2], cna[3], k));
-    }
-#define TR_CSWAP(a, b)                                                            \
-    if (key[b] < key[a]) {                                                        \
-        float tk = key[a]; key[a] = key[b]; key[b] = tk;                          \
-        int ti = idx[a]; idx[a] = idx[b]; idx[b] = ti;                            \
-    }
-    TR_CSWAP(0, 1) TR_CSWAP(2, 3) TR_CSWAP(0, 2) TR_CSWAP(1, 3) TR_CSWAP(1, 2)
-#undef TR_CSWAP
-#pragma unroll
-    for (int k = 3; k >= 1; --k)
-        if (idx[k] >= 0) {
-            if constexpr (SK == kStack32) stack[sp * stride + tid] = uint32_t(idx[k]);
-            else stack[sp * stride + tid] = (__float_as_uint(key[k]) & 0xFFFF0000u) | uint32_t(idx[k]);
-            ++sp;
-        }
-    int32_t next = idx[0];
-    while (next < 0 && sp > 0) {
-        --sp;
-        const uint32_t e = stack[sp * stride + tid];
-        if constexpr (SK == kStack32) {
-            next = int32_t(e);
-        } else {
-            if (__uint_as_float(e & 0xFFFF0000u) > tfar * 1.00000036f) continue;
-            next = int32_t(e & 0xFFFFu);
-        }
-    }
-    st.node = next;
-    st.sp = sp;
-    return next < 0 && st.leaves == 0;
-}
-
-// One triangle of the lane's pending leaves. Returns true when the query is complete.
-__device__ __forceinline__ bool trace4_leaf_pp(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                               const RayPre& r, float tnear, Trav4& st, bool& blocked)
-{
-    tri_hit(r, reinterpret_cast<const float*>(tris + 4 * size_t(st.tri)), tnear, st.tfar, st.hit);
-    if (++st.tri == st.tri_end) {
-        const uint32_t rest = st.leaves & (st.leaves - 1u);
-        st.leaves = rest;
-        if (rest) {
-            const uint4 w3 = reinterpret_cast<const uint4*>(nodes)[4 * size_t(st.pnode) + 3];
-            const int k = __builtin_ctz(rest);
-            const uint32_t ref = uint32_t(sel4(int32_t(w3.x), int32_t(w3.y), int32_t(w3.z), int32_t(w3.w), k));
-            st.tri = ref & 0x1FFFFFFFu;
-            st.tri_end = st.tri + (ref >> 29);
-        } else {
-            blocked = false;
-        }
-    }
-    return st.leaves == 0 && st.node < 0;
-}
-
-template <bool ANY, int SK>
+template <bool ANY, int SK, bool POS>
 __device__ __forceinline__ int32_t trace4(const float4* __restrict__ nodes, const float4* __restrict__ tris,
-                                          const RayPre& r, float tnear, float& tfar, uint32_t* stack, int tid,
-                                          int stride)
+                                          const RayPre& r, float tnear, float& tfar, uint32_t* stack, uint32_t tid,
+                                          uint32_t stride)
 {
     Trav4 st;
-    trav4_begin(st, tfar);
-    while (!trace4_step<ANY, SK>(nodes, tris, r, tnear, st, stack, tid, stride)) {
+    trav4_begin(st, tfar, tid);
+    while (!trace4_step<ANY, SK, POS>(nodes, tris, r, tnear, st, stack, tid, stride)) {
     }
     tfar = st.tfar;
     return st.hit;

@@ -102,6 +102,36 @@ std::vector<Bvh4QNodeHost> quantize_bvh4(const Bvh4& b4);
 // every plane of the quantized BVH, which the traversal's per-ray slab margins are sized by.
 float qbvh_plane_bound(const std::vector<Bvh4QNodeHost>& q4);
 
+// ---- node of the device's 4-wide BVH: 64 bytes (four 16-byte words) -----------------------------
+//   word 0: origin xyz, w = first inner child (the inner children are consecutive nodes)
+//   word 1: child box bytes lo_x[4], hi_x[4], lo_y[4], hi_y[4]
+//   word 2: lo_z[4], hi_z[4], z = triangle masks (byte k: child k's triangles, bit j = slot tri0 + j; 0
+//           for inner and empty children), w = tri0, the node's first triangle slot
+//   word 3: grid steps xyz times 2^24 (the traversal multiplies them by q * 2^-24), w = inner children
+// The quantized node with its children in the order inner, leaf, empty; the triangles of a node's
+// leaves are consecutive slots, so that a query keeps the triangles it has to test as one bit mask
+// and its children as one index.
+struct alignas(16) Bvh4DevNode {
+    float origin[3];
+    uint32_t child0;
+    uint8_t q[24];
+    uint32_t tri_masks;
+    uint32_t tri0;
+    float step24[3];
+    uint32_t n_inner;
+};
+static_assert(sizeof(Bvh4DevNode) == 64, "device node layout");
+static_assert(4 * kLeafMax <= 8, "a node's triangles fit the bits of a mask byte");
+
+struct Bvh4Device {
+    std::vector<Bvh4DevNode> nodes;   // root = node 0, depth-first, siblings together
+    std::vector<uint32_t> tri_order;  // slot -> index in the builder's leaf order
+    std::vector<uint32_t> tri_slot;   // index in the builder's leaf order -> slot
+    bool scaled = true;               // every step * 2^24 (and its product with the slab test's largest
+                                      // reciprocal, 1e20) is finite
+};
+Bvh4Device device_bvh4(const std::vector<Bvh4QNodeHost>& q4, size_t n_tris);
+
 // ---- lights ------------------------------------------------------------------------------
 enum : int32_t { kLightPoint = 0, kLightRect = 1 };
 struct alignas(16) LightHost {

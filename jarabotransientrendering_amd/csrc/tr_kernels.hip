@@ -92,9 +92,9 @@ __host__ __device__ constexpr uint32_t part_word(uint32_t part, uint32_t w) { re
 
 struct SceneDev {
     const float4* nodes;       // binary BVH (4 float4 per node)
-    const float4* nodes4;      // quantized 4-wide BVH (4 x 16 bytes per node, Bvh4QNodeHost)
-    const float4* tris;        // rotated triangle records in leaf order (4 float4 each, see TriRot)
-    const float4* tri_normal;  // per scene triangle: geometric normal xyz, w = material bits (int)
+    const float4* nodes4;      // quantized 4-wide BVH (4 x 16 bytes per node, Bvh4DevNode)
+    const float4* tris;        // rotated triangle records in slot order (4 float4 each, see TriRot)
+    const float4* tri_normal;  // per slot: geometric normal xyz, w = material bits (int)
     const float4* tri_vn;      // smooth triangles: p0, e1, e2, n0, n1, n2 (null if none)
     const float4* mats;        // Kd xyz, w = mean albedo used by the roulette
     const LightHost* lights;
@@ -140,7 +140,7 @@ struct WaveDev {
     float4* thr[2];   // throughput xyz (with the pending BSDF/phase weight and roulette), w = time
     uint4* misc[2];   // x = path id lo, y = path id hi, z/w = path-stream PCG32 state
     uint4* extra[2];  // x/y = light-stream PCG32 state, z = level | film pixel << 8, w = unwarp distance (float bits)
-    float2* hit;      // per record of the current bounce: x = distance, y = scene triangle (int bits) or -1
+    float2* hit;      // per record of the current bounce: x = distance, y = triangle slot (int bits) or -1
     float4* sh_o;     // light point xyz, w = distance
     float4* sh_d;     // direction xyz, w = film element index (uint bits)
     float4* sh_c;     // contribution rgb, w = film pixel (uint bits)
@@ -263,30 +263,23 @@ __global__ void __launch_bounds__(kBlock) camera_kernel(SceneDev S0, RenderDev R
 // ---------------------------------------------------------------------------------------------
 // Traversal variants: the binary BVH, or the 4-wide BVH with 32-bit, 16-bit or keyed 16-bit stack
 // entries (trd::kStack*). Any-hit queries of a keyed launch use the 16-bit format.
-// kTravWidePP: keyed stack and closest hits with postponed leaves (trace4_node_pp / trace4_leaf_pp);
-// its any-hit launches use the 16-bit stack.
-enum { kTravBinary = 0, kTravWide = 1, kTravWide16 = 2, kTravWideKeyed = 3, kTravWidePP = 4 };
-// postponed leaves: a triangle phase runs once this many lanes of a wavefront hold pending leaves
-constexpr int kLeafPhaseMin = 32;
+enum { kTravBinary = 0, kTravWide = 1, kTravWide16 = 2, kTravWideKeyed = 3 };
 
 // LDS words per thread of a traversal block for a stack of STACK entries
 template <int TRAV, int STACK>
 constexpr int stack_words() { return TRAV == kTravWide16 ? (STACK + 1) / 2 : STACK; }
 
+// one query to its end (public queries, whose tnear may be any number, and the binary BVH)
 template <bool ANY, int TRAV>
 __device__ __forceinline__ int32_t trace_scene(const SceneDev& S, const RayPre& r, float tnear, float& tfar,
                                                uint32_t* stack)
 {
+    static_assert(TRAV != kTravWideKeyed, "keyed entries need a positive tnear");
     if constexpr (TRAV == kTravBinary)
         return trace<ANY>(S.nodes, S.tris, r, tnear, tfar, reinterpret_cast<int32_t*>(stack) + threadIdx.x, kTraceBlock);
-    else if constexpr (TRAV == kTravWide)
-        return trace4<ANY, kStack32>(S.nodes4, S.tris, r, tnear, tfar, stack, threadIdx.x, kTraceBlock);
-    else if constexpr (TRAV == kTravWide16 || ANY)
-        return trace4<ANY, kStack16>(S.nodes4, S.tris, r, tnear, tfar, stack, threadIdx.x, kTraceBlock);
-    else if constexpr (TRAV == kTravWidePP)
-        return trace4<ANY, kStackKeyed>(S.nodes4, S.tris, r, tnear, tfar, stack, threadIdx.x, kTraceBlock);
     else
-        return trace4<ANY, kStackKeyed>(S.nodes4, S.tris, r, tnear, tfar, stack, threadIdx.x, kTraceBlock);
+        return trace4<ANY, TRAV == kTravWide ? kStack32 : kStack16, false>(S.nodes4, S.tris, r, tnear, tfar, stack,
+                                                                           threadIdx.x, kTraceBlock);
 }
 
 template <int TRAV>
@@ -296,7 +289,8 @@ constexpr int stack_kind() { return TRAV == kTravWide ? kStack32 : TRAV == kTrav
 // takes the next ray at once instead of waiting for the wavefront's slowest ray. The wavefront
 // claims `chunk` queue entries at a time (its static share first, then through its partition's
 // fetch cursor) and hands them to its idle lanes in lane order. Call with every lane of the
-// wavefront; `busy` marks the lanes with a query.
+// wavefront; `rec` is the queue entry of the lane's query, kIdle if it has none.
+constexpr uint32_t kIdle = 0xFFFFFFFFu;
 // idle lanes that trigger a refill (unless the whole wavefront is idle): closest-hit and any-hit launches
 // (with camera rays in their own packet kernel, 16 and 32 for either were 0.2-0.7 % slower than 24)
 constexpr int kRefillMinExtend = 24;
@@ -337,28 +331,27 @@ struct RayRefill {
         part = blockIdx.x % parts;
     }
 
-    // Assigns queue entries to idle lanes; `start(i)` begins the query of entry i on this lane.
+    // Assigns queue entries to idle lanes (their `rec`) and begins their queries with `start(i)`.
     // `cursor` is the partition word (P_FETCH_EXT / P_FETCH_SHADOW) of the launch's queue.
     template <int kRefillMin = kRefillMinExtend, class Start>
-    __device__ __forceinline__ void run(uint32_t count, uint32_t chunk, uint32_t* counters, uint32_t cursor, bool& busy,
-                                        Start start)
+    __device__ __forceinline__ void run(uint32_t count, uint32_t chunk, uint32_t* counters, uint32_t cursor,
+                                        uint32_t& rec, Start start)
     {
-        const uint32_t lane = __lane_id();
-        const uint64_t below = lane ? (~0ull >> (64u - lane)) : 0ull;
-        uint64_t need = __ballot(!busy);
+        uint64_t idle = __ballot(rec == kIdle);
         // refill in bulk: ray set-up runs once for many idle lanes instead of once per finished ray
         // (24 idle lanes measured best on the 82k-triangle scene: 1-2 % faster than 16 or 32, 4 % than 48,
         // and 13 % faster than refilling each lane at once)
-        if (__popcll(need) < kRefillMin && need != ~0ull) return;
-        while (need && !drained) {
+        if (drained || (__popcll(idle) < kRefillMin && idle != ~0ull)) return;
+        uint32_t take = kIdle;
+        do {
             if (pos >= end) {
                 if (dyn_base >= count) {  // nothing beyond the static shares
                     drained = true;
                     break;
                 }
                 uint32_t k = 0;
-                if (lane == 0) k = atomicAdd(counters + part_word(part, cursor), 1u);
-                k = __shfl(k, 0);
+                if (__lane_id() == 0) k = atomicAdd(counters + part_word(part, cursor), 1u);
+                k = uint32_t(__builtin_amdgcn_readfirstlane(int(k)));
                 const uint64_t b = uint64_t(dyn_base) + (uint64_t(k) * parts + part) * chunk;
                 if (b >= count) {
                     drained = true;
@@ -368,13 +361,14 @@ struct RayRefill {
                 end = uint32_t(min(b + chunk, uint64_t(count)));
             }
             const uint32_t avail = end - pos;
-            const uint32_t rank = uint32_t(__popcll(need & below));
-            if (!busy && rank < avail) {
-                start(pos + rank);
-                busy = true;
-            }
-            pos += min(uint32_t(__popcll(need)), avail);
-            need = __ballot(!busy);
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
+            if (rec == kIdle && take == kIdle && rank < avail) take = pos + rank;
+            pos += min(uint32_t(__popcll(idle)), avail);
+            idle = __ballot(rec == kIdle && take == kIdle);
+        } while (idle);
+        if (take != kIdle) {
+            rec = take;
+            start(take);
         }
     }
 };
@@ -398,59 +392,15 @@ __global__ void __launch_bounds__(kTraceBlock, 7) extend_kernel(SceneDev S0, con
     }
     if (gid < kParts) Wv.counters[part_word(gid, P_FETCH_SHADOW)] = 0;
     const uint32_t chunk = fetch_chunk(count);
-    if constexpr (TRAV == kTravWidePP) {
-        // persistent grid with per-lane refill; node steps and triangle steps in wavefront-wide phases
-        RayRefill rf(count, chunk);
-        bool busy = false, blocked = false;
-        uint32_t rec = 0;
-        RayPre r;
-        Trav4 st;
-        const float4 *nodes = S0.nodes4, *tris = S0.tris;
-        for (;;) {
-            rf.run(count, chunk, Wv.counters, P_FETCH_EXT, busy, [&](uint32_t i) {
-                rec = i;
-                const float4 d = Wv.ray_d[cur][i];
-                float3 c = Wv.cpos;
-                float pb = S0.plane_bound;
-                if constexpr (BATCH) {
-                    const JobDev& J = jobs[__float_as_uint(d.w)];
-                    nodes = J.S.nodes4;
-                    tris = J.S.tris;
-                    c = J.R.cpos;
-                    pb = J.S.plane_bound;
-                }
-                const float4 o = first ? make_float4(c.x, c.y, c.z, 0.0f) : Wv.ray_o[cur][i];
-                r = ray_pre(mk(o), mk(d), pb);
-                trav4_begin(st, __int_as_float(0x7f800000));
-                blocked = false;
-            });
-            if (__ballot(busy) == 0ull) break;  // the queue is drained and every query complete
-            const bool can = busy && trav4_pp_can_step(st, blocked);
-            const bool pend = busy && st.leaves != 0u;
-            const uint64_t cm = __ballot(can), pm = __ballot(pend);
-            bool done = busy && !can && !pend;  // (every busy lane can step or holds leaves)
-            if (cm == 0ull || __popcll(pm) >= kLeafPhaseMin) {
-                if (pend) done = trace4_leaf_pp(nodes, tris, r, kSigmaVisibility, st, blocked);
-            } else if (can) {
-                done = trace4_node_pp<kStackKeyed>(nodes, r, kSigmaVisibility, st, stack, threadIdx.x, kTraceBlock,
-                                                   blocked);
-            }
-            if (busy && done) {
-                Wv.hit[rec] = make_float2(st.hit >= 0 ? st.tfar : -1.0f, __int_as_float(st.hit));
-                busy = false;
-            }
-        }
-    } else if constexpr (TRAV != kTravBinary) {
+    if constexpr (TRAV != kTravBinary) {
         // persistent grid with per-lane refill: every lane steps its own query one node at a time
         RayRefill rf(count, chunk);
-        bool busy = false;
-        uint32_t rec = 0;
+        uint32_t rec = kIdle;
         RayPre r;
         Trav4 st;
         const float4 *nodes = S0.nodes4, *tris = S0.tris;
         for (;;) {
-            rf.run(count, chunk, Wv.counters, P_FETCH_EXT, busy, [&](uint32_t i) {
-                rec = i;
+            rf.run(count, chunk, Wv.counters, P_FETCH_EXT, rec, [&](uint32_t i) {
                 const float4 d = Wv.ray_d[cur][i];
                 float3 c = Wv.cpos;
                 float pb = S0.plane_bound;
@@ -461,15 +411,18 @@ __global__ void __launch_bounds__(kTraceBlock, 7) extend_kernel(SceneDev S0, con
                     c = J.R.cpos;
                     pb = J.S.plane_bound;
                 }
-                const float4 o = first ? make_float4(c.x, c.y, c.z, 0.0f) : Wv.ray_o[cur][i];
-                r = ray_pre(mk(o), mk(d), pb);
-                trav4_begin(st, __int_as_float(0x7f800000));
+                f3 o = mk(c.x, c.y, c.z);
+                // (in registers: otherwise the compiler selects between two addresses and uses flat loads)
+                asm("" : "+v"(o.x), "+v"(o.y), "+v"(o.z));
+                if (!first) o = mk(Wv.ray_o[cur][i]);
+                r = ray_pre(o, mk(d), pb);
+                trav4_begin(st, __int_as_float(0x7f800000), threadIdx.x);
             });
-            if (__ballot(busy) == 0ull) break;  // the queue is drained and every query complete
-            if (busy && trace4_step<false, stack_kind<TRAV>()>(nodes, tris, r, kSigmaVisibility, st, stack, threadIdx.x,
-                                                                kTraceBlock)) {
+            if (__ballot(rec != kIdle) == 0ull) break;  // the queue is drained and every query complete
+            if (rec != kIdle && trace4_step<false, stack_kind<TRAV>(), true>(nodes, tris, r, kSigmaVisibility, st, stack,
+                                                                             threadIdx.x, kTraceBlock)) {
                 Wv.hit[rec] = make_float2(st.hit >= 0 ? st.tfar : -1.0f, __int_as_float(st.hit));
-                busy = false;
+                rec = kIdle;
             }
         }
     } else {
@@ -517,24 +470,21 @@ __global__ void __launch_bounds__(kTraceBlock, 7) extend_camera_kernel(SceneDev 
     if (gid < kParts) Wv.counters[part_word(gid, P_FETCH_SHADOW)] = 0;
     const uint32_t chunk = fetch_chunk(count);
     RayRefill rf(count, chunk);
-    bool busy = false;
-    uint32_t rec = 0;
+    uint32_t rec = kIdle;
     RayPre r;
     const int col = int(threadIdx.x & ~63u);
     const f3 cam = mk(Wv.cpos.x, Wv.cpos.y, Wv.cpos.z);
     for (;;) {
-        rf.run(count, chunk, Wv.counters, P_FETCH_EXT, busy, [&](uint32_t i) {
-            rec = i;
-            r = ray_pre(cam, mk(Wv.ray_d[cur][i]), S0.plane_bound);
-        });
-        if (__ballot(busy) == 0ull) break;  // the queue is drained
+        rf.run(count, chunk, Wv.counters, P_FETCH_EXT, rec,
+               [&](uint32_t i) { r = ray_pre(cam, mk(Wv.ray_d[cur][i]), S0.plane_bound); });
+        if (__ballot(rec != kIdle) == 0ull) break;  // the queue is drained
         float tfar = __int_as_float(0x7f800000);
         int32_t hit = -1;
-        trace4_packet<stack_kind<TRAV>()>(S0.nodes4, S0.tris, r, kSigmaVisibility, busy, tfar, hit, stack, col,
+        trace4_packet<stack_kind<TRAV>()>(S0.nodes4, S0.tris, r, kSigmaVisibility, rec != kIdle, tfar, hit, stack, col,
                                           kTraceBlock);
-        if (busy) {
+        if (rec != kIdle) {
             Wv.hit[rec] = make_float2(hit >= 0 ? tfar : -1.0f, __int_as_float(hit));
-            busy = false;
+            rec = kIdle;
         }
     }
 }
@@ -1059,14 +1009,12 @@ __global__ void __launch_bounds__(kTraceBlock, 7) shadow_kernel(SceneDev S0, con
     if constexpr (TRAV != kTravBinary) {
         // persistent grid with per-lane refill (see extend_kernel)
         RayRefill rf(count, chunk);
-        bool busy = false;
-        uint32_t rec = 0;
+        uint32_t rec = kIdle;
         RayPre r;
         Trav4 st;
         const float4 *nodes = S0.nodes4, *tris = S0.tris;
         for (;;) {
-            rf.run<kRefillMinShadow>(count, chunk, Wv.counters, P_FETCH_SHADOW, busy, [&](uint32_t i) {
-                rec = i;
+            rf.run<kRefillMinShadow>(count, chunk, Wv.counters, P_FETCH_SHADOW, rec, [&](uint32_t i) {
                 float pb = S0.plane_bound;
                 if constexpr (BATCH) {
                     const SceneDev& S = jobs[Wv.sh_job[i]].S;
@@ -1076,16 +1024,17 @@ __global__ void __launch_bounds__(kTraceBlock, 7) shadow_kernel(SceneDev S0, con
                 }
                 const float4 o = Wv.sh_o[i], d = Wv.sh_d[i];
                 r = ray_pre(mk(o), mk(d), pb);
-                trav4_begin(st, o.w - kSigmaVisibility);
+                trav4_begin(st, o.w - kSigmaVisibility, threadIdx.x);
             });
-            if (__ballot(busy) == 0ull) break;
+            if (__ballot(rec != kIdle) == 0ull) break;
             // any hit: a keyed launch uses the 16-bit format (its LDS holds either)
             constexpr int SK = stack_kind<TRAV>() == kStackKeyed ? kStack16 : stack_kind<TRAV>();
-            if (busy && trace4_step<true, SK>(nodes, tris, r, kSigmaVisibility, st, stack, threadIdx.x, kTraceBlock)) {
+            if (rec != kIdle && trace4_step<true, SK, true>(nodes, tris, r, kSigmaVisibility, st, stack, threadIdx.x,
+                                                            kTraceBlock)) {
                 const bool vis = st.hit < 0;
                 Wv.sh_vis[rec] = vis ? 1 : 0;
                 visible += vis ? 1u : 0u;
-                busy = false;
+                rec = kIdle;
             }
         }
     } else {
@@ -1344,7 +1293,7 @@ __global__ void __launch_bounds__(kNormBlock) film_normalize_kernel(const float*
 // batch closest hit for the public query entry point
 template <int TRAV, int STACK>
 __global__ void __launch_bounds__(kTraceBlock) intersect_kernel(SceneDev S, const tr_ray* __restrict__ rays,
-                                                                tr_hit* __restrict__ hits, const uint2* __restrict__ ids,
+                                                                tr_hit* __restrict__ hits, const uint4* __restrict__ ids,
                                                                 uint32_t n)
 {
     __shared__ uint32_t stack[stack_words<TRAV, STACK>() * kTraceBlock];
@@ -1353,14 +1302,14 @@ __global__ void __launch_bounds__(kTraceBlock) intersect_kernel(SceneDev S, cons
         tr_ray q = rays[i];
         RayPre r = ray_pre(mk(q.org[0], q.org[1], q.org[2]), mk(q.dir[0], q.dir[1], q.dir[2]), S.plane_bound);
         float tfar = q.tfar;
-        int32_t tri = trace_scene<false, TRAV>(S, r, q.tnear, tfar, stack);
+        const int32_t slot = trace_scene<false, TRAV>(S, r, q.tnear, tfar, stack);
         tr_hit h;
-        if (tri >= 0) {
-            uint2 gp = ids[tri];
+        if (slot >= 0) {
+            const uint4 id = ids[slot];
             h.t = tfar;
-            h.geom_id = gp.x;
-            h.prim_id = gp.y;
-            h.tri = uint32_t(tri);
+            h.geom_id = id.x;
+            h.prim_id = id.y;
+            h.tri = id.z;
         } else {
             h.t = -1.0f;
             h.geom_id = 0xFFFFFFFFu;
@@ -1419,7 +1368,6 @@ void launch_timed(void (*k)(P...), uint32_t grid, uint32_t block, hipStream_t s,
         case kTravBinary: TR_STACK_DISPATCH3B(kTravBinary, bound, batch, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break; \
         case kTravWide: TR_STACK_DISPATCH3B(kTravWide, bound, batch, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break;     \
         case kTravWide16: TR_STACK_DISPATCH3B(kTravWide16, bound, batch, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break; \
-        case kTravWidePP: TR_STACK_DISPATCH3B(kTravWidePP, bound, batch, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break; \
         default: TR_STACK_DISPATCH3B(kTravWideKeyed, bound, batch, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break;       \
         }                                                                                                   \
     } while (0)
@@ -1444,8 +1392,7 @@ void launch_timed(void (*k)(P...), uint32_t grid, uint32_t block, hipStream_t s,
         switch (trav) {                                                                                   \
         case kTravBinary: TR_STACK_DISPATCH_T(kTravBinary, bound, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break; \
         case kTravWide: TR_STACK_DISPATCH_T(kTravWide, bound, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break;     \
-        case kTravWide16: TR_STACK_DISPATCH_T(kTravWide16, bound, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break; \
-        default: TR_STACK_DISPATCH_T(kTravWideKeyed, bound, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break;       \
+        default: TR_STACK_DISPATCH_T(kTravWide16, bound, KERNEL, GRID, BLOCK, STREAM, __VA_ARGS__); break;          \
         }                                                                                                 \
     } while (0)
 
@@ -1525,11 +1472,12 @@ struct LaunchCfg {
 // launch flags -> stack format
 static int stack_fmt_of(uint32_t flags)
 {
-    return (flags & TR_RENDER_POSTPONE_LEAVES) ? 3 : (flags & TR_RENDER_STACK32) ? 1 : (flags & TR_RENDER_STACK_KEYED) ? 2 : 0;
+    if (flags & TR_RENDER_POSTPONE_LEAVES) return 2;
+    return (flags & TR_RENDER_STACK32) ? 1 : (flags & TR_RENDER_STACK_KEYED) ? 2 : 0;
 }
 static uint32_t stack_flags_of(int fmt)
 {
-    return fmt == 1 ? TR_RENDER_STACK32 : fmt == 2 ? TR_RENDER_STACK_KEYED : fmt == 3 ? TR_RENDER_POSTPONE_LEAVES : 0u;
+    return fmt == 1 ? TR_RENDER_STACK32 : fmt == 2 ? TR_RENDER_STACK_KEYED : 0u;
 }
 
 struct WaveBuffers {
@@ -1667,10 +1615,10 @@ struct tr_scene_s {
     float4 *d_nodes = nullptr, *d_nodes4 = nullptr, *d_tris = nullptr, *d_tri_normal = nullptr, *d_mats = nullptr;
     float4* d_tri_vn = nullptr;  // smooth triangles: p0, e1, e2, n0, n1, n2 (6 float4 per triangle)
     LightHost* d_lights = nullptr;
-    uint2* d_ids = nullptr;
+    uint4* d_ids = nullptr;     // per triangle slot: geometry, primitive, scene triangle
     uint32_t n_nodes = 0, n_nodes4 = 0;
     int depth = 0, depth4 = 0, stack4 = 0;
-    bool wide = true;   // traverse the 4-wide BVH (tr_render_desc flags can select the binary one)
+    bool wide = true;   // the 4-wide BVH can be traversed (its scaled grid steps are finite; otherwise the binary one is)
     float bb_lo[3] = {0, 0, 0}, bb_hi[3] = {1, 1, 1};  // bounds of the triangles (set at commit)
     float plane_bound = 1.0f;  // largest |plane| of the quantized BVH (set at commit)
     LaunchCfg tune;     // launch shape used by renders of this scene (tr_autotune sets it)
@@ -1913,17 +1861,25 @@ int tr_scene_commit(tr_scene s)
     if (b4.nodes.size() >= (size_t(1) << 29) || b.tris.size() >= (size_t(1) << 29))
         return fail(TR_ERR_INVALID, "tr_scene_commit: more than 2^29 nodes or triangles");
     const std::vector<Bvh4QNodeHost> q4 = quantize_bvh4(b4);
+    const Bvh4Device dev4 = device_bvh4(q4, b.tris.size());
+    // the binary BVH's leaves refer to the same triangle slots
+    for (BvhNodeHost& nd : b.nodes)
+        for (int side = 0; side < 2; ++side)
+            if (nd.d[2 + side] > 0) nd.d[side] = int32_t(dev4.tri_slot[size_t(nd.d[side])]);
+    // per-triangle arrays are in slot order: scene triangle of each slot
+    std::vector<uint32_t> slot_tri(n);
+    for (uint32_t i = 0; i < n; ++i) std::memcpy(&slot_tri[i], &b.tris[dev4.tri_order[i]].p0[3], 4);
     HIP_TRY(hipStreamSynchronize(s->stream));
     s->release_device();
     std::vector<float4> normals(n > 0 ? n : 1);
     for (uint32_t i = 0; i < n; ++i) {
-        const float* t = &s->tris[9 * size_t(i)];
+        const float* t = &s->tris[9 * size_t(slot_tri[i])];
         // ng = normalize(cross(p2 - p0, p1 - p0)) (World.h:449)
         float e2[3] = {t[6] - t[0], t[7] - t[1], t[8] - t[2]}, e1[3] = {t[3] - t[0], t[4] - t[1], t[5] - t[2]};
         float c[3] = {e2[1] * e1[2] - e2[2] * e1[1], e2[2] * e1[0] - e2[0] * e1[2], e2[0] * e1[1] - e2[1] * e1[0]};
         float l = std::sqrt(c[0] * c[0] + c[1] * c[1] + c[2] * c[2]);
         float inv = l > 0.f ? float(1. / double(l)) : 0.f;
-        int32_t mi = s->tri_mat[i];
+        int32_t mi = s->tri_mat[slot_tri[i]];
         float w;
         std::memcpy(&w, &mi, 4);
         normals[i] = make_float4(c[0] * inv, c[1] * inv, c[2] * inv, w);
@@ -1937,8 +1893,9 @@ int tr_scene_commit(tr_scene s)
             s->bb_lo[k] = std::min(s->bb_lo[k], s->tris[3 * v + size_t(k)]);
             s->bb_hi[k] = std::max(s->bb_hi[k], s->tris[3 * v + size_t(k)]);
         }
-    std::vector<uint2> ids(n > 0 ? n : 1);
-    for (uint32_t i = 0; i < n; ++i) ids[i] = make_uint2(s->tri_geom[i], s->tri_prim[i]);
+    std::vector<uint4> ids(n > 0 ? n : 1);
+    for (uint32_t i = 0; i < n; ++i)
+        ids[i] = make_uint4(s->tri_geom[slot_tri[i]], s->tri_prim[slot_tri[i]], slot_tri[i], 0u);
     size_t nn = b.nodes.size(), nt = b.tris.size(), nm = std::max<size_t>(1, s->mats.size() / 4),
            nl = std::max<size_t>(1, s->lights.size());
     int rc;
@@ -1949,11 +1906,11 @@ int tr_scene_commit(tr_scene s)
         return rc;
     }
     HIP_TRY(hipMemcpyAsync(s->d_nodes, b.nodes.data(), nn * sizeof(BvhNodeHost), hipMemcpyHostToDevice, s->stream));
-    HIP_TRY(hipMemcpyAsync(s->d_nodes4, q4.data(), q4.size() * sizeof(Bvh4QNodeHost), hipMemcpyHostToDevice, s->stream));
+    HIP_TRY(hipMemcpyAsync(s->d_nodes4, dev4.nodes.data(), dev4.nodes.size() * sizeof(Bvh4DevNode), hipMemcpyHostToDevice, s->stream));
     // rotated triangle records (TriRot): per vertex x y z x y, then the scene triangle index
     std::vector<float> trot(16 * std::max<size_t>(1, nt), 0.f);
     for (size_t i = 0; i < nt; ++i) {
-        const TriHost& t = b.tris[i];
+        const TriHost& t = b.tris[dev4.tri_order[i]];
         const float* P[3] = {t.p0, t.p1, t.p2};
         float* o = &trot[16 * i];
         for (int v = 0; v < 3; ++v) {
@@ -1971,14 +1928,14 @@ int tr_scene_commit(tr_scene s)
         HIP_TRY(hipMemcpyAsync(s->d_mats, s->mats.data(), s->mats.size() * sizeof(float), hipMemcpyHostToDevice, s->stream));
     if (!s->lights.empty())
         HIP_TRY(hipMemcpyAsync(s->d_lights, s->lights.data(), s->lights.size() * sizeof(LightHost), hipMemcpyHostToDevice, s->stream));
-    HIP_TRY(hipMemcpyAsync(s->d_ids, ids.data(), ids.size() * sizeof(uint2), hipMemcpyHostToDevice, s->stream));
+    HIP_TRY(hipMemcpyAsync(s->d_ids, ids.data(), ids.size() * sizeof(uint4), hipMemcpyHostToDevice, s->stream));
     std::vector<float4> vn;
     if (!s->tri_vn.empty()) {
         // smooth triangles: the plane frame for barycentrics from a hit point, and corner normals
         vn.resize(size_t(n) * 6);
         for (uint32_t i = 0; i < n; ++i) {
-            const float* t = &s->tris[9 * size_t(i)];
-            const float* q = &s->tri_vn[9 * size_t(i)];
+            const float* t = &s->tris[9 * size_t(slot_tri[i])];
+            const float* q = &s->tri_vn[9 * size_t(slot_tri[i])];
             vn[6 * size_t(i) + 0] = make_float4(t[0], t[1], t[2], 0.f);
             vn[6 * size_t(i) + 1] = make_float4(t[3] - t[0], t[4] - t[1], t[5] - t[2], 0.f);
             vn[6 * size_t(i) + 2] = make_float4(t[6] - t[0], t[7] - t[1], t[8] - t[2], 0.f);
@@ -1997,6 +1954,7 @@ int tr_scene_commit(tr_scene s)
     s->depth4 = b4.depth;
     s->stack4 = b4.stack_bound;
     s->plane_bound = qbvh_plane_bound(q4);
+    s->wide = dev4.scaled;
     s->build_ms = b.build_ms;
     s->committed = true;
     return TR_OK;
@@ -2746,18 +2704,19 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     uint64_t total = 0;
     int bounces = 0, stack_bound = 0;
     uint32_t max_nodes4 = 0;
+    bool wide = cfg.wide;
+    for (auto& j : jobs) wide = wide && j.scene->wide;
     for (auto& j : jobs) {
         j.dev.path_begin = total;
         total += j.paths;
         bounces = std::max(bounces, j.max_bounces);
-        stack_bound = std::max(stack_bound, cfg.wide ? j.scene->stack4 : j.scene->depth);
+        stack_bound = std::max(stack_bound, wide ? j.scene->stack4 : j.scene->depth);
         max_nodes4 = std::max(max_nodes4, j.scene->n_nodes4);
     }
     // 16-bit stack entries hold node indices below 65,536
     const bool small = max_nodes4 <= 65536u && cfg.stack_fmt != 1;
-    const int trav_ext = !cfg.wide ? kTravBinary : !small ? kTravWide : cfg.stack_fmt == 2 ? kTravWideKeyed
-                                                                      : cfg.stack_fmt == 3 ? kTravWidePP : kTravWide16;
-    const int trav_sh = !cfg.wide ? kTravBinary : !small ? kTravWide : kTravWide16;
+    const int trav_ext = !wide ? kTravBinary : !small ? kTravWide : cfg.stack_fmt == 2 ? kTravWideKeyed : kTravWide16;
+    const int trav_sh = !wide ? kTravBinary : !small ? kTravWide : kTravWide16;
     const bool mb = jobs[0].dev.R.layers > 0;
     for (auto& j : jobs)
         if (j.dev.R.layers > 0 && (batch || guide))
@@ -3192,7 +3151,7 @@ int tr_autotune(tr_batch b, tr_launch_desc* best, double* ms_best)
         if (ms[1] < ms[0] * kTuneMargin) bestc.per_job = true;
     }
     // stage 4: traversal stack formats
-    for (int fmt : {1, 2, 3}) {
+    for (int fmt : {1, 2}) {
         LaunchCfg c = bestc;
         if (!c.wide || c.stack_fmt == fmt) continue;
         c.stack_fmt = fmt;
