@@ -57,6 +57,32 @@ __device__ __forceinline__ uint64_t pcg_seed(uint64_t initstate, uint64_t seq)
     return s;
 }
 
+// The state of the stream with increment `inc` after n draws. A step is s -> a s + inc, so n + 1 steps
+// from (inc + seed) (where pcg_seed stands before its last one) give A (inc + seed) + C inc with
+// A = a^(n + 1) and C = 1 + a + ... + a^n mod 2^64 (F. Brown, "Random number generation with arbitrary
+// strides", 1994), read from a table: a path keeps a stream as its number of draws instead of a state.
+constexpr uint32_t kPcgJumps = 768;  // three draws per vertex, at most 255 vertices
+struct PcgJumps {
+    uint64_t ac[kPcgJumps][2];
+};
+constexpr PcgJumps pcg_jumps()
+{
+    PcgJumps t{};
+    uint64_t a = 1, c = 0;
+    for (uint32_t n = 0; n < kPcgJumps; ++n) {
+        c += a;
+        a *= 6364136223846793005ULL;
+        t.ac[n][0] = a;
+        t.ac[n][1] = c;
+    }
+    return t;
+}
+__device__ __constant__ const PcgJumps kPcgJump = pcg_jumps();
+__device__ __forceinline__ uint64_t pcg_at(uint64_t initstate, uint64_t inc, uint32_t n)
+{
+    return kPcgJump.ac[n][0] * (inc + initstate) + kPcgJump.ac[n][1] * inc;
+}
+
 // ---- wave-aggregated queue append (one atomic per wavefront) -------------------------------
 __device__ __forceinline__ uint32_t wave_append(uint32_t* counter, bool pred)
 {

@@ -127,19 +127,22 @@ struct RenderDev {
     // Transient sampling mode (-time-sampling): free-flight rate 4 / (T * exposure); 0 = steady state
     float ts_lambda;
     int32_t time_sampling;
+    uint64_t pid0;             // path id of the job's first path (row0 * W * spp2 * n_inc)
 };
 
 struct WaveDev {
     // path records of the current ([cur]) and the next ([cur ^ 1]) bounce. The camera kernel writes
-    // no origin and no throughput: every camera ray starts at the camera with unit throughput at
-    // time 0, so the first bounce takes them from the camera set-up (and the sampled free-flight
-    // distance from extra.w, which holds the unwarp distance only from the first hit on).
+    // the direction alone (and the job of batched renders): every camera ray starts at the camera
+    // with unit throughput at time 0 and its streams at their seeds, so the first bounce makes the
+    // rest from the path's index. All paths of a wavefront are at the same level. A path id follows
+    // from the index and the light stream's state from its number of draws (pcg_at): 64 bytes per
+    // continuing path instead of 80, 16 instead of 48 for a camera ray (33.5 M camera rays 253 ->
+    // 179 us, shading of the 67 M-path frame 4.64 -> 4.32 ms, of the media scanline 0.59 -> 0.55 ms).
     float4* ray_o[2]; // origin xyz, w = sampled free-flight distance of this segment (inf without medium)
-    float4* ray_d[2]; // direction xyz, w = batched renders: job (uint bits); otherwise the path's
-                      // index in its wavefront (uint bits)
+    float4* ray_d[2]; // direction xyz, w = the path's index in its wavefront (uint bits)
     float4* thr[2];   // throughput xyz (with the pending BSDF/phase weight and roulette), w = time
-    uint4* misc[2];   // x = path id lo, y = path id hi, z/w = path-stream PCG32 state
-    uint4* extra[2];  // x/y = light-stream PCG32 state, z = level | film pixel << 8, w = unwarp distance (float bits)
+    uint4* st[2];     // x = film pixel, y = light-stream draws so far | job << 16, z/w = path-stream PCG32 state
+    float* uw[2];     // unwarp distance (renders with camera unwarp only)
     float2* hit;      // per record of the current bounce: x = distance, y = triangle slot (int bits) or -1
     float4* sh_o;     // light point xyz, w = distance
     float4* sh_d;     // direction xyz, w = film element index (uint bits)
@@ -221,10 +224,8 @@ __global__ void __launch_bounds__(kBlock) camera_kernel(SceneDev S0, RenderDev R
     } else {
         pid_local = uint32_t(ctl.base) + slot;
     }
-    const SceneDev& S = BATCH ? jobs[jid].S : S0;
     const RenderDev& R = BATCH ? jobs[jid].R : R0;
     uint32_t cs_local = pid_local / uint32_t(R.n_inc);
-    uint32_t inc_i = pid_local - cs_local * uint32_t(R.n_inc);
     uint32_t pix_local = cs_local / uint32_t(R.spp2);   // film pixel (row relative)
     uint32_t sub = cs_local - pix_local * uint32_t(R.spp2);
     uint32_t rowl = pix_local / uint32_t(R.W);
@@ -233,7 +234,6 @@ __global__ void __launch_bounds__(kBlock) camera_kernel(SceneDev S0, RenderDev R
     uint32_t sy = sub / uint32_t(R.spp);
     uint32_t sx = sub - sy * uint32_t(R.spp);
     uint64_t cs = (uint64_t(y) * uint64_t(R.W) + xr) * uint64_t(R.spp2) + sub;
-    uint64_t pid = cs * uint64_t(R.n_inc) + inc_i;
 
     // StratifiedSampler::get_next_sample: jittered position clamped inside the pixel
     uint64_t cinc = pcg_inc((1ull << 62) | cs);
@@ -248,16 +248,8 @@ __global__ void __launch_bounds__(kBlock) camera_kernel(SceneDev S0, RenderDev R
     f3 dir = nv * R.fd + uv * (2.0f * ic0) - vv * (2.0f * ic1);
     dir = normalize(normalize(dir));  // get_ray_direction normalises, Ray3D normalises again
 
-    uint64_t pinc = pcg_inc(2 * pid);
-    uint64_t pst = pcg_seed(R.seed, 2 * pid);
-    uint64_t nst = pcg_seed(R.seed, 2 * pid + 1);
-    float sampled = __int_as_float(0x7f800000);
-    if (S.has_medium) {
-        sampled = free_flight(pcg_float(pst, pinc), R.time_sampling ? R.ts_lambda : S.lambda);
-    }
-    Wv.ray_d[0][slot] = make_float4(dir.x, dir.y, dir.z, __uint_as_float(BATCH ? jid : slot));
-    Wv.misc[0][slot] = make_uint4(uint32_t(pid), uint32_t(pid >> 32), uint32_t(pst), uint32_t(pst >> 32));
-    Wv.extra[0][slot] = make_uint4(uint32_t(nst), uint32_t(nst >> 32), pix_local << 8, __float_as_uint(sampled));
+    Wv.ray_d[0][slot] = make_float4(dir.x, dir.y, dir.z, __uint_as_float(slot));
+    if constexpr (BATCH) Wv.st[0][slot] = make_uint4(pix_local, jid << 16, 0u, 0u);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -405,7 +397,7 @@ __global__ void __launch_bounds__(kTraceBlock, 7) extend_kernel(SceneDev S0, con
                 float3 c = Wv.cpos;
                 float pb = S0.plane_bound;
                 if constexpr (BATCH) {
-                    const JobDev& J = jobs[__float_as_uint(d.w)];
+                    const JobDev& J = jobs[Wv.st[cur][i].y >> 16];
                     nodes = J.S.nodes4;
                     tris = J.S.tris;
                     c = J.R.cpos;
@@ -438,8 +430,9 @@ __global__ void __launch_bounds__(kTraceBlock, 7) extend_kernel(SceneDev S0, con
                 const uint32_t i = base + j + lane;
                 if (i < count) {
                     const float4 d = Wv.ray_d[cur][i];
-                    const SceneDev& S = BATCH ? jobs[__float_as_uint(d.w)].S : S0;
-                    const float3 c = BATCH ? jobs[__float_as_uint(d.w)].R.cpos : Wv.cpos;
+                    const uint32_t jid = BATCH ? Wv.st[cur][i].y >> 16 : 0u;
+                    const SceneDev& S = BATCH ? jobs[jid].S : S0;
+                    const float3 c = BATCH ? jobs[jid].R.cpos : Wv.cpos;
                     const float4 o = first ? make_float4(c.x, c.y, c.z, 0.0f) : Wv.ray_o[cur][i];
                     RayPre r = ray_pre(mk(o), mk(d), S.plane_bound);
                     float tfar = __int_as_float(0x7f800000);
@@ -661,13 +654,16 @@ __device__ __forceinline__ float mean3(f3 v) { return (v.x + v.y + v.z) * (1.0f 
 
 template <int MODE, bool BATCH>
 __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kShadeBlock)
-    shade_kernel(SceneDev S0, RenderDev R0, const JobDev* __restrict__ jobs, WaveDev Wv, int cur, trg::GuideView G)
+    shade_kernel(SceneDev S0, RenderDev R0, const JobDev* __restrict__ jobs, WaveDev Wv, int cur_level, trg::GuideView G)
 {
     static_assert(!(BATCH && MODE == kShadeGuided), "guided renders take one job");
     constexpr bool GUIDED = MODE == kShadeGuided;
     __shared__ uint32_t scan[kShadeBlock / 64 + 2];
     __shared__ float glds[GUIDED ? (kShadeBlockGuided / 64) * 64 * trg::kRow : 1];
     __shared__ uint4 gfrag[GUIDED ? trg::kFwdFrags * 64 : 1];
+    const int cur = cur_level & 1;
+    const uint32_t level = uint32_t(cur_level >> 1);  // of every path of the launch
+    const uint64_t wave_base = Wv.ctl->base;
     const uint32_t count = Wv.counters[qword(cur)];
     if (blockIdx.x == 0 && threadIdx.x < kParts) Wv.counters[part_word(threadIdx.x, P_FETCH_EXT)] = 0;  // for the next extend
     if (blockIdx.x * blockDim.x >= count) return;  // no paths for this block (the last bounces' launches)
@@ -682,45 +678,56 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
         const uint32_t i = base + threadIdx.x;
         bool live = i < count;
         const float4 d4 = live ? Wv.ray_d[cur][i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        // batched renders: the path's job; otherwise its index in the wavefront
-        const uint32_t slot = __float_as_uint(d4.w);
-        const uint32_t jid = BATCH ? slot : 0u;
+        const uint32_t slot = __float_as_uint(d4.w);  // the path's index in its wavefront
+        uint4 st = {};
+        if (live && (BATCH || level > 0)) st = Wv.st[cur][i];
+        const uint32_t jid = BATCH ? st.y >> 16 : 0u;
         const SceneDev& S = BATCH ? jobs[jid].S : S0;
         const RenderDev& R = BATCH ? jobs[jid].R : R0;
         bool emit_shadow = false, cont = false, want = false;
         float4 sh_o = {}, sh_d = {}, sh_c = {};
         float4 n_o = {}, n_d = {}, n_thr = {};
-        uint4 n_misc = {}, n_extra = {};
         uint32_t sh_tag = 0xFFFFFFFFu, tag = 0xFFFFFFFFu;
         // state of a vertex that goes on to sample a direction
         f3 f = {}, pos = {}, n = {}, d = {};
         bool medium_event = false, two_sided = false;
         int32_t mat = -1;
         float pi = 1.0f, time = 0.0f, nsampled = 0.0f;
-        uint64_t pst = 0, nst = 0, pinc = 0;
-        uint4 misc = {}, extra = {};
+        uint64_t pst = 0, pinc = 0, pid = 0;
+        uint32_t nee = 0;    // light-stream draws
+        float uw = 0.0f;     // unwarp distance
         if (live) {
-            misc = Wv.misc[cur][i];
-            extra = Wv.extra[cur][i];
             float2 h = Wv.hit[i];
             int32_t tri = __float_as_int(h.y);
-            uint32_t level = extra.z & 0xFFu;
-            // a camera ray starts at the camera with unit throughput; extra.w holds its sampled
-            // free-flight distance until the unwarp distance replaces it below
-            const float4 o4 = level == 0 ? make_float4(R.cpos.x, R.cpos.y, R.cpos.z, __uint_as_float(extra.w))
-                                         : Wv.ray_o[cur][i];
-            const float4 thr = level == 0 ? make_float4(1.0f, 1.0f, 1.0f, 0.0f) : Wv.thr[cur][i];
-            f3 o = mk(o4);
+            const float lam = R.time_sampling ? R.ts_lambda : S.lambda;  // NextEventSampling::Time / MeanFreePath
+            const uint32_t pid_local = uint32_t(wave_base + slot - (BATCH ? jobs[jid].path_begin : 0ull));
+            pid = R.pid0 + pid_local;
+            pinc = pcg_inc(2 * pid);
+            f3 o = mk(R.cpos.x, R.cpos.y, R.cpos.z);
+            float4 thr = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
+            float sampled = __int_as_float(0x7f800000);
+            if (level == 0) {
+                // a camera ray: unit throughput, the path stream at its seed
+                pst = pcg_seed(R.seed, 2 * pid);
+                if (S.has_medium) sampled = free_flight(pcg_float(pst, pinc), lam);
+                if (!BATCH) st.x = pid_local / (uint32_t(R.n_inc) * uint32_t(R.spp2));
+                if (R.unwarp) uw = tri >= 0 ? h.x : 3.402823466e+38f;
+            } else {
+                const float4 o4 = Wv.ray_o[cur][i];
+                o = mk(o4);
+                sampled = o4.w;
+                thr = Wv.thr[cur][i];
+                pst = u64(st.z, st.w);
+                nee = st.y & 0xFFFFu;
+                if (R.unwarp) uw = Wv.uw[cur][i];
+            }
             d = mk(d4);
-            float sampled = o4.w;
-            if (level == 0 && R.unwarp) extra.w = __float_as_uint(tri >= 0 ? h.x : 3.402823466e+38f);
             if constexpr (GUIDED) {
                 if (slot % G.stride == 0u && slot / G.stride < G.train_paths) tag = (slot / G.stride) * G.max_levels;
             }
             // correct_next_event_distance (BidirectionalPathTracing.h:275-307)
             float dist, pd = 1.0f;
             bool alive = true;
-            const float lam = R.time_sampling ? R.ts_lambda : S.lambda;  // NextEventSampling::Time / MeanFreePath
             if (!S.has_medium) {
                 alive = tri >= 0;
                 dist = h.x;
@@ -749,14 +756,14 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                     if (mat & kMatSmooth) n = smooth_normal(S.tri_vn + 6 * size_t(tri), pos);
                     mat &= kMatIndex;
                 }
-                nst = u64(extra.x, extra.y);
-                uint64_t pid = u64(misc.x, misc.y);
-                uint64_t ninc = pcg_inc(2 * pid + 1);
-                pinc = pcg_inc(2 * pid);
+                // the light stream (sequence 2 pid + 1) after `nee` draws
+                const uint64_t ninc = pcg_inc(2 * pid + 1);
+                uint64_t nst = pcg_at(R.seed, ninc, nee);
                 // ---- next-event estimation at this vertex (connect_paths :976-1045,
                 //      connect_vertex_with_light :650-692)
                 if (int(level) + 1 <= R.max_bounces && time <= R.total_time) {
                     float u = pcg_float(nst, ninc);
+                    ++nee;
                     int li = min(int(u * float(S.n_lights)), S.n_lights - 1);
                     const LightHost& L = S.lights[li];
                     int type = int(L.I[3]);
@@ -774,6 +781,7 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                         irr = mk(L.I[0] * att, L.I[1] * att, L.I[2] * att);
                     } else {
                         float uu = pcg_float(nst, ninc), vv = pcg_float(nst, ninc);
+                        nee += 2;
                         lp = mk(L.pos[0], L.pos[1], L.pos[2]) + mk(L.left[0], L.left[1], L.left[2]) * uu +
                              mk(L.up[0], L.up[1], L.up[2]) * vv;
                         f3 v = pos - lp;
@@ -803,7 +811,7 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                         float scale = R.inv_inc / (pl2 / float(S.n_lights));
                         f3 val = mul(mul(f, fe), mul(irr, att)) * scale;
                         float ts = ldist + time;
-                        float cam_time = R.unwarp ? ts - __uint_as_float(extra.w) : ts;
+                        float cam_time = R.unwarp ? ts - uw : ts;
                         float sensor = (cam_time - R.offset) / R.exposure;
                         bool finite = isfinite(val.x) && isfinite(val.y) && isfinite(val.z);
                         bool nonzero = val.x != 0.0f || val.y != 0.0f || val.z != 0.0f;
@@ -815,21 +823,21 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                             const uint32_t layer = min(level, uint32_t(R.layers - 1));
                             uint32_t fidx = 0xFFFFFFFFu;
                             if (in_window)
-                                fidx = layer * R.layer_stride + (extra.z >> 8) * uint32_t(R.T) +
+                                fidx = layer * R.layer_stride + st.x * uint32_t(R.T) +
                                        min(uint32_t(floorf(sensor)), uint32_t(R.T - 1));
                             if (!finite) val = mk(0.0f, 0.0f, 0.0f);  // TransientRenderer.h:167-171
                             emit_shadow = true;
                             sh_o = make_float4(lp.x, lp.y, lp.z, ldist);
                             sh_d = make_float4(ldir.x, ldir.y, ldir.z, __uint_as_float(fidx));
-                            sh_c = make_float4(val.x, val.y, val.z, __uint_as_float(extra.z >> 8));
+                            sh_c = make_float4(val.x, val.y, val.z, __uint_as_float(st.x));
                             sh_tag = ((slot / uint32_t(R.n_inc)) << kMaxLayersTagBits) | layer;
                         } else if (in_window && finite && nonzero) {
                             uint32_t bin = min(uint32_t(floorf(sensor)), uint32_t(R.T - 1));
-                            uint32_t fidx = (extra.z >> 8) * uint32_t(R.T) + bin;
+                            uint32_t fidx = st.x * uint32_t(R.T) + bin;
                             emit_shadow = true;
                             sh_o = make_float4(lp.x, lp.y, lp.z, ldist);
                             sh_d = make_float4(ldir.x, ldir.y, ldir.z, __uint_as_float(fidx));
-                            sh_c = make_float4(val.x, val.y, val.z, __uint_as_float(extra.z >> 8));
+                            sh_c = make_float4(val.x, val.y, val.z, __uint_as_float(st.x));
                             if (GUIDED && tag != 0xFFFFFFFFu) sh_tag = tag + level;
                         }
                     }
@@ -838,7 +846,6 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                 //      film window; otherwise Russian roulette on the mean albedo, or in the
                 //      Transient mode the film's time length alone (TotalTime) (:447-481)
                 if (int(level) + 1 < R.max_bounces && time <= R.total_time) {
-                    pst = u64(misc.z, misc.w);
                     float albedo = medium_event ? S.medium_albedo : S.mats[mat].w;
                     float eps = R.time_sampling ? 0.0f : pcg_float(pst, pinc);
                     if (!(eps > albedo)) {
@@ -887,7 +894,7 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                 if (medium_event) {
                     bool timed = false;
                     if (R.time_sampling) {
-                        const f3 tg = light_target(S, R.seed, u64(misc.x, misc.y));
+                        const f3 tg = light_target(S, R.seed, pid);
                         f3 l;
                         float modl;
                         {
@@ -967,8 +974,7 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                 n_o = make_float4(pos.x, pos.y, pos.z, nsampled);
                 n_d = make_float4(nd.x, nd.y, nd.z, d4.w);
                 n_thr = make_float4(nf.x, nf.y, nf.z, time);
-                n_misc = make_uint4(misc.x, misc.y, uint32_t(pst), uint32_t(pst >> 32));
-                n_extra = make_uint4(uint32_t(nst), uint32_t(nst >> 32), extra.z + 1u, extra.w);
+                st = make_uint4(st.x, nee | (jid << 16), uint32_t(pst), uint32_t(pst >> 32));
             }
         }
         uint32_t q_pos, sh_pos;
@@ -984,8 +990,8 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
             Wv.ray_o[cur ^ 1][q_pos] = n_o;
             Wv.ray_d[cur ^ 1][q_pos] = n_d;
             Wv.thr[cur ^ 1][q_pos] = n_thr;
-            Wv.misc[cur ^ 1][q_pos] = n_misc;
-            Wv.extra[cur ^ 1][q_pos] = n_extra;
+            Wv.st[cur ^ 1][q_pos] = st;
+            if (R.unwarp) Wv.uw[cur ^ 1][q_pos] = uw;
         }
     }
 }
@@ -1483,7 +1489,8 @@ static uint32_t stack_flags_of(int fmt)
 struct WaveBuffers {
     uint32_t cap = 0;
     float4 *ray_o[2] = {}, *ray_d[2] = {}, *thr[2] = {};
-    uint4 *misc[2] = {}, *extra[2] = {};
+    uint4* st[2] = {};
+    float* uw[2] = {};  // allocated by the first render with camera unwarp
     float2* hit = nullptr;
     float4 *sh_o = nullptr, *sh_d = nullptr, *sh_c = nullptr;
     uint8_t* sh_vis = nullptr;
@@ -1503,7 +1510,7 @@ struct WaveBuffers {
     void release()
     {
         for (int b = 0; b < 2; ++b) {
-            dev_free(ray_o[b]); dev_free(ray_d[b]); dev_free(thr[b]); dev_free(misc[b]); dev_free(extra[b]);
+            dev_free(ray_o[b]); dev_free(ray_d[b]); dev_free(thr[b]); dev_free(st[b]); dev_free(uw[b]);
         }
         dev_free(hit); dev_free(sh_o); dev_free(sh_d); dev_free(sh_c); dev_free(sh_vis); dev_free(counters);
         dev_free(sh_tag); dev_free(sh_job); dev_free(ctl); dev_free(d_jobs); dev_free(cs_bits);
@@ -1547,6 +1554,13 @@ struct WaveBuffers {
         }
         return TR_OK;
     }
+    int ensure_unwarp()
+    {
+        int rc;
+        for (int b = 0; b < 2; ++b)
+            if (!uw[b] && cap && (rc = dev_alloc(&uw[b], cap))) return rc;
+        return TR_OK;
+    }
     int ensure_tags()
     {
         if (sh_tag || cap == 0) return TR_OK;
@@ -1559,7 +1573,7 @@ struct WaveBuffers {
         int rc;
         for (int b = 0; b < 2; ++b)
             if ((rc = dev_alloc(&ray_o[b], n)) || (rc = dev_alloc(&ray_d[b], n)) || (rc = dev_alloc(&thr[b], n)) ||
-                (rc = dev_alloc(&misc[b], n)) || (rc = dev_alloc(&extra[b], n))) {
+                (rc = dev_alloc(&st[b], n))) {
                 release();
                 return rc;
             }
@@ -1576,7 +1590,7 @@ struct WaveBuffers {
     {
         WaveDev w;
         for (int b = 0; b < 2; ++b) {
-            w.ray_o[b] = ray_o[b]; w.ray_d[b] = ray_d[b]; w.thr[b] = thr[b]; w.misc[b] = misc[b]; w.extra[b] = extra[b];
+            w.ray_o[b] = ray_o[b]; w.ray_d[b] = ray_d[b]; w.thr[b] = thr[b]; w.st[b] = st[b]; w.uw[b] = uw[b];
         }
         w.hit = hit;
         w.sh_o = sh_o; w.sh_d = sh_d; w.sh_c = sh_c; w.sh_vis = sh_vis; w.sh_tag = sh_tag;
@@ -2500,6 +2514,7 @@ int make_job(tr_scene s, const tr_camera* cam, tr_film f, const tr_render_desc* 
     R.ts_lambda = 4.0f / (float(fd.time_bins) * fd.exposure / 1.0f / 1.0f);
     R.inv_inc = float(1. / double(float(d->n_incoming)));
     R.unwarp = fd.camera_unwarp ? 1 : 0;
+    R.pid0 = uint64_t(R.row0) * uint64_t(R.W) * spp2 * uint64_t(R.n_inc);
     R.max_bounces = d->max_bounces;
     R.cpos = make_float3(cam->position[0], cam->position[1], cam->position[2]);
     R.nv = make_float3(nv[0], nv[1], nv[2]);
@@ -2648,15 +2663,15 @@ struct Launch {
             if ((rc = begin(TR_K_SHADE))) return rc;
             if (batch) {
                 if (c.mode == kShadeOnb)
-                    shade_kernel<kShadeOnb, true><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur, GV);
+                    shade_kernel<kShadeOnb, true><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur | (b << 1), GV);
                 else
-                    shade_kernel<kShadeRef, true><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur, GV);
+                    shade_kernel<kShadeRef, true><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur | (b << 1), GV);
             } else if (c.mode == kShadeGuided) {
-                shade_kernel<kShadeGuided, false><<<sg, kShadeBlockGuided, 0, stream>>>(S0, R0, dj, Wv, cur, GV);
+                shade_kernel<kShadeGuided, false><<<sg, kShadeBlockGuided, 0, stream>>>(S0, R0, dj, Wv, cur | (b << 1), GV);
             } else if (c.mode == kShadeOnb) {
-                shade_kernel<kShadeOnb, false><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur, GV);
+                shade_kernel<kShadeOnb, false><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur | (b << 1), GV);
             } else {
-                shade_kernel<kShadeRef, false><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur, GV);
+                shade_kernel<kShadeRef, false><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur | (b << 1), GV);
             }
             if ((rc = end())) return rc;
             if ((rc = begin(TR_K_SHADOW))) return rc;
@@ -2732,6 +2747,8 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     }
     int rc = wb.ensure(c.wave);
     if (rc) return rc;
+    for (auto& j : jobs)
+        if (j.dev.R.unwarp && (rc = wb.ensure_unwarp())) return rc;
     if (mb) {
         const uint32_t ncs = c.wave / uint32_t(jobs[0].dev.R.n_inc);
         if ((rc = wb.ensure_tags()) || (rc = wb.ensure_cs(ncs))) return rc;
