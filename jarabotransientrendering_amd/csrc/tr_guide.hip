@@ -19,6 +19,7 @@
 #include "tr_guide.h"
 #include "tr_guide_host.h"
 #include "tr_internal.h"
+#include "tr_readback.h"
 
 using namespace trg;
 
@@ -620,7 +621,6 @@ struct tr_guide_s {
     size_t rec_cap = 0, tp_cap = 0;
     float4* grad_rec = nullptr;  // records of tr_guide_gradient (at most batch_size)
     uint32_t grad_cap = 0;
-    float* h_out = nullptr;      // pinned: a gradient and its loss
     trg::GuideView view{};
     uint64_t steps = 0, records = 0;
     double train_ms = 0.0;
@@ -637,7 +637,6 @@ struct tr_guide_s {
         release_render();
         gfree(master), gfree(m), gfree(v), gfree(bias), gfree(fwd), gfree(bwd), gfree(partial), gfree(partial_loss);
         gfree(part2), gfree(loss2), gfree(count), gfree(wsum), gfree(grad_rec);
-        if (h_out) (void)hipHostFree(h_out);
         for (auto& e : ev)
             if (e) (void)hipEventDestroy(e);
         if (stream) (void)hipStreamDestroy(stream);
@@ -785,11 +784,6 @@ int tr_guide_create(tr_guide* out, const tr_guide_desc* d)
         (rc = galloc(&g->part2, size_t(kReduceSlices) * kParams)) || (rc = galloc(&g->loss2, kReduceSlices)) ||
         (rc = galloc(&g->count, 4)) || (rc = galloc(&g->wsum, 4)))
         return bail(rc);
-    if (hipHostMalloc(reinterpret_cast<void**>(&g->h_out), (kParams + 1) * sizeof(float), hipHostMallocDefault) !=
-        hipSuccess) {
-        g->h_out = nullptr;
-        return bail(tri::fail(TR_ERR_NOMEM, "tr_guide_create: hipHostMalloc"));
-    }
     std::vector<float> p = initial_params(D.init_seed);
     if ((rc = tr_guide_set_params(g, p.data()))) return bail(rc);
     *out = g;
@@ -913,13 +907,15 @@ int tr_guide_gradient(tr_guide g, const float* records, uint32_t n, float* grad,
     const uint32_t tg = train_grid(n);
     train_kernel<<<tg, kTrainBlock, 0, g->stream>>>(T);
     GHIP_TRY(hipGetLastError());
-    grad_kernel<<<(kParams + kGradCols) / kGradCols, kGradCols * kGradRows, 0, g->stream>>>(g->partial, g->partial_loss, tg,
-                                                                                          n, g->part2);
-    GHIP_TRY(hipGetLastError());
-    GHIP_TRY(hipMemcpyAsync(g->h_out, g->part2, (kParams + 1) * sizeof(float), hipMemcpyDeviceToHost, g->stream));
-    GHIP_TRY(hipStreamSynchronize(g->stream));
-    std::memcpy(grad, g->h_out, kParams * sizeof(float));
-    if (loss) *loss = g->h_out[kParams];
+    std::vector<float> out(kParams + 1);  // the gradient, then the loss
+    const hipError_t e = trb::read_back(out.data(), out.size() * sizeof(float), [&](hipStream_t stream, void* dst, size_t, size_t) {
+        grad_kernel<<<(kParams + kGradCols) / kGradCols, kGradCols * kGradRows, 0, stream>>>(
+            g->partial, g->partial_loss, tg, n, static_cast<float*>(dst));
+        return hipGetLastError();
+    }, g->stream);
+    if (e != hipSuccess) return tri::fail(TR_ERR_DEVICE, std::string("tr_guide_gradient: ") + hipGetErrorString(e));
+    std::memcpy(grad, out.data(), kParams * sizeof(float));
+    if (loss) *loss = out[kParams];
     return TR_OK;
 }
 
@@ -942,9 +938,10 @@ int tr_guide_train_batch(tr_guide g, const float* records, uint32_t n, float* lo
     GHIP_TRY(hipGetLastError());
     int rc = g->train(g->stream, 1);
     if (rc) return rc;
-    GHIP_TRY(hipMemcpyAsync(g->h_out, g->wsum, 2 * sizeof(float), hipMemcpyDeviceToHost, g->stream));
+    float lv[2];
+    GHIP_TRY(hipMemcpyAsync(lv, g->wsum, sizeof lv, hipMemcpyDeviceToHost, g->stream));
     GHIP_TRY(hipStreamSynchronize(g->stream));
-    if (loss) *loss = g->h_out[1];
+    if (loss) *loss = lv[1];
     g->records += n;
     return TR_OK;
 }

@@ -36,6 +36,7 @@
 #include "tr_guide.h"
 #include "tr_guide_host.h"
 #include "tr_internal.h"
+#include "tr_readback.h"
 
 using namespace trd;
 
@@ -1259,30 +1260,92 @@ __global__ void __launch_bounds__(kBlock) film_batch_kernel(const JobDev* __rest
 }
 
 // ---------------------------------------------------------------------------------------------
-// film read-back: one block per pixel writes (sum + comp) / weight of its T x RGB bins (0/0 -> 0,
-// ImageRow::weight, Image.h:153-162) in double precision, and the pixel's steady value (the sum
-// over its bins) for the steady image (StreakCameraFilm.h:369-397)
+// film read-back. The weight of a pixel: one for all of them (films that only renders added to), one
+// per pixel, or one per pixel of each bounce film.
+struct FilmWeight {
+    double same;
+    const double* pixel;
+    const float* layer;
+    __device__ __forceinline__ double at(size_t p) const { return pixel ? pixel[p] : layer ? double(layer[p]) : same; }
+};
+// (sum + comp) / weight (0/0 -> 0, ImageRow::weight, Image.h:153-162) in double precision, rounded
+// (StreakCameraFilm.h:369-397)
+__device__ __forceinline__ void film_value(float s, float c, double w, float* o)
+{
+    const double v = (double(s) + double(c)) / w;
+    *o = isfinite(v) ? float(v) : 0.0f;
+}
+// or the compensated sum itself
+__device__ __forceinline__ void film_value(float s, float c, double, double* o) { *o = double(s) + double(c); }
+
+// `n` values from element 0 of `sum` / `comp` (at bin `j0` of pixel `p0`) on, written to pinned host memory;
+// bound by PCIe (50 GB/s). Four values per thread (16-byte stores); `vec`: sum and comp are 16-byte
+// aligned and can be read so.
+constexpr uint32_t kValuesPerBlock = 1024;
+template <class Out>
+__global__ void __launch_bounds__(kValuesPerBlock / 4) film_values_kernel(const float* __restrict__ sum,
+                                                                          const float* __restrict__ comp, FilmWeight weight,
+                                                                          size_t p0, uint32_t j0, uint32_t T3, uint32_t n,
+                                                                          bool vec, Out* __restrict__ out)
+{
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) * 4u;
+    if (i < n) {
+        const uint64_t q = uint64_t(j0) + i;
+        size_t p = p0 + q / T3;
+        uint32_t j = uint32_t(q % T3);
+        float s[4], c[4];
+        if (vec && i + 4u <= n) {
+            const float4 a = *reinterpret_cast<const float4*>(sum + i), b = *reinterpret_cast<const float4*>(comp + i);
+            s[0] = a.x, s[1] = a.y, s[2] = a.z, s[3] = a.w;
+            c[0] = b.x, c[1] = b.y, c[2] = b.z, c[3] = b.w;
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < 4; ++k) {
+                s[k] = i + k < n ? sum[i + k] : 0.0f;
+                c[k] = i + k < n ? comp[i + k] : 0.0f;
+            }
+        }
+        double w = weight.at(p);
+        struct alignas(16) Four {
+            Out v[4];
+        } r;
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            film_value(s[k], c[k], w, &r.v[k]);
+            if (++j == T3) {
+                j = 0;
+                ++p;
+                if (k < 3 && i + k + 1 < n) w = weight.at(p);
+            }
+        }
+        Out* o = out + i;
+        if (i + 4u <= n) {
+            *reinterpret_cast<Four*>(o) = r;
+        } else {
+            for (uint32_t k = 0; i + k < n; ++k) o[k] = r.v[k];
+        }
+    }
+}
+
+// the steady image (StreakCameraFilm.h:369-397): one block per pixel sums its T x RGB values
 constexpr int kNormBlock = 256;
-__global__ void __launch_bounds__(kNormBlock) film_normalize_kernel(const float* __restrict__ sum,
-                                                                   const float* __restrict__ comp,
-                                                                   const double* __restrict__ weight, uint32_t T3,
-                                                                   float* __restrict__ out, float* __restrict__ steady)
+__global__ void __launch_bounds__(kNormBlock) film_steady_kernel(const float* __restrict__ sum,
+                                                                const float* __restrict__ comp, FilmWeight weight,
+                                                                size_t p0, uint32_t T3, float* __restrict__ steady)
 {
     __shared__ double part[kNormBlock / 64][3];
     const size_t p = blockIdx.x;
-    const double w = weight[p];
+    const double w = weight.at(p0 + p);
     double acc[3] = {0.0, 0.0, 0.0};
     for (uint32_t j = threadIdx.x; j < T3; j += kNormBlock) {
         const size_t i = p * T3 + j;
         double v = (double(sum[i]) + double(comp[i])) / w;
         if (!isfinite(v)) v = 0.0;
-        if (out) out[i] = float(v);
         const uint32_t k = j % 3u;
         acc[0] += k == 0 ? v : 0.0;
         acc[1] += k == 1 ? v : 0.0;
         acc[2] += k == 2 ? v : 0.0;
     }
-    if (!steady) return;
 #pragma unroll
     for (int k = 0; k < 3; ++k)
         for (int off = 32; off > 0; off >>= 1) acc[k] += __shfl_xor(acc[k], off);
@@ -1678,10 +1741,10 @@ struct tr_film_s {
     size_t n_elems = 0;  // max(layers, 1) * rows*W*T*3
     float *d_sum = nullptr, *d_comp = nullptr;        // compensated sums: sum + comp = film
     float *d_layer_w = nullptr, *d_steady = nullptr;  // multibounce films only (steady: sums, then comps)
-    float *d_read = nullptr, *d_read_steady = nullptr;  // read-back staging (allocated by the first read)
-    size_t read_cap = 0;                                // floats d_read holds
-    double* d_read_w = nullptr;
-    std::vector<double> weight;  // rows*W
+    float* d_read_steady = nullptr;  // steady image on its way to the host (allocated by the first read of one)
+    double* d_read_w = nullptr;      // per-pixel weights, uploaded by reads of films with caller-made samples
+    std::vector<double> weight;      // rows*W
+    bool same_weight = true;         // every pixel has the same weight (no caller-made samples)
     hipStream_t stream = nullptr;
 };
 
@@ -2194,7 +2257,7 @@ int tr_film_destroy(tr_film f)
     if (!f) return TR_OK;
     if (f->stream) (void)hipStreamSynchronize(f->stream);
     dev_free(f->d_sum); dev_free(f->d_comp); dev_free(f->d_layer_w); dev_free(f->d_steady);
-    dev_free(f->d_read); dev_free(f->d_read_steady); dev_free(f->d_read_w);
+    dev_free(f->d_read_steady); dev_free(f->d_read_w);
     if (f->stream) (void)hipStreamDestroy(f->stream);
     delete f;
     return TR_OK;
@@ -2213,18 +2276,43 @@ int tr_film_clear(tr_film f)
     }
     HIP_TRY(hipStreamSynchronize(f->stream));
     std::fill(f->weight.begin(), f->weight.end(), 0.0);
+    f->same_weight = true;
     return TR_OK;
 }
+
+}  // extern "C"
+
+namespace {
+
+// values of the film's elements [first, first + n) (n > 0) into the host array `out`: normalised (float) or
+// the compensated sums (double). Every entry point that writes a film returns after its work has completed,
+// so the staging's streams can read it.
+template <class Out>
+int film_values(tr_film f, size_t first, size_t n, const FilmWeight& w, Out* out)
+{
+    static_assert(trb::kChunk % (4 * sizeof(Out)) == 0, "chunks hold whole groups of four values");
+    const uint32_t T3 = 3u * uint32_t(f->desc.time_bins);
+    const hipError_t e = trb::read_back(out, n * sizeof(Out), [&](hipStream_t stream, void* dst, size_t at, size_t size) {
+        const size_t i = first + at / sizeof(Out);
+        const uint32_t m = uint32_t(size / sizeof(Out));
+        film_values_kernel<Out><<<(m + kValuesPerBlock - 1) / kValuesPerBlock, kValuesPerBlock / 4, 0, stream>>>(
+            f->d_sum + i, f->d_comp + i, w, i / T3, uint32_t(i % T3), T3, m, i % 4 == 0, static_cast<Out*>(dst));
+        return hipGetLastError();
+    });
+    if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string("tr_film_read: ") + hipGetErrorString(e));
+    return TR_OK;
+}
+
+}  // namespace
+
+extern "C" {
 
 int tr_film_read_sums(tr_film f, double* sums, double* weights)
 {
     if (!f) return fail(TR_ERR_INVALID, "tr_film_read_sums: null film");
     if (sums) {
-        std::vector<float> s(f->n_elems), c(f->n_elems);
-        HIP_TRY(hipMemcpyAsync(s.data(), f->d_sum, f->n_elems * sizeof(float), hipMemcpyDeviceToHost, f->stream));
-        HIP_TRY(hipMemcpyAsync(c.data(), f->d_comp, f->n_elems * sizeof(float), hipMemcpyDeviceToHost, f->stream));
-        HIP_TRY(hipStreamSynchronize(f->stream));
-        for (size_t i = 0; i < f->n_elems; ++i) sums[i] = double(s[i]) + double(c[i]);
+        const int rc = film_values(f, 0, f->n_elems, FilmWeight{}, sums);
+        if (rc) return rc;
     }
     if (weights) {
         if (f->layers) {
@@ -2247,31 +2335,25 @@ int tr_film_read_rows(tr_film f, int32_t row_begin, int32_t row_count, float* ou
     if (row_begin < 0 || row_count < 0 || row_begin + int64_t(row_count) > f->rows)
         return fail(TR_ERR_INVALID, "tr_film_read_rows: rows outside the film");
     if ((!out && !steady) || row_count == 0) return TR_OK;
-    const size_t W = size_t(f->desc.width), T = size_t(f->desc.time_bins), P = size_t(f->rows) * W;
-    const size_t p0 = size_t(row_begin) * W, np = size_t(row_count) * W, n = np * T * 3;
-    // normalised on the device; one copy of the result instead of both raw arrays
+    const size_t W = size_t(f->desc.width), T3 = size_t(f->desc.time_bins) * 3, P = size_t(f->rows) * W;
+    const size_t p0 = size_t(row_begin) * W, np = size_t(row_count) * W;
     int rc;
-    if (!f->d_read_w && (rc = dev_alloc(&f->d_read_w, P))) return rc;
-    if (out && f->read_cap < n) {
-        dev_free(f->d_read);
-        f->read_cap = 0;
-        if ((rc = dev_alloc(&f->d_read, n))) return rc;
-        f->read_cap = n;
+    FilmWeight w{f->weight[0], nullptr, nullptr};
+    if (!f->same_weight) {
+        if (!f->d_read_w && (rc = dev_alloc(&f->d_read_w, P))) return rc;
+        HIP_TRY(hipMemcpyAsync(f->d_read_w, f->weight.data(), P * sizeof(double), hipMemcpyHostToDevice, f->stream));
+        HIP_TRY(hipStreamSynchronize(f->stream));  // the upload reads f->weight asynchronously
+        w.pixel = f->d_read_w;
     }
     if (steady && !f->d_read_steady && (rc = dev_alloc(&f->d_read_steady, P * 3))) return rc;
-    HIP_TRY(hipMemcpyAsync(f->d_read_w, f->weight.data(), P * sizeof(double), hipMemcpyHostToDevice, f->stream));
-    film_normalize_kernel<<<uint32_t(np), kNormBlock, 0, f->stream>>>(f->d_sum + p0 * T * 3, f->d_comp + p0 * T * 3,
-                                                                     f->d_read_w + p0, uint32_t(3 * T),
-                                                                     out ? f->d_read : nullptr,
-                                                                     steady ? f->d_read_steady : nullptr);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && out) e = hipMemcpyAsync(out, f->d_read, n * sizeof(float), hipMemcpyDeviceToHost, f->stream);
-    if (e == hipSuccess && steady)
-        e = hipMemcpyAsync(steady, f->d_read_steady, np * 3 * sizeof(float), hipMemcpyDeviceToHost, f->stream);
-    // the weight upload reads f->weight asynchronously: always wait
-    const hipError_t se = hipStreamSynchronize(f->stream);
-    if (e == hipSuccess) e = se;
-    if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string("tr_film_read: ") + hipGetErrorString(e));
+    if (out && (rc = film_values(f, p0 * T3, np * T3, w, out))) return rc;
+    if (steady) {
+        film_steady_kernel<<<uint32_t(np), kNormBlock, 0, f->stream>>>(f->d_sum + p0 * T3, f->d_comp + p0 * T3, w, p0,
+                                                                      uint32_t(T3), f->d_read_steady);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipMemcpyAsync(steady, f->d_read_steady, np * 3 * sizeof(float), hipMemcpyDeviceToHost, f->stream));
+        HIP_TRY(hipStreamSynchronize(f->stream));
+    }
     return TR_OK;
 }
 
@@ -2279,37 +2361,23 @@ int tr_film_read(tr_film f, float* out, float* steady)
 {
     if (!f) return fail(TR_ERR_INVALID, "tr_film_read: null film");
     if (!out && !steady) return TR_OK;
-    const size_t W = size_t(f->desc.width), T = size_t(f->desc.time_bins), P = size_t(f->rows) * W;
     if (!f->layers) return tr_film_read_rows(f, 0, f->rows, out, steady);
-    std::vector<float> s(f->n_elems), c(f->n_elems);
-    HIP_TRY(hipMemcpyAsync(s.data(), f->d_sum, f->n_elems * sizeof(float), hipMemcpyDeviceToHost, f->stream));
-    HIP_TRY(hipMemcpyAsync(c.data(), f->d_comp, f->n_elems * sizeof(float), hipMemcpyDeviceToHost, f->stream));
-    HIP_TRY(hipStreamSynchronize(f->stream));
-    {
-        // multibounce films: each bounce film divided by its own weights; the steady image holds
-        // every sample
-        std::vector<float> lw(size_t(f->layers) * P), st(P * 6);
-        HIP_TRY(hipMemcpyAsync(lw.data(), f->d_layer_w, lw.size() * sizeof(float), hipMemcpyDeviceToHost, f->stream));
+    // multibounce films: each bounce film divided by its own weights; the steady image holds every
+    // sample
+    int rc;
+    if (out && (rc = film_values(f, 0, f->n_elems, FilmWeight{0.0, nullptr, f->d_layer_w}, out))) return rc;
+    if (steady) {
+        const size_t P = f->weight.size();
+        std::vector<float> st(P * 6);
         HIP_TRY(hipMemcpyAsync(st.data(), f->d_steady, st.size() * sizeof(float), hipMemcpyDeviceToHost, f->stream));
         HIP_TRY(hipStreamSynchronize(f->stream));
-        if (out)
-            for (size_t l = 0; l < size_t(f->layers); ++l)
-                for (size_t p = 0; p < P; ++p) {
-                    double w = lw[l * P + p];
-                    for (size_t t = 0; t < T * 3; ++t) {
-                        size_t i = ((l * P + p) * T) * 3 + t;
-                        double v = (double(s[i]) + double(c[i])) / w;
-                        out[i] = std::isfinite(v) ? float(v) : 0.0f;
-                    }
-                }
-        if (steady)
-            for (size_t p = 0; p < P; ++p)
-                for (int k = 0; k < 3; ++k) {
-                    double v = (double(st[p * 3 + size_t(k)]) + double(st[(P + p) * 3 + size_t(k)])) / f->weight[p];
-                    steady[p * 3 + size_t(k)] = std::isfinite(v) ? float(v) : 0.0f;
-                }
-        return TR_OK;
+        for (size_t p = 0; p < P; ++p)
+            for (size_t k = 0; k < 3; ++k) {
+                const double v = (double(st[p * 3 + k]) + double(st[(P + p) * 3 + k])) / f->weight[p];
+                steady[p * 3 + k] = std::isfinite(v) ? float(v) : 0.0f;
+            }
     }
+    return TR_OK;
 }
 
 int tr_film_write(tr_film f, const char* name, const char* ext)
@@ -2439,6 +2507,7 @@ int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
     if (e == hipSuccess) e = se;
     release();
     if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string("tr_film_add_samples: ") + hipGetErrorString(e));
+    f->same_weight = false;
     for (size_t p = 0; p < wadd.size(); ++p) f->weight[p] += wadd[p];
     return TR_OK;
 }
