@@ -1137,12 +1137,24 @@ constexpr uint32_t kFilmMaxSlots = 8;
 constexpr int kFilmRounds = 2;
 static_assert(kFilmRange <= uint32_t(kFilmBlock), "one record of a range per thread");
 
-template <bool GUIDED>
-__global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev Wv, int sh, uint32_t pix_slots, float* contrib)
+// Where the contributions come from: a render's shadow records, those of a guided render (whose
+// contributions are also credited to training records), or samples that the caller made.
+enum { kFilmRender = 0, kFilmGuided = 1, kFilmSamples = 2 };
+struct SamplesDev {
+    const tr_film_sample* samples;
+    uint32_t n;
+    const uint32_t* bad;  // index of the first sample outside the film (~0: none): then nothing is added
+};
+
+template <int SRC>
+__global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev Wv, int sh, uint32_t pix_slots,
+                                                          float* contrib, SamplesDev Q)
 {
+    constexpr bool GUIDED = SRC == kFilmGuided;
     extern __shared__ double hist[];         // pix_slots * T * 3 partials
     __shared__ uint32_t slot_pix[kFilmMaxSlots];
-    const uint32_t count = Wv.counters[shword(sh)];
+    const uint32_t count = SRC == kFilmSamples ? Q.n : Wv.counters[shword(sh)];
+    if (SRC == kFilmSamples && *Q.bad != 0xFFFFFFFFu) return;
     // guided renders: ranges of 256 records, about one append chunk of the guided shading kernel's
     // 256-thread blocks, so a range spans fewer pixels (guided passes' film time -11 %)
     constexpr uint32_t kRange = GUIDED ? 256u : kFilmRange;
@@ -1157,7 +1169,16 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
         bool pending = false;
         float4 c = {};
         uint32_t pix = 0, bin = 0;
-        if (threadIdx.x < kRange && r < count && Wv.sh_vis[r]) {
+        if constexpr (SRC == kFilmSamples) {
+            if (threadIdx.x < kRange && r < count) {
+                const tr_film_sample q = Q.samples[r];
+                const float sensor = (q.time - R.offset) / R.exposure;
+                c = make_float4(q.rgb[0], q.rgb[1], q.rgb[2], 0.0f);
+                pix = uint32_t(q.y - R.row0) * uint32_t(R.W) + uint32_t(q.x);
+                pending = sensor < float(T) && sensor >= 0.0f;
+                bin = pending ? min(uint32_t(floorf(sensor)), T - 1u) : 0u;
+            }
+        } else if (threadIdx.x < kRange && r < count && Wv.sh_vis[r]) {
             c = Wv.sh_c[r];
             if constexpr (GUIDED) {
                 // luminance of the contribution, credited to the training record of its vertex
@@ -1205,6 +1226,27 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
             }
             __syncthreads();
         }
+    }
+}
+
+// caller-made samples before they are deposited: the first one outside the film (of `rows` rows), and
+// each pixel's added weight
+__global__ void __launch_bounds__(kBlock) samples_begin_kernel(double* __restrict__ weight, uint32_t pixels, uint32_t* bad)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < pixels) weight[i] = 0.0;
+    if (i == 0) *bad = 0xFFFFFFFFu;
+}
+__global__ void __launch_bounds__(kBlock) samples_check_kernel(const tr_film_sample* __restrict__ samples, uint32_t n,
+                                                               int32_t W, int32_t row0, int32_t rows,
+                                                               double* __restrict__ weight, uint32_t* bad)
+{
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const int2 at = *reinterpret_cast<const int2*>(samples + i);
+        const int32_t row = int32_t(uint32_t(at.y) - uint32_t(row0));
+        if (at.x < 0 || at.x >= W || row < 0 || row >= rows) atomicMin(bad, i);
+        else if (samples[i].weight != 0.0f)
+            unsafeAtomicAdd(weight + size_t(row) * size_t(W) + size_t(at.x), double(samples[i].weight));
     }
 }
 
@@ -1742,7 +1784,10 @@ struct tr_film_s {
     float *d_sum = nullptr, *d_comp = nullptr;        // compensated sums: sum + comp = film
     float *d_layer_w = nullptr, *d_steady = nullptr;  // multibounce films only (steady: sums, then comps)
     float* d_read_steady = nullptr;  // steady image on its way to the host (allocated by the first read of one)
-    double* d_read_w = nullptr;      // per-pixel weights, uploaded by reads of films with caller-made samples
+    double* d_read_w = nullptr;      // per-pixel weights: uploaded by reads of films with caller-made samples,
+                                     // summed by tr_film_add_samples
+    tr_film_sample* d_samples = nullptr;  // caller-made samples being added, behind a 256-byte head (first bad index)
+    size_t samples_cap = 0;
     std::vector<double> weight;      // rows*W
     bool same_weight = true;         // every pixel has the same weight (no caller-made samples)
     hipStream_t stream = nullptr;
@@ -2257,7 +2302,7 @@ int tr_film_destroy(tr_film f)
     if (!f) return TR_OK;
     if (f->stream) (void)hipStreamSynchronize(f->stream);
     dev_free(f->d_sum); dev_free(f->d_comp); dev_free(f->d_layer_w); dev_free(f->d_steady);
-    dev_free(f->d_read_steady); dev_free(f->d_read_w);
+    dev_free(f->d_samples); dev_free(f->d_read_steady); dev_free(f->d_read_w);
     if (f->stream) (void)hipStreamDestroy(f->stream);
     delete f;
     return TR_OK;
@@ -2432,9 +2477,10 @@ int tr_film_device_buffers(tr_film f, float** d_sum, float** d_comp)
     return TR_OK;
 }
 
-// StreakCameraFilm::add_samples for caller-made samples: binned on the host as the reference bins
-// (pos_sensor = (time - offset) / exposure, kept if 0 <= pos_sensor < T; StreakCameraFilm.h:165-171),
-// then deposited by the renders' own film kernel from shadow-record-shaped staging buffers.
+// StreakCameraFilm::add_samples for caller-made samples: checked, binned as the reference bins
+// (pos_sensor = (time - offset) / exposure, kept if 0 <= pos_sensor < T; StreakCameraFilm.h:165-171) and
+// deposited on the device, by the renders' own film kernel. (Binned on the host into shadow-record
+// arrays, 500,000 samples took 1.5 ms on one thread and 0.6 ms of allocations and extra copies.)
 int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
 {
     if (!f) return fail(TR_ERR_INVALID, "tr_film_add_samples: null film");
@@ -2443,70 +2489,59 @@ int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
     if (!samples) return fail(TR_ERR_INVALID, "tr_film_add_samples: null samples");
     if (n > (1u << 31)) return fail(TR_ERR_INVALID, "tr_film_add_samples: more than 2^31 samples in one call");
     const tr_film_desc& fd = f->desc;
-    const uint32_t W = uint32_t(fd.width), T = uint32_t(fd.time_bins);
-    const int row0 = fd.scanline >= 0 ? fd.scanline : 0;
-    std::vector<float4> hc(n), hd(n);
-    std::vector<uint8_t> hv(n);
-    std::vector<double> wadd(f->weight.size(), 0.0);
-    auto bits = [](uint32_t u) {
-        float v;
-        std::memcpy(&v, &u, sizeof v);
-        return v;
-    };
-    for (uint32_t i = 0; i < n; ++i) {
-        const tr_film_sample& q = samples[i];
-        const int row = q.y - row0;
-        if (q.x < 0 || uint32_t(q.x) >= W || row < 0 || row >= f->rows)
-            return fail(TR_ERR_INVALID, "tr_film_add_samples: sample " + std::to_string(i) + " lies outside the film");
-        const uint32_t pix = uint32_t(row) * W + uint32_t(q.x);
-        wadd[pix] += double(q.weight);
-        const float sensor = (q.time - fd.offset) / fd.exposure;
-        const bool in_window = sensor < float(T) && sensor >= 0.0f;
-        const uint32_t bin = in_window ? std::min(uint32_t(std::floor(sensor)), T - 1u) : 0u;
-        hc[i] = make_float4(q.rgb[0], q.rgb[1], q.rgb[2], bits(pix));
-        hd[i] = make_float4(0.0f, 0.0f, 0.0f, bits(pix * T + bin));
-        hv[i] = in_window ? 1 : 0;
-    }
-    float4 *dc = nullptr, *dd = nullptr;
-    uint8_t* dv = nullptr;
-    uint32_t* dcount = nullptr;
-    auto release = [&]() {
-        dev_free(dc); dev_free(dd); dev_free(dv); dev_free(dcount);
-    };
+    const uint32_t T = uint32_t(fd.time_bins), P = uint32_t(f->weight.size());
+    const int32_t row0 = fd.scanline >= 0 ? fd.scanline : 0;
+    constexpr size_t kHead = 256 / sizeof(tr_film_sample), kKept = size_t(32) << 20;  // samples buffers up to 32 MiB are kept
     int rc;
-    if ((rc = dev_alloc(&dc, n)) || (rc = dev_alloc(&dd, n)) || (rc = dev_alloc(&dv, n)) || (rc = dev_alloc(&dcount, C_WORDS))) {
-        release();
-        return rc;
+    if (!f->d_read_w && (rc = dev_alloc(&f->d_read_w, P))) return rc;
+    if (f->samples_cap < n) {
+        dev_free(f->d_samples);
+        f->samples_cap = 0;
+        if ((rc = dev_alloc(&f->d_samples, kHead + n))) return rc;
+        f->samples_cap = n;
     }
-    uint32_t counts[C_WORDS] = {};
-    counts[shword(0)] = n;
+    uint32_t* bad = reinterpret_cast<uint32_t*>(f->d_samples);
+    tr_film_sample* d = f->d_samples + kHead;
     RenderDev R{};
     R.film = f->d_sum;
     R.film_comp = f->d_comp;
     R.W = fd.width;
     R.H = fd.height;
     R.T = fd.time_bins;
-    WaveDev Wv{};
-    Wv.sh_c = dc;
-    Wv.sh_d = dd;
-    Wv.sh_vis = dv;
-    Wv.counters = dcount;
+    R.row0 = row0;
+    R.offset = fd.offset;
+    R.exposure = fd.exposure;
     const uint32_t pix_slots = std::min<uint32_t>(kFilmMaxSlots, kFilmLdsBytes / (T * 24u));
     const size_t lds = size_t(pix_slots) * size_t(T) * 24u;
-    const uint32_t fg = std::max(1u, std::min((n + kFilmRange - 1) / kFilmRange, uint32_t(tri::compute_units()) * 4u));
-    hipError_t e = hipMemcpyAsync(dc, hc.data(), size_t(n) * sizeof(float4), hipMemcpyHostToDevice, f->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dd, hd.data(), size_t(n) * sizeof(float4), hipMemcpyHostToDevice, f->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dv, hv.data(), size_t(n), hipMemcpyHostToDevice, f->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dcount, counts, sizeof counts, hipMemcpyHostToDevice, f->stream);
+    const uint32_t cu = uint32_t(tri::compute_units());
+    const uint32_t fg = std::max(1u, std::min((n + kFilmRange - 1) / kFilmRange, cu * 4u));
+    samples_begin_kernel<<<(P + kBlock - 1) / kBlock, kBlock, 0, f->stream>>>(f->d_read_w, P, bad);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(d, samples, size_t(n) * sizeof(tr_film_sample), hipMemcpyHostToDevice, f->stream);
     if (e == hipSuccess) {
-        film_kernel<false><<<fg, kFilmBlock, lds, f->stream>>>(R, Wv, 0, pix_slots, nullptr);
+        samples_check_kernel<<<std::min((n + kBlock - 1) / kBlock, cu * 16u), kBlock, 0, f->stream>>>(d, n, fd.width, row0,
+                                                                                                   f->rows, f->d_read_w, bad);
+        film_kernel<kFilmSamples><<<fg, kFilmBlock, lds, f->stream>>>(R, WaveDev{}, 0, pix_slots, nullptr, SamplesDev{d, n, bad});
         e = hipGetLastError();
     }
-    // the staging vectors above are read by the copies: wait before they go out of scope
+    std::vector<double> wadd(P);
+    uint32_t first_bad = 0xFFFFFFFFu;
+    if (e == hipSuccess) e = hipMemcpyAsync(&first_bad, bad, sizeof first_bad, hipMemcpyDeviceToHost, f->stream);
+    // the copies read the caller's samples and write this frame's variables: wait in any case
     const hipError_t se = hipStreamSynchronize(f->stream);
     if (e == hipSuccess) e = se;
-    release();
+    if (e == hipSuccess && first_bad == 0xFFFFFFFFu) {
+        e = trb::read_back(wadd.data(), P * sizeof(double), [&](hipStream_t stream, void* dst, size_t at, size_t size) {
+            return hipMemcpyAsync(dst, reinterpret_cast<const char*>(f->d_read_w) + at, size, hipMemcpyDeviceToHost, stream);
+        });
+    }
+    if (f->samples_cap * sizeof(tr_film_sample) > kKept) {
+        dev_free(f->d_samples);
+        f->samples_cap = 0;
+    }
     if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string("tr_film_add_samples: ") + hipGetErrorString(e));
+    if (first_bad != 0xFFFFFFFFu)
+        return fail(TR_ERR_INVALID, "tr_film_add_samples: sample " + std::to_string(first_bad) + " lies outside the film");
     f->same_weight = false;
     for (size_t p = 0; p < wadd.size(); ++p) f->weight[p] += wadd[p];
     return TR_OK;
@@ -2752,9 +2787,9 @@ struct Launch {
             else if (R0.layers > 0)
                 film_mb_kernel<<<std::max(1u, std::min((wave + kBlock - 1) / kBlock, cu * 16u)), kBlock, 0, stream>>>(R0, Wv, cur ^ 1);
             else if (guide)
-                film_kernel<true><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, cur ^ 1, pix_slots, GV.contrib);
+                film_kernel<kFilmGuided><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, cur ^ 1, pix_slots, GV.contrib, SamplesDev{});
             else
-                film_kernel<false><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, cur ^ 1, pix_slots, nullptr);
+                film_kernel<kFilmRender><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, cur ^ 1, pix_slots, nullptr, SamplesDev{});
             if ((rc = end())) return rc;
             cur ^= 1;
         }

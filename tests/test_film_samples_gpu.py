@@ -1,0 +1,59 @@
+"""Caller-made samples checked, binned and deposited on the device (tr_film_add_samples), at the edges of
+the film kernel's 512-record ranges and of the kept sample buffer (32 MiB, 1,048,576 samples)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _samples(n, w, rows, row0, seed):
+    from jarabotransientrendering_amd import renderer
+    rng = np.random.default_rng(seed)
+    a = np.zeros(n, renderer.nat.FILM_SAMPLE_DTYPE)
+    a["x"], a["y"] = rng.integers(0, w, n), row0 + rng.integers(0, rows, n)
+    a["time"], a["rgb"], a["weight"] = rng.uniform(-1.0, 12.0, n), rng.normal(size=(n, 3)), rng.integers(0, 3, n) * 0.5
+    return a
+
+
+@pytest.mark.parametrize("scanline", [False, True])
+@pytest.mark.parametrize("n", [1, 511, 512, 513, 20011, (1 << 20) + 1])
+def test_samples_land_in_their_bins(n, scanline):
+    from jarabotransientrendering_amd import renderer
+    w, h, t = 13, 7, 97
+    film = renderer.StreakCameraFilm(w, h, t, 0.1)
+    film.set_offset(0.5)
+    if scanline:
+        film.set_streak(4)
+    rows, row0 = (1, 4) if scanline else (h, 0)
+    a = _samples(n, w, rows, row0, n)
+    film.add_samples(a)
+    film.add_samples(a[: n // 2 + 1])  # a second call into the same film and buffer
+    a = np.concatenate([a, a[: n // 2 + 1]])
+    sums, weight = film.read_sums()
+    sensor = (a["time"] - np.float32(0.5)) / np.float32(0.1)
+    inside = (sensor >= 0) & (sensor < t)
+    at = (a["y"][inside] - row0, a["x"][inside], np.floor(sensor[inside]).astype(int))
+    ref, mag = np.zeros((rows, w, t, 3)), np.zeros((rows, w, t, 3))
+    np.add.at(ref, at, a["rgb"][inside].astype(np.float64))
+    np.add.at(mag, at, np.abs(a["rgb"][inside].astype(np.float64)))
+    # the film's bound: 2 u of the magnitudes (u = 2^-24), and n u^2 far below it
+    assert (np.abs(sums - ref) <= 2.0 ** -22 * mag).all()
+    ref_w = np.zeros((rows, w))
+    np.add.at(ref_w, (a["y"] - row0, a["x"]), a["weight"].astype(np.float64))
+    assert np.array_equal(weight, ref_w)  # halves add exactly
+
+
+@pytest.mark.parametrize("field,value", [("x", -1), ("x", 13), ("y", -1), ("y", 7), ("y", -(1 << 31)), ("x", (1 << 31) - 1)])
+@pytest.mark.parametrize("at", [0, 1023, 20010])
+def test_a_sample_outside_the_film_adds_nothing(field, value, at):
+    from jarabotransientrendering_amd import _native as nat, renderer
+    film = renderer.StreakCameraFilm(13, 7, 97, 0.1)
+    a = _samples(20011, 13, 7, 0, 1)
+    film.add_samples(a[:100])
+    before = film.read_sums()
+    a[field][at] = value
+    a[field][20010] = value
+    with pytest.raises(nat.TrError, match=f"sample {at} lies outside the film"):
+        film.add_samples(a)
+    after = film.read_sums()
+    assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
