@@ -45,7 +45,19 @@ namespace {
 constexpr int kTraceBlock = 128;   // traversal kernels: 128 threads, STACK ints of LDS each
 constexpr int kBlock = 256;        // other kernels
 constexpr int kShadeBlock = 1024;  // shade: one queue atomic per 1024 paths
-constexpr uint32_t kDefaultWave = 1u << 25;
+// Paths per wavefront: the launches of a wavefront's last bounces hold few rays each and run at the
+// length of their longest query (100-190 us on the 82k-triangle scene), so fewer, larger wavefronts are
+// faster: a 67 M-path frame takes 20.7 ms in one wavefront, 22.2 in two, 24.0 in four, 27.2 in eight.
+constexpr uint32_t kDefaultWave = 1u << 26;
+// Shadow records a wavefront may collect before they are traced and deposited, for the same reason:
+// with room for them, the shadow rays of several bounces share one shadow and one film launch. All of
+// a media scanline's 16 bounces together: shadow 0.33 -> 0.15 ms, film 0.44 -> 0.23 ms per pass (1.75 ->
+// 1.41 ms in all); a 67 M-path frame in wavefronts of 2^25: 24.3 ms with one bounce per launch,
+// 23.3 with two, 22.6 with four, 22.1 with all eight.
+constexpr uint32_t kShadowRecords = 1u << 28;
+// Device memory of the two: wavefronts of more than kSmallWave paths and groups of bounces are made
+// smaller where their buffers would take more than a quarter of the free memory.
+constexpr uint32_t kSmallWave = 1u << 25;
 constexpr uint32_t kFetchMax = 512;  // rays per work fetch of a traversal wavefront (upper bound)
 constexpr uint32_t kTraceRaysPerThread = 8;   // lower bound on a full wavefront's rays per traversal thread
 constexpr uint32_t kTraceMinPerCu = 4;        // traversal blocks per CU below which that bound yields
@@ -79,8 +91,8 @@ constexpr uint32_t kParts = 8;
 constexpr uint32_t kPartBase = 64;
 constexpr uint32_t kPartWords = 64;
 // Queue lengths come in two 64-bit pairs, one per record buffer k: (rays of buffer k, shadow
-// rays made from the paths of the other buffer), so that shade appends to both of its output
-// queues with one atomic.
+// records: those carried over from earlier bounces and those made from the paths of the other
+// buffer), so that shade appends to both of its output queues with one atomic.
 enum {
     C_Q0 = 0,                                            // pairs: words 2k (rays), 2k + 1 (shadow rays)
     C_STAT_EXT = 4, C_STAT_SHADOW = 6,                   // 64-bit statistics
@@ -376,11 +388,12 @@ __global__ void __launch_bounds__(kTraceBlock, 7) extend_kernel(SceneDev S0, con
     __shared__ uint32_t stack[stack_words<TRAV, STACK>() * kTraceBlock];
     const int cur = cur_first & 1;
     const bool first = (cur_first & 2) != 0;  // camera rays: the origin is the camera's
+    const bool carry = (cur_first & 4) != 0;  // earlier bounces' shadow records are still in the queue
     const uint32_t count = Wv.counters[qword(cur)];
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid == 0) {
         Wv.counters[qword(cur ^ 1)] = 0;
-        Wv.counters[shword(cur ^ 1)] = 0;
+        Wv.counters[shword(cur ^ 1)] = carry ? Wv.counters[shword(cur)] : 0u;
         atomicAdd(reinterpret_cast<unsigned long long*>(Wv.counters + C_STAT_EXT), (unsigned long long)count);
     }
     if (gid < kParts) Wv.counters[part_word(gid, P_FETCH_SHADOW)] = 0;
@@ -453,12 +466,13 @@ template <int TRAV, int STACK>
 __global__ void __launch_bounds__(kTraceBlock, 7) extend_camera_kernel(SceneDev S0, WaveDev Wv, int cur)
 {
     static_assert(TRAV == kTravWide || TRAV == kTravWide16 || TRAV == kTravWideKeyed, "4-wide stacks");
+    constexpr bool carry = false;
     __shared__ uint32_t stack[stack_words<TRAV, STACK>() * kTraceBlock];
     const uint32_t count = Wv.counters[qword(cur)];
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid == 0) {
         Wv.counters[qword(cur ^ 1)] = 0;
-        Wv.counters[shword(cur ^ 1)] = 0;
+        Wv.counters[shword(cur ^ 1)] = carry ? Wv.counters[shword(cur)] : 0u;
         atomicAdd(reinterpret_cast<unsigned long long*>(Wv.counters + C_STAT_EXT), (unsigned long long)count);
     }
     if (gid < kParts) Wv.counters[part_word(gid, P_FETCH_SHADOW)] = 0;
@@ -1592,7 +1606,7 @@ static uint32_t stack_flags_of(int fmt)
 }
 
 struct WaveBuffers {
-    uint32_t cap = 0;
+    uint32_t cap = 0, sh_cap = 0;  // path records, shadow records
     float4 *ray_o[2] = {}, *ray_d[2] = {}, *thr[2] = {};
     uint4* st[2] = {};
     float* uw[2] = {};  // allocated by the first render with camera unwarp
@@ -1622,6 +1636,7 @@ struct WaveBuffers {
         if (h_jobs) (void)hipHostFree(h_jobs);
         h_jobs = nullptr;
         cap = 0;
+        sh_cap = 0;
         jobs_cap = 0;
         cs_cap = 0;
     }
@@ -1637,7 +1652,7 @@ struct WaveBuffers {
     int ensure_batch(uint32_t n_jobs)
     {
         int rc;
-        if (!sh_job && cap && (rc = dev_alloc(&sh_job, cap))) return rc;
+        if (!sh_job && sh_cap && (rc = dev_alloc(&sh_job, sh_cap))) return rc;
         if (n_jobs + 1 > jobs_cap) {
             // an earlier upload from the pinned table may still be queued (a render that failed
             // before its final synchronisation): drain the device before freeing it
@@ -1668,12 +1683,31 @@ struct WaveBuffers {
     }
     int ensure_tags()
     {
-        if (sh_tag || cap == 0) return TR_OK;
-        return dev_alloc(&sh_tag, cap);
+        if (sh_tag || sh_cap == 0) return TR_OK;
+        return dev_alloc(&sh_tag, sh_cap);
     }
-    int ensure(uint32_t n)
+    // device bytes of n path records and n_sh shadow records (with every optional array)
+    static uint64_t bytes(uint64_t n, uint64_t n_sh)
     {
-        if (n <= cap) return TR_OK;
+        return n * (2 * (3 * sizeof(float4) + sizeof(uint4) + sizeof(float)) + sizeof(float2)) +
+               n_sh * (3 * sizeof(float4) + sizeof(uint8_t) + 2 * sizeof(uint32_t));
+    }
+    // makes `group` bounces per shadow launch and then `wave` (whole units of paths) smaller until
+    // their buffers fit a quarter of the device memory that is free or held by this object
+    void fit(uint32_t& wave, uint32_t& group, uint32_t unit) const
+    {
+        if (wave <= cap && uint64_t(wave) * group <= sh_cap) return;
+        size_t free_bytes = 0, total_bytes = 0;
+        if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) return;
+        const uint64_t room = (uint64_t(free_bytes) + bytes(cap, sh_cap)) / 4;
+        while (group > 1 && bytes(wave, uint64_t(wave) * group) > room) group = (group + 1) / 2;
+        while (wave > kSmallWave && wave / 2 >= unit && bytes(wave, wave) > room) wave = wave / 2 / unit * unit;
+    }
+    int ensure(uint32_t n, uint32_t n_sh)
+    {
+        if (n <= cap && n_sh <= sh_cap) return TR_OK;
+        n = std::max(n, cap);
+        n_sh = std::max(n_sh, sh_cap);
         release();
         int rc;
         for (int b = 0; b < 2; ++b)
@@ -1682,13 +1716,14 @@ struct WaveBuffers {
                 release();
                 return rc;
             }
-        if ((rc = dev_alloc(&hit, n)) || (rc = dev_alloc(&sh_o, n)) ||
-            (rc = dev_alloc(&sh_d, n)) || (rc = dev_alloc(&sh_c, n)) || (rc = dev_alloc(&sh_vis, n)) ||
+        if ((rc = dev_alloc(&hit, n)) || (rc = dev_alloc(&sh_o, n_sh)) ||
+            (rc = dev_alloc(&sh_d, n_sh)) || (rc = dev_alloc(&sh_c, n_sh)) || (rc = dev_alloc(&sh_vis, n_sh)) ||
             (rc = dev_alloc(&counters, C_WORDS)) || (rc = dev_alloc(&ctl, 1))) {
             release();
             return rc;
         }
         cap = n;
+        sh_cap = n_sh;
         return TR_OK;
     }
     WaveDev view() const
@@ -2659,6 +2694,7 @@ struct Launch {
     hipEvent_t* ev;
     bool batch;
     int bounces;
+    int group;  // bounces whose shadow rays are traced and deposited together
     int stack_bound;
     int trav_ext, trav_sh;  // kTrav* of the closest-hit and any-hit launches
     uint32_t pix_slots;
@@ -2761,7 +2797,7 @@ struct Launch {
                 else TR_CAMERA_DISPATCH_T(kTravWideKeyed, stack_bound, tg, kTraceBlock, stream, S0, Wv, cur);
             } else {
                 TR_TRACE_DISPATCH(trav_ext, stack_bound, batch, extend_kernel, tg, kTraceBlock, stream, S0, dj, Wv,
-                                  cur | (b == 0 ? 2 : 0));
+                                  cur | (b == 0 ? 2 : 0) | (b % group != 0 ? 4 : 0));
             }
             if ((rc = end())) return rc;
             if ((rc = begin(TR_K_SHADE))) return rc;
@@ -2778,6 +2814,10 @@ struct Launch {
                 shade_kernel<kShadeRef, false><<<sg, kShadeBlock, 0, stream>>>(S0, R0, dj, Wv, cur | (b << 1), GV);
             }
             if ((rc = end())) return rc;
+            if ((b + 1) % group != 0 && b + 1 < bounces) {
+                cur ^= 1;
+                continue;
+            }
             if ((rc = begin(TR_K_SHADOW))) return rc;
             TR_TRACE_DISPATCH(trav_sh, stack_bound, batch, shadow_kernel, tg, kTraceBlock, stream, S0, dj, Wv, cur ^ 1);
             if ((rc = end())) return rc;
@@ -2849,7 +2889,10 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
         const uint32_t ni = uint32_t(jobs[0].dev.R.n_inc);
         c.wave = mb_wave(c.wave, ni);
     }
-    int rc = wb.ensure(c.wave);
+    // bounces whose shadow rays one launch takes
+    uint32_t group = std::max(1u, std::min(uint32_t(std::max(bounces, 1)), kShadowRecords / c.wave));
+    wb.fit(c.wave, group, guide ? c.wave : mb ? uint32_t(jobs[0].dev.R.n_inc) : 1u);
+    int rc = wb.ensure(c.wave, c.wave * group);
     if (rc) return rc;
     for (auto& j : jobs)
         if (j.dev.R.unwarp && (rc = wb.ensure_unwarp())) return rc;
@@ -2869,6 +2912,7 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     L.ev = ev;
     L.batch = batch;
     L.bounces = bounces;
+    L.group = int(group);
     L.stack_bound = stack_bound;
     L.trav_ext = trav_ext;
     L.trav_sh = trav_sh;
@@ -2975,7 +3019,8 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
             }
             // count the kernels each replay runs
             L.launches[TR_K_CAMERA] += 1;
-            for (int k : {TR_K_EXTEND, TR_K_SHADE, TR_K_SHADOW, TR_K_FILM}) L.launches[k] += uint32_t(bounces);
+            for (int k : {TR_K_EXTEND, TR_K_SHADE}) L.launches[k] += uint32_t(bounces);
+            for (int k : {TR_K_SHADOW, TR_K_FILM}) L.launches[k] += (uint32_t(bounces) + group - 1) / group;
             if (mb) L.launches[TR_K_FILM] += 1;
             hipError_t le = hipGraphLaunch(exec, stream);
             if (le != hipSuccess) {
@@ -3028,6 +3073,7 @@ int render_impl(tr_scene s, const tr_camera* cam, tr_film f, const tr_render_des
     if (rc) return rc;
     LaunchCfg c = s->tune;
     if (d->wave_paths) c.wave = d->wave_paths;
+    else if (guide && c.wave == kDefaultWave) c.wave = kSmallWave;  // (a guide trains after each wavefront)
     c.wide = (d->flags & TR_RENDER_BINARY_BVH) == 0;
     c.graph = (d->flags & TR_RENDER_GRAPH) != 0;
     c.prof = (d->flags & (TR_RENDER_PROFILE | TR_RENDER_PROFILE_EXTEND)) != 0;
