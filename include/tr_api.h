@@ -284,7 +284,8 @@ enum {
 };
 
 enum {
-    /* TR_K_FILM_MERGE: no longer launched (films accumulate compensated sums directly); kept so the
+    /* wavefronts of few paths run all bounces and their shadow rays in one launch, counted as EXTEND.
+     * TR_K_FILM_MERGE: no longer launched (films accumulate compensated sums directly); kept so the
      * statistics layout does not change */
     TR_K_CAMERA = 0, TR_K_EXTEND = 1, TR_K_SHADE = 2, TR_K_SHADOW = 3, TR_K_FILM_MERGE = 4, TR_K_FILM = 5,
     TR_K_GUIDE = 6, /* guided renders: training-record bookkeeping and Adam steps */

@@ -12,6 +12,7 @@
 //     shadow_kernel               occlusion of every shadow ray             (World::intersects)
 //     film_kernel                 visible contributions binned into the
 //                                 film's compensated FP32 (sum, comp) pairs (StreakCameraFilm.h:139-192)
+// A wavefront of few paths runs camera, bounces and shadow rays in one launch (path_kernel), then film_kernel.
 //
 // Path state lives in HBM as structure-of-arrays float4/uint4 records in two buffers: the rays of
 // bounce k are records [0, count) of buffer k & 1, and shade writes the paths that continue,
@@ -58,6 +59,16 @@ constexpr uint32_t kShadowRecords = 1u << 28;
 // Device memory of the two: wavefronts of more than kSmallWave paths and groups of bounces are made
 // smaller where their buffers would take more than a quarter of the free memory.
 constexpr uint32_t kSmallWave = 1u << 25;
+// Largest wavefronts whose bounces run in one launch (path_kernel) instead of two per bounce. A render of
+// 2^10 paths through the two: 163 and 84 us (22 triangles), 642 and 363 (81,930 triangles), 370 and 183 (a
+// medium, 16 bounces); of 2^18 paths 200 and 100, 1,074 and 586, 540 and 224; of 2^20 paths 303 and 219,
+// 1,476 and 1,210, 933 and 530; and 751 and 746 with 1,290 triangles, where longer queues win from here on
+// (2^21 paths: 948 and 1,337). In a medium over a shallow tree, where a path has many vertices and a ray's
+// length hardly varies, the launch still wins with 2^22 paths (2,183 and 1,640; 2^24: 6,833 and 6,213).
+constexpr uint32_t kPathWave = 1u << 20;
+constexpr uint32_t kPathWaveMedium = 1u << 22;
+constexpr uint32_t kShallowNodes = 64;  // 4-wide nodes of a shallow tree
+constexpr int kPathRefill = 8;  // idle lanes that begin new paths (24: 2 % slower in a medium)
 constexpr uint32_t kFetchMax = 512;  // rays per work fetch of a traversal wavefront (upper bound)
 constexpr uint32_t kTraceRaysPerThread = 8;   // lower bound on a full wavefront's rays per traversal thread
 constexpr uint32_t kTraceMinPerCu = 4;        // traversal blocks per CU below which that bound yields
@@ -100,7 +111,7 @@ enum {
 };
 __host__ __device__ constexpr uint32_t qword(int k) { return uint32_t(2 * k); }
 __host__ __device__ constexpr uint32_t shword(int k) { return uint32_t(2 * k + 1); }
-enum { P_FETCH_EXT = 0, P_FETCH_SHADOW = 1, P_STAT_CONTRIB = 2 };  // words of a partition (P_STAT_CONTRIB: 64-bit)
+enum { P_FETCH_EXT = 0, P_FETCH_SHADOW = 1, P_STAT_CONTRIB = 2, P_STAT_EXT = 4, P_STAT_SHADOW = 6 };  // words of a partition (P_STAT_*: 64-bit)
 __host__ __device__ constexpr uint32_t part_word(uint32_t part, uint32_t w) { return kPartBase + part * kPartWords + w; }
 
 struct SceneDev {
@@ -163,6 +174,10 @@ struct WaveDev {
     uint8_t* sh_vis;  // 1 if the shadow ray is unoccluded
     uint32_t* sh_tag; // guided renders: training record of the contribution (or ~0)
     uint32_t* sh_job; // batched renders: job of each shadow record
+    // path launches: GPU wavefront w runs seg_paths paths, from w * seg_paths on, and their shadow records are
+    // w * seg_cap + j for j below seg_n[w] (seg_cap = 0: the records are one queue, whose length is a counter)
+    uint32_t* seg_n;
+    uint32_t seg_cap, seg_paths;
     struct WaveCtl* ctl;
     uint32_t* counters;
     float3 cpos;      // single-job renders: camera position (batched renders: their job's R.cpos)
@@ -209,37 +224,23 @@ __device__ __forceinline__ f3 point_on_ray(f3 o, f3 d, float t)
     return mk(o.x + d.x * t, o.y + d.y * t, o.z + d.z * t);
 }
 
-// ---------------------------------------------------------------------------------------------
-// camera: one thread per path of the wavefront
-template <bool BATCH>
-__global__ void __launch_bounds__(kBlock) camera_kernel(SceneDev S0, RenderDev R0, const JobDev* __restrict__ jobs,
-                                                        uint32_t n_jobs, WaveDev Wv)
+// the last job whose first path is <= the global path index
+__device__ __forceinline__ uint32_t job_of(const JobDev* __restrict__ jobs, uint32_t n_jobs, uint64_t gidx)
 {
-    const WaveCtl ctl = *Wv.ctl;
-    const uint32_t n = ctl.n;
-    uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot == 0) Wv.counters[C_Q0] = n;
-    if (slot < kParts) Wv.counters[part_word(slot, P_FETCH_EXT)] = 0;
-    if (slot >= n) return;
-    // a job holds fewer than 2^32 paths: 32-bit index arithmetic within the job
-    uint32_t jid = 0, pid_local;
-    if constexpr (BATCH) {
-        // job of this path: the last job whose first path is <= the global path index
-        const uint64_t gidx = ctl.base + slot;
-        uint32_t lo = 0, hi = n_jobs;
-        while (hi - lo > 1u) {
-            uint32_t mid = (lo + hi) >> 1;
-            if (jobs[mid].path_begin <= gidx) lo = mid;
-            else hi = mid;
-        }
-        jid = lo;
-        pid_local = uint32_t(gidx - jobs[lo].path_begin);
-    } else {
-        pid_local = uint32_t(ctl.base) + slot;
+    uint32_t lo = 0, hi = n_jobs;
+    while (hi - lo > 1u) {
+        uint32_t mid = (lo + hi) >> 1;
+        if (jobs[mid].path_begin <= gidx) lo = mid;
+        else hi = mid;
     }
-    const RenderDev& R = BATCH ? jobs[jid].R : R0;
+    return lo;
+}
+
+// direction of the camera ray of a job's path (fewer than 2^32: 32-bit index arithmetic) and its film pixel
+__device__ __forceinline__ f3 camera_ray(const RenderDev& R, uint32_t pid_local, uint32_t& pix_local)
+{
     uint32_t cs_local = pid_local / uint32_t(R.n_inc);
-    uint32_t pix_local = cs_local / uint32_t(R.spp2);   // film pixel (row relative)
+    pix_local = cs_local / uint32_t(R.spp2);   // film pixel (row relative)
     uint32_t sub = cs_local - pix_local * uint32_t(R.spp2);
     uint32_t rowl = pix_local / uint32_t(R.W);
     uint32_t xr = pix_local - rowl * uint32_t(R.W);
@@ -259,8 +260,26 @@ __global__ void __launch_bounds__(kBlock) camera_kernel(SceneDev S0, RenderDev R
     float ic1 = (py - R.yw2) / float(R.H) / R.ratio;
     f3 nv = mk(R.nv.x, R.nv.y, R.nv.z), uv = mk(R.uv.x, R.uv.y, R.uv.z), vv = mk(R.vv.x, R.vv.y, R.vv.z);
     f3 dir = nv * R.fd + uv * (2.0f * ic0) - vv * (2.0f * ic1);
-    dir = normalize(normalize(dir));  // get_ray_direction normalises, Ray3D normalises again
+    return normalize(normalize(dir));  // get_ray_direction normalises, Ray3D normalises again
+}
 
+// ---------------------------------------------------------------------------------------------
+// camera: one thread per path of the wavefront
+template <bool BATCH>
+__global__ void __launch_bounds__(kBlock) camera_kernel(SceneDev S0, RenderDev R0, const JobDev* __restrict__ jobs,
+                                                        uint32_t n_jobs, WaveDev Wv)
+{
+    const WaveCtl ctl = *Wv.ctl;
+    const uint32_t n = ctl.n;
+    uint32_t slot = blockIdx.x * blockDim.x + threadIdx.x;
+    if (slot == 0) Wv.counters[C_Q0] = n;
+    if (slot < kParts) Wv.counters[part_word(slot, P_FETCH_EXT)] = 0;
+    if (slot >= n) return;
+    const uint64_t gidx = ctl.base + slot;
+    const uint32_t jid = BATCH ? job_of(jobs, n_jobs, gidx) : 0u;
+    const uint32_t pid_local = BATCH ? uint32_t(gidx - jobs[jid].path_begin) : uint32_t(gidx);
+    uint32_t pix_local;
+    const f3 dir = camera_ray(BATCH ? jobs[jid].R : R0, pid_local, pix_local);
     Wv.ray_d[0][slot] = make_float4(dir.x, dir.y, dir.z, __uint_as_float(slot));
     if constexpr (BATCH) Wv.st[0][slot] = make_uint4(pix_local, jid << 16, 0u, 0u);
 }
@@ -296,6 +315,11 @@ constexpr int stack_kind() { return TRAV == kTravWide ? kStack32 : TRAV == kTrav
 // fetch cursor) and hands them to its idle lanes in lane order. Call with every lane of the
 // wavefront; `rec` is the queue entry of the lane's query, kIdle if it has none.
 constexpr uint32_t kIdle = 0xFFFFFFFFu;
+// lanes of `mask` below this one
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), 0u));
+}
 // idle lanes that trigger a refill (unless the whole wavefront is idle): closest-hit and any-hit launches
 // (with camera rays in their own packet kernel, 16 and 32 for either were 0.2-0.7 % slower than 24)
 constexpr int kRefillMinExtend = 24;
@@ -366,7 +390,7 @@ struct RayRefill {
                 end = uint32_t(min(b + chunk, uint64_t(count)));
             }
             const uint32_t avail = end - pos;
-            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(uint32_t(idle >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(idle), 0u));
+            const uint32_t rank = lanes_below(idle);
             if (rec == kIdle && take == kIdle && rank < avail) take = pos + rank;
             pos += min(uint32_t(__popcll(idle)), avail);
             idle = __ballot(rec == kIdle && take == kIdle);
@@ -657,6 +681,216 @@ __device__ __forceinline__ f3 light_target(const SceneDev& S, uint64_t seed, uin
     return p;
 }
 
+// A path's vertex: what sampling its next direction needs.
+struct Vertex {
+    f3 f, pos, n;   // throughput up to here, position, shading normal
+    bool medium_event, two_sided;
+    bool want;      // the path goes on
+    int32_t mat;
+    float pi, time, nsampled;  // roulette probability, time of arrival, next free flight
+};
+// Its connection to a light, if it has one (`emit`): a shadow record.
+struct Connection {
+    float4 o, d, c;
+    uint32_t tag;
+    bool emit;
+};
+
+__device__ __forceinline__ float flight_rate(const SceneDev& S, const RenderDev& R)
+{
+    return R.time_sampling ? R.ts_lambda : S.lambda;  // NextEventSampling::Time / MeanFreePath
+}
+
+// The vertex at the end of the ray (o, d), whose closest hit is `h`: the free flight's correction, the
+// connection to a light and the decision to go on. thr: throughput and time of the path before it,
+// sampled: its free flight, pst / pinc: the path's stream, nee: light-stream draws so far. LAYERS: the
+// film may be a multibounce one.
+template <bool LAYERS>
+__device__ __forceinline__ void path_vertex(const SceneDev& S, const RenderDev& R, uint32_t level, uint32_t slot, uint64_t pid,
+                                            uint64_t pinc, uint32_t pix, float2 h, f3 o, f3 d, float4 thr, float sampled,
+                                            float uw, uint64_t& pst, uint32_t& nee, Vertex& vx, Connection& sh)
+{
+    const int32_t tri = __float_as_int(h.y);
+    const float lam = flight_rate(S, R);
+    f3 &f = vx.f, &pos = vx.pos, &n = vx.n;
+    bool &medium_event = vx.medium_event, &two_sided = vx.two_sided;
+    int32_t& mat = vx.mat;
+    float &pi = vx.pi, &time = vx.time, &nsampled = vx.nsampled;
+    // correct_next_event_distance (BidirectionalPathTracing.h:275-307)
+    float dist, pd = 1.0f;
+    bool alive = true;
+    if (!S.has_medium) {
+        alive = tri >= 0;
+        dist = h.x;
+    } else if (tri >= 0 && h.x < sampled) {
+        dist = h.x;
+        pd = expf(-dist * lam);
+    } else {
+        dist = sampled;
+        medium_event = true;
+        pd = expf(-dist * lam) * lam;
+    }
+    if (alive) {
+        f = mk(thr);
+        if (S.has_medium) {
+            f = mk(f.x * expf(-dist * S.sigma_t.x), f.y * expf(-dist * S.sigma_t.y), f.z * expf(-dist * S.sigma_t.z));
+            f = f * (1.0f / pd);
+        }
+        time = thr.w + dist;
+        pos = point_on_ray(o, d, dist);
+        n = mk(0.0f, 0.0f, 0.0f);
+        if (!medium_event) {
+            float4 nn = S.tri_normal[tri];
+            n = mk(nn);
+            mat = __float_as_int(nn.w);
+            two_sided = (mat & kMatTwoSided) != 0;
+            if (mat & kMatSmooth) n = smooth_normal(S.tri_vn + 6 * size_t(tri), pos);
+            mat &= kMatIndex;
+        }
+        // the light stream (sequence 2 pid + 1) after `nee` draws
+        const uint64_t ninc = pcg_inc(2 * pid + 1);
+        uint64_t nst = pcg_at(R.seed, ninc, nee);
+        // ---- next-event estimation at this vertex (connect_paths :976-1045,
+        //      connect_vertex_with_light :650-692)
+        if (int(level) + 1 <= R.max_bounces && time <= R.total_time) {
+            float u = pcg_float(nst, ninc);
+            ++nee;
+            int li = min(int(u * float(S.n_lights)), S.n_lights - 1);
+            const LightHost& L = S.lights[li];
+            int type = int(L.I[3]);
+            f3 lp, ldir;
+            float ldist, pl2 = 1.0f;
+            f3 irr;
+            bool ok = true;
+            if (type == kLightPoint) {
+                lp = mk(L.pos[0], L.pos[1], L.pos[2]);
+                f3 v = pos - lp;
+                float d2 = dot(v, v);
+                ldist = sqrtf(d2);
+                ldir = v * (1.0f / ldist);
+                float att = 1.0f / d2;
+                irr = mk(L.I[0] * att, L.I[1] * att, L.I[2] * att);
+            } else {
+                float uu = pcg_float(nst, ninc), vv = pcg_float(nst, ninc);
+                nee += 2;
+                lp = mk(L.pos[0], L.pos[1], L.pos[2]) + mk(L.left[0], L.left[1], L.left[2]) * uu +
+                     mk(L.up[0], L.up[1], L.up[2]) * vv;
+                f3 v = pos - lp;
+                ldist = sqrtf(dot(v, v));
+                ldir = v * (1.0f / ldist);
+                float dl = dot(ldir, mk(L.normal[0], L.normal[1], L.normal[2]));
+                ok = dl > 0.0f;
+                float a = L.I[0] * dl / (ldist * ldist);
+                irr = mk(a, a, a);
+                pl2 = L.normal[3];
+                ldir = normalize(ldir);
+            }
+            if (ok) {
+                f3 fe;
+                if (medium_event) {
+                    fe = mk(S.sigma_s.x, S.sigma_s.y, S.sigma_s.z) * kInv4Pi;
+                } else {
+                    float4 kd = S.mats[mat];
+                    // dot_clamped, or dot_abs for a two-sided material (Path.h:188-193)
+                    float cd = -dot(ldir, n);
+                    float c = two_sided ? fabsf(cd) : fmaxf(cd, 0.0f);
+                    fe = mk(kd.x, kd.y, kd.z) * (kInvPi * c);
+                }
+                f3 att = mk(1.0f, 1.0f, 1.0f);
+                if (S.has_medium)
+                    att = mk(expf(-S.sigma_t.x * ldist), expf(-S.sigma_t.y * ldist), expf(-S.sigma_t.z * ldist));
+                float scale = R.inv_inc / (pl2 / float(S.n_lights));
+                f3 val = mul(mul(f, fe), mul(irr, att)) * scale;
+                float ts = ldist + time;
+                float cam_time = R.unwarp ? ts - uw : ts;
+                float sensor = (cam_time - R.offset) / R.exposure;
+                bool finite = isfinite(val.x) && isfinite(val.y) && isfinite(val.z);
+                bool nonzero = val.x != 0.0f || val.y != 0.0f || val.z != 0.0f;
+                const bool in_window = sensor >= 0.0f && sensor < float(R.T);
+                if (LAYERS && R.layers > 0) {
+                    // multibounce film: every connected sample counts for its layer's
+                    // weight and the steady image, in the time window or not
+                    // (MultibounceStreakCameraFilm.h:137-157, Film.h:263-283)
+                    const uint32_t layer = min(level, uint32_t(R.layers - 1));
+                    uint32_t fidx = 0xFFFFFFFFu;
+                    if (in_window)
+                        fidx = layer * R.layer_stride + pix * uint32_t(R.T) +
+                               min(uint32_t(floorf(sensor)), uint32_t(R.T - 1));
+                    if (!finite) val = mk(0.0f, 0.0f, 0.0f);  // TransientRenderer.h:167-171
+                    sh.emit = true;
+                    sh.o = make_float4(lp.x, lp.y, lp.z, ldist);
+                    sh.d = make_float4(ldir.x, ldir.y, ldir.z, __uint_as_float(fidx));
+                    sh.c = make_float4(val.x, val.y, val.z, __uint_as_float(pix));
+                    sh.tag = ((slot / uint32_t(R.n_inc)) << kMaxLayersTagBits) | layer;
+                } else if (in_window && finite && nonzero) {
+                    uint32_t bin = min(uint32_t(floorf(sensor)), uint32_t(R.T - 1));
+                    uint32_t fidx = pix * uint32_t(R.T) + bin;
+                    sh.emit = true;
+                    sh.o = make_float4(lp.x, lp.y, lp.z, ldist);
+                    sh.d = make_float4(ldir.x, ldir.y, ldir.z, __uint_as_float(fidx));
+                    sh.c = make_float4(val.x, val.y, val.z, __uint_as_float(pix));
+                }
+            }
+        }
+        // ---- termination: later vertices cannot contribute past the bounce cap or the
+        //      film window; otherwise Russian roulette on the mean albedo, or in the
+        //      Transient mode the film's time length alone (TotalTime) (:447-481)
+        if (int(level) + 1 < R.max_bounces && time <= R.total_time) {
+            float albedo = medium_event ? S.medium_albedo : S.mats[mat].w;
+            float eps = R.time_sampling ? 0.0f : pcg_float(pst, pinc);
+            if (!(eps > albedo)) {
+                pi = R.time_sampling ? 1.0f : albedo;
+                nsampled = __int_as_float(0x7f800000);
+                if (S.has_medium) nsampled = free_flight(pcg_float(pst, pinc), lam);
+                vx.want = true;
+            }
+        }
+    }
+}
+
+// The direction that an unguided path goes on in, its BSDF (with the cosine) or phase function and its
+// density. onb: orthonormal shading frame.
+__device__ __forceinline__ void path_direction(const SceneDev& S, const RenderDev& R, bool onb, uint64_t pid, uint64_t pinc, f3 d,
+                                               const Vertex& vx, uint64_t& pst, f3& nd, f3& fa, float& pa)
+{
+    const f3 pos = vx.pos, n = vx.n;
+    const float time = vx.time, nsampled = vx.nsampled;
+    if (vx.medium_event) {
+        bool timed = false;
+        if (R.time_sampling) {
+            const f3 tg = light_target(S, R.seed, pid);
+            f3 l;
+            float modl;
+            {
+#pragma clang fp contract(off)
+                l = mk(tg.x - pos.x, tg.y - pos.y, tg.z - pos.z);
+                modl = sqrtf((l.x * l.x + l.y * l.y) + l.z * l.z);
+            }
+            if (time_angular_window(modl, time, nsampled, R.total_time, R.exposure)) {
+                float e1 = pcg_float(pst, pinc), e2 = pcg_float(pst, pinc);
+                timed = sample_time_angular(l, modl, time, nsampled, R.total_time, e1, e2, &nd, &pa);
+            }
+        }
+        if (!timed) {
+            float e1 = pcg_float(pst, pinc), e2 = pcg_float(pst, pinc);
+            nd = sample_isotropic(d, e1, e2);
+            pa = kInv4Pi;
+        }
+        fa = mk(S.sigma_s.x, S.sigma_s.y, S.sigma_s.z) * kInv4Pi;
+    } else {
+        (void)pcg_float(pst, pinc);  // BSDF pick of a single-BSDF UberMaterial
+        float e1 = pcg_float(pst, pinc), e2 = pcg_float(pst, pinc);
+        float ct;
+        nd = onb ? sample_lambert_onb(n, e1, e2, &ct) : sample_lambert(n, e1, e2, &ct);
+        // a two-sided material hit from behind samples in its inverted frame
+        // (TwoSided.h:80-88, Intersection.h:180-185)
+        if (vx.two_sided && dot(d, n) > 0.0f) nd = nd * -1.0f;
+        float4 kd = S.mats[vx.mat];
+        fa = mk(kd.x, kd.y, kd.z) * (kInvPi * fabsf(dot(n, nd)));
+        pa = ct * kInvPi;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // shade: one thread per queued path whose ray has just been traced
 // Shading modes: the reference's shading frame (default), an orthonormal frame (same estimator
@@ -699,22 +933,20 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
         const uint32_t jid = BATCH ? st.y >> 16 : 0u;
         const SceneDev& S = BATCH ? jobs[jid].S : S0;
         const RenderDev& R = BATCH ? jobs[jid].R : R0;
-        bool emit_shadow = false, cont = false, want = false;
-        float4 sh_o = {}, sh_d = {}, sh_c = {};
+        bool cont = false;
         float4 n_o = {}, n_d = {}, n_thr = {};
-        uint32_t sh_tag = 0xFFFFFFFFu, tag = 0xFFFFFFFFu;
-        // state of a vertex that goes on to sample a direction
-        f3 f = {}, pos = {}, n = {}, d = {};
-        bool medium_event = false, two_sided = false;
-        int32_t mat = -1;
-        float pi = 1.0f, time = 0.0f, nsampled = 0.0f;
+        uint32_t tag = 0xFFFFFFFFu;  // guided: training record of this vertex
+        Vertex vx = {};              // a vertex that goes on to sample a direction
+        vx.mat = -1;
+        vx.pi = 1.0f;
+        Connection sh = {};
+        sh.tag = 0xFFFFFFFFu;
+        f3 d = {};
         uint64_t pst = 0, pinc = 0, pid = 0;
         uint32_t nee = 0;    // light-stream draws
         float uw = 0.0f;     // unwarp distance
         if (live) {
-            float2 h = Wv.hit[i];
-            int32_t tri = __float_as_int(h.y);
-            const float lam = R.time_sampling ? R.ts_lambda : S.lambda;  // NextEventSampling::Time / MeanFreePath
+            const float2 h = Wv.hit[i];
             const uint32_t pid_local = uint32_t(wave_base + slot - (BATCH ? jobs[jid].path_begin : 0ull));
             pid = R.pid0 + pid_local;
             pinc = pcg_inc(2 * pid);
@@ -724,9 +956,9 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
             if (level == 0) {
                 // a camera ray: unit throughput, the path stream at its seed
                 pst = pcg_seed(R.seed, 2 * pid);
-                if (S.has_medium) sampled = free_flight(pcg_float(pst, pinc), lam);
+                if (S.has_medium) sampled = free_flight(pcg_float(pst, pinc), flight_rate(S, R));
                 if (!BATCH) st.x = pid_local / (uint32_t(R.n_inc) * uint32_t(R.spp2));
-                if (R.unwarp) uw = tri >= 0 ? h.x : 3.402823466e+38f;
+                if (R.unwarp) uw = __float_as_int(h.y) >= 0 ? h.x : 3.402823466e+38f;
             } else {
                 const float4 o4 = Wv.ray_o[cur][i];
                 o = mk(o4);
@@ -737,157 +969,26 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                 if (R.unwarp) uw = Wv.uw[cur][i];
             }
             d = mk(d4);
+            path_vertex<!BATCH && !GUIDED>(S, R, level, slot, pid, pinc, st.x, h, o, d, thr, sampled, uw, pst, nee, vx, sh);
             if constexpr (GUIDED) {
-                if (slot % G.stride == 0u && slot / G.stride < G.train_paths) tag = (slot / G.stride) * G.max_levels;
-            }
-            // correct_next_event_distance (BidirectionalPathTracing.h:275-307)
-            float dist, pd = 1.0f;
-            bool alive = true;
-            if (!S.has_medium) {
-                alive = tri >= 0;
-                dist = h.x;
-            } else if (tri >= 0 && h.x < sampled) {
-                dist = h.x;
-                pd = expf(-dist * lam);
-            } else {
-                dist = sampled;
-                medium_event = true;
-                pd = expf(-dist * lam) * lam;
-            }
-            if (alive) {
-                f = mk(thr);
-                if (S.has_medium) {
-                    f = mk(f.x * expf(-dist * S.sigma_t.x), f.y * expf(-dist * S.sigma_t.y), f.z * expf(-dist * S.sigma_t.z));
-                    f = f * (1.0f / pd);
-                }
-                time = thr.w + dist;
-                pos = point_on_ray(o, d, dist);
-                n = mk(0.0f, 0.0f, 0.0f);
-                if (!medium_event) {
-                    float4 nn = S.tri_normal[tri];
-                    n = mk(nn);
-                    mat = __float_as_int(nn.w);
-                    two_sided = (mat & kMatTwoSided) != 0;
-                    if (mat & kMatSmooth) n = smooth_normal(S.tri_vn + 6 * size_t(tri), pos);
-                    mat &= kMatIndex;
-                }
-                // the light stream (sequence 2 pid + 1) after `nee` draws
-                const uint64_t ninc = pcg_inc(2 * pid + 1);
-                uint64_t nst = pcg_at(R.seed, ninc, nee);
-                // ---- next-event estimation at this vertex (connect_paths :976-1045,
-                //      connect_vertex_with_light :650-692)
-                if (int(level) + 1 <= R.max_bounces && time <= R.total_time) {
-                    float u = pcg_float(nst, ninc);
-                    ++nee;
-                    int li = min(int(u * float(S.n_lights)), S.n_lights - 1);
-                    const LightHost& L = S.lights[li];
-                    int type = int(L.I[3]);
-                    f3 lp, ldir;
-                    float ldist, pl2 = 1.0f;
-                    f3 irr;
-                    bool ok = true;
-                    if (type == kLightPoint) {
-                        lp = mk(L.pos[0], L.pos[1], L.pos[2]);
-                        f3 v = pos - lp;
-                        float d2 = dot(v, v);
-                        ldist = sqrtf(d2);
-                        ldir = v * (1.0f / ldist);
-                        float att = 1.0f / d2;
-                        irr = mk(L.I[0] * att, L.I[1] * att, L.I[2] * att);
-                    } else {
-                        float uu = pcg_float(nst, ninc), vv = pcg_float(nst, ninc);
-                        nee += 2;
-                        lp = mk(L.pos[0], L.pos[1], L.pos[2]) + mk(L.left[0], L.left[1], L.left[2]) * uu +
-                             mk(L.up[0], L.up[1], L.up[2]) * vv;
-                        f3 v = pos - lp;
-                        ldist = sqrtf(dot(v, v));
-                        ldir = v * (1.0f / ldist);
-                        float dl = dot(ldir, mk(L.normal[0], L.normal[1], L.normal[2]));
-                        ok = dl > 0.0f;
-                        float a = L.I[0] * dl / (ldist * ldist);
-                        irr = mk(a, a, a);
-                        pl2 = L.normal[3];
-                        ldir = normalize(ldir);
-                    }
-                    if (ok) {
-                        f3 fe;
-                        if (medium_event) {
-                            fe = mk(S.sigma_s.x, S.sigma_s.y, S.sigma_s.z) * kInv4Pi;
-                        } else {
-                            float4 kd = S.mats[mat];
-                            // dot_clamped, or dot_abs for a two-sided material (Path.h:188-193)
-                            float cd = -dot(ldir, n);
-                            float c = two_sided ? fabsf(cd) : fmaxf(cd, 0.0f);
-                            fe = mk(kd.x, kd.y, kd.z) * (kInvPi * c);
-                        }
-                        f3 att = mk(1.0f, 1.0f, 1.0f);
-                        if (S.has_medium)
-                            att = mk(expf(-S.sigma_t.x * ldist), expf(-S.sigma_t.y * ldist), expf(-S.sigma_t.z * ldist));
-                        float scale = R.inv_inc / (pl2 / float(S.n_lights));
-                        f3 val = mul(mul(f, fe), mul(irr, att)) * scale;
-                        float ts = ldist + time;
-                        float cam_time = R.unwarp ? ts - uw : ts;
-                        float sensor = (cam_time - R.offset) / R.exposure;
-                        bool finite = isfinite(val.x) && isfinite(val.y) && isfinite(val.z);
-                        bool nonzero = val.x != 0.0f || val.y != 0.0f || val.z != 0.0f;
-                        const bool in_window = sensor >= 0.0f && sensor < float(R.T);
-                        if (!BATCH && !GUIDED && R.layers > 0) {
-                            // multibounce film: every connected sample counts for its layer's
-                            // weight and the steady image, in the time window or not
-                            // (MultibounceStreakCameraFilm.h:137-157, Film.h:263-283)
-                            const uint32_t layer = min(level, uint32_t(R.layers - 1));
-                            uint32_t fidx = 0xFFFFFFFFu;
-                            if (in_window)
-                                fidx = layer * R.layer_stride + st.x * uint32_t(R.T) +
-                                       min(uint32_t(floorf(sensor)), uint32_t(R.T - 1));
-                            if (!finite) val = mk(0.0f, 0.0f, 0.0f);  // TransientRenderer.h:167-171
-                            emit_shadow = true;
-                            sh_o = make_float4(lp.x, lp.y, lp.z, ldist);
-                            sh_d = make_float4(ldir.x, ldir.y, ldir.z, __uint_as_float(fidx));
-                            sh_c = make_float4(val.x, val.y, val.z, __uint_as_float(st.x));
-                            sh_tag = ((slot / uint32_t(R.n_inc)) << kMaxLayersTagBits) | layer;
-                        } else if (in_window && finite && nonzero) {
-                            uint32_t bin = min(uint32_t(floorf(sensor)), uint32_t(R.T - 1));
-                            uint32_t fidx = st.x * uint32_t(R.T) + bin;
-                            emit_shadow = true;
-                            sh_o = make_float4(lp.x, lp.y, lp.z, ldist);
-                            sh_d = make_float4(ldir.x, ldir.y, ldir.z, __uint_as_float(fidx));
-                            sh_c = make_float4(val.x, val.y, val.z, __uint_as_float(st.x));
-                            if (GUIDED && tag != 0xFFFFFFFFu) sh_tag = tag + level;
-                        }
-                    }
-                }
-                // ---- termination: later vertices cannot contribute past the bounce cap or the
-                //      film window; otherwise Russian roulette on the mean albedo, or in the
-                //      Transient mode the film's time length alone (TotalTime) (:447-481)
-                if (int(level) + 1 < R.max_bounces && time <= R.total_time) {
-                    float albedo = medium_event ? S.medium_albedo : S.mats[mat].w;
-                    float eps = R.time_sampling ? 0.0f : pcg_float(pst, pinc);
-                    if (!(eps > albedo)) {
-                        pi = R.time_sampling ? 1.0f : albedo;
-                        nsampled = __int_as_float(0x7f800000);
-                        if (S.has_medium) nsampled = free_flight(pcg_float(pst, pinc), lam);
-                        want = true;
-                        if (GUIDED && tag != 0xFFFFFFFFu) tag += level;
-                    }
-                }
+                if (slot % G.stride == 0u && slot / G.stride < G.train_paths) sh.tag = tag = (slot / G.stride) * G.max_levels + level;
             }
         }
-        if (!want) tag = 0xFFFFFFFFu;
+        if (!vx.want) tag = 0xFFFFFFFFu;
         // ---- guided: the network's mixture for every vertex of this wavefront that samples a
         //      direction (all 64 lanes take part in the matrix-core evaluation)
         float raw[GUIDED ? trg::kRaw : 1];
         float* mine = glds + (GUIDED ? (threadIdx.x >> 6) * 64 * trg::kRow : 0);
         if constexpr (GUIDED) {
-            const f3 pn = mk((pos.x - G.bb_lo.x) * G.bb_inv.x, (pos.y - G.bb_lo.y) * G.bb_inv.y,
-                             (pos.z - G.bb_lo.z) * G.bb_inv.z);
+            const f3 pn = mk((vx.pos.x - G.bb_lo.x) * G.bb_inv.x, (vx.pos.y - G.bb_lo.y) * G.bb_inv.y,
+                             (vx.pos.z - G.bb_lo.z) * G.bb_inv.z);
             raw[0] = pn.x, raw[1] = pn.y, raw[2] = pn.z;
             raw[3] = -d.x, raw[4] = -d.y, raw[5] = -d.z;
-            raw[6] = n.x, raw[7] = n.y, raw[8] = n.z;
-            raw[9] = fminf(fmaxf(time / R.total_time, 0.0f), 1.0f);
-            raw[10] = medium_event ? 1.0f : 0.0f;
+            raw[6] = vx.n.x, raw[7] = vx.n.y, raw[8] = vx.n.z;
+            raw[9] = fminf(fmaxf(vx.time / R.total_time, 0.0f), 1.0f);
+            raw[10] = vx.medium_event ? 1.0f : 0.0f;
             raw[11] = 0.0f;
-            if (__ballot(want) != 0ull) {
+            if (__ballot(vx.want) != 0ull) {
                 const int lane = int(__lane_id());
                 float feat[trg::kFeat];
                 trg::encode_features(raw, feat);
@@ -901,45 +1002,16 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             }
         }
-        if (want) {
+        if (vx.want) {
+            const f3 f = vx.f, pos = vx.pos, n = vx.n;
+            const bool medium_event = vx.medium_event, two_sided = vx.two_sided;
+            const int32_t mat = vx.mat;
+            const float pi = vx.pi;
             f3 nd, fa;
             float pa;
             bool ok = true;
             if constexpr (!GUIDED) {
-                if (medium_event) {
-                    bool timed = false;
-                    if (R.time_sampling) {
-                        const f3 tg = light_target(S, R.seed, pid);
-                        f3 l;
-                        float modl;
-                        {
-#pragma clang fp contract(off)
-                            l = mk(tg.x - pos.x, tg.y - pos.y, tg.z - pos.z);
-                            modl = sqrtf((l.x * l.x + l.y * l.y) + l.z * l.z);
-                        }
-                        if (time_angular_window(modl, time, nsampled, R.total_time, R.exposure)) {
-                            float e1 = pcg_float(pst, pinc), e2 = pcg_float(pst, pinc);
-                            timed = sample_time_angular(l, modl, time, nsampled, R.total_time, e1, e2, &nd, &pa);
-                        }
-                    }
-                    if (!timed) {
-                        float e1 = pcg_float(pst, pinc), e2 = pcg_float(pst, pinc);
-                        nd = sample_isotropic(d, e1, e2);
-                        pa = kInv4Pi;
-                    }
-                    fa = mk(S.sigma_s.x, S.sigma_s.y, S.sigma_s.z) * kInv4Pi;
-                } else {
-                    (void)pcg_float(pst, pinc);  // BSDF pick of a single-BSDF UberMaterial
-                    float e1 = pcg_float(pst, pinc), e2 = pcg_float(pst, pinc);
-                    float ct;
-                    nd = MODE == kShadeRef ? sample_lambert(n, e1, e2, &ct) : sample_lambert_onb(n, e1, e2, &ct);
-                    // a two-sided material hit from behind samples in its inverted frame
-                    // (TwoSided.h:80-88, Intersection.h:180-185)
-                    if (two_sided && dot(d, n) > 0.0f) nd = nd * -1.0f;
-                    float4 kd = S.mats[mat];
-                    fa = mk(kd.x, kd.y, kd.z) * (kInvPi * fabsf(dot(n, nd)));
-                    pa = ct * kInvPi;
-                }
+                path_direction(S, R, MODE == kShadeOnb, pid, pinc, d, vx, pst, nd, fa, pa);
             } else {
                 const float alpha = G.alpha;
                 const f3 nside = (two_sided && dot(d, n) > 0.0f) ? n * -1.0f : n;  // side the path arrives on
@@ -986,19 +1058,19 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
             if (ok) {
                 f3 nf = mul(f, fa) * (1.0f / (pi * pa));
                 cont = true;
-                n_o = make_float4(pos.x, pos.y, pos.z, nsampled);
+                n_o = make_float4(pos.x, pos.y, pos.z, vx.nsampled);
                 n_d = make_float4(nd.x, nd.y, nd.z, d4.w);
-                n_thr = make_float4(nf.x, nf.y, nf.z, time);
+                n_thr = make_float4(nf.x, nf.y, nf.z, vx.time);
                 st = make_uint4(st.x, nee | (jid << 16), uint32_t(pst), uint32_t(pst >> 32));
             }
         }
         uint32_t q_pos, sh_pos;
-        block_append2(Wv.counters + qword(cur ^ 1), cont ? 1u : 0u, emit_shadow ? 1u : 0u, scan, &q_pos, &sh_pos);
-        if (emit_shadow) {
-            Wv.sh_o[sh_pos] = sh_o;
-            Wv.sh_d[sh_pos] = sh_d;
-            Wv.sh_c[sh_pos] = sh_c;
-            if (GUIDED || (!BATCH && R.layers > 0)) Wv.sh_tag[sh_pos] = sh_tag;
+        block_append2(Wv.counters + qword(cur ^ 1), cont ? 1u : 0u, sh.emit ? 1u : 0u, scan, &q_pos, &sh_pos);
+        if (sh.emit) {
+            Wv.sh_o[sh_pos] = sh.o;
+            Wv.sh_d[sh_pos] = sh.d;
+            Wv.sh_c[sh_pos] = sh.c;
+            if (GUIDED || (!BATCH && R.layers > 0)) Wv.sh_tag[sh_pos] = sh.tag;
             if constexpr (BATCH) Wv.sh_job[sh_pos] = jid;
         }
         if (cont) {
@@ -1008,6 +1080,164 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
             Wv.st[cur ^ 1][q_pos] = st;
             if (R.unwarp) Wv.uw[cur ^ 1][q_pos] = uw;
         }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// path: all bounces of a small wavefront's paths in one launch, a path per lane, and then their shadow rays,
+// in place of the camera launch, an extend and a shade launch per bounce and the shadow launch. Those take
+// 10-20 us each however few paths there are (a launch, and a ray's chain of node reads), and each waits for
+// the longest ray of the one before it; here a GPU wavefront waits for its own rays only. It loses lanes as
+// paths end, which the queues' compaction avoids, so it begins new paths in them where it has more than 64
+// (media: 2^21 paths 1,116 us with 64 paths per wavefront, 898 with 256; where paths are short, or none
+// ends early, 64 are as fast or faster), and large wavefronts keep the queues (kPathWave). Its shadow
+// records are a segment of its own: appending each bounce's to one queue took 12 ns per atomic, 2.2 ms of a
+// 2^20-path medium render that takes 0.6. Lanes and order aside, every path is computed as by the queue's
+// kernels.
+template <int TRAV, int STACK, bool BATCH>
+__global__ void __launch_bounds__(kTraceBlock, 4) path_kernel(SceneDev S0, RenderDev R0, const JobDev* __restrict__ jobs,
+                                                             uint32_t n_jobs, WaveDev Wv, bool onb)
+{
+    static_assert(TRAV == kTravWide || TRAV == kTravWide16, "4-wide BVH, plain stacks");
+    __shared__ uint32_t stack[stack_words<TRAV, STACK>() * kTraceBlock];
+    const WaveCtl ctl = *Wv.ctl;
+    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, rec0 = wave * Wv.seg_cap;
+    const uint32_t end = min(ctl.n, (wave + 1u) * Wv.seg_paths);
+    uint32_t fresh = wave * Wv.seg_paths;  // the wavefront's next path to begin
+    if (fresh >= ctl.n) return;
+    uint32_t traced = 0, n_rec = 0;
+    bool live = false;
+    uint32_t slot = 0, jid = 0, level = 0, pix = 0, nee = 0;
+    uint64_t pid = 0, pst = 0;
+    f3 o = {}, d = {};
+    float4 thr = {};
+    float sampled = 0.0f, uw = 0.0f;
+    for (;;) {
+        const uint64_t idle = __ballot(!live);
+        if (fresh < end && (__popcll(idle) >= kPathRefill || idle == ~0ull)) {
+            const uint32_t i = fresh + lanes_below(idle);
+            if (!live && i < end) {
+                const uint64_t gidx = ctl.base + i;
+                slot = i;
+                if constexpr (BATCH) jid = job_of(jobs, n_jobs, gidx);
+                const SceneDev& S = BATCH ? jobs[jid].S : S0;
+                const RenderDev& R = BATCH ? jobs[jid].R : R0;
+                const uint32_t pid_local = BATCH ? uint32_t(gidx - jobs[jid].path_begin) : uint32_t(gidx);
+                pid = R.pid0 + pid_local;
+                o = mk(R.cpos.x, R.cpos.y, R.cpos.z);
+                d = camera_ray(R, pid_local, pix);
+                thr = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
+                sampled = __int_as_float(0x7f800000);
+                pst = pcg_seed(R.seed, 2 * pid);
+                if (S.has_medium) sampled = free_flight(pcg_float(pst, pcg_inc(2 * pid)), flight_rate(S, R));
+                level = nee = 0;
+                live = true;
+            }
+            fresh += uint32_t(__popcll(idle));
+        }
+        const uint64_t active = __ballot(live);
+        if (active == 0ull) break;  // every path of the wavefront is done
+        traced += uint32_t(__popcll(active));
+        Connection sh = {};
+        if (live) {
+            const SceneDev& S = BATCH ? jobs[jid].S : S0;
+            const RenderDev& R = BATCH ? jobs[jid].R : R0;
+            const uint64_t pinc = pcg_inc(2 * pid);
+            float tfar = __int_as_float(0x7f800000);
+            const int32_t hit = trace4<false, stack_kind<TRAV>(), true>(S.nodes4, S.tris, ray_pre(o, d, S.plane_bound),
+                                                                        kSigmaVisibility, tfar, stack, threadIdx.x, kTraceBlock);
+            const float2 h = make_float2(hit >= 0 ? tfar : -1.0f, __int_as_float(hit));
+            if (level == 0 && R.unwarp) uw = hit >= 0 ? tfar : 3.402823466e+38f;
+            Vertex vx = {};
+            vx.mat = -1;
+            vx.pi = 1.0f;
+            path_vertex<!BATCH>(S, R, level, slot, pid, pinc, pix, h, o, d, thr, sampled, uw, pst, nee, vx, sh);
+            live = vx.want;
+            if (live) {
+                f3 nd, fa;
+                float pa;
+                path_direction(S, R, onb, pid, pinc, d, vx, pst, nd, fa, pa);
+                const f3 nf = mul(vx.f, fa) * (1.0f / (vx.pi * pa));
+                o = vx.pos;
+                d = nd;
+                sampled = vx.nsampled;
+                thr = make_float4(nf.x, nf.y, nf.z, vx.time);
+                ++level;
+            }
+        }
+        const uint64_t emitted = __ballot(sh.emit);
+        if (sh.emit) {
+            const uint32_t at = rec0 + n_rec + lanes_below(emitted);
+            Wv.sh_o[at] = sh.o;
+            Wv.sh_d[at] = sh.d;
+            Wv.sh_c[at] = sh.c;
+            if (!BATCH && R0.layers > 0) Wv.sh_tag[at] = sh.tag;
+            if constexpr (BATCH) Wv.sh_job[at] = jid;
+        }
+        n_rec += uint32_t(__popcll(emitted));
+    }
+    // the wavefront's shadow rays, handed to idle lanes as in shadow_kernel
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    uint32_t next = 0, rec = kIdle, visible = 0;
+    RayPre r;
+    Trav4 st;
+    const float4 *nodes = S0.nodes4, *tris = S0.tris;
+    for (;;) {
+        const uint64_t idle = __ballot(rec == kIdle);
+        if (next < n_rec && (__popcll(idle) >= kRefillMinShadow || idle == ~0ull)) {
+            const uint32_t i = next + lanes_below(idle);
+            if (rec == kIdle && i < n_rec) {
+                rec = i;
+                float pb = S0.plane_bound;
+                if constexpr (BATCH) {
+                    const SceneDev& J = jobs[Wv.sh_job[rec0 + i]].S;
+                    nodes = J.nodes4;
+                    tris = J.tris;
+                    pb = J.plane_bound;
+                }
+                const float4 so = Wv.sh_o[rec0 + i], sd = Wv.sh_d[rec0 + i];
+                r = ray_pre(mk(so), mk(sd), pb);
+                trav4_begin(st, so.w - kSigmaVisibility, threadIdx.x);
+            }
+            next += uint32_t(__popcll(idle));
+        }
+        if (__ballot(rec != kIdle) == 0ull) break;  // none left
+        if (rec != kIdle && trace4_step<true, stack_kind<TRAV>(), true>(nodes, tris, r, kSigmaVisibility, st, stack, threadIdx.x,
+                                                                        kTraceBlock)) {
+            const bool vis = st.hit < 0;
+            Wv.sh_vis[rec0 + rec] = vis ? 1 : 0;
+            visible += vis ? 1u : 0u;
+            rec = kIdle;
+        }
+    }
+    visible = wave_sum(visible);
+    if (__lane_id() == 0) {
+        Wv.seg_n[wave] = n_rec;
+        uint32_t* part = Wv.counters + part_word(blockIdx.x % kParts, 0);
+        if (traced) atomicAdd(reinterpret_cast<unsigned long long*>(part + P_STAT_EXT), (unsigned long long)traced);
+        if (n_rec) atomicAdd(reinterpret_cast<unsigned long long*>(part + P_STAT_SHADOW), (unsigned long long)n_rec);
+        if (visible) atomicAdd(reinterpret_cast<unsigned long long*>(part + P_STAT_CONTRIB), (unsigned long long)visible);
+    }
+}
+
+// calls f(r) for every shadow record of the launch that is visible: those of the queue `sh`, or, of path
+// launches, those of every wavefront's segment
+template <class F>
+__device__ __forceinline__ void each_visible(const WaveDev& Wv, int sh, F f)
+{
+    if (Wv.seg_cap == 0u) {
+        const uint32_t count = Wv.counters[shword(sh)];
+        for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < count; r += gridDim.x * blockDim.x)
+            if (Wv.sh_vis[r]) f(r);
+        return;
+    }
+    const uint32_t segs = (Wv.ctl->n + Wv.seg_paths - 1u) / Wv.seg_paths;
+    for (uint32_t w = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; w < segs; w += (gridDim.x * blockDim.x) >> 6) {
+        const uint32_t n = Wv.seg_n[w], r0 = w * Wv.seg_cap;
+        for (uint32_t j = __lane_id(); j < n; j += 64u)
+            if (Wv.sh_vis[r0 + j]) f(r0 + j);
     }
 }
 
@@ -1149,11 +1379,13 @@ constexpr uint32_t kFilmRange = 512;
 constexpr uint32_t kFilmLdsBytes = 72 * 1024;  // FP64 histograms: pix_slots * T * 3 * 8 bytes (3 pixels of 1024 bins)
 constexpr uint32_t kFilmMaxSlots = 8;
 constexpr int kFilmRounds = 2;
+constexpr uint32_t kFilmSegs = 8;
 static_assert(kFilmRange <= uint32_t(kFilmBlock), "one record of a range per thread");
 
-// Where the contributions come from: a render's shadow records, those of a guided render (whose
-// contributions are also credited to training records), or samples that the caller made.
-enum { kFilmRender = 0, kFilmGuided = 1, kFilmSamples = 2 };
+// Where the contributions come from: a render's queue of shadow records, that of a guided render (whose
+// contributions are also credited to training records), samples that the caller made, or the shadow
+// records of a path launch, of which a block takes those of 512 paths (kFilmSegs segments) in turn.
+enum { kFilmRender = 0, kFilmGuided = 1, kFilmSamples = 2, kFilmPath = 3 };
 struct SamplesDev {
     const tr_film_sample* samples;
     uint32_t n;
@@ -1167,24 +1399,57 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
     constexpr bool GUIDED = SRC == kFilmGuided;
     extern __shared__ double hist[];         // pix_slots * T * 3 partials
     __shared__ uint32_t slot_pix[kFilmMaxSlots];
-    const uint32_t count = SRC == kFilmSamples ? Q.n : Wv.counters[shword(sh)];
+    constexpr bool SEGS = SRC == kFilmPath;
+    __shared__ uint32_t seg_end[SEGS ? kFilmSegs : 1];  // records of the block's segments up to and with each
+    const uint32_t segs = SEGS ? (Wv.ctl->n + Wv.seg_paths - 1u) / Wv.seg_paths : 0u;
+    const uint32_t count = SRC == kFilmSamples ? Q.n : SEGS ? 0u : Wv.counters[shword(sh)];
     if (SRC == kFilmSamples && *Q.bad != 0xFFFFFFFFu) return;
     // guided renders: ranges of 256 records, about one append chunk of the guided shading kernel's
     // 256-thread blocks, so a range spans fewer pixels (guided passes' film time -11 %)
     constexpr uint32_t kRange = GUIDED ? 256u : kFilmRange;
-    if (blockIdx.x * kRange >= count) return;  // no range for this block (the last bounces' launches)
+    const uint32_t groups = SEGS ? (segs + kFilmSegs - 1) / kFilmSegs : (count + kRange - 1) / kRange;
+    if (blockIdx.x >= groups) return;  // no range for this block (the last bounces' launches)
     const uint32_t T = uint32_t(R.T), T3 = 3u * T, hsize = pix_slots * T3;
     const int rounds = pix_slots ? kFilmRounds : 1;
     // the histograms start at zero; each flush reads and clears only the slots that were used
     for (uint32_t i = threadIdx.x; i < hsize; i += blockDim.x) hist[i] = 0.0;
-    for (uint32_t start = blockIdx.x * kRange; start < count; start += gridDim.x * kRange) {
+    uint32_t group = blockIdx.x, start = 0;  // the range's group of records and first record in it
+    while (group < groups) {
+        uint32_t total = kRange;
+        if constexpr (SEGS) {
+            if (start == 0) {
+                if (threadIdx.x < 64) {
+                    const uint32_t w = group * kFilmSegs + threadIdx.x;
+                    uint32_t x = threadIdx.x < kFilmSegs && w < segs ? Wv.seg_n[w] : 0u;
+                    for (uint32_t off = 1; off < kFilmSegs; off <<= 1) {
+                        const uint32_t y = __shfl_up(x, off);
+                        if (threadIdx.x >= off) x += y;
+                    }
+                    if (threadIdx.x < kFilmSegs) seg_end[threadIdx.x] = x;
+                }
+                __syncthreads();
+            }
+            total = seg_end[kFilmSegs - 1];
+        }
         // this thread's record of the range, if it is a visible contribution
-        const uint32_t r = start + threadIdx.x;
+        uint32_t r = SEGS ? 0xFFFFFFFFu : group * kRange + threadIdx.x;
+        bool mine = threadIdx.x < kRange && (SEGS ? start + threadIdx.x < total : r < count);
+        if (SEGS && mine) {
+            const uint32_t j = start + threadIdx.x;
+            uint32_t k = 0;
+            while (j >= seg_end[k]) ++k;
+            r = (group * kFilmSegs + k) * Wv.seg_cap + j - (k ? seg_end[k - 1] : 0u);
+        }
+        start += kRange;
+        if (start >= total) {
+            start = 0;
+            group += gridDim.x;
+        }
         bool pending = false;
         float4 c = {};
         uint32_t pix = 0, bin = 0;
         if constexpr (SRC == kFilmSamples) {
-            if (threadIdx.x < kRange && r < count) {
+            if (mine) {
                 const tr_film_sample q = Q.samples[r];
                 const float sensor = (q.time - R.offset) / R.exposure;
                 c = make_float4(q.rgb[0], q.rgb[1], q.rgb[2], 0.0f);
@@ -1192,7 +1457,7 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
                 pending = sensor < float(T) && sensor >= 0.0f;
                 bin = pending ? min(uint32_t(floorf(sensor)), T - 1u) : 0u;
             }
-        } else if (threadIdx.x < kRange && r < count && Wv.sh_vis[r]) {
+        } else if (mine && Wv.sh_vis[r]) {
             c = Wv.sh_c[r];
             if constexpr (GUIDED) {
                 // luminance of the contribution, credited to the training record of its vertex
@@ -1268,9 +1533,7 @@ __global__ void __launch_bounds__(kBlock) samples_check_kernel(const tr_film_sam
 // steady image, and (inside the time window) to their layer's film
 __global__ void __launch_bounds__(kBlock) film_mb_kernel(RenderDev R, WaveDev Wv, int sh)
 {
-    const uint32_t count = Wv.counters[shword(sh)];
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < count; r += gridDim.x * blockDim.x) {
-        if (!Wv.sh_vis[r]) continue;
+    each_visible(Wv, sh, [&](uint32_t r) {
         const float4 c = Wv.sh_c[r];
         const uint32_t tag = Wv.sh_tag[r], pix = __float_as_uint(c.w), fidx = __float_as_uint(Wv.sh_d[r].w);
         atomicOr(R.cs_bits + (tag >> kMaxLayersTagBits), 1u << (tag & ((1u << kMaxLayersTagBits) - 1u)));
@@ -1280,7 +1543,7 @@ __global__ void __launch_bounds__(kBlock) film_mb_kernel(RenderDev R, WaveDev Wv
                 film_add3(R.film, R.film_comp, size_t(fidx) * 3, c.x, c.y, c.z);
             }
         }
-    }
+    });
 }
 
 // multibounce films, after a wavefront: each camera sample adds 1 to the weight of every layer it
@@ -1304,15 +1567,13 @@ __global__ void __launch_bounds__(kBlock) mb_weight_kernel(RenderDev R, WaveDev 
 // batched renders: visible contributions go straight to their job's film, one compensated add each
 __global__ void __launch_bounds__(kBlock) film_batch_kernel(const JobDev* __restrict__ jobs, WaveDev Wv, int sh)
 {
-    const uint32_t count = Wv.counters[shword(sh)];
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < count; r += gridDim.x * blockDim.x) {
-        if (!Wv.sh_vis[r]) continue;
+    each_visible(Wv, sh, [&](uint32_t r) {
         const RenderDev& R = jobs[Wv.sh_job[r]].R;
         float4 c = Wv.sh_c[r];
         uint32_t pix = __float_as_uint(c.w);
         uint32_t bin = __float_as_uint(Wv.sh_d[r].w) - pix * uint32_t(R.T);
         film_add3(R.film, R.film_comp, (size_t(pix) * uint32_t(R.T) + bin) * 3, c.x, c.y, c.z);
-    }
+    });
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1504,6 +1765,14 @@ void launch_timed(void (*k)(P...), uint32_t grid, uint32_t block, hipStream_t s,
         else if ((bound) < 32) launch_timed(extend_camera_kernel<T, 32>, GRID, BLOCK, STREAM, ev_start, ev_stop, __VA_ARGS__); \
         else launch_timed(extend_camera_kernel<T, kBvhStack>, GRID, BLOCK, STREAM, ev_start, ev_stop, __VA_ARGS__);      \
     } while (0)
+// path launches (path_kernel), timed like them
+#define TR_PATH_DISPATCH_T(T, bound, B, GRID, BLOCK, STREAM, ...)                                                    \
+    do {                                                                                                            \
+        if ((bound) < 16) launch_timed(path_kernel<T, 16, B>, GRID, BLOCK, STREAM, ev_start, ev_stop, __VA_ARGS__); \
+        else if ((bound) < 24) launch_timed(path_kernel<T, 24, B>, GRID, BLOCK, STREAM, ev_start, ev_stop, __VA_ARGS__); \
+        else if ((bound) < 32) launch_timed(path_kernel<T, 32, B>, GRID, BLOCK, STREAM, ev_start, ev_stop, __VA_ARGS__); \
+        else launch_timed(path_kernel<T, kBvhStack, B>, GRID, BLOCK, STREAM, ev_start, ev_stop, __VA_ARGS__);        \
+    } while (0)
 #define TR_STACK_DISPATCH_T(T, bound, KERNEL, GRID, BLOCK, STREAM, ...)                   \
     do {                                                                                   \
         if ((bound) < 16) KERNEL<T, 16><<<GRID, BLOCK, 0, STREAM>>>(__VA_ARGS__);          \
@@ -1615,6 +1884,7 @@ struct WaveBuffers {
     uint8_t* sh_vis = nullptr;
     uint32_t* sh_tag = nullptr;  // allocated by the first guided render
     uint32_t* sh_job = nullptr;  // allocated by the first batched render
+    uint32_t* seg_n = nullptr;   // shadow records per wavefront of a path launch
     WaveCtl* ctl = nullptr;
     JobDev* d_jobs = nullptr;
     // pinned host staging of the job table: the upload is asynchronous, so its source must stay
@@ -1632,7 +1902,7 @@ struct WaveBuffers {
             dev_free(ray_o[b]); dev_free(ray_d[b]); dev_free(thr[b]); dev_free(st[b]); dev_free(uw[b]);
         }
         dev_free(hit); dev_free(sh_o); dev_free(sh_d); dev_free(sh_c); dev_free(sh_vis); dev_free(counters);
-        dev_free(sh_tag); dev_free(sh_job); dev_free(ctl); dev_free(d_jobs); dev_free(cs_bits);
+        dev_free(sh_tag); dev_free(sh_job); dev_free(seg_n); dev_free(ctl); dev_free(d_jobs); dev_free(cs_bits);
         if (h_jobs) (void)hipHostFree(h_jobs);
         h_jobs = nullptr;
         cap = 0;
@@ -1718,7 +1988,8 @@ struct WaveBuffers {
             }
         if ((rc = dev_alloc(&hit, n)) || (rc = dev_alloc(&sh_o, n_sh)) ||
             (rc = dev_alloc(&sh_d, n_sh)) || (rc = dev_alloc(&sh_c, n_sh)) || (rc = dev_alloc(&sh_vis, n_sh)) ||
-            (rc = dev_alloc(&counters, C_WORDS)) || (rc = dev_alloc(&ctl, 1))) {
+            (rc = dev_alloc(&counters, C_WORDS)) || (rc = dev_alloc(&ctl, 1)) ||
+            (rc = dev_alloc(&seg_n, (std::min(n, kPathWaveMedium) + 63) / 64))) {
             release();
             return rc;
         }
@@ -1735,6 +2006,8 @@ struct WaveBuffers {
         w.hit = hit;
         w.sh_o = sh_o; w.sh_d = sh_d; w.sh_c = sh_c; w.sh_vis = sh_vis; w.sh_tag = sh_tag;
         w.sh_job = sh_job; w.ctl = ctl;
+        w.seg_n = seg_n;
+        w.seg_cap = w.seg_paths = 0u;
         w.counters = counters;
         return w;
     }
@@ -2695,6 +2968,8 @@ struct Launch {
     bool batch;
     int bounces;
     int group;  // bounces whose shadow rays are traced and deposited together
+    bool path_launch;  // a wavefront's bounces run in one launch (path_kernel), path_per_wave paths per GPU wavefront
+    uint32_t path_per_wave;
     int stack_bound;
     int trav_ext, trav_sh;  // kTrav* of the closest-hit and any-hit launches
     uint32_t pix_slots;
@@ -2753,7 +3028,8 @@ struct Launch {
         return TR_OK;
     }
 
-    // the kernels of one wavefront: camera, then per bounce extend / shade / shadow / film
+    // the kernels of one wavefront: camera, then per bounce extend / shade and per group of bounces shadow /
+    // film; or path, shadow, film
     int enqueue_wave()
     {
         int rc;
@@ -2774,7 +3050,6 @@ struct Launch {
         const uint32_t by_rays = std::max((wave + kTraceBlock * kTraceRaysPerThread - 1) / (kTraceBlock * kTraceRaysPerThread),
                                           cu * kTraceMinPerCu);
         const uint32_t tg = std::max(1u, std::min({(wave + kTraceBlock - 1) / kTraceBlock, cu * c.trace_per_cu, by_rays}));
-        const uint32_t fg = std::max(1u, std::min((wave + kFilmRange - 1) / kFilmRange, cu * 4u));
         const uint32_t sblock = c.mode == kShadeGuided ? kShadeBlockGuided : kShadeBlock;
         // guided shading: 2 blocks per CU (its LDS allows no more), persistent over the wavefront, so
         // each block stages the network's 38 KB of weights once per launch instead of once per
@@ -2782,6 +3057,23 @@ struct Launch {
         const uint32_t scap = cu * (c.mode == kShadeGuided ? 2u : c.shade_per_cu);
         const uint32_t sg = std::max(1u, std::min((wave + sblock - 1) / sblock, scap));
         const uint32_t cg = (wave + kBlock - 1) / kBlock;
+        if (path_launch) {
+            const bool onb = c.mode == kShadeOnb;
+            Wv.seg_paths = path_per_wave;
+            Wv.seg_cap = Wv.seg_paths * uint32_t(bounces);
+            const uint32_t waves = (wave + Wv.seg_paths - 1) / Wv.seg_paths, pg = (waves * 64u + kTraceBlock - 1) / kTraceBlock;
+            if ((rc = begin(TR_K_EXTEND))) return rc;
+            if (trav_ext == kTravWide16 && batch)
+                TR_PATH_DISPATCH_T(kTravWide16, stack_bound, true, pg, kTraceBlock, stream, S0, R0, dj, nj, Wv, onb);
+            else if (trav_ext == kTravWide16)
+                TR_PATH_DISPATCH_T(kTravWide16, stack_bound, false, pg, kTraceBlock, stream, S0, R0, dj, nj, Wv, onb);
+            else if (batch)
+                TR_PATH_DISPATCH_T(kTravWide, stack_bound, true, pg, kTraceBlock, stream, S0, R0, dj, nj, Wv, onb);
+            else
+                TR_PATH_DISPATCH_T(kTravWide, stack_bound, false, pg, kTraceBlock, stream, S0, R0, dj, nj, Wv, onb);
+            if ((rc = end()) || (rc = enqueue_film(Wv, 0))) return rc;
+            return enqueue_layer_weights();
+        }
         if ((rc = begin(TR_K_CAMERA))) return rc;
         if (batch) camera_kernel<true><<<cg, kBlock, 0, stream>>>(S0, R0, dj, nj, Wv);
         else camera_kernel<false><<<cg, kBlock, 0, stream>>>(S0, R0, dj, nj, Wv);
@@ -2820,26 +3112,41 @@ struct Launch {
             }
             if ((rc = begin(TR_K_SHADOW))) return rc;
             TR_TRACE_DISPATCH(trav_sh, stack_bound, batch, shadow_kernel, tg, kTraceBlock, stream, S0, dj, Wv, cur ^ 1);
-            if ((rc = end())) return rc;
-            if ((rc = begin(TR_K_FILM))) return rc;
-            if (batch)
-                film_batch_kernel<<<std::max(1u, std::min((wave + kBlock - 1) / kBlock, cu * 16u)), kBlock, 0, stream>>>(dj, Wv, cur ^ 1);
-            else if (R0.layers > 0)
-                film_mb_kernel<<<std::max(1u, std::min((wave + kBlock - 1) / kBlock, cu * 16u)), kBlock, 0, stream>>>(R0, Wv, cur ^ 1);
-            else if (guide)
-                film_kernel<kFilmGuided><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, cur ^ 1, pix_slots, GV.contrib, SamplesDev{});
-            else
-                film_kernel<kFilmRender><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, cur ^ 1, pix_slots, nullptr, SamplesDev{});
-            if ((rc = end())) return rc;
+            if ((rc = end()) || (rc = enqueue_film(Wv, cur ^ 1))) return rc;
             cur ^= 1;
         }
-        if (!batch && R0.layers > 0) {
-            if ((rc = begin(TR_K_FILM))) return rc;
-            const uint32_t ncs = wave / uint32_t(R0.n_inc);
-            mb_weight_kernel<<<std::max(1u, std::min((ncs + kBlock - 1) / kBlock, cu * 16u)), kBlock, 0, stream>>>(R0, Wv);
-            if ((rc = end())) return rc;
-        }
-        return TR_OK;
+        return enqueue_layer_weights();
+    }
+
+    // the traced shadow records deposited: those of queue `sh`, or of a path launch (Wv.seg_cap)
+    int enqueue_film(const WaveDev& Wv, int sh)
+    {
+        int rc;
+        const RenderDev R0 = (*jobs)[0].dev.R;
+        const uint32_t wave = cfg->wave, cu = uint32_t(std::max(compute_units, 1));
+        const uint32_t fg = std::max(1u, std::min((wave + kFilmRange - 1) / kFilmRange, cu * 4u));
+        const uint32_t rg = std::max(1u, std::min((wave + kBlock - 1) / kBlock, cu * 16u));
+        if ((rc = begin(TR_K_FILM))) return rc;
+        if (batch) film_batch_kernel<<<rg, kBlock, 0, stream>>>(wb->d_jobs, Wv, sh);
+        else if (R0.layers > 0) film_mb_kernel<<<rg, kBlock, 0, stream>>>(R0, Wv, sh);
+        else if (guide)
+            film_kernel<kFilmGuided><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, sh, pix_slots, GV.contrib, SamplesDev{});
+        else if (Wv.seg_cap)
+            film_kernel<kFilmPath><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, sh, pix_slots, nullptr, SamplesDev{});
+        else film_kernel<kFilmRender><<<fg, kFilmBlock, film_lds, stream>>>(R0, Wv, sh, pix_slots, nullptr, SamplesDev{});
+        return end();
+    }
+
+    // multibounce films, after a wavefront
+    int enqueue_layer_weights()
+    {
+        const RenderDev R0 = (*jobs)[0].dev.R;
+        if (batch || R0.layers == 0) return TR_OK;
+        int rc;
+        if ((rc = begin(TR_K_FILM))) return rc;
+        const uint32_t ncs = cfg->wave / uint32_t(R0.n_inc), cu = uint32_t(std::max(compute_units, 1));
+        mb_weight_kernel<<<std::max(1u, std::min((ncs + kBlock - 1) / kBlock, cu * 16u)), kBlock, 0, stream>>>(R0, wb->view());
+        return end();
     }
 };
 
@@ -2863,8 +3170,11 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     uint64_t total = 0;
     int bounces = 0, stack_bound = 0;
     uint32_t max_nodes4 = 0;
-    bool wide = cfg.wide;
-    for (auto& j : jobs) wide = wide && j.scene->wide;
+    bool wide = cfg.wide, shallow_medium = true;
+    for (auto& j : jobs) {
+        wide = wide && j.scene->wide;
+        shallow_medium = shallow_medium && j.scene->has_medium && j.scene->n_nodes4 <= kShallowNodes;
+    }
     for (auto& j : jobs) {
         j.dev.path_begin = total;
         total += j.paths;
@@ -2913,6 +3223,9 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     L.batch = batch;
     L.bounces = bounces;
     L.group = int(group);
+    L.path_launch = !guide && bounces > 0 && c.wave <= (shallow_medium ? kPathWaveMedium : kPathWave) &&
+                    group == uint32_t(bounces) && (trav_ext == kTravWide || trav_ext == kTravWide16);
+    L.path_per_wave = shallow_medium && !jobs[0].dev.R.time_sampling ? 64u * std::max(1u, c.wave >> 19) : 64u;
     L.stack_bound = stack_bound;
     L.trav_ext = trav_ext;
     L.trav_sh = trav_sh;
@@ -3052,7 +3365,11 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
         auto rd64 = [&](int w) { return uint64_t(counters[w]) | (uint64_t(counters[w + 1]) << 32); };
         stats->extension_rays = rd64(C_STAT_EXT);
         stats->shadow_rays = rd64(C_STAT_SHADOW);
-        for (uint32_t p = 0; p < kParts; ++p) stats->contributions += rd64(int(part_word(p, P_STAT_CONTRIB)));
+        for (uint32_t p = 0; p < kParts; ++p) {
+            stats->extension_rays += rd64(int(part_word(p, P_STAT_EXT)));
+            stats->shadow_rays += rd64(int(part_word(p, P_STAT_SHADOW)));
+            stats->contributions += rd64(int(part_word(p, P_STAT_CONTRIB)));
+        }
         stats->waves = n_waves;
         stats->bounces_max = uint32_t(bounces);
         for (int k = 0; k < TR_K_COUNT; ++k) {
