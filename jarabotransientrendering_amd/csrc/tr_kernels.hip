@@ -68,6 +68,7 @@ constexpr uint32_t kSmallWave = 1u << 25;
 constexpr uint32_t kPathWave = 1u << 20;
 constexpr uint32_t kPathWaveMedium = 1u << 22;
 constexpr uint32_t kShallowNodes = 64;  // 4-wide nodes of a shallow tree
+constexpr uint32_t kPathSegs = kPathWaveMedium / 64;  // GPU wavefronts of a path launch, at most
 constexpr int kPathRefill = 8;  // idle lanes that begin new paths (24: 2 % slower in a medium)
 constexpr uint32_t kFetchMax = 512;  // rays per work fetch of a traversal wavefront (upper bound)
 constexpr uint32_t kTraceRaysPerThread = 8;   // lower bound on a full wavefront's rays per traversal thread
@@ -1090,7 +1091,11 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
 // the longest ray of the one before it; here a GPU wavefront waits for its own rays only. It loses lanes as
 // paths end, which the queues' compaction avoids, so it begins new paths in them where it has more than 64
 // (media: 2^21 paths 1,116 us with 64 paths per wavefront, 898 with 256; where paths are short, or none
-// ends early, 64 are as fast or faster), and large wavefronts keep the queues (kPathWave). Its shadow
+// ends early, 64 are as fast or faster), and large wavefronts keep the queues (kPathWave). Where there are
+// fewer than two GPU wavefronts of 64 per SIMD, each takes 32 or 16 paths: fewer lanes wait for the longest
+// ray and for each other's branches (1,290 triangles, 2^14 paths: 267, 227, 207 us with 64, 32, 16;
+// 81,930 triangles 444, 366, 343; a medium 169, 162, 158), but not over 22 triangles without a medium,
+// where all rays are short (2^10 paths: 85, 91, 98; cold caches in more compute units). Its shadow
 // records are a segment of its own: appending each bounce's to one queue took 12 ns per atomic, 2.2 ms of a
 // 2^20-path medium render that takes 0.6. Lanes and order aside, every path is computed as by the queue's
 // kernels.
@@ -1379,12 +1384,12 @@ constexpr uint32_t kFilmRange = 512;
 constexpr uint32_t kFilmLdsBytes = 72 * 1024;  // FP64 histograms: pix_slots * T * 3 * 8 bytes (3 pixels of 1024 bins)
 constexpr uint32_t kFilmMaxSlots = 8;
 constexpr int kFilmRounds = 2;
-constexpr uint32_t kFilmSegs = 8;
+constexpr uint32_t kFilmSegs = 32;  // segments of a path launch that a block takes at a time, at most
 static_assert(kFilmRange <= uint32_t(kFilmBlock), "one record of a range per thread");
 
 // Where the contributions come from: a render's queue of shadow records, that of a guided render (whose
 // contributions are also credited to training records), samples that the caller made, or the shadow
-// records of a path launch, of which a block takes those of 512 paths (kFilmSegs segments) in turn.
+// records of a path launch, of which a block takes those of 512 paths, or of 8 segments, in turn.
 enum { kFilmRender = 0, kFilmGuided = 1, kFilmSamples = 2, kFilmPath = 3 };
 struct SamplesDev {
     const tr_film_sample* samples;
@@ -1401,13 +1406,14 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
     __shared__ uint32_t slot_pix[kFilmMaxSlots];
     constexpr bool SEGS = SRC == kFilmPath;
     __shared__ uint32_t seg_end[SEGS ? kFilmSegs : 1];  // records of the block's segments up to and with each
+    const uint32_t per_group = SEGS ? min(max(kFilmRange / Wv.seg_paths, 8u), kFilmSegs) : 1u;
     const uint32_t segs = SEGS ? (Wv.ctl->n + Wv.seg_paths - 1u) / Wv.seg_paths : 0u;
     const uint32_t count = SRC == kFilmSamples ? Q.n : SEGS ? 0u : Wv.counters[shword(sh)];
     if (SRC == kFilmSamples && *Q.bad != 0xFFFFFFFFu) return;
     // guided renders: ranges of 256 records, about one append chunk of the guided shading kernel's
     // 256-thread blocks, so a range spans fewer pixels (guided passes' film time -11 %)
     constexpr uint32_t kRange = GUIDED ? 256u : kFilmRange;
-    const uint32_t groups = SEGS ? (segs + kFilmSegs - 1) / kFilmSegs : (count + kRange - 1) / kRange;
+    const uint32_t groups = SEGS ? (segs + per_group - 1) / per_group : (count + kRange - 1) / kRange;
     if (blockIdx.x >= groups) return;  // no range for this block (the last bounces' launches)
     const uint32_t T = uint32_t(R.T), T3 = 3u * T, hsize = pix_slots * T3;
     const int rounds = pix_slots ? kFilmRounds : 1;
@@ -1419,8 +1425,8 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
         if constexpr (SEGS) {
             if (start == 0) {
                 if (threadIdx.x < 64) {
-                    const uint32_t w = group * kFilmSegs + threadIdx.x;
-                    uint32_t x = threadIdx.x < kFilmSegs && w < segs ? Wv.seg_n[w] : 0u;
+                    const uint32_t w = group * per_group + threadIdx.x;
+                    uint32_t x = threadIdx.x < per_group && w < segs ? Wv.seg_n[w] : 0u;
                     for (uint32_t off = 1; off < kFilmSegs; off <<= 1) {
                         const uint32_t y = __shfl_up(x, off);
                         if (threadIdx.x >= off) x += y;
@@ -1438,7 +1444,7 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
             const uint32_t j = start + threadIdx.x;
             uint32_t k = 0;
             while (j >= seg_end[k]) ++k;
-            r = (group * kFilmSegs + k) * Wv.seg_cap + j - (k ? seg_end[k - 1] : 0u);
+            r = (group * per_group + k) * Wv.seg_cap + j - (k ? seg_end[k - 1] : 0u);
         }
         start += kRange;
         if (start >= total) {
@@ -1989,7 +1995,7 @@ struct WaveBuffers {
         if ((rc = dev_alloc(&hit, n)) || (rc = dev_alloc(&sh_o, n_sh)) ||
             (rc = dev_alloc(&sh_d, n_sh)) || (rc = dev_alloc(&sh_c, n_sh)) || (rc = dev_alloc(&sh_vis, n_sh)) ||
             (rc = dev_alloc(&counters, C_WORDS)) || (rc = dev_alloc(&ctl, 1)) ||
-            (rc = dev_alloc(&seg_n, (std::min(n, kPathWaveMedium) + 63) / 64))) {
+            (rc = dev_alloc(&seg_n, kPathSegs))) {
             release();
             return rc;
         }
@@ -3170,10 +3176,11 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     uint64_t total = 0;
     int bounces = 0, stack_bound = 0;
     uint32_t max_nodes4 = 0;
-    bool wide = cfg.wide, shallow_medium = true;
+    bool wide = cfg.wide, medium = true, shallow = true;
     for (auto& j : jobs) {
         wide = wide && j.scene->wide;
-        shallow_medium = shallow_medium && j.scene->has_medium && j.scene->n_nodes4 <= kShallowNodes;
+        medium = medium && j.scene->has_medium;
+        shallow = shallow && j.scene->n_nodes4 <= kShallowNodes;
     }
     for (auto& j : jobs) {
         j.dev.path_begin = total;
@@ -3223,9 +3230,12 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     L.batch = batch;
     L.bounces = bounces;
     L.group = int(group);
-    L.path_launch = !guide && bounces > 0 && c.wave <= (shallow_medium ? kPathWaveMedium : kPathWave) &&
+    L.path_launch = !guide && bounces > 0 && c.wave <= (medium && shallow ? kPathWaveMedium : kPathWave) &&
                     group == uint32_t(bounces) && (trav_ext == kTravWide || trav_ext == kTravWide16);
-    L.path_per_wave = shallow_medium && !jobs[0].dev.R.time_sampling ? 64u * std::max(1u, c.wave >> 19) : 64u;
+    L.path_per_wave = 64u;
+    if (medium && shallow && !jobs[0].dev.R.time_sampling) L.path_per_wave *= std::max(1u, c.wave >> 19);
+    if (medium || !shallow)
+        while (L.path_per_wave > 16u && c.wave <= L.path_per_wave * 1024u) L.path_per_wave /= 2u;
     L.stack_bound = stack_bound;
     L.trav_ext = trav_ext;
     L.trav_sh = trav_sh;

@@ -33,7 +33,7 @@ def _render(R, scene, flags):
     return st, *film.read_sums()
 
 
-@pytest.mark.parametrize("paths", [1, 63, 64, 65, 129, 8 * 64, 8 * 64 + 1, 1 << 20, (1 << 20) + 1])
+@pytest.mark.parametrize("paths", [1, 15, 17, 63, 64, 65, 129, 8 * 64, 8 * 64 + 1, (1 << 15) + 1, (1 << 16) + 1, 1 << 20, (1 << 20) + 1])
 @pytest.mark.parametrize("name", ["icosphere", "media", "media_time", "multibounce"])
 def test_path_launch_against_the_queues(name, paths):
     from jarabotransientrendering_amd import renderer as R
