@@ -1394,7 +1394,8 @@ enum { kFilmRender = 0, kFilmGuided = 1, kFilmSamples = 2, kFilmPath = 3 };
 struct SamplesDev {
     const tr_film_sample* samples;
     uint32_t n;
-    const uint32_t* bad;  // index of the first sample outside the film (~0: none): then nothing is added
+    const uint32_t* bad;  // index of the first sample outside the film (~0: none): then nothing is added;
+                          // null if the host has checked them
 };
 
 template <int SRC>
@@ -1409,7 +1410,7 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
     const uint32_t per_group = SEGS ? min(max(kFilmRange / Wv.seg_paths, 8u), kFilmSegs) : 1u;
     const uint32_t segs = SEGS ? (Wv.ctl->n + Wv.seg_paths - 1u) / Wv.seg_paths : 0u;
     const uint32_t count = SRC == kFilmSamples ? Q.n : SEGS ? 0u : Wv.counters[shword(sh)];
-    if (SRC == kFilmSamples && *Q.bad != 0xFFFFFFFFu) return;
+    if (SRC == kFilmSamples && Q.bad && *Q.bad != 0xFFFFFFFFu) return;
     // guided renders: ranges of 256 records, about one append chunk of the guided shading kernel's
     // 256-thread blocks, so a range spans fewer pixels (guided passes' film time -11 %)
     constexpr uint32_t kRange = GUIDED ? 256u : kFilmRange;
@@ -2647,7 +2648,7 @@ namespace {
 // the compensated sums (double). Every entry point that writes a film returns after its work has completed,
 // so the staging's streams can read it.
 template <class Out>
-int film_values(tr_film f, size_t first, size_t n, const FilmWeight& w, Out* out)
+int film_values(tr_film f, size_t first, size_t n, const FilmWeight& w, Out* out, hipStream_t own = nullptr)
 {
     static_assert(trb::kChunk % (4 * sizeof(Out)) == 0, "chunks hold whole groups of four values");
     const uint32_t T3 = 3u * uint32_t(f->desc.time_bins);
@@ -2657,7 +2658,7 @@ int film_values(tr_film f, size_t first, size_t n, const FilmWeight& w, Out* out
         film_values_kernel<Out><<<(m + kValuesPerBlock - 1) / kValuesPerBlock, kValuesPerBlock / 4, 0, stream>>>(
             f->d_sum + i, f->d_comp + i, w, i / T3, uint32_t(i % T3), T3, m, i % 4 == 0, static_cast<Out*>(dst));
         return hipGetLastError();
-    });
+    }, own);
     if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string("tr_film_read: ") + hipGetErrorString(e));
     return TR_OK;
 }
@@ -2697,15 +2698,18 @@ int tr_film_read_rows(tr_film f, int32_t row_begin, int32_t row_count, float* ou
     const size_t W = size_t(f->desc.width), T3 = size_t(f->desc.time_bins) * 3, P = size_t(f->rows) * W;
     const size_t p0 = size_t(row_begin) * W, np = size_t(row_count) * W;
     int rc;
+    if (steady && !f->d_read_steady && (rc = dev_alloc(&f->d_read_steady, P * 3))) return rc;
     FilmWeight w{f->weight[0], nullptr, nullptr};
+    hipStream_t own = nullptr;  // a read of one chunk follows the upload of its weights on the film's stream
     if (!f->same_weight) {
         if (!f->d_read_w && (rc = dev_alloc(&f->d_read_w, P))) return rc;
         HIP_TRY(hipMemcpyAsync(f->d_read_w, f->weight.data(), P * sizeof(double), hipMemcpyHostToDevice, f->stream));
-        HIP_TRY(hipStreamSynchronize(f->stream));  // the upload reads f->weight asynchronously
         w.pixel = f->d_read_w;
+        // (the upload reads f->weight, which stays as it is until this call returns)
+        if (out && np * T3 * sizeof(float) <= trb::kChunk) own = f->stream;
+        else HIP_TRY(hipStreamSynchronize(f->stream));
     }
-    if (steady && !f->d_read_steady && (rc = dev_alloc(&f->d_read_steady, P * 3))) return rc;
-    if (out && (rc = film_values(f, p0 * T3, np * T3, w, out))) return rc;
+    if (out && (rc = film_values(f, p0 * T3, np * T3, w, out, own))) return rc;
     if (steady) {
         film_steady_kernel<<<uint32_t(np), kNormBlock, 0, f->stream>>>(f->d_sum + p0 * T3, f->d_comp + p0 * T3, w, p0,
                                                                       uint32_t(T3), f->d_read_steady);
@@ -2794,7 +2798,9 @@ int tr_film_device_buffers(tr_film f, float** d_sum, float** d_comp)
 // StreakCameraFilm::add_samples for caller-made samples: checked, binned as the reference bins
 // (pos_sensor = (time - offset) / exposure, kept if 0 <= pos_sensor < T; StreakCameraFilm.h:165-171) and
 // deposited on the device, by the renders' own film kernel. (Binned on the host into shadow-record
-// arrays, 500,000 samples took 1.5 ms on one thread and 0.6 ms of allocations and extra copies.)
+// arrays, 500,000 samples took 1.5 ms on one thread and 0.6 ms of allocations and extra copies.) Up to
+// kHostSamples are checked and their weights summed by the host, 1-2 ns each, while the device's two more
+// launches and two more copies take 30 us.
 int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
 {
     if (!f) return fail(TR_ERR_INVALID, "tr_film_add_samples: null film");
@@ -2806,8 +2812,20 @@ int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
     const uint32_t T = uint32_t(fd.time_bins), P = uint32_t(f->weight.size());
     const int32_t row0 = fd.scanline >= 0 ? fd.scanline : 0;
     constexpr size_t kHead = 256 / sizeof(tr_film_sample), kKept = size_t(32) << 20;  // samples buffers up to 32 MiB are kept
+    constexpr uint32_t kHostSamples = 16384;
+    const bool on_host = n <= kHostSamples;
+    uint32_t first_bad = 0xFFFFFFFFu;
+    auto outside = [&]() {
+        return fail(TR_ERR_INVALID, "tr_film_add_samples: sample " + std::to_string(first_bad) + " lies outside the film");
+    };
+    if (on_host) {
+        for (uint32_t i = 0; i < n && first_bad == 0xFFFFFFFFu; ++i)
+            if (samples[i].x < 0 || samples[i].x >= fd.width || samples[i].y < row0 || int64_t(samples[i].y) - row0 >= f->rows)
+                first_bad = i;
+        if (first_bad != 0xFFFFFFFFu) return outside();
+    }
     int rc;
-    if (!f->d_read_w && (rc = dev_alloc(&f->d_read_w, P))) return rc;
+    if (!on_host && !f->d_read_w && (rc = dev_alloc(&f->d_read_w, P))) return rc;
     if (f->samples_cap < n) {
         dev_free(f->d_samples);
         f->samples_cap = 0;
@@ -2829,22 +2847,26 @@ int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
     const size_t lds = size_t(pix_slots) * size_t(T) * 24u;
     const uint32_t cu = uint32_t(tri::compute_units());
     const uint32_t fg = std::max(1u, std::min((n + kFilmRange - 1) / kFilmRange, cu * 4u));
-    samples_begin_kernel<<<(P + kBlock - 1) / kBlock, kBlock, 0, f->stream>>>(f->d_read_w, P, bad);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = hipMemcpyAsync(d, samples, size_t(n) * sizeof(tr_film_sample), hipMemcpyHostToDevice, f->stream);
-    if (e == hipSuccess) {
-        samples_check_kernel<<<std::min((n + kBlock - 1) / kBlock, cu * 16u), kBlock, 0, f->stream>>>(d, n, fd.width, row0,
-                                                                                                   f->rows, f->d_read_w, bad);
-        film_kernel<kFilmSamples><<<fg, kFilmBlock, lds, f->stream>>>(R, WaveDev{}, 0, pix_slots, nullptr, SamplesDev{d, n, bad});
+    hipError_t e = hipSuccess;
+    if (!on_host) {
+        samples_begin_kernel<<<(P + kBlock - 1) / kBlock, kBlock, 0, f->stream>>>(f->d_read_w, P, bad);
         e = hipGetLastError();
     }
-    std::vector<double> wadd(P);
-    uint32_t first_bad = 0xFFFFFFFFu;
-    if (e == hipSuccess) e = hipMemcpyAsync(&first_bad, bad, sizeof first_bad, hipMemcpyDeviceToHost, f->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(d, samples, size_t(n) * sizeof(tr_film_sample), hipMemcpyHostToDevice, f->stream);
+    if (e == hipSuccess) {
+        if (!on_host)
+            samples_check_kernel<<<std::min((n + kBlock - 1) / kBlock, cu * 16u), kBlock, 0, f->stream>>>(
+                d, n, fd.width, row0, f->rows, f->d_read_w, bad);
+        film_kernel<kFilmSamples><<<fg, kFilmBlock, lds, f->stream>>>(R, WaveDev{}, 0, pix_slots, nullptr,
+                                                                     SamplesDev{d, n, on_host ? nullptr : bad});
+        e = hipGetLastError();
+    }
+    if (!on_host && e == hipSuccess) e = hipMemcpyAsync(&first_bad, bad, sizeof first_bad, hipMemcpyDeviceToHost, f->stream);
     // the copies read the caller's samples and write this frame's variables: wait in any case
     const hipError_t se = hipStreamSynchronize(f->stream);
     if (e == hipSuccess) e = se;
-    if (e == hipSuccess && first_bad == 0xFFFFFFFFu) {
+    std::vector<double> wadd(on_host ? 0 : P);
+    if (!on_host && e == hipSuccess && first_bad == 0xFFFFFFFFu) {
         e = trb::read_back(wadd.data(), P * sizeof(double), [&](hipStream_t stream, void* dst, size_t at, size_t size) {
             return hipMemcpyAsync(dst, reinterpret_cast<const char*>(f->d_read_w) + at, size, hipMemcpyDeviceToHost, stream);
         });
@@ -2854,10 +2876,12 @@ int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
         f->samples_cap = 0;
     }
     if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string("tr_film_add_samples: ") + hipGetErrorString(e));
-    if (first_bad != 0xFFFFFFFFu)
-        return fail(TR_ERR_INVALID, "tr_film_add_samples: sample " + std::to_string(first_bad) + " lies outside the film");
+    if (first_bad != 0xFFFFFFFFu) return outside();
     f->same_weight = false;
     for (size_t p = 0; p < wadd.size(); ++p) f->weight[p] += wadd[p];
+    if (on_host)
+        for (uint32_t i = 0; i < n; ++i)
+            f->weight[size_t(samples[i].y - row0) * size_t(fd.width) + size_t(samples[i].x)] += double(samples[i].weight);
     return TR_OK;
 }
 

@@ -57,3 +57,25 @@ def test_a_sample_outside_the_film_adds_nothing(field, value, at):
         film.add_samples(a)
     after = film.read_sums()
     assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
+
+
+@pytest.mark.parametrize("n", [16384, 16385])
+def test_samples_checked_by_the_host_or_the_device(n):
+    """Around the largest call that the host checks: the film is what it is for two halves of the samples."""
+    from jarabotransientrendering_amd import _native as nat, renderer
+    whole, halves = (renderer.StreakCameraFilm(13, 7, 97, 0.1) for _ in range(2))
+    a = _samples(n, 13, 7, 0, n)
+    whole.add_samples(a)
+    halves.add_samples(a[: n // 2])
+    halves.add_samples(a[n // 2:])
+    # each side within the film's 2 u of the magnitudes in a bin, of which there are at most all samples'
+    bound = 2.0 ** -22 * np.abs(a["rgb"].astype(np.float64)).sum(axis=0)
+    assert (np.abs(whole.read_sums()[0] - halves.read_sums()[0]) <= 2 * bound).all()
+    assert np.array_equal(whole.read_sums()[1], halves.read_sums()[1])  # weights of halves add exactly
+    assert np.isfinite(whole.read()).all()
+    before = halves.read_sums()
+    a["y"][n - 1] = 7
+    with pytest.raises(nat.TrError, match=f"sample {n - 1} lies outside the film"):
+        halves.add_samples(a)
+    after = halves.read_sums()
+    assert np.array_equal(before[0], after[0]) and np.array_equal(before[1], after[1])
