@@ -132,6 +132,11 @@ int tr_intersect_batch(tr_scene scene, const tr_ray* rays, uint32_t n, tr_hit* h
 /* Same, on device pointers, asynchronously on `stream` (a hipStream_t; NULL = library stream). */
 int tr_intersect_batch_device(tr_scene scene, const tr_ray* d_rays, uint32_t n, tr_hit* d_hits,
                               void* stream);
+/* tr_intersect_batch for rays and answers in separate arrays: org and dir hold 3 n floats; tnear and tfar
+ * one value for all rays (n_tnear, n_tfar = 1) or one per ray (= n); t, geom_id, prim_id and tri n each. */
+int tr_intersect_arrays(tr_scene scene, const float* org, const float* dir, const float* tnear, uint32_t n_tnear,
+                        const float* tfar, uint32_t n_tfar, uint32_t n, float* t, uint32_t* geom_id, uint32_t* prim_id,
+                        uint32_t* tri);
 /* tr_intersect_batch without allocating device memory. No counterpart in the reference: it is for
  * callers that cannot allocate (code under HIP graph capture, serving loops, harnesses that forbid
  * hipMalloc). Rays and hits are staged in a static device array of TR_NOALLOC_MAX_RAYS x 48 bytes
@@ -149,6 +154,9 @@ int tr_intersect_batch_noalloc(tr_scene scene, const tr_ray* rays, uint32_t n, t
  * tr_intersect_batch, so occluded[i] == (tr_intersect_batch finds a hit) for every ray.
  * Host pointers; n may be 0. */
 int tr_occluded_batch(tr_scene scene, const tr_ray* rays, uint32_t n, uint8_t* occluded);
+/* Same for rays in separate arrays (see tr_intersect_arrays), up to tfar - shorten (in double, rounded). */
+int tr_occluded_arrays(tr_scene scene, const float* org, const float* dir, const float* tnear, uint32_t n_tnear,
+                       const float* tfar, uint32_t n_tfar, double shorten, uint32_t n, uint8_t* occluded);
 /* Same, on device pointers, asynchronously on `stream` (a hipStream_t; NULL = library stream). */
 int tr_occluded_batch_device(tr_scene scene, const tr_ray* d_rays, uint32_t n, uint8_t* d_occluded,
                              void* stream);

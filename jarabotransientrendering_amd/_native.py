@@ -150,6 +150,10 @@ SIGNATURES = {
     "tr_scene_commit": (ctypes.c_int, [ctypes.c_void_p]),
     "tr_scene_info_get": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(SceneInfo)]),
     "tr_intersect_batch": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint32, ctypes.c_void_p]),
+    "tr_intersect_arrays": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_uint32, ctypes.c_void_p, ctypes.c_uint32,
+                                                                  ctypes.c_uint32] + [ctypes.c_void_p] * 4),
+    "tr_occluded_arrays": (ctypes.c_int, [ctypes.c_void_p] * 4 + [ctypes.c_uint32, ctypes.c_void_p, ctypes.c_uint32,
+                                                                 ctypes.c_double, ctypes.c_uint32, ctypes.c_void_p]),
     "tr_intersect_batch_device": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint32,
                                                  ctypes.c_void_p, ctypes.c_void_p]),
     "tr_intersect_batch_noalloc": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint32,

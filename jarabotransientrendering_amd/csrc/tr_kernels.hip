@@ -294,8 +294,8 @@ enum { kTravBinary = 0, kTravWide = 1, kTravWide16 = 2, kTravWideKeyed = 3 };
 template <int TRAV, int STACK>
 constexpr int stack_words() { return TRAV == kTravWide16 ? (STACK + 1) / 2 : STACK; }
 
-// one query to its end (public queries, whose tnear may be any number, and the binary BVH)
-template <bool ANY, int TRAV>
+// one query to its end (public queries, whose tnear may be any number unless POS, and the binary BVH)
+template <bool ANY, int TRAV, bool POS = false>
 __device__ __forceinline__ int32_t trace_scene(const SceneDev& S, const RayPre& r, float tnear, float& tfar,
                                                uint32_t* stack)
 {
@@ -303,7 +303,7 @@ __device__ __forceinline__ int32_t trace_scene(const SceneDev& S, const RayPre& 
     if constexpr (TRAV == kTravBinary)
         return trace<ANY>(S.nodes, S.tris, r, tnear, tfar, reinterpret_cast<int32_t*>(stack) + threadIdx.x, kTraceBlock);
     else
-        return trace4<ANY, TRAV == kTravWide ? kStack32 : kStack16, false>(S.nodes4, S.tris, r, tnear, tfar, stack,
+        return trace4<ANY, TRAV == kTravWide ? kStack32 : kStack16, POS>(S.nodes4, S.tris, r, tnear, tfar, stack,
                                                                            threadIdx.x, kTraceBlock);
 }
 
@@ -1728,6 +1728,77 @@ __global__ void __launch_bounds__(kTraceBlock) occluded_kernel(SceneDev S, const
     }
 }
 
+// Queries of host rays, read from and answered into pinned host memory by the kernel itself: no copy, no
+// device buffer. A ray is words of four arrays, each at its own stride (0: the same for every ray), so
+// that records and separate arrays are read alike.
+struct RayArrays {
+    const uint32_t *org, *dir, *tnear, *tfar;
+    uint32_t so, sd, sn, sf;  // words from ray to ray
+    double shorten;           // taken off tfar in double
+};
+struct HitArrays {
+    uint32_t *t, *geom, *prim, *tri;
+    uint32_t stride;
+    uint8_t* occluded;
+};
+constexpr uint32_t kQueryRayWords = 8;  // words of a ray at most
+
+// `per_wave` rays per wavefront: the kernel is bound by each ray's chain of node reads, and lanes wait for the
+// longest of their wavefront and for each other's branches, so calls are spread over the chip: one ray per
+// wavefront up to 2,048 rays, then as many as make 2,048 wavefronts, at most 16 (81,930 triangles, closest
+// hits: 1,000 rays 116, 81, 65 us with 64, 8, 1 per wavefront; 16,384 rays 139, 100, 154; 262,144 rays 562
+// with 8, 460 with 16). Host memory is
+// read coalesced, each word once, by way of the LDS: lanes that read their own ray's words (12 or 32 bytes
+// apart) fetch every line over PCIe several times. POS: tnear is positive.
+template <bool ANY, int TRAV, int STACK, bool POS>
+__global__ void __launch_bounds__(kTraceBlock) query_kernel(SceneDev S, RayArrays in, HitArrays out,
+                                                           const uint4* __restrict__ ids, uint32_t n, uint32_t per_wave)
+{
+    __shared__ uint32_t stack[stack_words<TRAV, STACK>() * kTraceBlock];
+    __shared__ uint32_t words[kTraceBlock * kQueryRayWords];
+    const uint32_t per_block = per_wave * (kTraceBlock / 64), first = blockIdx.x * per_block;
+    const uint32_t rays = min(per_block, n - first);
+    // words [first * stride, (first + rays) * stride) of each array; arrays inside another's records are not copied again
+    auto stage = [&](const uint32_t* a, uint32_t stride, uint32_t at) {
+        for (uint32_t k = threadIdx.x; k < rays * stride; k += kTraceBlock) words[at + k] = a[size_t(first) * stride + k];
+    };
+    const bool records = in.so == kQueryRayWords;
+    const uint32_t at_d = records ? 4u : 3u * per_block, at_n = records ? 3u : 6u * per_block, at_f = records ? 7u : 7u * per_block;
+    stage(in.org, in.so, 0u);
+    if (!records) {
+        stage(in.dir, in.sd, at_d);
+        if (in.sn) stage(in.tnear, in.sn, at_n);
+        if (in.sf) stage(in.tfar, in.sf, at_f);
+    }
+    const float near0 = __uint_as_float(in.sn ? 0u : *in.tnear), far0 = __uint_as_float(in.sf ? 0u : *in.tfar);
+    __syncthreads();
+    const uint32_t j = (threadIdx.x >> 6) * per_wave + (threadIdx.x & 63u);
+    if ((threadIdx.x & 63u) >= per_wave || j >= rays) return;
+    const uint32_t i = first + j;
+    auto word = [&](uint32_t at, uint32_t stride, uint32_t k) { return __uint_as_float(words[at + j * stride + k]); };
+    const f3 o = mk(word(0, in.so, 0), word(0, in.so, 1), word(0, in.so, 2));
+    const f3 d = mk(word(at_d, in.sd, 0), word(at_d, in.sd, 1), word(at_d, in.sd, 2));
+    const float tnear = in.sn ? word(at_n, in.sn, 0) : near0;
+    float tfar = float(double(in.sf ? word(at_f, in.sf, 0) : far0) - in.shorten);
+    int32_t slot = -1;
+    if (tfar > tnear)  // (nothing to hit otherwise, also where either is NaN)
+        slot = trace_scene<ANY, TRAV, POS>(S, ray_pre(o, d, S.plane_bound), tnear, tfar, stack);
+    if (ANY) {
+        out.occluded[i] = slot >= 0 ? 1 : 0;
+        return;
+    }
+    const uint4 id = slot >= 0 ? ids[slot] : make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0xFFFFFFFFu, 0u);
+    const uint32_t t = __float_as_uint(slot >= 0 ? tfar : -1.0f);
+    if (out.stride == 4u) {
+        reinterpret_cast<uint4*>(out.t)[i] = make_uint4(t, id.x, id.y, id.z);
+    } else {
+        out.t[i] = t;
+        out.geom[i] = id.x;
+        out.prim[i] = id.y;
+        out.tri[i] = id.z;
+    }
+}
+
 // The traversal stack holds at most one entry per BVH level; the smallest instantiation that
 // covers the scene's depth keeps LDS per block (and so occupancy) in check.
 // `bound` = entries the traversal stack can hold at most (binary: depth; 4-wide: 3 per level).
@@ -2437,29 +2508,146 @@ int tr_intersect_batch_device(tr_scene s, const tr_ray* d_rays, uint32_t n, tr_h
     return TR_OK;
 }
 
+}  // extern "C"
+
+namespace {
+
+template <bool ANY, int TRAV, bool POS>
+void launch_query(int bound, uint32_t grid, hipStream_t q, const SceneDev& S, const RayArrays& in, const HitArrays& out,
+                  const uint4* ids, uint32_t n, uint32_t per_wave)
+{
+    if (bound < 16) query_kernel<ANY, TRAV, 16, POS><<<grid, kTraceBlock, 0, q>>>(S, in, out, ids, n, per_wave);
+    else if (bound < 24) query_kernel<ANY, TRAV, 24, POS><<<grid, kTraceBlock, 0, q>>>(S, in, out, ids, n, per_wave);
+    else if (bound < 32) query_kernel<ANY, TRAV, 32, POS><<<grid, kTraceBlock, 0, q>>>(S, in, out, ids, n, per_wave);
+    else query_kernel<ANY, TRAV, kBvhStack, POS><<<grid, kTraceBlock, 0, q>>>(S, in, out, ids, n, per_wave);
+}
+
+// Host rays of a call: records (tr_ray), or separate arrays with one or a per-ray tnear and tfar.
+struct HostRays {
+    const float *org, *dir, *tnear, *tfar;
+    bool records, many_near, many_far;
+    double shorten;
+};
+struct HostHits {
+    tr_hit* records;
+    float* t;
+    uint32_t *geom, *prim, *tri;
+    uint8_t* occluded;
+};
+
+// Rays of a launch. Several threads each copy a launch's rays into pinned memory, wait for it and copy the
+// answers out, so that copies and launches overlap. A launch lasts as long as its longest ray, 50-80 us over
+// 81,930 triangles however many rays it has: 262,144 rays take 885 us with 4 threads and launches of 8,192
+// rays, 625 with 16,384, 562 with 32,768; 1,001 with one thread, 480 with 8 (1,000,000 rays: 4 threads
+// 1.60 ms, 8 threads 1.47). In all, with buffers made for each call, the runtime's copies and records
+// packed by the caller, 262,144 rays took 2,700 us and take 500; 1,000 took 74 and take 50.
+constexpr uint32_t kQueryChunk = 32768;
+constexpr uint32_t kMaxQueryThreads = trb::kStreams;
+constexpr uint32_t kQueryPerWave = 16;
+static_assert(kQueryChunk * (sizeof(tr_ray) + sizeof(tr_hit)) + 64 <= trb::kChunk, "a launch's rays and answers fit a chunk");
+
+template <bool ANY>
+int query_host(tr_scene s, const HostRays& in, uint32_t n, const HostHits& out, const char* who)
+{
+    const int trav = !s->wide ? kTravBinary : s->n_nodes4 <= 65536u ? kTravWide16 : kTravWide;
+    const int bound = s->wide ? s->stack4 : s->depth;
+    const bool pos = !in.records && !in.many_near && *in.tnear > 0.0f;
+    uint32_t per_wave = 1;
+    while (per_wave < kQueryPerWave && per_wave * 2048u < n) per_wave *= 2u;
+    const SceneDev S = s->view();
+    const uint32_t threads = uint32_t(std::min<uint64_t>(kMaxQueryThreads, (uint64_t(n) + kQueryChunk - 1) / kQueryChunk));
+    const hipError_t e = trb::run_chunks(n, kQueryChunk, threads, [&](hipStream_t q, hipEvent_t done, char* host, size_t first, size_t m) {
+        // in: the rays; then, 16-byte aligned, the answers
+        RayArrays r{};
+        r.shorten = in.shorten;
+        uint32_t* w = reinterpret_cast<uint32_t*>(host);
+        auto put = [&](const float* from, size_t count) {
+            uint32_t* at = w;
+            std::memcpy(at, from, count * sizeof(float));
+            w += count;
+            return static_cast<const uint32_t*>(at);
+        };
+        if (in.records) {
+            r.org = put(in.org + first * kQueryRayWords, m * kQueryRayWords);
+            r.dir = r.tnear = r.tfar = r.org;
+            r.so = r.sd = r.sn = r.sf = kQueryRayWords;
+        } else {
+            r.org = put(in.org + 3 * first, 3 * m);
+            r.dir = put(in.dir + 3 * first, 3 * m);
+            r.tnear = put(in.tnear + (in.many_near ? first : 0), in.many_near ? m : 1);
+            r.tfar = put(in.tfar + (in.many_far ? first : 0), in.many_far ? m : 1);
+            r.so = r.sd = 3u;
+            r.sn = in.many_near ? 1u : 0u;
+            r.sf = in.many_far ? 1u : 0u;
+        }
+        w += (4 - (w - reinterpret_cast<uint32_t*>(host)) % 4) % 4;
+        HitArrays h{};
+        h.occluded = reinterpret_cast<uint8_t*>(w);
+        h.stride = out.records ? 4u : 1u;
+        h.t = w;
+        h.geom = w + m;
+        h.prim = w + 2 * m;
+        h.tri = w + 3 * m;
+        const uint32_t per_block = per_wave * (kTraceBlock / 64), grid = uint32_t((m + per_block - 1) / per_block);
+        if (trav == kTravBinary) launch_query<ANY, kTravBinary, false>(bound, grid, q, S, r, h, s->d_ids, uint32_t(m), per_wave);
+        else if (!ANY && pos && trav == kTravWide16)
+            launch_query<ANY, kTravWide16, !ANY>(bound, grid, q, S, r, h, s->d_ids, uint32_t(m), per_wave);
+        else if (trav == kTravWide16)
+            launch_query<ANY, kTravWide16, false>(bound, grid, q, S, r, h, s->d_ids, uint32_t(m), per_wave);
+        else launch_query<ANY, kTravWide, false>(bound, grid, q, S, r, h, s->d_ids, uint32_t(m), per_wave);
+        hipError_t err = hipGetLastError();
+        if (err == hipSuccess) err = hipEventRecord(done, q);
+        if (err == hipSuccess) err = hipEventSynchronize(done);
+        if (err != hipSuccess) return err;
+        if (ANY) {
+            std::memcpy(out.occluded + first, h.occluded, m);
+        } else if (out.records) {
+            std::memcpy(out.records + first, h.t, m * sizeof(tr_hit));
+        } else {
+            std::memcpy(out.t + first, h.t, m * 4);
+            std::memcpy(out.geom + first, h.geom, m * 4);
+            std::memcpy(out.prim + first, h.prim, m * 4);
+            std::memcpy(out.tri + first, h.tri, m * 4);
+        }
+        return hipSuccess;
+    });
+    if (e == hipErrorOutOfMemory) return fail(TR_ERR_NOMEM, std::string(who) + ": " + hipGetErrorString(e));
+    if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string(who) + ": " + hipGetErrorString(e));
+    return TR_OK;
+}
+
+HostRays host_records(const tr_ray* rays)
+{
+    const float* w = reinterpret_cast<const float*>(rays);
+    return HostRays{w, w, w, w, true, true, true, 0.0};
+}
+
+}  // namespace
+
+extern "C" {
+
 int tr_intersect_batch(tr_scene s, const tr_ray* rays, uint32_t n, tr_hit* hits)
 {
     if (!s) return fail(TR_ERR_INVALID, "tr_intersect_batch: null scene");
     if (!s->committed) return fail(TR_ERR_STATE, "tr_intersect_batch: scene not committed");
     if (n == 0) return TR_OK;
     if (!rays || !hits) return fail(TR_ERR_INVALID, "tr_intersect_batch: null buffer");
-    tr_ray* dr = nullptr;
-    tr_hit* dh = nullptr;
-    int rc;
-    if ((rc = dev_alloc(&dr, n)) || (rc = dev_alloc(&dh, n))) {
-        dev_free(dr);
-        return rc;
-    }
-    int out = TR_OK;
-    if (hipMemcpyAsync(dr, rays, size_t(n) * sizeof(tr_ray), hipMemcpyHostToDevice, s->stream) != hipSuccess)
-        out = fail(TR_ERR_DEVICE, "tr_intersect_batch: upload failed");
-    if (!out) out = tr_intersect_batch_device(s, dr, n, dh, s->stream);
-    if (!out && hipMemcpyAsync(hits, dh, size_t(n) * sizeof(tr_hit), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-        out = fail(TR_ERR_DEVICE, "tr_intersect_batch: download failed");
-    if (!out && hipStreamSynchronize(s->stream) != hipSuccess) out = fail(TR_ERR_DEVICE, "tr_intersect_batch: kernel failed");
-    dev_free(dr);
-    dev_free(dh);
-    return out;
+    return query_host<false>(s, host_records(rays), n, HostHits{hits, nullptr, nullptr, nullptr, nullptr, nullptr},
+                             "tr_intersect_batch");
+}
+
+int tr_intersect_arrays(tr_scene s, const float* org, const float* dir, const float* tnear, uint32_t n_tnear, const float* tfar,
+                        uint32_t n_tfar, uint32_t n, float* t, uint32_t* geom_id, uint32_t* prim_id, uint32_t* tri)
+{
+    if (!s) return fail(TR_ERR_INVALID, "tr_intersect_arrays: null scene");
+    if (!s->committed) return fail(TR_ERR_STATE, "tr_intersect_arrays: scene not committed");
+    if (n == 0) return TR_OK;
+    if (!org || !dir || !tnear || !tfar || !t || !geom_id || !prim_id || !tri)
+        return fail(TR_ERR_INVALID, "tr_intersect_arrays: null buffer");
+    if ((n_tnear != 1 && n_tnear != n) || (n_tfar != 1 && n_tfar != n))
+        return fail(TR_ERR_INVALID, "tr_intersect_arrays: tnear and tfar hold one value or one per ray");
+    return query_host<false>(s, HostRays{org, dir, tnear, tfar, false, n_tnear > 1, n_tfar > 1, 0.0}, n,
+                             HostHits{nullptr, t, geom_id, prim_id, tri, nullptr}, "tr_intersect_arrays");
 }
 
 }  // extern "C"
@@ -2547,23 +2735,21 @@ int tr_occluded_batch(tr_scene s, const tr_ray* rays, uint32_t n, uint8_t* occlu
     if (!s->committed) return fail(TR_ERR_STATE, "tr_occluded_batch: scene not committed");
     if (n == 0) return TR_OK;
     if (!rays || !occluded) return fail(TR_ERR_INVALID, "tr_occluded_batch: null buffer");
-    tr_ray* dr = nullptr;
-    uint8_t* dq = nullptr;
-    int rc;
-    if ((rc = dev_alloc(&dr, n)) || (rc = dev_alloc(&dq, n))) {
-        dev_free(dr);
-        return rc;
-    }
-    int out = TR_OK;
-    if (hipMemcpyAsync(dr, rays, size_t(n) * sizeof(tr_ray), hipMemcpyHostToDevice, s->stream) != hipSuccess)
-        out = fail(TR_ERR_DEVICE, "tr_occluded_batch: upload failed");
-    if (!out) out = tr_occluded_batch_device(s, dr, n, dq, s->stream);
-    if (!out && hipMemcpyAsync(occluded, dq, size_t(n), hipMemcpyDeviceToHost, s->stream) != hipSuccess)
-        out = fail(TR_ERR_DEVICE, "tr_occluded_batch: download failed");
-    if (!out && hipStreamSynchronize(s->stream) != hipSuccess) out = fail(TR_ERR_DEVICE, "tr_occluded_batch: kernel failed");
-    dev_free(dr);
-    dev_free(dq);
-    return out;
+    return query_host<true>(s, host_records(rays), n, HostHits{nullptr, nullptr, nullptr, nullptr, nullptr, occluded},
+                            "tr_occluded_batch");
+}
+
+int tr_occluded_arrays(tr_scene s, const float* org, const float* dir, const float* tnear, uint32_t n_tnear, const float* tfar,
+                       uint32_t n_tfar, double shorten, uint32_t n, uint8_t* occluded)
+{
+    if (!s) return fail(TR_ERR_INVALID, "tr_occluded_arrays: null scene");
+    if (!s->committed) return fail(TR_ERR_STATE, "tr_occluded_arrays: scene not committed");
+    if (n == 0) return TR_OK;
+    if (!org || !dir || !tnear || !tfar || !occluded) return fail(TR_ERR_INVALID, "tr_occluded_arrays: null buffer");
+    if ((n_tnear != 1 && n_tnear != n) || (n_tfar != 1 && n_tfar != n))
+        return fail(TR_ERR_INVALID, "tr_occluded_arrays: tnear and tfar hold one value or one per ray");
+    return query_host<true>(s, HostRays{org, dir, tnear, tfar, false, n_tnear > 1, n_tfar > 1, shorten}, n,
+                            HostHits{nullptr, nullptr, nullptr, nullptr, nullptr, occluded}, "tr_occluded_arrays");
 }
 
 int tr_film_create(tr_film* out, const tr_film_desc* d)

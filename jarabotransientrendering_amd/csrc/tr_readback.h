@@ -22,16 +22,17 @@ namespace trb {
 constexpr size_t kChunk = size_t(2) << 20;
 constexpr size_t kPiece = size_t(512) << 10;  // bytes a thread copies at a time
 constexpr uint32_t kSlots = 8;                // chunks in a large staging block
+constexpr uint32_t kStreams = 4;              // streams of a staging block (hardware queues of a process)
 constexpr int kHelpers = 3;                   // copying threads besides the caller's
 constexpr size_t kPerThread = size_t(1) << 20;  // least bytes per copying thread (starting one takes ~20 us)
 
-// A pinned block with an event per chunk slot, and two streams that take the chunks in turn. Made for
+// A pinned block with an event per chunk slot, and streams that take the chunks in turn. Made for
 // one device, used by one read at a time.
 struct Staging {
     int device = 0;
     uint32_t slots = 0;
     char* host = nullptr;
-    hipStream_t stream[2] = {};
+    hipStream_t stream[kStreams] = {};
     hipEvent_t done[kSlots] = {};
 
     bool make(int dev, uint32_t n)
@@ -180,6 +181,45 @@ hipError_t read_back(void* out, size_t bytes, Launch launch, hipStream_t own = n
     for (int t = 0; t < n_helpers; ++t) helpers[t].join();
     if (error.load() != int(hipSuccess))  // nothing writes the block any more
         for (hipStream_t q : {st->stream[0], st->stream[1], own ? own : st->stream[0]}) (void)hipStreamSynchronize(q);
+    Pool::get().give(st);
+    return hipError_t(error.load());
+}
+
+// Calls work(stream, event, pinned, first, count) for every range of at most `per` items of [0, n), by
+// `threads` threads at once, each with a chunk of pinned memory, an event and (up to kStreams) a stream
+// of its own. `work` returns with nothing of its own in flight, unless it fails. Returns when
+// all ranges are done, or on an error, when nothing is in flight.
+template <class Work>
+hipError_t run_chunks(size_t n, size_t per, uint32_t threads, Work work)
+{
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess) return e;
+    threads = std::min(std::max(threads, 1u), kSlots);
+    Staging* st = Pool::get().take(device, threads * kChunk);
+    if (!st) return hipErrorOutOfMemory;
+    std::atomic<size_t> next{0};
+    std::atomic<int> error{int(hipSuccess)};
+    auto run = [&](uint32_t t) {
+        for (size_t first; error.load() == int(hipSuccess) && (first = next.fetch_add(per)) < n;) {
+            const hipError_t w = work(st->stream[t % kStreams], st->done[t], st->host + t * kChunk, first, std::min(per, n - first));
+            if (w != hipSuccess) error = int(w);
+        }
+    };
+    std::thread helpers[kSlots];
+    uint32_t started = 0;
+    try {
+        for (uint32_t t = 1; t < threads; ++t, ++started)
+            helpers[started] = std::thread([&run, t, device] {
+                (void)hipSetDevice(device);
+                run(t);
+            });
+    } catch (...) {  // no more threads: those that started and this one do the work
+    }
+    run(0);
+    for (uint32_t t = 0; t < started; ++t) helpers[t].join();
+    if (error.load() != int(hipSuccess))  // nothing uses the block any more
+        for (hipStream_t q : st->stream) (void)hipStreamSynchronize(q);
     Pool::get().give(st);
     return hipError_t(error.load());
 }

@@ -60,6 +60,23 @@ class HomogeneousMedium:
         self.sigma_s = tuple(float(x) for x in sigma_s)
 
 
+def _ray_arrays(origins, directions, tnear, tfar):
+    """Number of rays, the arrays that hold them and the arguments that hand those to the library."""
+    o = np.ascontiguousarray(np.asarray(origins, dtype=np.float32).reshape(-1, 3))
+    n = o.shape[0]
+    d = np.asarray(directions, dtype=np.float32).reshape(-1, 3)
+    d = np.ascontiguousarray(d if d.shape[0] == n else np.broadcast_to(d, (n, 3)))
+    kept, args = [o, d], [nat.as_ptr(o), nat.as_ptr(d)]
+    for b in (tnear, tfar):  # one value for all rays, or one each
+        b = np.asarray(b).astype(np.float32, copy=False)
+        while b.ndim > 1 and b.shape[0] == 1:
+            b = b[0]
+        b = b.reshape(1) if b.ndim == 0 else np.ascontiguousarray(np.broadcast_to(b, (n,)))
+        kept.append(b)
+        args += [nat.as_ptr(b), b.shape[0]]
+    return n, kept, args
+
+
 class World:
     """World (src/RayTracing/World.h:95-789): geometry, lights, medium; freeze() builds the BVH."""
 
@@ -155,35 +172,25 @@ class World:
                            tfar: float = math.inf):
         """Batched World::first_intersection (World.h:566-615): returns (t, geom_id, prim_id, tri);
         misses have t = -1 and ids 0xFFFFFFFF."""
-        o = np.asarray(origins, dtype=np.float32).reshape(-1, 3)
-        d = np.asarray(directions, dtype=np.float32).reshape(-1, 3)
-        n = o.shape[0]
-        rays = np.zeros((n, 8), dtype=np.float32)
-        rays[:, 0:3] = o
-        rays[:, 3] = tnear
-        rays[:, 4:7] = d
-        rays[:, 7] = tfar
-        hits = np.zeros((n, 4), dtype=np.uint32)
-        nat.check(nat.lib().tr_intersect_batch(self._h, nat.as_ptr(rays), n, nat.as_ptr(hits)))
-        t = hits[:, 0].view(np.float32).copy()
-        return t, hits[:, 1].copy(), hits[:, 2].copy(), hits[:, 3].copy()
+        n, kept, rays = _ray_arrays(origins, directions, tnear, tfar)
+        t = np.empty(n, dtype=np.float32)
+        ids = [np.empty(n, dtype=np.uint32) for _ in range(3)]
+        nat.check(nat.lib().tr_intersect_arrays(self._h, *rays, n, nat.as_ptr(t), *map(nat.as_ptr, ids)))
+        return t, ids[0], ids[1], ids[2]
 
     def intersects(self, origins: np.ndarray, directions: np.ndarray, max_length=math.inf,
                    epsilon: float = 1e-5) -> np.ndarray:
         """Batched World::intersects (World.h:617-639): True where some triangle is hit in
         (epsilon, max_length - epsilon]; `max_length` may be a scalar or one value per ray, and
         epsilon defaults to _SIGMA_VISIBILITY_ (1e-5), as in the reference."""
-        o = np.asarray(origins, dtype=np.float32).reshape(-1, 3)
-        d = np.asarray(directions, dtype=np.float32).reshape(-1, 3)
-        n = o.shape[0]
-        rays = np.zeros((n, 8), dtype=np.float32)
-        rays[:, 0:3] = o
-        rays[:, 3] = epsilon
-        rays[:, 4:7] = d
-        rays[:, 7] = np.asarray(max_length, dtype=np.float64) - epsilon
-        occ = np.zeros(n, dtype=np.uint8)
-        nat.check(nat.lib().tr_occluded_batch(self._h, nat.as_ptr(rays), n, nat.as_ptr(occ)))
-        return occ.astype(bool)
+        # the length less epsilon in 64 bits; of 32-bit lengths the library takes it off
+        length, shorten = np.asarray(max_length), float(epsilon) if np.ndim(epsilon) == 0 else 0.0
+        if length.dtype != np.float32 or np.ndim(epsilon):
+            length, shorten = np.asarray(max_length, dtype=np.float64) - epsilon, 0.0
+        n, kept, rays = _ray_arrays(origins, directions, epsilon, length)
+        occ = np.empty(n, dtype=bool)  # written as 0 or 1
+        nat.check(nat.lib().tr_occluded_arrays(self._h, *rays, shorten, n, nat.as_ptr(occ)))
+        return occ
 
 
 class PinholeCamera:
