@@ -1360,21 +1360,20 @@ __device__ __forceinline__ void film_add_partial(float* __restrict__ sum, float*
     if (c != 0.0f) unsafeAtomicAdd(comp + i, c);
 }
 
-// film: bins the visible contributions of this bounce into the film. A block takes a range of
+// film: bins the visible contributions of this bounce into the film. A block takes ranges of
 // kFilmRange consecutive shadow records; their pixels are few (paths are enumerated pixel-major
 // and queue compaction keeps runs of neighbouring paths together), so each block accumulates into
 // LDS histograms of up to `pix_slots` pixels x T bins x RGB and flushes each non-zero bin with one
-// compensated add. Records of pixels that find no slot try again after the flush, in a second
-// round with the slots free, and only those left after kFilmRounds rounds go straight to HBM: the
-// range's records come from a few append chunks of the shading kernel, each holding paths of one
-// or two pixels, and the 256-path chunks of guided shading put more pixels in a range than the
-// slots hold (the second round: film time -4 % on the 1024-spp icosphere frames, -7 % on guided
-// media passes).
-// The LDS histograms hold FP64 partials (non-returning LDS atomic adds): a partial of at most
-// kFilmRange float contributions is exact to within 2^-44 of their magnitude sum, far inside the
-// film's compensated FP32 bound, and is flushed as the float pair (hi, lo) = (float(p),
-// float(p - hi)). Short ranges (512 records) measured best: 1.6x faster than 4096-record ranges on
-// the 1024-bin films, whose per-pixel records spread over many bins. The kernel waits on its loads
+// compensated add. A block takes kFilmRun ranges in a row, or the segments of 512 or more paths, and
+// flushes at their end or when a range's pixels find no slot; the records left out then try again, and only
+// those left after kFilmRounds rounds go straight to HBM (a range's records come from a few append chunks of
+// the shading kernel, each holding paths of one or two pixels). Flushing after every range instead made up
+// to three times as many returning atomics as bins: media scanline 164 -> 78 us, guided 366 -> 327, 67 M-path
+// icosphere frame 2.20 -> 2.04 ms (runs of 1, 4, 16 ranges: 2.36, 2.04, 2.13).
+// The LDS histograms hold FP64 partials (non-returning LDS atomic adds): a partial of n float
+// contributions is exact to within n 2^-53 of their magnitude sum (2^-36 for the 130,000 of a group of
+// 4,096 paths with 32 vertices), far inside the film's compensated FP32 bound, and is flushed as the float
+// pair (hi, lo) = (float(p), float(p - hi)). The kernel waits on its loads
 // and returning atomics: 1024-thread blocks (two per CU, 32 wavefronts) ran it 12-16 % faster than
 // 256-thread blocks (three per CU, 12 wavefronts), and 72 KB of LDS per block (three 1024-bin
 // pixels instead of two, still two blocks per CU) 10-14 % faster again.
@@ -1383,7 +1382,8 @@ constexpr int kFilmBlock = 1024;
 constexpr uint32_t kFilmRange = 512;
 constexpr uint32_t kFilmLdsBytes = 72 * 1024;  // FP64 histograms: pix_slots * T * 3 * 8 bytes (3 pixels of 1024 bins)
 constexpr uint32_t kFilmMaxSlots = 8;
-constexpr int kFilmRounds = 2;
+constexpr int kFilmRounds = 3;
+constexpr uint32_t kFilmRun = 4;
 constexpr uint32_t kFilmSegs = 32;  // segments of a path launch that a block takes at a time, at most
 static_assert(kFilmRange <= uint32_t(kFilmBlock), "one record of a range per thread");
 
@@ -1411,18 +1411,35 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
     const uint32_t segs = SEGS ? (Wv.ctl->n + Wv.seg_paths - 1u) / Wv.seg_paths : 0u;
     const uint32_t count = SRC == kFilmSamples ? Q.n : SEGS ? 0u : Wv.counters[shword(sh)];
     if (SRC == kFilmSamples && Q.bad && *Q.bad != 0xFFFFFFFFu) return;
-    // guided renders: ranges of 256 records, about one append chunk of the guided shading kernel's
-    // 256-thread blocks, so a range spans fewer pixels (guided passes' film time -11 %)
-    constexpr uint32_t kRange = GUIDED ? 256u : kFilmRange;
-    const uint32_t groups = SEGS ? (segs + per_group - 1) / per_group : (count + kRange - 1) / kRange;
+    // records that a block takes in a row: a path launch's group of segments, or kFilmRun ranges (fewer where
+    // blocks would go without)
+    const uint32_t run = min(max((count + kFilmRange - 1) / kFilmRange / gridDim.x, 1u), kFilmRun) * kFilmRange;
+    const uint32_t groups = SEGS ? (segs + per_group - 1) / per_group : (count + run - 1) / run;
     if (blockIdx.x >= groups) return;  // no range for this block (the last bounces' launches)
     const uint32_t T = uint32_t(R.T), T3 = 3u * T, hsize = pix_slots * T3;
     const int rounds = pix_slots ? kFilmRounds : 1;
     // the histograms start at zero; each flush reads and clears only the slots that were used
     for (uint32_t i = threadIdx.x; i < hsize; i += blockDim.x) hist[i] = 0.0;
+    if (threadIdx.x < kFilmMaxSlots) slot_pix[threadIdx.x] = 0xFFFFFFFFu;
+    __syncthreads();
+    auto flush = [&]() {
+        for (uint32_t i = threadIdx.x; i < hsize; i += blockDim.x) {
+            const uint32_t k = i / T3;
+            if (slot_pix[k] == 0xFFFFFFFFu) continue;
+            const double v = hist[i];
+            if (v != 0.0) {
+                const float hi = float(v), lo = float(v - double(hi));
+                film_add_partial(R.film, R.film_comp, size_t(slot_pix[k]) * T3 + (i - k * T3), hi, lo);
+                hist[i] = 0.0;
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < kFilmMaxSlots) slot_pix[threadIdx.x] = 0xFFFFFFFFu;
+        __syncthreads();
+    };
     uint32_t group = blockIdx.x, start = 0;  // the range's group of records and first record in it
     while (group < groups) {
-        uint32_t total = kRange;
+        uint32_t total = SEGS ? 0u : min(run, count - group * run);
         if constexpr (SEGS) {
             if (start == 0) {
                 if (threadIdx.x < 64) {
@@ -1439,16 +1456,17 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
             total = seg_end[kFilmSegs - 1];
         }
         // this thread's record of the range, if it is a visible contribution
-        uint32_t r = SEGS ? 0xFFFFFFFFu : group * kRange + threadIdx.x;
-        bool mine = threadIdx.x < kRange && (SEGS ? start + threadIdx.x < total : r < count);
+        const uint32_t j = start + threadIdx.x;
+        const bool mine = threadIdx.x < kFilmRange && j < total;
+        uint32_t r = group * run + j;
         if (SEGS && mine) {
-            const uint32_t j = start + threadIdx.x;
             uint32_t k = 0;
             while (j >= seg_end[k]) ++k;
             r = (group * per_group + k) * Wv.seg_cap + j - (k ? seg_end[k - 1] : 0u);
         }
-        start += kRange;
-        if (start >= total) {
+        start += kFilmRange;
+        const bool last = start >= total;  // of its group
+        if (last) {
             start = 0;
             group += gridDim.x;
         }
@@ -1476,16 +1494,18 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
             pending = true;
         }
         for (int round = 0; round < rounds; ++round) {
-            if (threadIdx.x < kFilmMaxSlots) slot_pix[threadIdx.x] = 0xFFFFFFFFu;
-            if (!__syncthreads_or(pending)) break;
             if (pending) {
+                // neighbouring pixels begin at different slots, so the first one tried is mostly the right one
                 int slot = -1;
-                for (uint32_t k = 0; k < pix_slots; ++k) {
-                    uint32_t v = atomicCAS(&slot_pix[k], 0xFFFFFFFFu, pix);
+                uint32_t k = pix_slots ? pix % pix_slots : 0u;
+                for (uint32_t t = 0; t < pix_slots; ++t) {
+                    uint32_t v = *static_cast<volatile uint32_t*>(&slot_pix[k]);
+                    if (v == 0xFFFFFFFFu) v = atomicCAS(&slot_pix[k], 0xFFFFFFFFu, pix);
                     if (v == 0xFFFFFFFFu || v == pix) {
                         slot = int(k);
                         break;
                     }
+                    k = k + 1 == pix_slots ? 0u : k + 1;
                 }
                 if (slot >= 0) {
                     double* h = hist + uint32_t(slot) * T3 + bin * 3u;
@@ -1498,20 +1518,10 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
                     pending = false;
                 }
             }
-            __syncthreads();
-            uint32_t used = 0;  // slots are claimed in order
-            while (used < pix_slots && slot_pix[used] != 0xFFFFFFFFu) ++used;
-            for (uint32_t i = threadIdx.x; i < used * T3; i += blockDim.x) {
-                const double v = hist[i];
-                if (v != 0.0) {
-                    const uint32_t k = i / T3;
-                    const float hi = float(v), lo = float(v - double(hi));
-                    film_add_partial(R.film, R.film_comp, size_t(slot_pix[k]) * T3 + (i - k * T3), hi, lo);
-                    hist[i] = 0.0;
-                }
-            }
-            __syncthreads();
+            if (!__syncthreads_or(pending)) break;
+            flush();
         }
+        if (last) flush();
     }
 }
 
