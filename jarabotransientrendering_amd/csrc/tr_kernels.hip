@@ -199,11 +199,21 @@ struct WaveCtl {
     uint32_t pad;
 };
 
-__global__ void set_wave_kernel(WaveCtl* ctl, uint64_t base, uint32_t n)
+// (the first wavefront of a render also clears the counters)
+__global__ void __launch_bounds__(kBlock) set_wave_kernel(WaveCtl* ctl, uint64_t base, uint32_t n, uint32_t* counters)
 {
-    ctl->base = base;
-    ctl->n = n;
-    ctl->pad = 0u;
+    if (threadIdx.x == 0) {
+        ctl->base = base;
+        ctl->n = n;
+        ctl->pad = 0u;
+    }
+    if (base == 0)
+        for (uint32_t k = threadIdx.x; k < C_WORDS; k += kBlock) counters[k] = 0u;
+}
+// the counters of a finished render, to pinned host memory
+__global__ void __launch_bounds__(kBlock) read_counters_kernel(const uint32_t* __restrict__ counters, uint32_t* __restrict__ out)
+{
+    for (uint32_t k = threadIdx.x; k < C_WORDS; k += kBlock) out[k] = counters[k];
 }
 
 __device__ __forceinline__ uint64_t u64(uint32_t lo, uint32_t hi) { return uint64_t(lo) | (uint64_t(hi) << 32); }
@@ -2227,8 +2237,11 @@ struct tr_film_s {
     int rows = 0;
     int layers = 0;      // multibounce bounce films (0: one streak film)
     size_t n_elems = 0;  // max(layers, 1) * rows*W*T*3
-    float *d_sum = nullptr, *d_comp = nullptr;        // compensated sums: sum + comp = film
-    float *d_layer_w = nullptr, *d_steady = nullptr;  // multibounce films only (steady: sums, then comps)
+    // one allocation, cleared as a whole: compensated sums (sum + comp = film) and, of multibounce films, the
+    // layers' weights and the steady image (sums, then comps)
+    float *d_sum = nullptr, *d_comp = nullptr;
+    float *d_layer_w = nullptr, *d_steady = nullptr;
+    size_t device_floats = 0;
     float* d_read_steady = nullptr;  // steady image on its way to the host (allocated by the first read of one)
     double* d_read_w = nullptr;      // per-pixel weights: uploaded by reads of films with caller-made samples,
                                      // summed by tr_film_add_samples
@@ -2833,18 +2846,25 @@ int tr_film_create(tr_film* out, const tr_film_desc* d)
     f->rows = rows;
     f->layers = layers;
     f->n_elems = n;
-    auto release = [&]() {
-        dev_free(f->d_sum); dev_free(f->d_comp); dev_free(f->d_layer_w); dev_free(f->d_steady);
+    auto part = [&](size_t count) {  // 256-byte aligned
+        const size_t at = f->device_floats;
+        f->device_floats += (count + 63) / 64 * 64;
+        return at;
     };
-    if ((rc = dev_alloc(&f->d_sum, n)) || (rc = dev_alloc(&f->d_comp, n)) ||
-        (layers && ((rc = dev_alloc(&f->d_layer_w, size_t(layers) * rows * size_t(d->width))) ||
-                    (rc = dev_alloc(&f->d_steady, size_t(rows) * size_t(d->width) * 6))))) {
-        release();
+    const size_t px = size_t(rows) * size_t(d->width);
+    part(n);
+    const size_t comp = part(n), layer_w = part(size_t(layers) * px), steady = part(layers ? px * 6 : 0);
+    if ((rc = dev_alloc(&f->d_sum, f->device_floats))) {
         delete f;
         return rc;
     }
+    f->d_comp = f->d_sum + comp;
+    if (layers) {
+        f->d_layer_w = f->d_sum + layer_w;
+        f->d_steady = f->d_sum + steady;
+    }
     if (hipStreamCreateWithFlags(&f->stream, hipStreamNonBlocking) != hipSuccess) {
-        release();
+        dev_free(f->d_sum);
         delete f;
         return fail(TR_ERR_DEVICE, "tr_film_create: hipStreamCreate failed");
     }
@@ -2862,7 +2882,7 @@ int tr_film_destroy(tr_film f)
 {
     if (!f) return TR_OK;
     if (f->stream) (void)hipStreamSynchronize(f->stream);
-    dev_free(f->d_sum); dev_free(f->d_comp); dev_free(f->d_layer_w); dev_free(f->d_steady);
+    dev_free(f->d_sum);
     dev_free(f->d_samples); dev_free(f->d_read_steady); dev_free(f->d_read_w);
     if (f->stream) (void)hipStreamDestroy(f->stream);
     delete f;
@@ -2872,14 +2892,7 @@ int tr_film_destroy(tr_film f)
 int tr_film_clear(tr_film f)
 {
     if (!f) return fail(TR_ERR_INVALID, "tr_film_clear: null film");
-    const size_t bytes = f->n_elems * sizeof(float);
-    HIP_TRY(hipMemsetAsync(f->d_sum, 0, bytes, f->stream));
-    HIP_TRY(hipMemsetAsync(f->d_comp, 0, bytes, f->stream));
-    if (f->layers) {
-        const size_t px = size_t(f->rows) * size_t(f->desc.width);
-        HIP_TRY(hipMemsetAsync(f->d_layer_w, 0, size_t(f->layers) * px * sizeof(float), f->stream));
-        HIP_TRY(hipMemsetAsync(f->d_steady, 0, px * 6 * sizeof(float), f->stream));
-    }
+    HIP_TRY(hipMemsetAsync(f->d_sum, 0, f->device_floats * sizeof(float), f->stream));
     HIP_TRY(hipStreamSynchronize(f->stream));
     std::fill(f->weight.begin(), f->weight.end(), 0.0);
     f->same_weight = true;
@@ -3437,10 +3450,12 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     if (jobs.empty()) return fail(TR_ERR_INVALID, "render: no job");
     // every return drains the stream, so no queued copy or kernel outlives the host buffers and
     // device views it was given (the normal path synchronises as well, to read the counters)
+    trb::Lease pinned;  // (given back after that)
     struct Drain {
         hipStream_t s;
         ~Drain() { (void)hipStreamSynchronize(s); }
     } drain{stream};
+    if (!pinned.take()) return fail(TR_ERR_NOMEM, "render: pinned memory");
     const bool batch = jobs.size() > 1;
     if (batch && guide) return fail(TR_ERR_INVALID, "render: guided renders take one job");
     uint64_t total = 0;
@@ -3542,7 +3557,6 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
         L.pix_slots = std::min<uint32_t>(kFilmMaxSlots, kFilmLdsBytes / (T * 24u));
         L.film_lds = size_t(L.pix_slots) * size_t(T) * 24u;
     }
-    HIP_TRY(hipMemsetAsync(wb.counters, 0, C_WORDS * sizeof(uint32_t), stream));
     // pass buffers are written on this stream; order it after any pending film work
     for (auto& j : jobs) HIP_TRY(hipStreamSynchronize(j.film->stream));
 
@@ -3563,7 +3577,7 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
         for (uint64_t base = 0; base < total && !rc; base += c.wave) {
             const uint32_t n = uint32_t(std::min<uint64_t>(c.wave, total - base));
             ++n_waves;
-            set_wave_kernel<<<1, 1, 0, stream>>>(wb.ctl, base, n);
+            set_wave_kernel<<<1, kBlock, 0, stream>>>(wb.ctl, base, n, wb.counters);
             rc = L.enqueue_wave();
         }
         const hipError_t ce = hipStreamEndCapture(stream, &graph);
@@ -3591,7 +3605,7 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
                 return rc;
             }
         }
-        set_wave_kernel<<<1, 1, 0, stream>>>(wb.ctl, base, n);
+        set_wave_kernel<<<1, kBlock, 0, stream>>>(wb.ctl, base, n, wb.counters);
         if (c.graph) {
             if (!exec) {
                 uint32_t launches_before[TR_K_COUNT];
@@ -3630,8 +3644,9 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
             }
         }
     }
-    uint32_t counters[C_WORDS];
-    hipError_t e = hipMemcpyAsync(counters, wb.counters, sizeof counters, hipMemcpyDeviceToHost, stream);
+    uint32_t* const counters = reinterpret_cast<uint32_t*>(pinned.host());
+    read_counters_kernel<<<1, kBlock, 0, stream>>>(wb.counters, counters);
+    hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(stream);
     drop_graph();
     if (rc) return rc;

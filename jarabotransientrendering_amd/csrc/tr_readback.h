@@ -26,7 +26,7 @@ constexpr uint32_t kStreams = 4;              // streams of a staging block (har
 constexpr int kHelpers = 3;                   // copying threads besides the caller's
 constexpr size_t kPerThread = size_t(1) << 20;  // least bytes per copying thread (starting one takes ~20 us)
 
-// A pinned block with an event per chunk slot, and streams that take the chunks in turn. Made for
+// A pinned block with an event per chunk slot, and streams that take the chunks in turn (one for one slot). Made for
 // one device, used by one read at a time.
 struct Staging {
     int device = 0;
@@ -43,11 +43,16 @@ struct Staging {
             host = nullptr;
             return false;
         }
-        for (hipStream_t& q : stream)
-            if (hipStreamCreateWithFlags(&q, hipStreamNonBlocking) != hipSuccess) return q = nullptr, false;
+        for (uint32_t k = 0; k < std::min(n, kStreams); ++k)
+            if (hipStreamCreateWithFlags(&stream[k], hipStreamNonBlocking) != hipSuccess) return stream[k] = nullptr, false;
         for (uint32_t k = 0; k < n; ++k)
             if (hipEventCreateWithFlags(&done[k], hipEventDisableTiming) != hipSuccess) return done[k] = nullptr, false;
         return true;
+    }
+    void wait()
+    {
+        for (hipStream_t q : stream)
+            if (q) (void)hipStreamSynchronize(q);
     }
     ~Staging()
     {
@@ -59,7 +64,8 @@ struct Staging {
     }
 };
 
-// Blocks kept between reads, for any thread: at most kKept of each size, 36 MiB in all. The pool
+// Blocks kept between calls, for any thread: at most 8 of one chunk (a render holds one too) and 2 large
+// ones, 48 MiB in all. The pool
 // lives until the process ends (its blocks are not freed after the runtime has shut down).
 class Pool {
 public:
@@ -93,7 +99,7 @@ public:
             std::lock_guard<std::mutex> lock(mutex_);
             int same = 0;
             for (Staging* f : free_) same += f && f->slots == s->slots;
-            if (same < kKept)
+            if (same < (s->slots == 1 ? kKeptSmall : kKeptLarge))
                 for (Staging*& f : free_)
                     if (!f) {
                         f = s;
@@ -104,9 +110,32 @@ public:
     }
 
 private:
-    static constexpr int kKept = 2;
+    static constexpr int kKeptSmall = 8, kKeptLarge = 2;
     std::mutex mutex_;
-    Staging* free_[2 * kKept] = {};
+    Staging* free_[kKeptSmall + kKeptLarge] = {};
+};
+
+// A small pinned block for as long as this object lives.
+class Lease {
+public:
+    Lease() = default;
+    Lease(const Lease&) = delete;
+    Lease& operator=(const Lease&) = delete;
+    ~Lease()
+    {
+        if (block_) Pool::get().give(block_);
+    }
+    bool take()
+    {
+        int device = 0;
+        if (hipGetDevice(&device) != hipSuccess) return false;
+        block_ = Pool::get().take(device, 1);
+        return block_ != nullptr;
+    }
+    char* host() const { return block_->host; }
+
+private:
+    Staging* block_ = nullptr;
 };
 
 // Fills out[0, bytes) with what `launch(stream, dst, offset, size)` makes the GPU write to the pinned
@@ -179,8 +208,10 @@ hipError_t read_back(void* out, size_t bytes, Launch launch, hipStream_t own = n
         }
     }
     for (int t = 0; t < n_helpers; ++t) helpers[t].join();
-    if (error.load() != int(hipSuccess))  // nothing writes the block any more
-        for (hipStream_t q : {st->stream[0], st->stream[1], own ? own : st->stream[0]}) (void)hipStreamSynchronize(q);
+    if (error.load() != int(hipSuccess)) {  // nothing writes the block any more
+        st->wait();
+        if (own) (void)hipStreamSynchronize(own);
+    }
     Pool::get().give(st);
     return hipError_t(error.load());
 }
@@ -218,8 +249,7 @@ hipError_t run_chunks(size_t n, size_t per, uint32_t threads, Work work)
     }
     run(0);
     for (uint32_t t = 0; t < started; ++t) helpers[t].join();
-    if (error.load() != int(hipSuccess))  // nothing uses the block any more
-        for (hipStream_t q : st->stream) (void)hipStreamSynchronize(q);
+    if (error.load() != int(hipSuccess)) st->wait();  // nothing uses the block any more
     Pool::get().give(st);
     return hipError_t(error.load());
 }
