@@ -60,15 +60,16 @@ constexpr uint32_t kShadowRecords = 1u << 28;
 // smaller where their buffers would take more than a quarter of the free memory.
 constexpr uint32_t kSmallWave = 1u << 25;
 // Largest wavefronts whose bounces run in one launch (path_kernel) instead of two per bounce. A render of
-// 2^10 paths through the two: 163 and 84 us (22 triangles), 642 and 363 (81,930 triangles), 370 and 183 (a
-// medium, 16 bounces); of 2^18 paths 200 and 100, 1,074 and 586, 540 and 224; of 2^20 paths 303 and 219,
-// 1,476 and 1,210, 933 and 530; and 751 and 746 with 1,290 triangles, where longer queues win from here on
-// (2^21 paths: 948 and 1,337). In a medium over a shallow tree, where a path has many vertices and a ray's
-// length hardly varies, the launch still wins with 2^22 paths (2,183 and 1,640; 2^24: 6,833 and 6,213).
+// 2^10 paths through the two: 163 and 84 us (22 triangles), 642 and 266 (81,930 triangles), 370 and 161 (a
+// medium, 16 bounces); of 2^18 paths 200 and 100, 1,074 and 586, 540 and 224; of 2^20 paths 276 and 196,
+// 1,450 and 1,196, 906 and 484; and 719 and 718 with 1,290 triangles, where longer queues win from here on
+// (2^21 paths: 915 and 1,158). Over a tree of a few nodes, where a ray's length hardly varies, the launch
+// still wins with 2^22 paths (618 and 571; medium 2,137 and 1,525) and 2^23 (1,134 and 971; 3,745 and 2,840),
+// but no longer with 2^24 (1,929 and 2,026; 6,485 and 5,494), nor over 90 triangles (2^22: 1,285 and 1,585).
 constexpr uint32_t kPathWave = 1u << 20;
-constexpr uint32_t kPathWaveMedium = 1u << 22;
-constexpr uint32_t kShallowNodes = 64;  // 4-wide nodes of a shallow tree
-constexpr uint32_t kPathSegs = kPathWaveMedium / 64;  // GPU wavefronts of a path launch, at most
+constexpr uint32_t kPathWaveShallow = 1u << 23;
+constexpr uint32_t kShallowNodes = 5;  // 4-wide nodes of a shallow tree
+constexpr uint32_t kPathSegs = 1u << 15;  // GPU wavefronts of a path launch, at most
 constexpr int kPathRefill = 8;  // idle lanes that begin new paths (24: 2 % slower in a medium)
 constexpr uint32_t kFetchMax = 512;  // rays per work fetch of a traversal wavefront (upper bound)
 constexpr uint32_t kTraceRaysPerThread = 8;   // lower bound on a full wavefront's rays per traversal thread
@@ -1099,9 +1100,10 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
 // in place of the camera launch, an extend and a shade launch per bounce and the shadow launch. Those take
 // 10-20 us each however few paths there are (a launch, and a ray's chain of node reads), and each waits for
 // the longest ray of the one before it; here a GPU wavefront waits for its own rays only. It loses lanes as
-// paths end, which the queues' compaction avoids, so it begins new paths in them where it has more than 64
-// (media: 2^21 paths 1,116 us with 64 paths per wavefront, 898 with 256; where paths are short, or none
-// ends early, 64 are as fast or faster), and large wavefronts keep the queues (kPathWave). Where there are
+// paths end, which the queues' compaction avoids, so over shallow trees it begins new paths in them: it takes
+// 256 paths from 2^21 on and 512 of 2^23 (a medium, 2^21 paths: 1,062 us with 64 paths per wavefront, 828
+// with 256; 2^23: 3,971 and, with 512, 2,840; over larger trees 64 are as fast or faster where the launch
+// wins), and large wavefronts keep the queues (kPathWave). Where there are
 // fewer than two GPU wavefronts of 64 per SIMD, each takes 32 or 16 paths: fewer lanes wait for the longest
 // ray and for each other's branches (1,290 triangles, 2^14 paths: 267, 227, 207 us with 64, 32, 16;
 // 81,930 triangles 444, 366, 343; a medium 169, 162, 158), but not over 22 triangles without a medium,
@@ -3515,10 +3517,10 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     L.batch = batch;
     L.bounces = bounces;
     L.group = int(group);
-    L.path_launch = !guide && bounces > 0 && c.wave <= (medium && shallow ? kPathWaveMedium : kPathWave) &&
+    L.path_launch = !guide && bounces > 0 && c.wave <= (shallow ? kPathWaveShallow : kPathWave) &&
                     group == uint32_t(bounces) && (trav_ext == kTravWide || trav_ext == kTravWide16);
     L.path_per_wave = 64u;
-    if (medium && shallow && !jobs[0].dev.R.time_sampling) L.path_per_wave *= std::max(1u, c.wave >> 19);
+    if (shallow) L.path_per_wave *= std::max({1u, std::min(4u, c.wave >> 19), c.wave >> 20});
     if (medium || !shallow)
         while (L.path_per_wave > 16u && c.wave <= L.path_per_wave * 1024u) L.path_per_wave /= 2u;
     L.stack_bound = stack_bound;
