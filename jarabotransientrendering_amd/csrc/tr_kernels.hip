@@ -1039,7 +1039,7 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
                 if (!(usel < alpha)) {
                     float ul = pcg_float(pst, pinc);
                     e1 = pcg_float(pst, pinc), e2 = pcg_float(pst, pinc);
-                    trg::Lobe L = trg::lobe_of(mix, trg::pick_lobe(mix, ul));
+                    trg::Lobe L = trg::pick_lobe(mix, ul);
                     trg::vmf_sample(L, e1, e2, &nd.x, &nd.y, &nd.z);
                 }
                 float q = trg::mixture_pdf(mix, nd.x, nd.y, nd.z);
