@@ -30,6 +30,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "tr_api.h"
@@ -1536,24 +1537,15 @@ __global__ void __launch_bounds__(kFilmBlock) film_kernel(RenderDev R, WaveDev W
     }
 }
 
-// caller-made samples before they are deposited: the first one outside the film (of `rows` rows), and
-// each pixel's added weight
-__global__ void __launch_bounds__(kBlock) samples_begin_kernel(double* __restrict__ weight, uint32_t pixels, uint32_t* bad)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < pixels) weight[i] = 0.0;
-    if (i == 0) *bad = 0xFFFFFFFFu;
-}
+// index of the first caller-made sample outside the film (of `rows` rows), before they are deposited
+__global__ void samples_begin_kernel(uint32_t* bad) { *bad = 0xFFFFFFFFu; }
 __global__ void __launch_bounds__(kBlock) samples_check_kernel(const tr_film_sample* __restrict__ samples, uint32_t n,
-                                                               int32_t W, int32_t row0, int32_t rows,
-                                                               double* __restrict__ weight, uint32_t* bad)
+                                                               int32_t W, int32_t row0, int32_t rows, uint32_t* bad)
 {
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const int2 at = *reinterpret_cast<const int2*>(samples + i);
         const int32_t row = int32_t(uint32_t(at.y) - uint32_t(row0));
         if (at.x < 0 || at.x >= W || row < 0 || row >= rows) atomicMin(bad, i);
-        else if (samples[i].weight != 0.0f)
-            unsafeAtomicAdd(weight + size_t(row) * size_t(W) + size_t(at.x), double(samples[i].weight));
     }
 }
 
@@ -2245,12 +2237,12 @@ struct tr_film_s {
     float *d_layer_w = nullptr, *d_steady = nullptr;
     size_t device_floats = 0;
     float* d_read_steady = nullptr;  // steady image on its way to the host (allocated by the first read of one)
-    double* d_read_w = nullptr;      // per-pixel weights: uploaded by reads of films with caller-made samples,
-                                     // summed by tr_film_add_samples
+    double* d_read_w = nullptr;      // per-pixel weights, uploaded by reads of films with caller-made samples
     tr_film_sample* d_samples = nullptr;  // caller-made samples being added, behind a 256-byte head (first bad index)
     size_t samples_cap = 0;
     std::vector<double> weight;      // rows*W
     bool same_weight = true;         // every pixel has the same weight (no caller-made samples)
+    std::vector<double> added;       // weights of the samples being added, per pixel (zeros between calls)
     hipStream_t stream = nullptr;
 };
 
@@ -3059,9 +3051,13 @@ int tr_film_device_buffers(tr_film f, float** d_sum, float** d_comp)
 // StreakCameraFilm::add_samples for caller-made samples: checked, binned as the reference bins
 // (pos_sensor = (time - offset) / exposure, kept if 0 <= pos_sensor < T; StreakCameraFilm.h:165-171) and
 // deposited on the device, by the renders' own film kernel. (Binned on the host into shadow-record
-// arrays, 500,000 samples took 1.5 ms on one thread and 0.6 ms of allocations and extra copies.) Up to
-// kHostSamples are checked and their weights summed by the host, 1-2 ns each, while the device's two more
-// launches and two more copies take 30 us.
+// arrays, 500,000 samples took 1.5 ms on one thread and 0.6 ms of allocations and extra copies.) The
+// weights are summed by the host, per pixel in the order of the samples, so that the same calls give the
+// same bits: 1-2 ns each. Up to kHostSamples they are checked by the host too, as the device's two launches take
+// longer; larger calls sum while the device works, and calls of kThreadSamples or more already while the
+// runtime copies the samples (500,000: 480 us on one thread), by a second thread where there are at least as
+// many samples as pixels (fewer are scattered over lines of another core's cache: 17,000 over 256 x 256
+// pixels took 300 us, and take 66). Nothing that follows the deposit needs memory.
 int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
 {
     if (!f) return fail(TR_ERR_INVALID, "tr_film_add_samples: null film");
@@ -3073,25 +3069,65 @@ int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
     const uint32_t T = uint32_t(fd.time_bins), P = uint32_t(f->weight.size());
     const int32_t row0 = fd.scanline >= 0 ? fd.scanline : 0;
     constexpr size_t kHead = 256 / sizeof(tr_film_sample), kKept = size_t(32) << 20;  // samples buffers up to 32 MiB are kept
-    constexpr uint32_t kHostSamples = 16384;
+    constexpr uint32_t kHostSamples = 16384, kThreadSamples = 131072;
     const bool on_host = n <= kHostSamples;
+    try {
+        f->added.resize(P, 0.0);
+    } catch (const std::bad_alloc&) {
+        return fail(TR_ERR_NOMEM, "tr_film_add_samples: host allocation");
+    }
+    // sums the weights into f->added; stops at the first sample outside the film
     uint32_t first_bad = 0xFFFFFFFFu;
+    auto pixel = [&](uint32_t i) {
+        const uint32_t x = uint32_t(samples[i].x), row = uint32_t(samples[i].y) - uint32_t(row0);
+        return x < uint32_t(fd.width) && row < uint32_t(f->rows) ? row * uint32_t(fd.width) + x : 0xFFFFFFFFu;
+    };
+    auto sum_weights = [&]() {
+        uint32_t at = 0xFFFFFFFFu;  // a run of samples of one pixel
+        double sum = 0.0;
+        for (uint32_t i = 0; i < n; ++i) {
+            const uint32_t p = pixel(i);
+            if (p == 0xFFFFFFFFu) {
+                first_bad = i;
+                break;
+            }
+            if (p != at) {
+                if (at != 0xFFFFFFFFu) f->added[at] = sum;
+                at = p;
+                sum = f->added[p];
+            }
+            sum += double(samples[i].weight);
+        }
+        if (at != 0xFFFFFFFFu) f->added[at] = sum;
+    };
+    // calls use(p) at least once for each pixel that sum_weights has added to
+    auto each_pixel = [&](auto use) {
+        const uint32_t m = std::min(n, first_bad);
+        if (m < P / 16)
+            for (uint32_t i = 0; i < m; ++i) use(pixel(i));
+        else
+            for (uint32_t p = 0; p < P; ++p) use(p);
+    };
     auto outside = [&]() {
+        each_pixel([&](uint32_t p) { f->added[p] = 0.0; });
         return fail(TR_ERR_INVALID, "tr_film_add_samples: sample " + std::to_string(first_bad) + " lies outside the film");
     };
-    if (on_host) {
-        for (uint32_t i = 0; i < n && first_bad == 0xFFFFFFFFu; ++i)
-            if (samples[i].x < 0 || samples[i].x >= fd.width || samples[i].y < row0 || int64_t(samples[i].y) - row0 >= f->rows)
-                first_bad = i;
-        if (first_bad != 0xFFFFFFFFu) return outside();
-    }
     int rc;
-    if (!on_host && !f->d_read_w && (rc = dev_alloc(&f->d_read_w, P))) return rc;
     if (f->samples_cap < n) {
         dev_free(f->d_samples);
         f->samples_cap = 0;
         if ((rc = dev_alloc(&f->d_samples, kHead + n))) return rc;
         f->samples_cap = n;
+    }
+    std::thread summing;
+    if (on_host) {
+        sum_weights();
+        if (first_bad != 0xFFFFFFFFu) return outside();
+    } else if (n >= kThreadSamples && n >= P) {
+        try {
+            summing = std::thread(sum_weights);
+        } catch (...) {  // no more threads: below
+        }
     }
     uint32_t* bad = reinterpret_cast<uint32_t*>(f->d_samples);
     tr_film_sample* d = f->d_samples + kHead;
@@ -3108,41 +3144,37 @@ int tr_film_add_samples(tr_film f, const tr_film_sample* samples, uint32_t n)
     const size_t lds = size_t(pix_slots) * size_t(T) * 24u;
     const uint32_t cu = uint32_t(tri::compute_units());
     const uint32_t fg = std::max(1u, std::min((n + kFilmRange - 1) / kFilmRange, cu * 4u));
-    hipError_t e = hipSuccess;
-    if (!on_host) {
-        samples_begin_kernel<<<(P + kBlock - 1) / kBlock, kBlock, 0, f->stream>>>(f->d_read_w, P, bad);
+    hipError_t e = hipMemcpyAsync(d, samples, size_t(n) * sizeof(tr_film_sample), hipMemcpyHostToDevice, f->stream);
+    if (e == hipSuccess && !on_host) {
+        samples_begin_kernel<<<1, 1, 0, f->stream>>>(bad);
+        samples_check_kernel<<<std::min((n + kBlock - 1) / kBlock, cu * 16u), kBlock, 0, f->stream>>>(
+            d, n, fd.width, row0, f->rows, bad);
         e = hipGetLastError();
     }
-    if (e == hipSuccess) e = hipMemcpyAsync(d, samples, size_t(n) * sizeof(tr_film_sample), hipMemcpyHostToDevice, f->stream);
     if (e == hipSuccess) {
-        if (!on_host)
-            samples_check_kernel<<<std::min((n + kBlock - 1) / kBlock, cu * 16u), kBlock, 0, f->stream>>>(
-                d, n, fd.width, row0, f->rows, f->d_read_w, bad);
         film_kernel<kFilmSamples><<<fg, kFilmBlock, lds, f->stream>>>(R, WaveDev{}, 0, pix_slots, nullptr,
                                                                      SamplesDev{d, n, on_host ? nullptr : bad});
         e = hipGetLastError();
     }
-    if (!on_host && e == hipSuccess) e = hipMemcpyAsync(&first_bad, bad, sizeof first_bad, hipMemcpyDeviceToHost, f->stream);
-    // the copies read the caller's samples and write this frame's variables: wait in any case
+    if (summing.joinable()) summing.join();
+    else if (!on_host) sum_weights();
+    // the copy reads the caller's samples: wait in any case
     const hipError_t se = hipStreamSynchronize(f->stream);
     if (e == hipSuccess) e = se;
-    std::vector<double> wadd(on_host ? 0 : P);
-    if (!on_host && e == hipSuccess && first_bad == 0xFFFFFFFFu) {
-        e = trb::read_back(wadd.data(), P * sizeof(double), [&](hipStream_t stream, void* dst, size_t at, size_t size) {
-            return hipMemcpyAsync(dst, reinterpret_cast<const char*>(f->d_read_w) + at, size, hipMemcpyDeviceToHost, stream);
-        });
-    }
     if (f->samples_cap * sizeof(tr_film_sample) > kKept) {
         dev_free(f->d_samples);
         f->samples_cap = 0;
     }
-    if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string("tr_film_add_samples: ") + hipGetErrorString(e));
     if (first_bad != 0xFFFFFFFFu) return outside();
+    if (e != hipSuccess) {
+        each_pixel([&](uint32_t p) { f->added[p] = 0.0; });
+        return fail(TR_ERR_DEVICE, std::string("tr_film_add_samples: ") + hipGetErrorString(e));
+    }
     f->same_weight = false;
-    for (size_t p = 0; p < wadd.size(); ++p) f->weight[p] += wadd[p];
-    if (on_host)
-        for (uint32_t i = 0; i < n; ++i)
-            f->weight[size_t(samples[i].y - row0) * size_t(fd.width) + size_t(samples[i].x)] += double(samples[i].weight);
+    each_pixel([&](uint32_t p) {
+        f->weight[p] += f->added[p];
+        f->added[p] = 0.0;
+    });
     return TR_OK;
 }
 
