@@ -913,7 +913,8 @@ int tr_guide_gradient(tr_guide g, const float* records, uint32_t n, float* grad,
             g->partial, g->partial_loss, tg, n, static_cast<float*>(dst));
         return hipGetLastError();
     }, g->stream);
-    if (e != hipSuccess) return tri::fail(TR_ERR_DEVICE, std::string("tr_guide_gradient: ") + hipGetErrorString(e));
+    if (e != hipSuccess)
+        return tri::fail(e == hipErrorOutOfMemory ? TR_ERR_NOMEM : TR_ERR_DEVICE, std::string("tr_guide_gradient: ") + hipGetErrorString(e));
     std::memcpy(grad, out.data(), kParams * sizeof(float));
     if (loss) *loss = out[kParams];
     return TR_OK;

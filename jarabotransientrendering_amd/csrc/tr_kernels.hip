@@ -2609,7 +2609,7 @@ struct HostHits {
 // 1.60 ms, 8 threads 1.47). In all, with buffers made for each call, the runtime's copies and records
 // packed by the caller, 262,144 rays took 2,700 us and take 500; 1,000 took 74 and take 50.
 constexpr uint32_t kQueryChunk = 32768;
-constexpr uint32_t kMaxQueryThreads = trb::kStreams;
+constexpr uint32_t kMaxQueryThreads = 4;
 constexpr uint32_t kQueryPerWave = 16;
 static_assert(kQueryChunk * (sizeof(tr_ray) + sizeof(tr_hit)) + 64 <= trb::kChunk, "a launch's rays and answers fit a chunk");
 
@@ -2623,7 +2623,9 @@ int query_host(tr_scene s, const HostRays& in, uint32_t n, const HostHits& out, 
     while (per_wave < kQueryPerWave && per_wave * 2048u < n) per_wave *= 2u;
     const SceneDev S = s->view();
     const uint32_t threads = uint32_t(std::min<uint64_t>(kMaxQueryThreads, (uint64_t(n) + kQueryChunk - 1) / kQueryChunk));
-    const hipError_t e = trb::run_chunks(n, kQueryChunk, threads, [&](hipStream_t q, hipEvent_t done, char* host, size_t first, size_t m) {
+    const hipError_t e = trb::run_chunks(n, kQueryChunk, threads, [&](const trb::Chunk& chunk, size_t first, size_t m) {
+        const hipStream_t q = chunk.stream;
+        char* const host = chunk.host;
         // in: the rays; then, 16-byte aligned, the answers
         RayArrays r{};
         r.shorten = in.shorten;
@@ -2663,8 +2665,8 @@ int query_host(tr_scene s, const HostRays& in, uint32_t n, const HostHits& out, 
             launch_query<ANY, kTravWide16, false>(bound, grid, q, S, r, h, s->d_ids, uint32_t(m), per_wave);
         else launch_query<ANY, kTravWide, false>(bound, grid, q, S, r, h, s->d_ids, uint32_t(m), per_wave);
         hipError_t err = hipGetLastError();
-        if (err == hipSuccess) err = hipEventRecord(done, q);
-        if (err == hipSuccess) err = hipEventSynchronize(done);
+        if (err == hipSuccess) err = hipEventRecord(chunk.done, q);
+        if (err == hipSuccess) err = hipEventSynchronize(chunk.done);
         if (err != hipSuccess) return err;
         if (ANY) {
             std::memcpy(out.occluded + first, h.occluded, m);
@@ -2912,7 +2914,8 @@ int film_values(tr_film f, size_t first, size_t n, const FilmWeight& w, Out* out
             f->d_sum + i, f->d_comp + i, w, i / T3, uint32_t(i % T3), T3, m, i % 4 == 0, static_cast<Out*>(dst));
         return hipGetLastError();
     }, own);
-    if (e != hipSuccess) return fail(TR_ERR_DEVICE, std::string("tr_film_read: ") + hipGetErrorString(e));
+    if (e != hipSuccess)
+        return fail(e == hipErrorOutOfMemory ? TR_ERR_NOMEM : TR_ERR_DEVICE, std::string("tr_film_read: ") + hipGetErrorString(e));
     return TR_OK;
 }
 
@@ -3484,12 +3487,12 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     if (jobs.empty()) return fail(TR_ERR_INVALID, "render: no job");
     // every return drains the stream, so no queued copy or kernel outlives the host buffers and
     // device views it was given (the normal path synchronises as well, to read the counters)
-    trb::Lease pinned;  // (given back after that)
+    trb::Chunks pinned;  // (given back after that)
     struct Drain {
         hipStream_t s;
         ~Drain() { (void)hipStreamSynchronize(s); }
     } drain{stream};
-    if (!pinned.take()) return fail(TR_ERR_NOMEM, "render: pinned memory");
+    if (pinned.take(1) != hipSuccess) return fail(TR_ERR_NOMEM, "render: pinned memory");
     const bool batch = jobs.size() > 1;
     if (batch && guide) return fail(TR_ERR_INVALID, "render: guided renders take one job");
     uint64_t total = 0;
@@ -3678,7 +3681,7 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
             }
         }
     }
-    uint32_t* const counters = reinterpret_cast<uint32_t*>(pinned.host());
+    uint32_t* const counters = reinterpret_cast<uint32_t*>(pinned[0].host);
     read_counters_kernel<<<1, kBlock, 0, stream>>>(wb.counters, counters);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess) e = hipStreamSynchronize(stream);

@@ -21,52 +21,38 @@ namespace trb {
 // blocks raise a flag per MiB was slower, 24 GB/s: a release to the host per block costs more.)
 constexpr size_t kChunk = size_t(2) << 20;
 constexpr size_t kPiece = size_t(512) << 10;  // bytes a thread copies at a time
-constexpr uint32_t kSlots = 8;                // chunks in a large staging block
-constexpr uint32_t kStreams = 4;              // streams of a staging block (hardware queues of a process)
+constexpr uint32_t kSlots = 8;                // chunks that one call uses at most
 constexpr int kHelpers = 3;                   // copying threads besides the caller's
 constexpr size_t kPerThread = size_t(1) << 20;  // least bytes per copying thread (starting one takes ~20 us)
 
-// A pinned block with an event per chunk slot, and streams that take the chunks in turn (one for one slot). Made for
-// one device, used by one read at a time.
-struct Staging {
+// A chunk of pinned memory with a stream and an event, made for one device and used by one call at a time.
+struct Chunk {
     int device = 0;
-    uint32_t slots = 0;
     char* host = nullptr;
-    hipStream_t stream[kStreams] = {};
-    hipEvent_t done[kSlots] = {};
+    hipStream_t stream = nullptr;
+    hipEvent_t done = nullptr;
 
-    bool make(int dev, uint32_t n)
+    bool make(int dev)
     {
         device = dev;
-        slots = n;
-        if (hipHostMalloc(reinterpret_cast<void**>(&host), n * kChunk, hipHostMallocDefault) != hipSuccess) {
-            host = nullptr;
-            return false;
-        }
-        for (uint32_t k = 0; k < std::min(n, kStreams); ++k)
-            if (hipStreamCreateWithFlags(&stream[k], hipStreamNonBlocking) != hipSuccess) return stream[k] = nullptr, false;
-        for (uint32_t k = 0; k < n; ++k)
-            if (hipEventCreateWithFlags(&done[k], hipEventDisableTiming) != hipSuccess) return done[k] = nullptr, false;
+        if (hipHostMalloc(reinterpret_cast<void**>(&host), kChunk, hipHostMallocDefault) != hipSuccess) return host = nullptr, false;
+        if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) return stream = nullptr, false;
+        if (hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) return done = nullptr, false;
         return true;
     }
-    void wait()
+    ~Chunk()
     {
-        for (hipStream_t q : stream)
-            if (q) (void)hipStreamSynchronize(q);
-    }
-    ~Staging()
-    {
-        for (hipEvent_t e : done)
-            if (e) (void)hipEventDestroy(e);
-        for (hipStream_t q : stream)
-            if (q) (void)hipStreamDestroy(q);
+        if (done) (void)hipEventDestroy(done);
+        if (stream) (void)hipStreamDestroy(stream);
         if (host) (void)hipHostFree(host);
     }
 };
 
-// Blocks kept between calls, for any thread: at most 8 of one chunk (a render holds one too) and 2 large
-// ones, 48 MiB in all. The pool
-// lives until the process ends (its blocks are not freed after the runtime has shut down).
+// Chunks kept between calls, for any thread: kMost in all, 64 MiB. A call takes as many as it wants of those
+// that are free or may still be made, and at least one, which is freed again where there are kMost others; so
+// threads that read at once share the chunks instead of making more. (With blocks of eight chunks, two of them
+// kept, 4, 8 and 16 threads reading 6 MB each took 0.68, 2.1 and 5.0 ms; 0.50, 0.95 and 1.94 with this, the rate
+// of the link.) The pool lives until the process ends (its chunks are not freed after the runtime has shut down).
 class Pool {
 public:
     static Pool& get()
@@ -74,68 +60,128 @@ public:
         static Pool* p = new Pool;
         return *p;
     }
-    Staging* take(int device, size_t bytes)
+    // up to `want` chunks; how many (0: no memory for one)
+    uint32_t take(int device, uint32_t want, Chunk** out)
     {
-        const uint32_t slots = bytes <= kChunk ? 1u : kSlots;
+        uint32_t n = 0, make = 0;
         {
             std::lock_guard<std::mutex> lock(mutex_);
-            for (Staging*& f : free_)
-                if (f && f->device == device && f->slots == slots) {
-                    Staging* s = f;
-                    f = nullptr;
-                    return s;
+            for (uint32_t k = 0; k < kept_ && n < want;)
+                if (free_[k]->device == device) {
+                    out[n++] = free_[k];
+                    free_[k] = free_[--kept_];
+                } else {
+                    ++k;
                 }
+            make = std::min(want - n, alive_ < kMost ? kMost - alive_ : 0u);
+            if (n + make == 0) make = 1;
+            alive_ += make;
         }
-        Staging* s = new (std::nothrow) Staging;
-        if (s && !s->make(device, slots)) {
-            delete s;
-            s = nullptr;
+        for (; make; --make) {
+            Chunk* c = new (std::nothrow) Chunk;
+            if (!c || !c->make(device)) {
+                delete c;
+                break;
+            }
+            out[n++] = c;
         }
-        return s;
-    }
-    void give(Staging* s)
-    {
-        {
+        if (make) {
             std::lock_guard<std::mutex> lock(mutex_);
-            int same = 0;
-            for (Staging* f : free_) same += f && f->slots == s->slots;
-            if (same < (s->slots == 1 ? kKeptSmall : kKeptLarge))
-                for (Staging*& f : free_)
-                    if (!f) {
-                        f = s;
-                        return;
-                    }
+            alive_ -= make;
         }
-        delete s;
+        return n;
+    }
+    void give(Chunk* const* chunks, uint32_t n)
+    {
+        for (uint32_t k = 0; k < n; ++k) {
+            {
+                std::lock_guard<std::mutex> lock(mutex_);
+                if (alive_ <= kMost) {
+                    free_[kept_++] = chunks[k];
+                    continue;
+                }
+                --alive_;
+            }
+            delete chunks[k];
+        }
     }
 
 private:
-    static constexpr int kKeptSmall = 8, kKeptLarge = 2;
+    static constexpr uint32_t kMost = 32;
     std::mutex mutex_;
-    Staging* free_[kKeptSmall + kKeptLarge] = {};
+    Chunk* free_[kMost] = {};
+    uint32_t kept_ = 0, alive_ = 0;  // chunks in free_; with those in use
 };
 
-// A small pinned block for as long as this object lives.
-class Lease {
+// The chunks of one call.
+class Chunks {
 public:
-    Lease() = default;
-    Lease(const Lease&) = delete;
-    Lease& operator=(const Lease&) = delete;
-    ~Lease()
-    {
-        if (block_) Pool::get().give(block_);
-    }
-    bool take()
+    Chunks() = default;
+    Chunks(const Chunks&) = delete;
+    Chunks& operator=(const Chunks&) = delete;
+    ~Chunks() { Pool::get().give(chunk_, n_); }
+    hipError_t take(uint32_t want)
     {
         int device = 0;
-        if (hipGetDevice(&device) != hipSuccess) return false;
-        block_ = Pool::get().take(device, 1);
-        return block_ != nullptr;
+        const hipError_t e = hipGetDevice(&device);
+        if (e != hipSuccess) return e;
+        n_ = Pool::get().take(device, std::min(want, kSlots), chunk_);
+        return n_ ? hipSuccess : hipErrorOutOfMemory;
     }
-    char* host() const { return block_->host; }
+    uint32_t size() const { return n_; }
+    Chunk& operator[](uint32_t k) const { return *chunk_[k]; }
+    void wait() const
+    {
+        for (uint32_t k = 0; k < n_; ++k) (void)hipStreamSynchronize(chunk_[k]->stream);
+    }
 
 private:
-    Staging* block_ = nullptr;
+    Chunk* chunk_[kSlots] = {};
+    uint32_t n_ = 0;
+};
+
+// Threads that calls have started besides their own, kMost in all calls: more only take turns on the
+// processors (a GPU's share of its host's: 16) and on the link, which two reads fill.
+class Helpers {
+public:
+    Helpers() = default;
+    Helpers(const Helpers&) = delete;
+    Helpers& operator=(const Helpers&) = delete;
+    ~Helpers() { join(); }
+    template <class F>
+    void start(uint32_t n, F f)
+    {
+        for (n = std::min(n, kSlots); n_ < n;) {
+            if (running().fetch_add(1) >= kMost) {
+                running().fetch_sub(1);
+                return;
+            }
+            try {
+                thread_[n_] = std::thread(f, n_);
+                ++n_;
+            } catch (...) {  // no more threads: those that started and the caller's do the work
+                running().fetch_sub(1);
+                return;
+            }
+        }
+    }
+    void join()
+    {
+        for (; n_; --n_) {
+            thread_[n_ - 1].join();
+            running().fetch_sub(1);
+        }
+    }
+
+private:
+    static constexpr int kMost = 12;
+    static std::atomic<int>& running()
+    {
+        static std::atomic<int> n{0};
+        return n;
+    }
+    std::thread thread_[kSlots];
+    uint32_t n_ = 0;
 };
 
 // Fills out[0, bytes) with what `launch(stream, dst, offset, size)` makes the GPU write to the pinned
@@ -147,13 +193,14 @@ template <class Launch>
 hipError_t read_back(void* out, size_t bytes, Launch launch, hipStream_t own = nullptr)
 {
     if (bytes == 0) return hipSuccess;
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
-    if (e != hipSuccess) return e;
-    Staging* st = Pool::get().take(device, bytes);
-    if (!st) return hipErrorOutOfMemory;
     constexpr uint64_t kPieces = kChunk / kPiece;
     const uint64_t chunks = (bytes + kChunk - 1) / kChunk, pieces = (bytes + kPiece - 1) / kPiece;
+    Chunks st;
+    hipError_t e = st.take(uint32_t(std::min<uint64_t>(chunks, kSlots)));
+    if (e != hipSuccess) {
+        if (own) (void)hipStreamSynchronize(own);
+        return e;
+    }
     std::atomic<uint64_t> next{0}, submitted{0}, copied{0};  // pieces claimed / submitted / copied
     std::atomic<uint32_t> slot_copied[kSlots] = {};           // pieces copied of the chunk in each slot
     std::atomic<int> error{int(hipSuccess)};
@@ -163,94 +210,78 @@ hipError_t read_back(void* out, size_t bytes, Launch launch, hipStream_t own = n
         do {
             if (k >= submitted.load()) return false;
         } while (!next.compare_exchange_weak(k, k + 1));
-        const uint32_t slot = uint32_t((k / kPieces) % st->slots);
-        const hipError_t w = hipEventSynchronize(st->done[slot]);
+        const uint32_t slot = uint32_t((k / kPieces) % st.size());
+        const hipError_t w = hipEventSynchronize(st[slot].done);
         if (w != hipSuccess) {
             error = int(w);
             return false;
         }
         const size_t at = size_t(k) * kPiece;
-        std::memcpy(static_cast<char*>(out) + at, st->host + slot * kChunk + at % kChunk, std::min(kPiece, bytes - at));
+        std::memcpy(static_cast<char*>(out) + at, st[slot].host + at % kChunk, std::min(kPiece, bytes - at));
         slot_copied[slot].fetch_add(1);
         copied.fetch_add(1);
         return true;
     };
-    auto help = [&]() {
+    auto help = [&](uint32_t) {
         while (next.load() < pieces && error.load() == int(hipSuccess))
             if (!copy_one()) std::this_thread::yield();
     };
-    std::thread helpers[kHelpers];
-    int n_helpers = 0;
-    const int want = int(std::min<size_t>(kHelpers, bytes / kPerThread));
+    Helpers helpers;
+    const uint32_t want = uint32_t(std::min<size_t>(kHelpers, bytes / kPerThread));
     // the caller's thread submits chunks while slots are free and copies otherwise
     for (uint64_t k = 0; copied.load() < pieces && error.load() == int(hipSuccess);) {
-        const uint32_t slot = uint32_t(k % st->slots);
-        if (k < chunks && (k < st->slots || slot_copied[slot].load() == kPieces)) {
+        const uint32_t slot = uint32_t(k % st.size());
+        if (k < chunks && (k < st.size() || slot_copied[slot].load() == kPieces)) {
             slot_copied[slot].store(0);
             const size_t at = size_t(k) * kChunk;
-            const hipStream_t stream = own ? own : st->stream[k & 1];
-            e = launch(stream, st->host + slot * kChunk, at, std::min(kChunk, bytes - at));
-            if (e == hipSuccess) e = hipEventRecord(st->done[slot], stream);
+            const hipStream_t stream = own ? own : st[std::min(uint32_t(k & 1), st.size() - 1u)].stream;
+            e = launch(stream, st[slot].host, at, std::min(kChunk, bytes - at));
+            if (e == hipSuccess) e = hipEventRecord(st[slot].done, stream);
             if (e != hipSuccess) {
                 error = int(e);
                 break;
             }
             ++k;
             submitted.store(std::min(pieces, k * kPieces));
-            if (k == std::min<uint64_t>(chunks, 2)) {
-                try {
-                    while (n_helpers < want) helpers[n_helpers] = std::thread(help), ++n_helpers;
-                } catch (...) {  // no more threads: those that started and this one copy
-                }
-            }
+            if (k == std::min<uint64_t>(chunks, 2)) helpers.start(want, help);
         } else if (!copy_one()) {
             std::this_thread::yield();
         }
     }
-    for (int t = 0; t < n_helpers; ++t) helpers[t].join();
-    if (error.load() != int(hipSuccess)) {  // nothing writes the block any more
-        st->wait();
+    helpers.join();
+    if (error.load() != int(hipSuccess)) {  // nothing writes the chunks any more
+        st.wait();
         if (own) (void)hipStreamSynchronize(own);
     }
-    Pool::get().give(st);
     return hipError_t(error.load());
 }
 
-// Calls work(stream, event, pinned, first, count) for every range of at most `per` items of [0, n), by
-// `threads` threads at once, each with a chunk of pinned memory, an event and (up to kStreams) a stream
-// of its own. `work` returns with nothing of its own in flight, unless it fails. Returns when
-// all ranges are done, or on an error, when nothing is in flight.
+// Calls work(chunk, first, count) for every range of at most `per` items of [0, n), by up to `threads` threads
+// at once, each with a chunk of its own. `work` returns with nothing of its own in flight, unless it fails.
+// Returns when all ranges are done, or on an error, when nothing is in flight.
 template <class Work>
 hipError_t run_chunks(size_t n, size_t per, uint32_t threads, Work work)
 {
-    int device = 0;
-    hipError_t e = hipGetDevice(&device);
+    Chunks st;
+    const hipError_t e = st.take(threads);
     if (e != hipSuccess) return e;
-    threads = std::min(std::max(threads, 1u), kSlots);
-    Staging* st = Pool::get().take(device, threads * kChunk);
-    if (!st) return hipErrorOutOfMemory;
+    const int device = st[0].device;
     std::atomic<size_t> next{0};
     std::atomic<int> error{int(hipSuccess)};
     auto run = [&](uint32_t t) {
         for (size_t first; error.load() == int(hipSuccess) && (first = next.fetch_add(per)) < n;) {
-            const hipError_t w = work(st->stream[t % kStreams], st->done[t], st->host + t * kChunk, first, std::min(per, n - first));
+            const hipError_t w = work(st[t], first, std::min(per, n - first));
             if (w != hipSuccess) error = int(w);
         }
     };
-    std::thread helpers[kSlots];
-    uint32_t started = 0;
-    try {
-        for (uint32_t t = 1; t < threads; ++t, ++started)
-            helpers[started] = std::thread([&run, t, device] {
-                (void)hipSetDevice(device);
-                run(t);
-            });
-    } catch (...) {  // no more threads: those that started and this one do the work
-    }
+    Helpers helpers;
+    helpers.start(st.size() - 1u, [&](uint32_t t) {
+        (void)hipSetDevice(device);
+        run(t + 1u);
+    });
     run(0);
-    for (uint32_t t = 0; t < started; ++t) helpers[t].join();
-    if (error.load() != int(hipSuccess)) st->wait();  // nothing uses the block any more
-    Pool::get().give(st);
+    helpers.join();
+    if (error.load() != int(hipSuccess)) st.wait();  // nothing uses the chunks any more
     return hipError_t(error.load());
 }
 

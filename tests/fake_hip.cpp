@@ -4,6 +4,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <sys/mman.h>
+#include <unistd.h>
 
 #include <cstdlib>
 #include <cstring>
@@ -16,6 +17,9 @@ namespace {
 std::mutex m;
 size_t budget = size_t(288) << 30, used = 0;
 bool pinned_fails = false;
+std::map<void*, size_t> pinned;  // and the bytes of all that were ever made
+size_t pinned_live = 0, pinned_made = 0;
+int event_us = 0;  // a wait for an event takes that long
 long mallocs_left = -1;  // hipMalloc fails from the one after these on (-1: never)
 struct Block {
     size_t size, mapped;
@@ -45,6 +49,9 @@ void fake_budget(size_t bytes) { budget = bytes; }
 void fake_pinned_fails(int on) { pinned_fails = on != 0; }
 void fake_mallocs_left(long n) { mallocs_left = n; }
 size_t fake_used() { return used; }
+size_t fake_pinned_live() { return pinned_live; }
+size_t fake_pinned_made() { return pinned_made; }
+void fake_event_us(int us) { event_us = us; }
 const char* fake_log() { return log_.c_str(); }
 void fake_clear() { log_.clear(); }
 
@@ -74,10 +81,21 @@ hipError_t hipFree(void* p)
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
+    std::lock_guard<std::mutex> lock(m);
     *p = pinned_fails ? nullptr : std::calloc(1, n);
-    return *p ? hipSuccess : hipErrorOutOfMemory;
+    if (!*p) return hipErrorOutOfMemory;
+    pinned[*p] = n;
+    pinned_live += n;
+    pinned_made += n;
+    return hipSuccess;
 }
-hipError_t hipHostFree(void* p) { return std::free(p), hipSuccess; }
+hipError_t hipHostFree(void* p)
+{
+    std::lock_guard<std::mutex> lock(m);
+    pinned_live -= pinned[p];
+    pinned.erase(p);
+    return std::free(p), hipSuccess;
+}
 hipError_t hipMemGetInfo(size_t* f, size_t* t) { return *f = budget - used, *t = budget, hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t)
 {
@@ -116,7 +134,11 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return handle(rein
 hipError_t hipEventDestroy(hipEvent_t e) { return std::free(e), hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.0f, hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t)
+{
+    if (event_us) usleep(useconds_t(event_us));
+    return hipSuccess;
+}
 hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return handle(reinterpret_cast<void**>(s)); }
 hipError_t hipStreamDestroy(hipStream_t s) { return std::free(s), hipSuccess; }

@@ -18,6 +18,7 @@ import ctypes, sys
 sys.path.insert(0, {root!r})
 fake = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
 fake.fake_log.restype, fake.fake_used.restype = ctypes.c_char_p, ctypes.c_size_t
+fake.fake_pinned_live.restype = fake.fake_pinned_made.restype = ctypes.c_size_t
 fake.fake_budget.argtypes = [ctypes.c_size_t]
 fake.fake_mallocs_left.argtypes = [ctypes.c_long]
 import numpy as np
@@ -95,4 +96,41 @@ film.add_samples(a)
 nat.check(nat.lib().tr_film_read_sums(film.handle, None, nat.as_ptr(got)))
 pix[{n} - 1] = a["x"][{n} - 1]
 assert np.array_equal(got.ravel(), expect + np.bincount(pix, minlength={width * height}))
+""")
+
+
+@pytest.mark.parametrize("threads", [8, 40])
+def test_concurrent_reads_share_the_pinned_chunks(threads):
+    """Films of 6 MB read by several threads at once, again and again: at most 32 chunks of 2 MiB are kept, and
+    no more are made than those and one for each thread that finds none."""
+    run(f"""
+import threading
+films = [R.StreakCameraFilm(45, 45, 256, 0.1) for _ in range({threads})]
+for f in films:
+    f.handle
+fake.fake_event_us(300)
+def go(f):
+    for _ in range(6):
+        f.read()
+ts = [threading.Thread(target=go, args=(f,)) for f in films]
+[t.start() for t in ts]
+[t.join() for t in ts]
+assert fake.fake_pinned_live() <= 64 << 20, fake.fake_pinned_live()
+if {threads} <= 32:
+    assert fake.fake_pinned_made() <= 64 << 20, fake.fake_pinned_made()
+""")
+
+
+def test_a_read_without_pinned_memory_says_so():
+    run("""
+film = R.StreakCameraFilm(4, 4, 8, 0.1)
+film.handle
+fake.fake_pinned_fails(1)
+try:
+    film.read()
+    raise SystemExit("read")
+except nat.TrError as e:
+    assert e.code == nat.TR_ERR_NOMEM, e
+fake.fake_pinned_fails(0)
+film.read()
 """)
