@@ -2604,12 +2604,14 @@ struct HostHits {
 
 // Rays of a launch. Several threads each copy a launch's rays into pinned memory, wait for it and copy the
 // answers out, so that copies and launches overlap. A launch lasts as long as its longest ray, 50-80 us over
-// 81,930 triangles however many rays it has: 262,144 rays take 885 us with 4 threads and launches of 8,192
-// rays, 625 with 16,384, 562 with 32,768; 1,001 with one thread, 480 with 8 (1,000,000 rays: 4 threads
-// 1.60 ms, 8 threads 1.47). In all, with buffers made for each call, the runtime's copies and records
-// packed by the caller, 262,144 rays took 2,700 us and take 500; 1,000 took 74 and take 50.
+// 81,930 triangles however many rays it has: 262,144 rays took 885 us with 4 threads and launches of 8,192
+// rays, 625 with 16,384, 562 with 32,768. One thread per launch, up to a call's eight chunks: with 4, 6 and 8
+// threads 262,144 rays take 550, 510 and 525 us, 524,288 take 960, 900 and 885, 1,000,000 take 1.80, 1.64 and
+// 1.56 ms; visibility of 1,000,000 records 1.35, 1.21 and 1.16 ms, where a copy, a kernel and a copy
+// take 1.18 (up to 131,072 rays all are alike). In all, with buffers made for each call, the runtime's copies
+// and records packed by the caller, 262,144 rays took 2,700 us; 1,000 took 74 and take 50.
 constexpr uint32_t kQueryChunk = 32768;
-constexpr uint32_t kMaxQueryThreads = 4;
+constexpr uint32_t kMaxQueryThreads = trb::kSlots;
 constexpr uint32_t kQueryPerWave = 16;
 static_assert(kQueryChunk * (sizeof(tr_ray) + sizeof(tr_hit)) + 64 <= trb::kChunk, "a launch's rays and answers fit a chunk");
 
