@@ -493,10 +493,7 @@ Bvh4 collapse_bvh4_greedy(const BvhBuildResult& b)
 namespace {
 
 // float(origin + q * 2^(e - 127)) with q * 2^(e - 127) exact, as the device evaluates it
-float dequant(float origin, uint32_t q, int be)
-{
-    return origin + float(q) * std::ldexp(1.0f, be - 127);
-}
+float dequant(float origin, uint32_t q, float step) { return origin + float(q) * step; }
 
 }  // namespace
 
@@ -524,13 +521,19 @@ std::vector<Bvh4QNodeHost> quantize_bvh4(const Bvh4& b4)
             // smallest grid step 2^(e-127) whose 255th plane reaches the largest hi plane
             int e = 1;
             const double ext = double(h) - double(o);
-            if (ext > 0.0) e = std::max(1, std::min(254, int(std::ceil(std::log2(ext / 255.0))) + 127 - 1));
-            while (e < 254 && dequant(o, 255u, e) < h) ++e;
+            if (ext > 0.0) {
+                int p = 0;  // ceil(log2(ext / 255))
+                if (std::frexp(ext / 255.0, &p) == 0.5) --p;
+                e = std::max(1, std::min(254, p + 127 - 1));
+            }
+            while (e < 254 && dequant(o, 255u, std::ldexp(1.0f, e - 127)) < h) ++e;
             be[a] = e;
         }
         q.step_x = std::ldexp(1.0f, be[0] - 127);
         q.step_y = std::ldexp(1.0f, be[1] - 127);
         q.step_z = std::ldexp(1.0f, be[2] - 127);
+        const float steps[3] = {q.step_x, q.step_y, q.step_z};
+        const double per_step[3] = {std::ldexp(1.0, 127 - be[0]), std::ldexp(1.0, 127 - be[1]), std::ldexp(1.0, 127 - be[2])};
         // byte offsets: lo_x 0, hi_x 4, lo_y 8, hi_y 12 (word 1), lo_z 16, hi_z 20 (word 2)
         const int lo_off[3] = {0, 8, 16}, hi_off[3] = {4, 12, 20};
         for (int k = 0; k < 4; ++k) {
@@ -544,13 +547,15 @@ std::vector<Bvh4QNodeHost> quantize_bvh4(const Bvh4& b4)
             }
             for (int a = 0; a < 3; ++a) {
                 const float o = q.origin[a];
-                const double step = std::ldexp(1.0, be[a] - 127);
-                long ql = long(std::floor((double(lo[a][k]) - double(o)) / step));
+                const double xl = (double(lo[a][k]) - double(o)) * per_step[a];  // not negative: o is the lowest plane
+                const double xh = (double(hi[a][k]) - double(o)) * per_step[a];
+                long ql = long(xl);
                 ql = std::max(0L, std::min(255L, ql));
-                while (ql > 0 && dequant(o, uint32_t(ql), be[a]) > lo[a][k]) --ql;
-                long qh = long(std::ceil((double(hi[a][k]) - double(o)) / step));
+                while (ql > 0 && dequant(o, uint32_t(ql), steps[a]) > lo[a][k]) --ql;
+                long qh = long(xh);
+                if (double(qh) < xh) ++qh;
                 qh = std::max(0L, std::min(255L, qh));
-                while (qh < 255 && dequant(o, uint32_t(qh), be[a]) < hi[a][k]) ++qh;
+                while (qh < 255 && dequant(o, uint32_t(qh), steps[a]) < hi[a][k]) ++qh;
                 q.q[lo_off[a] + k] = uint8_t(ql);
                 q.q[hi_off[a] + k] = uint8_t(qh);
             }
