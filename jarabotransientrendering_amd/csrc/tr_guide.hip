@@ -566,8 +566,17 @@ template <class T>
 int galloc(T** p, size_t n)
 {
     *p = nullptr;
-    hipError_t e = hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(n, 1) * sizeof(T));
-    if (e != hipSuccess) return tri::fail(TR_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    const size_t bytes = std::max<size_t>(n, 1) * sizeof(T);
+    hipError_t e = hipMalloc(reinterpret_cast<void**>(p), bytes);
+    if (e == hipErrorOutOfMemory && tri::release_idle_buffers()) {
+        (void)hipGetLastError();  // (the next launch would report it)
+        e = hipMalloc(reinterpret_cast<void**>(p), bytes);
+    }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();
+        return tri::fail(TR_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     return TR_OK;
 }
 template <class T>

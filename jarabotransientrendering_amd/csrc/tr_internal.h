@@ -148,6 +148,7 @@ namespace tri {
 int fail(int code, const std::string& msg);  // records the message for tr_last_error, returns code
 int check_device();                          // TR_OK if the current device is a gfx950
 int compute_units();                         // compute units of the current device
+bool release_idle_buffers();                 // of renders, on the current device; false if there are none
 }  // namespace tri
 
 // ---- image output (tr_image_io.cpp) ---------------------------------------------------------

@@ -57,9 +57,10 @@ constexpr uint32_t kDefaultWave = 1u << 26;
 // 1.41 ms in all); a 67 M-path frame in wavefronts of 2^25: 24.3 ms with one bounce per launch,
 // 23.3 with two, 22.6 with four, 22.1 with all eight.
 constexpr uint32_t kShadowRecords = 1u << 28;
-// Device memory of the two: wavefronts of more than kSmallWave paths and groups of bounces are made
-// smaller where their buffers would take more than a quarter of the free memory.
+// Device memory of the two, up to 25 GB: see WaveBuffers::fit. Wavefronts of kSmallWave paths and one
+// bounce (6.7 GB) are always tried, and smaller ones down to kLeastWave where memory has run out.
 constexpr uint32_t kSmallWave = 1u << 25;
+constexpr uint32_t kLeastWave = 1u << 18;
 // Largest wavefronts whose bounces run in one launch (path_kernel) instead of two per bounce. A render of
 // 2^10 paths through the two: 163 and 84 us (22 triangles), 642 and 266 (81,930 triangles), 370 and 161 (a
 // medium, 16 bounces); of 2^18 paths 200 and 100, 1,074 and 586, 540 and 224; of 2^20 paths 276 and 196,
@@ -1967,13 +1968,23 @@ int check_device()
     return TR_OK;
 }
 
+bool release_idle_buffers();
+
 template <class T>
 int dev_alloc(T** p, size_t count, uint64_t* bytes = nullptr)
 {
     *p = nullptr;
     if (count == 0) count = 1;
     hipError_t e = hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
-    if (e != hipSuccess) return fail(TR_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    if (e == hipErrorOutOfMemory && release_idle_buffers()) {
+        (void)hipGetLastError();  // (the next launch would report it)
+        e = hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T));
+    }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        (void)hipGetLastError();
+        return fail(TR_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
     if (bytes) *bytes += count * sizeof(T);
     return TR_OK;
 }
@@ -2016,7 +2027,34 @@ static uint32_t stack_flags_of(int fmt)
     return fmt == 1 ? TR_RENDER_STACK32 : fmt == 2 ? TR_RENDER_STACK_KEYED : 0u;
 }
 
+struct WaveBuffers;
+
+// The wavefront buffers of every scene and batch: those that no render uses are given back when device
+// memory runs out, and what they hold bounds what another may take (WaveBuffers::fit).
+class BufferList {
+public:
+    static BufferList& get()
+    {
+        static BufferList* l = new BufferList;  // (outlives the scenes)
+        return *l;
+    }
+    void add(WaveBuffers* b);
+    void remove(WaveBuffers* b);
+    void use(WaveBuffers* b, int by);
+    bool release_idle();
+    uint64_t others(const WaveBuffers* b);
+
+private:
+    std::mutex mutex_;
+    WaveBuffers* first_ = nullptr;
+};
+
 struct WaveBuffers {
+    // renders at work in these buffers, the device they are on and their bytes (changed and read under the
+    // list's lock)
+    int users = 0, device = 0;
+    uint64_t held = 0;
+    WaveBuffers *prev = nullptr, *next = nullptr;
     uint32_t cap = 0, sh_cap = 0;  // path records, shadow records
     float4 *ray_o[2] = {}, *ray_d[2] = {}, *thr[2] = {};
     uint4* st[2] = {};
@@ -2038,6 +2076,15 @@ struct WaveBuffers {
     uint32_t cs_cap = 0;
     uint32_t* counters = nullptr;
 
+    WaveBuffers() { BufferList::get().add(this); }
+    ~WaveBuffers()
+    {
+        BufferList::get().remove(this);
+        release();
+    }
+    WaveBuffers(const WaveBuffers&) = delete;
+    WaveBuffers& operator=(const WaveBuffers&) = delete;
+
     void release()
     {
         for (int b = 0; b < 2; ++b) {
@@ -2056,6 +2103,7 @@ struct WaveBuffers {
     {
         if (n <= cs_cap) return TR_OK;
         dev_free(cs_bits);
+        cs_cap = 0;
         int rc = dev_alloc(&cs_bits, n);
         if (rc) return rc;
         cs_cap = n;
@@ -2080,6 +2128,7 @@ struct WaveBuffers {
                 hipSuccess) {
                 h_jobs = nullptr;
                 dev_free(d_jobs);
+                (void)hipGetLastError();
                 return fail(TR_ERR_NOMEM, "hipHostMalloc: job table");
             }
             jobs_cap = n_jobs + 1;
@@ -2104,16 +2153,31 @@ struct WaveBuffers {
         return n * (2 * (3 * sizeof(float4) + sizeof(uint4) + sizeof(float)) + sizeof(float2)) +
                n_sh * (3 * sizeof(float4) + sizeof(uint8_t) + 2 * sizeof(uint32_t));
     }
-    // makes `group` bounces per shadow launch and then `wave` (whole units of paths) smaller until
-    // their buffers fit a quarter of the device memory that is free or held by this object
+    // Makes `group` bounces per shadow launch and then `wave` (whole units of paths) smaller until their
+    // buffers fit a quarter of the device memory that is free or held by this object, and with those of other
+    // scenes and batches a quarter of all memory: a process with many scenes keeps a few of the large
+    // shapes, and 6.7 GB for each further one (a 67 M-path frame 24.3 ms instead of 20.7).
     void fit(uint32_t& wave, uint32_t& group, uint32_t unit) const
     {
         if (wave <= cap && uint64_t(wave) * group <= sh_cap) return;
         size_t free_bytes = 0, total_bytes = 0;
         if (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess) return;
-        const uint64_t room = (uint64_t(free_bytes) + bytes(cap, sh_cap)) / 4;
+        const uint64_t other = BufferList::get().others(this), quarter = uint64_t(total_bytes) / 4;
+        const uint64_t room = std::max(bytes(kSmallWave, kSmallWave), std::min((uint64_t(free_bytes) + bytes(cap, sh_cap)) / 4,
+                                                                              quarter > other ? quarter - other : 0));
         while (group > 1 && bytes(wave, uint64_t(wave) * group) > room) group = (group + 1) / 2;
-        while (wave > kSmallWave && wave / 2 >= unit && bytes(wave, wave) > room) wave = wave / 2 / unit * unit;
+        while (wave > kSmallWave && bytes(wave, wave) > room && smaller(wave, group, unit)) {}
+    }
+    // the next smaller shape: fewer bounces per group, then fewer paths (whole units of them)
+    static bool smaller(uint32_t& wave, uint32_t& group, uint32_t unit)
+    {
+        if (group > 1) {
+            group = (group + 1) / 2;
+            return true;
+        }
+        if (wave / 2 < std::max(kLeastWave, unit)) return false;
+        wave = wave / 2 / unit * unit;
+        return true;
     }
     int ensure(uint32_t n, uint32_t n_sh)
     {
@@ -2139,6 +2203,17 @@ struct WaveBuffers {
         sh_cap = n_sh;
         return TR_OK;
     }
+    // everything that a render of wavefronts of `wave` paths needs
+    int ensure_all(uint32_t wave, uint32_t group, bool unwarp, bool tags, uint32_t camera_samples, uint32_t jobs)
+    {
+        int rc = ensure(wave, wave * group);
+        if (!rc && unwarp) rc = ensure_unwarp();
+        if (!rc && tags) rc = ensure_tags();
+        if (!rc && camera_samples) rc = ensure_cs(camera_samples);
+        if (!rc && jobs) rc = ensure_batch(jobs);
+        if (rc) release();
+        return rc;
+    }
     WaveDev view() const
     {
         WaveDev w;
@@ -2155,10 +2230,62 @@ struct WaveBuffers {
     }
 };
 
+void BufferList::add(WaveBuffers* b)
+{
+    std::lock_guard<std::mutex> lock(mutex_);
+    b->next = first_;
+    if (first_) first_->prev = b;
+    first_ = b;
+}
+void BufferList::remove(WaveBuffers* b)
+{
+    std::lock_guard<std::mutex> lock(mutex_);
+    (b->prev ? b->prev->next : first_) = b->next;
+    if (b->next) b->next->prev = b->prev;
+}
+// a render begins (1) or ends (-1) in `b`
+void BufferList::use(WaveBuffers* b, int by)
+{
+    int device = 0;
+    (void)hipGetDevice(&device);
+    std::lock_guard<std::mutex> lock(mutex_);
+    b->users += by;
+    b->device = device;
+    b->held = WaveBuffers::bytes(b->cap, b->sh_cap);
+}
+// gives back the buffers on the current device that no render uses; false if there are none
+bool BufferList::release_idle()
+{
+    int device = 0;
+    if (hipGetDevice(&device) != hipSuccess) return false;
+    bool any = false;
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (WaveBuffers* b = first_; b; b = b->next)
+        if (b->users == 0 && b->held != 0 && b->device == device) {
+            b->release();
+            b->held = 0;
+            any = true;
+        }
+    return any;
+}
+// bytes that all but `b` hold on the current device
+uint64_t BufferList::others(const WaveBuffers* b)
+{
+    int device = 0;
+    (void)hipGetDevice(&device);
+    uint64_t sum = 0;
+    std::lock_guard<std::mutex> lock(mutex_);
+    for (const WaveBuffers* o = first_; o; o = o->next)
+        if (o != b && o->device == device) sum += o->held;
+    return sum;
+}
+bool release_idle_buffers() { return BufferList::get().release_idle(); }
+
 }  // namespace
 
 namespace tri {
 int fail(int code, const std::string& msg) { return ::fail(code, msg); }
+bool release_idle_buffers() { return ::release_idle_buffers(); }
 int check_device() { return ::check_device(); }
 int compute_units()
 {
@@ -2291,7 +2418,6 @@ int tr_scene_destroy(tr_scene s)
     if (!s) return TR_OK;
     if (s->stream) (void)hipStreamSynchronize(s->stream);
     s->release_device();
-    s->wave.release();
     if (s->ev_made)
         for (auto& e : s->ev) (void)hipEventDestroy(e);
     if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -3488,6 +3614,11 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     // every return drains the stream, so no queued copy or kernel outlives the host buffers and
     // device views it was given (the normal path synchronises as well, to read the counters)
     trb::Chunks pinned;  // (given back after that)
+    struct Use {
+        WaveBuffers* b;
+        explicit Use(WaveBuffers* wb) : b(wb) { BufferList::get().use(b, 1); }
+        ~Use() { BufferList::get().use(b, -1); }
+    } use(&wb);  // (until after that)
     struct Drain {
         hipStream_t s;
         ~Drain() { (void)hipStreamSynchronize(s); }
@@ -3530,15 +3661,20 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     }
     // bounces whose shadow rays one launch takes
     uint32_t group = std::max(1u, std::min(uint32_t(std::max(bounces, 1)), kShadowRecords / c.wave));
-    wb.fit(c.wave, group, guide ? c.wave : mb ? uint32_t(jobs[0].dev.R.n_inc) : 1u);
-    int rc = wb.ensure(c.wave, c.wave * group);
+    const uint32_t unit = guide ? c.wave : mb ? uint32_t(jobs[0].dev.R.n_inc) : 1u;
+    wb.fit(c.wave, group, unit);
+    bool unwarp = false;
+    for (auto& j : jobs) unwarp = unwarp || j.dev.R.unwarp;
+    int rc;
+    for (;;) {
+        const bool was = wb.cap != 0;  // (what it already has may have made the first try larger than the shape)
+        rc = wb.ensure_all(c.wave, group, unwarp, mb || guide, mb ? c.wave / uint32_t(jobs[0].dev.R.n_inc) : 0u,
+                           batch ? uint32_t(jobs.size()) : 0u);
+        if (rc != TR_ERR_NOMEM || (!was && !WaveBuffers::smaller(c.wave, group, unit))) break;
+    }
     if (rc) return rc;
-    for (auto& j : jobs)
-        if (j.dev.R.unwarp && (rc = wb.ensure_unwarp())) return rc;
     if (mb) {
-        const uint32_t ncs = c.wave / uint32_t(jobs[0].dev.R.n_inc);
-        if ((rc = wb.ensure_tags()) || (rc = wb.ensure_cs(ncs))) return rc;
-        HIP_TRY(hipMemsetAsync(wb.cs_bits, 0, size_t(ncs) * sizeof(uint32_t), stream));
+        HIP_TRY(hipMemsetAsync(wb.cs_bits, 0, size_t(c.wave / uint32_t(jobs[0].dev.R.n_inc)) * sizeof(uint32_t), stream));
         jobs[0].dev.R.cs_bits = wb.cs_bits;
     }
     Launch L{};
@@ -3564,13 +3700,11 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     if (guide) {
         const HostJob& j = jobs[0];
         if (j.max_bounces < 1) return fail(TR_ERR_INVALID, "tr_render_transient_guided: max_bounces must be >= 1");
-        if ((rc = wb.ensure_tags())) return rc;
         if ((rc = trg::guide_begin_render(guide, c.wave, uint32_t(j.max_bounces), j.scene->bb_lo, j.scene->bb_hi,
                                           stream, &L.GV)))
             return rc;
     }
     if (batch) {
-        if ((rc = wb.ensure_batch(uint32_t(jobs.size())))) return rc;
         // the previous render on this stream ended with a synchronisation, so the pinned table is
         // free to overwrite
         JobDev* dj = wb.h_jobs;
@@ -3775,7 +3909,6 @@ struct tr_batch_s {
     ~tr_batch_s()
     {
         if (stream) (void)hipStreamSynchronize(stream);
-        wave.release();
         if (ev_made)
             for (auto& e : ev) (void)hipEventDestroy(e);
         if (stream) (void)hipStreamDestroy(stream);

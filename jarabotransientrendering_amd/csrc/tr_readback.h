@@ -35,10 +35,12 @@ struct Chunk {
     bool make(int dev)
     {
         device = dev;
-        if (hipHostMalloc(reinterpret_cast<void**>(&host), kChunk, hipHostMallocDefault) != hipSuccess) return host = nullptr, false;
-        if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) return stream = nullptr, false;
-        if (hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) return done = nullptr, false;
-        return true;
+        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&host), kChunk, hipHostMallocDefault);
+        if (e != hipSuccess) host = nullptr;
+        if (e == hipSuccess && (e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking)) != hipSuccess) stream = nullptr;
+        if (e == hipSuccess && (e = hipEventCreateWithFlags(&done, hipEventDisableTiming)) != hipSuccess) done = nullptr;
+        if (e != hipSuccess) (void)hipGetLastError();  // (the next launch would report it)
+        return e == hipSuccess;
     }
     ~Chunk()
     {

@@ -19,6 +19,7 @@ size_t budget = size_t(288) << 30, used = 0;
 bool pinned_fails = false;
 std::map<void*, size_t> pinned;  // and the bytes of all that were ever made
 size_t pinned_live = 0, pinned_made = 0;
+bool freed = false;  // a kernel was given memory that is not allocated
 int event_us = 0;  // a wait for an event takes that long
 long mallocs_left = -1;  // hipMalloc fails from the one after these on (-1: never)
 struct Block {
@@ -37,6 +38,13 @@ bool backed(const void* p)
     if (static_cast<const char*>(p) >= it->first + it->second.mapped) return true;
     return it->second.size <= kBacked;
 }
+thread_local hipError_t last = hipSuccess;
+hipError_t failed(hipError_t e) { return last = e; }
+bool live(const void* p)
+{
+    auto it = blocks.upper_bound(static_cast<char*>(const_cast<void*>(p)));
+    return it != blocks.begin() && static_cast<const char*>(p) < (--it)->first + it->second.size;
+}
 thread_local struct {
     dim3 grid, block;
     size_t lds;
@@ -51,6 +59,7 @@ void fake_mallocs_left(long n) { mallocs_left = n; }
 size_t fake_used() { return used; }
 size_t fake_pinned_live() { return pinned_live; }
 size_t fake_pinned_made() { return pinned_made; }
+int fake_freed() { return freed; }
 void fake_event_us(int us) { event_us = us; }
 const char* fake_log() { return log_.c_str(); }
 void fake_clear() { log_.clear(); }
@@ -59,7 +68,7 @@ hipError_t hipMalloc(void** p, size_t n)
 {
     std::lock_guard<std::mutex> lock(m);
     *p = nullptr;
-    if (mallocs_left == 0 || used + n > budget) return hipErrorOutOfMemory;
+    if (mallocs_left == 0 || used + n > budget) return failed(hipErrorOutOfMemory);
     if (mallocs_left > 0) --mallocs_left;
     const size_t mapped = (n + 4095) / 4096 * 4096 + 4096;
     void* a = mmap(nullptr, mapped, n <= kBacked ? PROT_READ | PROT_WRITE : PROT_NONE, MAP_PRIVATE | MAP_ANONYMOUS | MAP_NORESERVE, -1, 0);
@@ -83,7 +92,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned)
 {
     std::lock_guard<std::mutex> lock(m);
     *p = pinned_fails ? nullptr : std::calloc(1, n);
-    if (!*p) return hipErrorOutOfMemory;
+    if (!*p) return failed(hipErrorOutOfMemory);
     pinned[*p] = n;
     pinned_live += n;
     pinned_made += n;
@@ -107,6 +116,7 @@ hipError_t hipMemsetAsync(void* d, int v, size_t n, hipStream_t)
 {
     std::lock_guard<std::mutex> lock(m);
     log_ += "memset\n";
+    if (!live(d)) return failed(hipErrorInvalidValue);
     if (backed(d)) std::memset(d, v, n);
     return hipSuccess;
 }
@@ -122,7 +132,12 @@ hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int)  // (the header renam
     return hipSuccess;
 }
 const char* hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError()
+{
+    const hipError_t e = last;
+    last = hipSuccess;
+    return e;
+}
 hipError_t hipGetSymbolAddress(void** p, const void*)
 {
     static char symbol[16 << 20];
@@ -142,7 +157,11 @@ hipError_t hipEventSynchronize(hipEvent_t)
 hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return handle(reinterpret_cast<void**>(s)); }
 hipError_t hipStreamDestroy(hipStream_t s) { return std::free(s), hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    if (event_us) usleep(useconds_t(event_us));
+    return hipSuccess;
+}
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { return handle(reinterpret_cast<void**>(g)); }
 hipError_t hipGraphDestroy(hipGraph_t g) { return std::free(g), hipSuccess; }
@@ -160,6 +179,10 @@ static hipError_t launched(const void* f, void** args)
     std::lock_guard<std::mutex> lock(m);
     const std::string& name = kernels[f];
     log_ += name;
+    // the buffers that the first and the last kernel of a render get
+    if ((name.find("set_wave_kernel") != std::string::npos || name.find("read_counters_kernel") != std::string::npos) &&
+        !live(*static_cast<void**>(args[0])))
+        freed = true;
     if (name.find("extend_kernel") != std::string::npos) log_ += " " + std::to_string(*static_cast<int*>(args[3]));
     log_ += "\n";
     // the first sample outside the film: none

@@ -134,3 +134,85 @@ except nat.TrError as e:
 fake.fake_pinned_fails(0)
 film.read()
 """)
+
+
+FRAME = """
+def frame(size, spp, bounces, layers=0, unwarp=False, n_inc=1):
+    s = scenes.icosphere_box(level=0, width=size, height=size, time_bins=4, exposure=1.0, sqrt_spp=spp, n_incoming=n_inc,
+                             max_bounces=bounces, seed=1)
+    s.film.bounce_layers, s.film.camera_unwarp = layers, unwarp
+    w, cam, sampler, film, integ = R.setup_scene(s)
+    return lambda **k: R.TransientRenderer().render(None, w, integ, cam, film, sampler, seed=1, **k)
+"""
+
+
+def test_a_process_may_hold_many_rendered_scenes():
+    """Frames of 67 M paths in as many scenes, all kept: a few take the large shape (25 GB), the others stay at
+    6.7 GB while there is memory, and then idle ones give theirs back."""
+    run(FRAME + """
+frames = [frame(256, 32, 8) for _ in range(60)]
+used = []
+for f in frames:
+    assert f()["paths"] == 1 << 26
+    used.append(fake.fake_used())
+assert used[0] > 20 << 30 and used[9] < 130 << 30, [u >> 30 for u in used]
+assert frames[0]()["paths"] == 1 << 26
+assert not fake.fake_freed()
+""")
+
+
+@pytest.mark.parametrize("budget", [1, 3, 5, 9, 20, 40])
+def test_renders_shrink_to_the_memory_there_is(budget):
+    """Whatever is left by the time buffers are made: fewer bounces per group, then fewer paths per wavefront, and
+    no error left behind for the next launch to report."""
+    run(FRAME + f"""
+fs = [frame(256, 32, 8), frame(128, 8, 255), frame(256, 16, 16, layers=3, unwarp=True, n_inc=3)]
+fake.fake_budget(({budget} << 30) + fake.fake_used())
+for f in fs + fs[::-1]:
+    f()
+assert not fake.fake_freed()
+""")
+
+
+def test_an_allocation_that_fails_leaves_a_scene_that_renders():
+    """hipMalloc failing at any point of a first, a larger and a multibounce render."""
+    run(FRAME + """
+for kind in (dict(size=16, spp=2, bounces=5), dict(size=16, spp=2, bounces=5, layers=2, unwarp=True)):
+    done = False
+    for k in range(60):
+        small, f = frame(size=4, spp=1, bounces=2, layers=kind.get("layers", 0)), frame(**kind)
+        small()
+        fake.fake_mallocs_left(k)
+        try:
+            f()
+            done = True
+        except nat.TrError as e:
+            assert e.code == nat.TR_ERR_NOMEM, e
+        fake.fake_mallocs_left(-1)
+        f()
+        small()
+    assert done and not fake.fake_freed()
+""")
+
+
+def test_idle_buffers_are_given_back_while_others_render():
+    """Threads that render in turn in more scenes than memory holds: no render loses its buffers."""
+    run(FRAME + """
+import threading
+fake.fake_budget((9 << 30) + fake.fake_used())
+wrong = []
+def go(k):
+    fs = [frame(64, 16, 4 + k) for _ in range(4)]
+    for _ in range(5):
+        for f in fs:
+            try:
+                assert f()["paths"] == 1 << 20
+            except nat.TrError as e:
+                if e.code != nat.TR_ERR_NOMEM:  # (the other threads may hold all there is)
+                    wrong.append(str(e))
+fake.fake_event_us(200)
+ts = [threading.Thread(target=go, args=(k,)) for k in range(8)]
+[t.start() for t in ts]
+[t.join() for t in ts]
+assert not wrong and not fake.fake_freed(), wrong[:3]
+""")
