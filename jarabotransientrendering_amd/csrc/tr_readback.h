@@ -28,19 +28,32 @@ constexpr size_t kPerThread = size_t(1) << 20;  // least bytes per copying threa
 // A chunk of pinned memory with a stream and an event, made for one device and used by one call at a time.
 struct Chunk {
     int device = 0;
+    uint32_t place = 0;  // in the pool
     char* host = nullptr;
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
 
-    bool make(int dev)
+    // without its memory
+    static Chunk* make(int dev, uint32_t place)
     {
-        device = dev;
-        hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&host), kChunk, hipHostMallocDefault);
-        if (e != hipSuccess) host = nullptr;
-        if (e == hipSuccess && (e = hipStreamCreateWithFlags(&stream, hipStreamNonBlocking)) != hipSuccess) stream = nullptr;
-        if (e == hipSuccess && (e = hipEventCreateWithFlags(&done, hipEventDisableTiming)) != hipSuccess) done = nullptr;
-        if (e != hipSuccess) (void)hipGetLastError();  // (the next launch would report it)
-        return e == hipSuccess;
+        Chunk* c = new (std::nothrow) Chunk;
+        if (!c) return nullptr;
+        c->device = dev;
+        c->place = place;
+        if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) c->stream = nullptr;
+        else if (hipEventCreateWithFlags(&c->done, hipEventDisableTiming) != hipSuccess) c->done = nullptr;
+        if (c->done) return c;
+        (void)hipGetLastError();  // (the next launch would report it)
+        delete c;
+        return nullptr;
+    }
+    bool fill()
+    {
+        if (host) return true;
+        if (hipHostMalloc(reinterpret_cast<void**>(&host), kChunk, hipHostMallocDefault) == hipSuccess) return true;
+        (void)hipGetLastError();
+        host = nullptr;
+        return false;
     }
     ~Chunk()
     {
@@ -51,10 +64,12 @@ struct Chunk {
 };
 
 // Chunks kept between calls, for any thread: kMost in all, 64 MiB. A call takes as many as it wants of those
-// that are free or may still be made, and at least one, which is freed again where there are kMost others; so
-// threads that read at once share the chunks instead of making more. (With blocks of eight chunks, two of them
-// kept, 4, 8 and 16 threads reading 6 MB each took 0.68, 2.1 and 5.0 ms; 0.50, 0.95 and 1.94 with this, the rate
-// of the link.) The pool lives until the process ends (its chunks are not freed after the runtime has shut down).
+// that are free, and at least one, which is freed again where none was; so threads that read at once share the
+// chunks instead of making more. (With blocks of eight chunks, two of them kept, 4, 8 and 16 threads reading
+// 6 MB each took 0.68, 2.1 and 5.0 ms; 0.50, 0.95 and 1.94 with this, the rate of the link.) The streams of
+// eight chunks are made together and the first chunks are taken first, so that a call that is alone has its
+// streams spread over the hardware queues whatever other streams the process has made between two calls. The
+// pool lives until the process ends (its chunks are not freed after the runtime has shut down).
 class Pool {
 public:
     static Pool& get()
@@ -65,54 +80,45 @@ public:
     // up to `want` chunks; how many (0: no memory for one)
     uint32_t take(int device, uint32_t want, Chunk** out)
     {
-        uint32_t n = 0, make = 0;
+        uint32_t n = 0;
         {
             std::lock_guard<std::mutex> lock(mutex_);
-            for (uint32_t k = 0; k < kept_ && n < want;)
-                if (free_[k]->device == device) {
-                    out[n++] = free_[k];
-                    free_[k] = free_[--kept_];
-                } else {
-                    ++k;
-                }
-            make = std::min(want - n, alive_ < kMost ? kMost - alive_ : 0u);
-            if (n + make == 0) make = 1;
-            alive_ += make;
-        }
-        for (; make; --make) {
-            Chunk* c = new (std::nothrow) Chunk;
-            if (!c || !c->make(device)) {
-                delete c;
-                break;
+            for (uint32_t k = 0; k < kMost && n < want; ++k) {
+                if (!at_[k])
+                    for (uint32_t j = k; j < k / kSlots * kSlots + kSlots; ++j)
+                        if (!at_[j]) at_[j] = Chunk::make(device, j);
+                if (!at_[k]) break;
+                if (used_[k] || at_[k]->device != device) continue;
+                used_[k] = true;
+                out[n++] = at_[k];
             }
-            out[n++] = c;
         }
-        if (make) {
-            std::lock_guard<std::mutex> lock(mutex_);
-            alive_ -= make;
+        uint32_t filled = 0;
+        while (filled < n && out[filled]->fill()) ++filled;
+        give(out + filled, n - filled);
+        if (n == 0 && (out[0] = Chunk::make(device, kMost))) {
+            if (out[0]->fill()) return 1;
+            delete out[0];
         }
-        return n;
+        return filled;
     }
     void give(Chunk* const* chunks, uint32_t n)
     {
         for (uint32_t k = 0; k < n; ++k) {
-            {
-                std::lock_guard<std::mutex> lock(mutex_);
-                if (alive_ <= kMost) {
-                    free_[kept_++] = chunks[k];
-                    continue;
-                }
-                --alive_;
+            if (chunks[k]->place == kMost) {
+                delete chunks[k];
+                continue;
             }
-            delete chunks[k];
+            std::lock_guard<std::mutex> lock(mutex_);
+            used_[chunks[k]->place] = false;
         }
     }
 
 private:
     static constexpr uint32_t kMost = 32;
     std::mutex mutex_;
-    Chunk* free_[kMost] = {};
-    uint32_t kept_ = 0, alive_ = 0;  // chunks in free_; with those in use
+    Chunk* at_[kMost] = {};
+    bool used_[kMost] = {};
 };
 
 // The chunks of one call.
