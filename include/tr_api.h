@@ -288,8 +288,14 @@ enum {
     /* camera rays (the first bounce of a single-job render) traced one query per lane like the
      * later bounces, instead of as packets of one pixel's 64 samples per wavefront. Launch tuning
      * and testing; results do not change. */
-    TR_RENDER_NO_CAMERA_PACKETS = 1024u
+    TR_RENDER_NO_CAMERA_PACKETS = 1024u,
+    /* wavefronts of few paths, too, as a launch per bounce over the ray and shadow queues, instead of all
+     * bounces in one launch. Launch tuning and testing; results do not change. */
+    TR_RENDER_QUEUES = 2048u
 };
+/* in the flags: shadow rays traced and deposited every n bounces at the latest (1..255; 0: as many bounces
+ * together as their buffers hold). Launch tuning and testing; results do not change. */
+#define TR_RENDER_SHADOW_GROUP(n) ((uint32_t)(n) << 24)
 
 enum {
     /* wavefronts of few paths run all bounces and their shadow rays in one launch, counted as EXTEND.
@@ -329,7 +335,8 @@ typedef struct tr_batch_s* tr_batch;
 typedef struct {
     uint32_t wave_paths;    /* paths per wavefront (0 = library default) */
     uint32_t flags;         /* TR_RENDER_PROFILE | TR_RENDER_BINARY_BVH | TR_RENDER_ORTHONORMAL_FRAME | TR_RENDER_GRAPH
-                             * | TR_RENDER_STACK32 | TR_RENDER_STACK_KEYED | TR_RENDER_PER_JOB */
+                             * | TR_RENDER_STACK32 | TR_RENDER_STACK_KEYED | TR_RENDER_PER_JOB | TR_RENDER_QUEUES
+                             * | TR_RENDER_SHADOW_GROUP(n) */
     uint32_t trace_per_cu;  /* persistent traversal blocks per compute unit (0 = default 24) */
     uint32_t shade_per_cu;  /* shading blocks per compute unit (0 = default 2) */
 } tr_launch_desc;

@@ -2014,6 +2014,8 @@ struct LaunchCfg {
     bool per_job = false;
     // single-job renders: camera rays traced as per-pixel packets (extend_camera_kernel)
     bool camera_packets = true;
+    bool path_launch = true;  // small wavefronts: all bounces in one launch (path_kernel)
+    uint32_t group = 0;       // bounces whose shadow rays are traced together, at most (0: as the buffers hold)
 };
 
 // launch flags -> stack format
@@ -3661,6 +3663,7 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     }
     // bounces whose shadow rays one launch takes
     uint32_t group = std::max(1u, std::min(uint32_t(std::max(bounces, 1)), kShadowRecords / c.wave));
+    if (c.group) group = std::min(group, c.group);
     const uint32_t unit = guide ? c.wave : mb ? uint32_t(jobs[0].dev.R.n_inc) : 1u;
     wb.fit(c.wave, group, unit);
     bool unwarp = false;
@@ -3688,7 +3691,7 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     L.batch = batch;
     L.bounces = bounces;
     L.group = int(group);
-    L.path_launch = !guide && bounces > 0 && c.wave <= (shallow ? kPathWaveShallow : kPathWave) &&
+    L.path_launch = c.path_launch && !guide && bounces > 0 && c.wave <= (shallow ? kPathWaveShallow : kPathWave) &&
                     group == uint32_t(bounces) && (trav_ext == kTravWide || trav_ext == kTravWide16);
     L.path_per_wave = 64u;
     if (shallow) L.path_per_wave *= std::max({1u, std::min(4u, c.wave >> 19), c.wave >> 20});
@@ -3864,6 +3867,8 @@ int render_impl(tr_scene s, const tr_camera* cam, tr_film f, const tr_render_des
     if (d->flags & (TR_RENDER_STACK32 | TR_RENDER_STACK_KEYED | TR_RENDER_POSTPONE_LEAVES)) c.stack_fmt = stack_fmt_of(d->flags);
     c.mode = guide ? kShadeGuided : ((d->flags & TR_RENDER_ORTHONORMAL_FRAME) ? kShadeOnb : kShadeRef);
     c.camera_packets = (d->flags & TR_RENDER_NO_CAMERA_PACKETS) == 0;
+    c.path_launch = (d->flags & TR_RENDER_QUEUES) == 0;
+    c.group = d->flags >> 24;
     return run_jobs(s->stream, s->wave, jobs, c, guide, s->compute_units, s->ev, &s->ev_made, stats, t_start);
 }
 
@@ -3931,6 +3936,8 @@ LaunchCfg launch_cfg(const tr_batch_s* b, const tr_launch_desc* L)
         c.mode = (L->flags & TR_RENDER_ORTHONORMAL_FRAME) ? kShadeOnb : kShadeRef;
         c.stack_fmt = stack_fmt_of(L->flags);
         c.per_job = (L->flags & TR_RENDER_PER_JOB) != 0;
+        c.path_launch = (L->flags & TR_RENDER_QUEUES) == 0;
+        c.group = L->flags >> 24;
     }
     return c;
 }

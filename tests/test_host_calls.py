@@ -216,3 +216,33 @@ ts = [threading.Thread(target=go, args=(k,)) for k in range(8)]
 [t.join() for t in ts]
 assert not wrong and not fake.fake_freed(), wrong[:3]
 """)
+
+
+@pytest.mark.parametrize("bounces,group", [(1, 1), (5, 1), (5, 2), (7, 3), (7, 6), (7, 7), (9, 0)])
+def test_launches_of_groups_of_bounces(bounces, group):
+    """Closest hits of a bounce carry the shadow queue over (flag 4) unless it begins a group; a group's shadow and
+    film launches follow its last bounce."""
+    out = run(FRAME + f"""
+for flags in (nat.TR_RENDER_QUEUES | nat.TR_RENDER_SHADOW_GROUP({group}), 1024 | nat.TR_RENDER_QUEUES | nat.TR_RENDER_SHADOW_GROUP({group})):
+    s = scenes.icosphere_box(level=0, width=4, height=4, time_bins=4, sqrt_spp=1, n_incoming=1, max_bounces={bounces}, seed=1)
+    w, cam, sampler, film, integ = R.setup_scene(s)
+    e = R.TransientRenderer()
+    e.extra_flags = flags
+    fake.fake_clear()
+    e.render(None, w, integ, cam, film, sampler, seed=1)
+    print("\\n".join(l for l in fake.fake_log().decode().split("\\n") if "extend" in l or "shadow_k" in l or "film_k" in l))
+    print("end")
+""")
+    first, second = out.split("end\n")[:2]
+    for lines, packets in ((first, True), (second, False)):
+        expect = []
+        for b in range(bounces):
+            flags = (b & 1) | (2 if b == 0 else 0) | (4 if b % (group or bounces) else 0)
+            expect.append("extend_camera" if packets and b == 0 else f"extend {flags}")
+            if (b + 1) % (group or bounces) == 0 or b + 1 == bounces:
+                expect += ["shadow", "film"]
+        got = []
+        for line in lines.strip().split("\n"):
+            kind = next(k for k in ("extend_camera", "extend", "shadow", "film") if k in line)
+            got.append(kind + (" " + line.split()[-1] if kind == "extend" else ""))
+        assert got == expect
