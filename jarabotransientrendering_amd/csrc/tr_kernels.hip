@@ -63,14 +63,21 @@ constexpr uint32_t kSmallWave = 1u << 25;
 constexpr uint32_t kLeastWave = 1u << 18;
 // Largest wavefronts whose bounces run in one launch (path_kernel) instead of two per bounce. A render of
 // 2^10 paths through the two: 163 and 84 us (22 triangles), 642 and 266 (81,930 triangles), 370 and 161 (a
-// medium, 16 bounces); of 2^18 paths 200 and 100, 1,074 and 586, 540 and 224; of 2^20 paths 276 and 196,
-// 1,450 and 1,196, 906 and 484; and 719 and 718 with 1,290 triangles, where longer queues win from here on
-// (2^21 paths: 915 and 1,158). Over a tree of a few nodes, where a ray's length hardly varies, the launch
-// still wins with 2^22 paths (618 and 571; medium 2,137 and 1,525) and 2^23 (1,134 and 971; 3,745 and 2,840),
-// but no longer with 2^24 (1,929 and 2,026; 6,485 and 5,494), nor over 90 triangles (2^22: 1,285 and 1,585).
+// medium, 16 bounces); of 2^18 paths 200 and 100, 1,074 and 586, 540 and 224. Where the line lies, in us through
+// the queues and in one launch, without and with a medium (16 bounces):
+//   4-wide nodes (triangles)   2^19              2^20                      2^21                      2^23
+//        4 (22)                                  578, 391   1,090,   665     839,   627  1,545, 1,102  2,277, 2,016  4,525, 3,628
+//       11 (58)                                  666, 461   1,170,   760     942,   752  1,638, 1,245  2,488, 2,423  4,538, 4,028
+//       16 (82)                                  738, 609   1,310,   907   1,040, 1,019  1,807, 1,569  2,746, 3,285  4,954, 5,044
+//       22 (90)                                  771, 686   1,403, 1,018   1,062, 1,127  1,917, 1,723  2,878, 3,752  5,366, 5,835
+//      287 (1,290)                               977, 1,013 1,697, 1,334   1,286, 1,651  2,244, 2,281  3,495, 5,506  5,900, 7,816
+//   18,388 (81,930)       1,381, 1,037         1,825, 1,604 2,812, 2,016   1,983, 2,717  3,269, 3,474
+//   73,614 (327,690)      1,800, 1,762         2,395, 2,861 3,503, 3,346   3,400, 4,689  4,923, 5,752
+// (the last with 32-bit stack entries, whose LDS leaves room for fewer wavefronts).
 constexpr uint32_t kPathWave = 1u << 20;
+constexpr uint32_t kPathWave32 = 1u << 19;       // with 32-bit stack entries
 constexpr uint32_t kPathWaveShallow = 1u << 23;
-constexpr uint32_t kShallowNodes = 5;  // 4-wide nodes of a shallow tree
+constexpr uint32_t kShallowNodes = 11;  // 4-wide nodes of a shallow tree
 constexpr uint32_t kPathSegs = 1u << 15;  // GPU wavefronts of a path launch, at most
 constexpr int kPathRefill = 8;  // idle lanes that begin new paths (24: 2 % slower in a medium)
 constexpr uint32_t kFetchMax = 512;  // rays per work fetch of a traversal wavefront (upper bound)
@@ -1102,14 +1109,14 @@ __global__ void __launch_bounds__(MODE == kShadeGuided ? kShadeBlockGuided : kSh
 // in place of the camera launch, an extend and a shade launch per bounce and the shadow launch. Those take
 // 10-20 us each however few paths there are (a launch, and a ray's chain of node reads), and each waits for
 // the longest ray of the one before it; here a GPU wavefront waits for its own rays only. It loses lanes as
-// paths end, which the queues' compaction avoids, so over shallow trees it begins new paths in them: it takes
-// 256 paths from 2^21 on and 512 of 2^23 (a medium, 2^21 paths: 1,062 us with 64 paths per wavefront, 828
-// with 256; 2^23: 3,971 and, with 512, 2,840; over larger trees 64 are as fast or faster where the launch
-// wins), and large wavefronts keep the queues (kPathWave). Where there are
+// paths end, which the queues' compaction avoids, so it begins new paths in them: it takes 128 paths from 2^20 on,
+// 256 from 2^21 and 512 of 2^23 (22 triangles, 2^21 paths: 796 us with 64 paths per wavefront, 627 with 256, in a
+// medium 1,347 and 1,102; 2^23: 2,920 and, with 512, 2,016, in a medium 4,850 and 3,628; 20,490 triangles,
+// 2^20: 1,417 and, with 128, 1,300), and large wavefronts keep the queues (kPathWave). Where there are
 // fewer than two GPU wavefronts of 64 per SIMD, each takes 32 or 16 paths: fewer lanes wait for the longest
 // ray and for each other's branches (1,290 triangles, 2^14 paths: 267, 227, 207 us with 64, 32, 16;
-// 81,930 triangles 444, 366, 343; a medium 169, 162, 158), but not over 22 triangles without a medium,
-// where all rays are short (2^10 paths: 85, 91, 98; cold caches in more compute units). Its shadow
+// 81,930 triangles 444, 366, 343; a medium 169, 162, 158; 22 triangles, 2^10 paths of 8 bounces: 73.4 and
+// 68.5 with 64 and 16, of 4 bounces 71.3 and 67.4, of 2 57.3 and 58.9). Its shadow
 // records are a segment of its own: appending each bounce's to one queue took 12 ns per atomic, 2.2 ms of a
 // 2^20-path medium render that takes 0.6. Lanes and order aside, every path is computed as by the queue's
 // kernels.
@@ -3631,10 +3638,9 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     uint64_t total = 0;
     int bounces = 0, stack_bound = 0;
     uint32_t max_nodes4 = 0;
-    bool wide = cfg.wide, medium = true, shallow = true;
+    bool wide = cfg.wide, shallow = true;
     for (auto& j : jobs) {
         wide = wide && j.scene->wide;
-        medium = medium && j.scene->has_medium;
         shallow = shallow && j.scene->n_nodes4 <= kShallowNodes;
     }
     for (auto& j : jobs) {
@@ -3691,12 +3697,11 @@ int run_jobs(hipStream_t stream, WaveBuffers& wb, std::vector<HostJob>& jobs, co
     L.batch = batch;
     L.bounces = bounces;
     L.group = int(group);
-    L.path_launch = c.path_launch && !guide && bounces > 0 && c.wave <= (shallow ? kPathWaveShallow : kPathWave) &&
+    const uint32_t path_wave = shallow ? kPathWaveShallow : trav_ext == kTravWide ? kPathWave32 : kPathWave;
+    L.path_launch = c.path_launch && !guide && bounces > 0 && c.wave <= path_wave &&
                     group == uint32_t(bounces) && (trav_ext == kTravWide || trav_ext == kTravWide16);
-    L.path_per_wave = 64u;
-    if (shallow) L.path_per_wave *= std::max({1u, std::min(4u, c.wave >> 19), c.wave >> 20});
-    if (medium || !shallow)
-        while (L.path_per_wave > 16u && c.wave <= L.path_per_wave * 1024u) L.path_per_wave /= 2u;
+    L.path_per_wave = 64u * std::max({1u, std::min(4u, c.wave >> 19), c.wave >> 20});
+    while (L.path_per_wave > 16u && c.wave <= L.path_per_wave * 1024u) L.path_per_wave /= 2u;
     L.stack_bound = stack_bound;
     L.trav_ext = trav_ext;
     L.trav_sh = trav_sh;

@@ -1,6 +1,6 @@
 """Renders through the ray and shadow queues where a small wavefront would take one launch for all its bounces:
 groups of fewer bounces than a render has, stack formats, camera-ray packets, graph replay, batches, and the
-oracle's rows of a full-size film."""
+oracle's rows of a full-size film, and the largest renders of one launch."""
 import numpy as np
 import pytest
 
@@ -130,3 +130,39 @@ def test_full_size_rows_match_the_oracle(R, oracle, flags):
     per_pix = np.abs(part - ref).sum(axis=(2, 3)) / np.maximum(np.abs(ref).sum(axis=(2, 3)), 1e-4)
     assert (per_pix < 1e-4).mean() >= 0.95
     assert abs(part.sum() / ref.sum() - 1) < 5e-3
+
+
+def _cubes(n):
+    """A box shell with n cubes in it: 4-wide trees of 2, 4, 6, 8, 11, 13 and 16 nodes for n from 0 to 6."""
+    rng = np.random.default_rng(n)
+    tris = [scenes.box_shell(inner_box=False)[0]]
+    for _ in range(n):
+        c, size = rng.uniform(0.1, 0.7, 3), rng.uniform(0.08, 0.25, 3)
+        v = np.array([[x, y, z] for x in (0, 1) for y in (0, 1) for z in (0, 1)]) * size + c
+        for a, b, d, e in ((0, 1, 3, 2), (4, 6, 7, 5), (0, 4, 5, 1), (2, 3, 7, 6), (0, 2, 6, 4), (1, 5, 7, 3)):
+            tris.append(np.array([[v[a], v[b], v[d]], [v[a], v[d], v[e]]], np.float32))
+    return np.concatenate(tris).astype(np.float32)
+
+
+@pytest.mark.parametrize("cubes,paths,flags,one_launch", [
+    (4, 1 << 23, 0, True), (4, (1 << 23) + 8, 0, False),      # the largest of a tree of eleven nodes
+    (6, 1 << 20, 0, True), (6, (1 << 20) + 8, 0, False),      # of more
+    (6, 1 << 19, nat.TR_RENDER_STACK32, True), (6, (1 << 19) + 8, nat.TR_RENDER_STACK32, False),  # with 32-bit stacks
+    (1, (1 << 10) + 8, 0, True), (1, (1 << 16) + 8, 0, True)])  # wavefronts of 16 and 64 paths
+def test_the_largest_path_launches(R, cubes, paths, flags, one_launch):
+    w = R.World()
+    w.add_triangles(_cubes(cubes), R.Lambertian((0.7, 0.6, 0.5)))
+    w.add_light(R.PointLightSource((0.5, 0.95, 0.5), (10, 10, 10)))
+    w.freeze()
+    camera = R.PinholeCamera((0.5, 0.5, -1.2), (0.5, 0.5, 0.5), (0.0, 1.0, 0.0), 45.0)
+    out = []
+    for queues in (0, QUEUES):
+        film = R.StreakCameraFilm(8, 1, 50, 0.1)
+        integ = R.BidirectionalPathTracing(w, paths // 8, None, film)
+        integ.set_max_path_size(4)
+        eng = R.TransientRenderer()
+        eng.extra_flags = flags | queues
+        st = eng.render(None, w, integ, camera, film, R.StratifiedSampler(8, 1, 1), seed=2)
+        assert (st["kernel_launches"]["shade"] == 0) == (one_launch and not queues)
+        out.append((st, *film.read_sums()))
+    _same(*out)
