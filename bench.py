@@ -34,6 +34,8 @@ BYTES_SHADOW_PER_RAY = 32 + 1           # shadow ray in, visibility byte out
 BYTES_FILM_PER_RECORD = 1               # visibility byte of every shadow record
 BYTES_FILM_PER_CONTRIB = 20 + 48        # record in (RGB, pixel, bin) + FP32 RGB sum and compensation RMW
 BYTES_SHADE_PER_SEGMENT = 64 + 64 + 20  # path state in + out, NEE record out
+BYTES_CAMERA_PER_RAY = 16               # direction and path index out
+BYTES_PATH_PER_RECORD = 48 + 32 + 1     # path launch: shadow record out, its ray in again, visibility byte out
 BYTES_PATH_PER_SEGMENT = 300            # whole segment: extension + shadow + state + record + film
 
 
@@ -402,11 +404,8 @@ def bench_batch(args) -> dict:
     # one profiled batch pass without graph replay for the per-kernel split
     prof = b.render({**launch, "flags": launch["flags"] & ~8 | 1})
     kern_ms, kern_n = prof["kernel_ms"], prof["kernel_launches"]
-    alg = {"extend": BYTES_EXTEND_PER_RAY * prof["extension_rays"],
-           "shadow": BYTES_SHADOW_PER_RAY * prof["shadow_rays"],
-           "shade": BYTES_SHADE_PER_SEGMENT * prof["extension_rays"],
-           "film": BYTES_FILM_PER_RECORD * prof["shadow_rays"] + BYTES_FILM_PER_CONTRIB * prof["contributions"],
-           "camera": 48 * prof["paths"]}
+    alg = stage_bytes(prof["paths"], prof["extension_rays"], prof["shadow_rays"], prof["contributions"], kern_n)
+    kern_ms, kern_n = stage_names(kern_ms, kern_n), stage_names(kern_n, kern_n)
     dom = max(kern_ms, key=lambda n: kern_ms[n])
     avg_ms = kern_ms[dom] / max(kern_n[dom], 1)
     bpl = alg[dom] / max(kern_n[dom], 1)
@@ -559,6 +558,21 @@ def guide_mlp_bench(n_eval: int = 1 << 22, reps: int = 5, train_sizes=(1 << 14, 
     return res
 
 
+def stage_bytes(paths: int, ext: int, shd: int, con: int, launches: dict) -> dict:
+    """Algorithmic bytes of each stage. Renders of few paths run camera, bounces and shadow rays in one launch,
+    which the library counts as extend: they have the stages path and film only."""
+    film = BYTES_FILM_PER_RECORD * shd + BYTES_FILM_PER_CONTRIB * con
+    if not launches["shade"]:
+        return {"path": BYTES_PATH_PER_RECORD * shd, "film": film}
+    return {"extend": BYTES_EXTEND_PER_RAY * ext, "shadow": BYTES_SHADOW_PER_RAY * shd, "film": film,
+            "shade": BYTES_SHADE_PER_SEGMENT * ext, "camera": BYTES_CAMERA_PER_RAY * paths}
+
+
+def stage_names(values: dict, launches: dict) -> dict:
+    """Per-kernel statistics with a path launch under its own name."""
+    return {"path" if k == "extend" and not launches["shade"] else k: v for k, v in values.items()}
+
+
 def copy_probe(nbytes: int, reps: int = 3) -> None:
     """Device-to-device copies of a known size (the HIP runtime's copy kernel), the calibration
     workload for the FETCH_SIZE / WRITE_SIZE counters."""
@@ -668,13 +682,9 @@ def main():
     ext = sum(s["extension_rays"] for s in steps)
     shd = sum(s["shadow_rays"] for s in steps)
     con = sum(s["contributions"] for s in steps)
-    alg_bytes = {
-        "extend": BYTES_EXTEND_PER_RAY * ext,
-        "shadow": BYTES_SHADOW_PER_RAY * shd,
-        "film": BYTES_FILM_PER_RECORD * shd + BYTES_FILM_PER_CONTRIB * con,
-        "shade": BYTES_SHADE_PER_SEGMENT * ext,
-        "camera": 48 * paths,  # direction, path id + stream state, light stream + pixel + free flight
-    }
+    alg_bytes = stage_bytes(paths, ext, shd, con, kern_n)
+    dom = next(iter(stage_names({dom: 0}, kern_n)))
+    kern_ms = stage_names(kern_ms, kern_n)
     avg_ms = dom_ms / max(dom_n, 1)
     bytes_per_launch = alg_bytes[dom] / max(dom_n, 1)
     achieved = bytes_per_launch / (avg_ms * 1e-3) / 1e9
