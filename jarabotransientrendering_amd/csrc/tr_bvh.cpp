@@ -447,10 +447,11 @@ struct SahCollapse {
     }
 };
 
-// Entries a traversal stack can hold at most: a node step pushes its entered inner children but the
-// one it descends into (or all of them when it also has entered leaves, for any-hit queries), so
-// along any root-to-node path at most sum(inner children - 1, or inner children next to a leaf)
-// entries wait; the largest such sum over the tree.
+// Entries that wait on a traversal stack at most: of a node's entered inner children all but the one that is
+// visited next (or all, while an any-hit query tests the node's leaves), so along any root-to-node path at
+// most sum(inner children - 1, or inner children next to a leaf); the largest such sum over the tree. Any-hit
+// steps push all entered inner children and then pop one: between the two they hold one entry more, so
+// stacks have room for at least this bound + 1.
 int stack_bound(const std::vector<Bvh4NodeHost>& nodes, int32_t n)
 {
     int inner = 0, best = 0;

@@ -68,7 +68,7 @@ static_assert(sizeof(Bvh4NodeHost) == 128, "node layout");
 struct Bvh4 {
     std::vector<Bvh4NodeHost> nodes;  // root = node 0
     int depth = 0;                     // levels of 4-wide nodes
-    int stack_bound = 0;               // entries a traversal stack may hold (3 per level)
+    int stack_bound = 0;               // entries that wait on a traversal stack at most (its capacity is larger)
 };
 
 // Collapses a binary BVH into a 4-wide one. collapse_bvh4 picks the binary nodes that become wide

@@ -511,13 +511,12 @@ template <int TRAV, int STACK>
 __global__ void __launch_bounds__(kTraceBlock, 7) extend_camera_kernel(SceneDev S0, WaveDev Wv, int cur)
 {
     static_assert(TRAV == kTravWide || TRAV == kTravWide16 || TRAV == kTravWideKeyed, "4-wide stacks");
-    constexpr bool carry = false;
     __shared__ uint32_t stack[stack_words<TRAV, STACK>() * kTraceBlock];
     const uint32_t count = Wv.counters[qword(cur)];
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid == 0) {
         Wv.counters[qword(cur ^ 1)] = 0;
-        Wv.counters[shword(cur ^ 1)] = carry ? Wv.counters[shword(cur)] : 0u;
+        Wv.counters[shword(cur ^ 1)] = 0;
         atomicAdd(reinterpret_cast<unsigned long long*>(Wv.counters + C_STAT_EXT), (unsigned long long)count);
     }
     if (gid < kParts) Wv.counters[part_word(gid, P_FETCH_SHADOW)] = 0;
@@ -1873,7 +1872,9 @@ __global__ void __launch_bounds__(kTraceBlock) query_kernel(SceneDev S, RayArray
 
 // The traversal stack holds at most one entry per BVH level; the smallest instantiation that
 // covers the scene's depth keeps LDS per block (and so occupancy) in check.
-// `bound` = entries the traversal stack can hold at most (binary: depth; 4-wide: 3 per level).
+// `bound` = entries that wait on the traversal stack at most (binary: depth; 4-wide: Bvh4::stack_bound). An
+// any-hit step pushes one more before it pops it, so a stack holds at least bound + 1 (tr_scene_commit refuses
+// trees with bound >= kBvhStack).
 // Launches kernel k on `s`; with a start event, through hipExtLaunchKernelGGL, which stamps the
 // start and stop events as part of the dispatch itself instead of as marker packets around it (a
 // marker pair between two launches drains the GPU: 3 % of a media-workload render timed this way).
