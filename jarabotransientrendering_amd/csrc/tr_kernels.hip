@@ -2469,7 +2469,9 @@ int tr_scene_add_mesh_ex(tr_scene s, const float* xyz, uint32_t nv, const uint32
     uint32_t g = s->n_geoms++;
     // material index with the two-sided flag (bit 30) and, per triangle, the smooth flag (bit 29)
     const int32_t mat_bits = mat | ((flags & TR_MATERIAL_TWO_SIDED) ? kMatTwoSided : 0);
-    if (normals && s->tri_vn.empty()) s->tri_vn.assign(s->tri_mat.size() * 9, 0.f);
+    // corner normals: none in the scene, or those of every triangle (zeros for meshes without)
+    const bool any_normals = normals || !s->tri_vn.empty();
+    if (normals) s->tri_vn.resize(s->tri_mat.size() * 9, 0.f);
     for (uint32_t t = 0; t < nt; ++t) {
         for (int k = 0; k < 3; ++k) {
             const float* p = xyz + 3 * size_t(idx[3 * t + k]);
@@ -2481,7 +2483,7 @@ int tr_scene_add_mesh_ex(tr_scene s, const float* xyz, uint32_t nv, const uint32
         s->tri_mat.push_back(smooth ? (mat_bits | kMatSmooth) : mat_bits);
         s->tri_geom.push_back(g);
         s->tri_prim.push_back(t);
-        if (!s->tri_vn.empty()) {
+        if (any_normals) {
             if (normals) s->tri_vn.insert(s->tri_vn.end(), normals + 9 * size_t(t), normals + 9 * size_t(t) + 9);
             else s->tri_vn.insert(s->tri_vn.end(), 9, 0.f);
         }

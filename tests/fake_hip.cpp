@@ -19,6 +19,7 @@ size_t budget = size_t(288) << 30, used = 0;
 bool pinned_fails = false;
 std::map<void*, size_t> pinned;  // and the bytes of all that were ever made
 size_t pinned_live = 0, pinned_made = 0;
+const void* shading_normals = nullptr;  // SceneDev::tri_vn of the last shading launch
 bool freed = false;  // a kernel was given memory that is not allocated
 int event_us = 0;  // a wait for an event takes that long
 long mallocs_left = -1;  // hipMalloc fails from the one after these on (-1: never)
@@ -59,6 +60,7 @@ void fake_mallocs_left(long n) { mallocs_left = n; }
 size_t fake_used() { return used; }
 size_t fake_pinned_live() { return pinned_live; }
 size_t fake_pinned_made() { return pinned_made; }
+const void* fake_shading_normals() { return shading_normals; }
 int fake_freed() { return freed; }
 void fake_event_us(int us) { event_us = us; }
 const char* fake_log() { return log_.c_str(); }
@@ -185,6 +187,8 @@ static hipError_t launched(const void* f, void** args)
         freed = true;
     if (name.find("extend_kernel") != std::string::npos) log_ += " " + std::to_string(*static_cast<int*>(args[3]));
     log_ += "\n";
+    if (name.find("shade_kernel") != std::string::npos || name.find("path_kernel") != std::string::npos)
+        shading_normals = static_cast<const void**>(args[0])[4];
     // the first sample outside the film: none
     if (name.find("samples_begin_kernel") != std::string::npos) **static_cast<uint32_t**>(args[0]) = 0xFFFFFFFFu;
     return hipSuccess;

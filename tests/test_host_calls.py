@@ -246,3 +246,37 @@ for flags in (nat.TR_RENDER_QUEUES | nat.TR_RENDER_SHADOW_GROUP({group}), 1024 |
             kind = next(k for k in ("extend_camera", "extend", "shadow", "film") if k in line)
             got.append(kind + (" " + line.split()[-1] if kind == "extend" else ""))
         assert got == expect
+
+
+@pytest.mark.parametrize("meshes", ["s", "sf", "fs", "sfs", "ss", "fsfs", "f"])
+def test_corner_normals_of_every_mesh_reach_the_device(meshes):
+    """Smooth (s) and flat (f) meshes in any order: a slot's shading frame holds its triangle's corners and normals,
+    zeros for a flat one; a scene of flat meshes alone has none."""
+    run(f"""
+rng = np.random.default_rng(3)
+w, tris, normals = R.World(), [], []
+for kind in {meshes!r}:
+    t = rng.normal(size=(5, 3, 3)).astype(np.float32)
+    n = rng.normal(size=(5, 3, 3)).astype(np.float32) if kind == "s" else None
+    w.add_triangles(t, R.Lambertian((0.5, 0.5, 0.5)), n)
+    tris.append(t)
+    normals.append(np.zeros((5, 3, 3), np.float32) if n is None else n)
+tris, normals = np.concatenate(tris), np.concatenate(normals)
+w.add_light(R.PointLightSource((0, 0, 5), (1, 1, 1)))
+w.freeze()
+film = R.StreakCameraFilm(4, 4, 4, 1.0)
+integ = R.BidirectionalPathTracing(w, 1, None, film)
+R.TransientRenderer().render(None, w, integ, R.PinholeCamera((0, 0, 4), (0, 0, 0), (0, 1, 0)), film, R.StratifiedSampler(4, 4, 1))
+fake.fake_shading_normals.restype = ctypes.c_void_p
+p = fake.fake_shading_normals()
+if "s" not in {meshes!r}:
+    assert not p
+else:
+    assert p
+    v = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), (len(tris), 6, 4))[:, :, :3]
+    for k in range(len(tris)):
+        slot = np.flatnonzero((v[:, 0] == tris[k, 0]).all(axis=1))
+        assert len(slot) == 1
+        assert np.array_equal(v[slot[0], 1:3], tris[k, 1:] - tris[k, 0])
+        assert np.array_equal(v[slot[0], 3:], normals[k]), k
+""")
