@@ -243,9 +243,9 @@ struct __attribute__((packed, aligned(4))) Packed3 {
     float x, y, z;
 };
 
-// The far bound of box tests for a hit at distance t: three ulp further, so that a box whose
-// triangle lies at exactly t is still entered.
-__device__ __forceinline__ float box_far(float t) { return t * 1.00000036f; }
+// The far bound of box tests for a hit at distance t: three ulp further (also behind the origin, where t is
+// negative), so that a box whose triangle lies at exactly t is still entered.
+__device__ __forceinline__ float box_far(float t) { return fmaf(fabsf(t), 0x1.8p-22f, t); }
 
 // Tests the triangle record at byte offset `off` of `tris` (its slot is `slot`) against the current
 // hit: updates hit (a slot) and tfar; equal-distance ties go to the lower scene triangle index, which
@@ -285,7 +285,7 @@ __device__ __forceinline__ void tri_hit(const RayPre& r, const char* __restrict_
     const float T = U * (r.Sz * Akz) + V * (r.Sz * Bkz) + W * (r.Sz * Ckz);
     // divide only when an estimate of the distance is near (tnear, tfar]
     const float te = T * __builtin_amdgcn_rcpf(det);
-    if (!((te >= tnear * 0.99999f) & (te <= tfar * 1.00001f))) return;
+    if (!((te >= fmaf(fabsf(tnear), -1e-5f, tnear)) & (te <= fmaf(fabsf(tfar), 1e-5f, tfar)))) return;
     const float th = T / det;
     if (!((th > tnear) & (th <= tfar))) return;
     if (th == tfar && hit >= 0) {
@@ -322,11 +322,11 @@ __device__ __forceinline__ int32_t trace(const float4* __restrict__ nodes, const
         float ry0 = (b.z - r.o.y) * r.inv.y, ry1 = (b.w - r.o.y) * r.inv.y;
         float rz0 = (c.z - r.o.z) * r.inv.z, rz1 = (c.w - r.o.z) * r.inv.z;
         float tl0 = fmaxf(fmaxf(fminf(lx0, lx1), fminf(ly0, ly1)), fmaxf(fminf(lz0, lz1), tnear));
-        float tl1 = fminf(fminf(fmaxf(lx0, lx1), fmaxf(ly0, ly1)), fminf(fmaxf(lz0, lz1), tfar)) * 1.00000036f;
+        float tl1 = fminf(fminf(fmaxf(lx0, lx1), fmaxf(ly0, ly1)), fminf(fmaxf(lz0, lz1), tfar));
         float tr0 = fmaxf(fmaxf(fminf(rx0, rx1), fminf(ry0, ry1)), fmaxf(fminf(rz0, rz1), tnear));
-        float tr1 = fminf(fminf(fmaxf(rx0, rx1), fmaxf(ry0, ry1)), fminf(fmaxf(rz0, rz1), tfar)) * 1.00000036f;
-        bool hl = (tl0 <= tl1) && dd.z >= 0;
-        bool hr = (tr0 <= tr1) && dd.w >= 0;
+        float tr1 = fminf(fminf(fmaxf(rx0, rx1), fmaxf(ry0, ry1)), fminf(fmaxf(rz0, rz1), tfar));
+        bool hl = (tl0 <= box_far(tl1)) && dd.z >= 0;
+        bool hr = (tr0 <= box_far(tr1)) && dd.w >= 0;
         // leaf children: test their triangles now
 #pragma unroll
         for (int side = 0; side < 2; ++side) {
