@@ -1,10 +1,8 @@
 """The library's host code over a HIP runtime that launches nothing (fake_hip.cpp): what a call does when memory
 runs out, and which kernels it launches. Each program runs in a process of its own."""
-import functools
 import os
 import subprocess
 import sys
-import tempfile
 
 import pytest
 
@@ -26,25 +24,23 @@ from jarabotransientrendering_amd import _native as nat, renderer as R, scenes
 """
 
 
-@functools.lru_cache(maxsize=None)
-def _fake():
-    d = tempfile.mkdtemp()
-    so = os.path.join(d, "libamdhip64.so.7")
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = os.path.join(tmp_path_factory.mktemp("hip"), "libamdhip64.so.7")
     subprocess.check_call(["g++", "-std=c++17", "-O1", "-w", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__",
                            "-I/opt/rocm/include", "-Wl,-soname,libamdhip64.so.7",
                            os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", so])
-    return so
 
-
-def run(program):
-    r = subprocess.run([sys.executable, "-c", HEAD.format(root=ROOT, fake=_fake()) + program], capture_output=True,
-                       text=True, timeout=120)
-    assert r.returncode == 0, r.stdout + r.stderr
-    return r.stdout
+    def program(text):
+        r = subprocess.run([sys.executable, "-c", HEAD.format(root=ROOT, fake=so) + text], capture_output=True, text=True,
+                           timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+        return r.stdout
+    return program
 
 
 @pytest.mark.parametrize("n", [1000, 20000])
-def test_samples_need_no_pinned_memory(n):
+def test_samples_need_no_pinned_memory(run, n):
     """Once a call has added its radiance nothing is left that can run out of memory: the weights are in too."""
     run(f"""
 film = R.StreakCameraFilm(13, 7, 20, 0.1)
@@ -61,7 +57,7 @@ assert np.array_equal(weights.ravel(), np.bincount(a["y"] * 13 + a["x"], minleng
 
 @pytest.mark.parametrize("n", [100, 16384, 16385, 131072])
 @pytest.mark.parametrize("width,height", [(13, 7), (300, 100)])
-def test_sample_weights_are_summed_in_order(n, width, height):
+def test_sample_weights_are_summed_in_order(run, n, width, height):
     """Weights of any magnitudes: each call's are summed in the order of the samples and then added to the
     film's, in double, so that the same calls give the same bits."""
     run(f"""
@@ -100,7 +96,7 @@ assert np.array_equal(got.ravel(), expect + np.bincount(pix, minlength={width * 
 
 
 @pytest.mark.parametrize("threads", [8, 40])
-def test_concurrent_reads_share_the_pinned_chunks(threads):
+def test_concurrent_reads_share_the_pinned_chunks(run, threads):
     """Films of 6 MB read by several threads at once, again and again: at most 32 chunks of 2 MiB are kept, and
     no more are made than those and one for each thread that finds none."""
     run(f"""
@@ -121,7 +117,7 @@ if {threads} <= 32:
 """)
 
 
-def test_a_read_without_pinned_memory_says_so():
+def test_a_read_without_pinned_memory_says_so(run):
     run("""
 film = R.StreakCameraFilm(4, 4, 8, 0.1)
 film.handle
@@ -146,7 +142,7 @@ def frame(size, spp, bounces, layers=0, unwarp=False, n_inc=1):
 """
 
 
-def test_a_process_may_hold_many_rendered_scenes():
+def test_a_process_may_hold_many_rendered_scenes(run):
     """Frames of 67 M paths in as many scenes, all kept: a few take the large shape (25 GB), the others stay at
     6.7 GB while there is memory, and then idle ones give theirs back."""
     run(FRAME + """
@@ -162,7 +158,7 @@ assert not fake.fake_freed()
 
 
 @pytest.mark.parametrize("budget", [1, 3, 5, 9, 20, 40])
-def test_renders_shrink_to_the_memory_there_is(budget):
+def test_renders_shrink_to_the_memory_there_is(run, budget):
     """Whatever is left by the time buffers are made: fewer bounces per group, then fewer paths per wavefront, and
     no error left behind for the next launch to report."""
     run(FRAME + f"""
@@ -174,7 +170,7 @@ assert not fake.fake_freed()
 """)
 
 
-def test_an_allocation_that_fails_leaves_a_scene_that_renders():
+def test_an_allocation_that_fails_leaves_a_scene_that_renders(run):
     """hipMalloc failing at any point of a first, a larger and a multibounce render."""
     run(FRAME + """
 for kind in (dict(size=16, spp=2, bounces=5), dict(size=16, spp=2, bounces=5, layers=2, unwarp=True)):
@@ -195,7 +191,7 @@ for kind in (dict(size=16, spp=2, bounces=5), dict(size=16, spp=2, bounces=5, la
 """)
 
 
-def test_idle_buffers_are_given_back_while_others_render():
+def test_idle_buffers_are_given_back_while_others_render(run):
     """Threads that render in turn in more scenes than memory holds: no render loses its buffers."""
     run(FRAME + """
 import threading
@@ -219,7 +215,7 @@ assert not wrong and not fake.fake_freed(), wrong[:3]
 
 
 @pytest.mark.parametrize("bounces,group", [(1, 1), (5, 1), (5, 2), (7, 3), (7, 6), (7, 7), (9, 0)])
-def test_launches_of_groups_of_bounces(bounces, group):
+def test_launches_of_groups_of_bounces(run, bounces, group):
     """Closest hits of a bounce carry the shadow queue over (flag 4) unless it begins a group; a group's shadow and
     film launches follow its last bounce."""
     out = run(FRAME + f"""
@@ -249,7 +245,7 @@ for flags in (nat.TR_RENDER_QUEUES | nat.TR_RENDER_SHADOW_GROUP({group}), 1024 |
 
 
 @pytest.mark.parametrize("meshes", ["s", "sf", "fs", "sfs", "ss", "fsfs", "f"])
-def test_corner_normals_of_every_mesh_reach_the_device(meshes):
+def test_corner_normals_of_every_mesh_reach_the_device(run, meshes):
     """Smooth (s) and flat (f) meshes in any order: a slot's shading frame holds its triangle's corners and normals,
     zeros for a flat one; a scene of flat meshes alone has none."""
     run(f"""
